@@ -454,6 +454,11 @@ bool gemm_i8_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K,
 size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, size_t N, size_t K, size_t M, int weights);
 int launch_gemm_i8(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                    size_t M, int out_dtype, void *scratch);
+// Tiled GEMM of K-quant weights and Q8_K activations on the fp16 matrix cores with integer operands (mh_gemm_int16.hip)
+bool gemm_x16_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights,
+                      const ActScratch &act);
+int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
+                    size_t M, int out_dtype);
 // Tiled int8 GEMM on Q8_0 activations (mh_gemm_i8.hip): Q8_0 and Q4_0 weights, K a multiple of 256, nine rows and more;
 // `scratch` holds gemm_i8_scratch_bytes for the K-split partial sums
 bool gemm_q23k_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,

@@ -1069,6 +1069,9 @@ int launch_mmq_set(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
         return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "small-batch MFMA matmul: unsupported kind or shape");
     }
     if (gemm_i8_applies(dev, kind, N, K, ws.w, ws.count, act)) {
+        if (gemm_x16_applies(dev, kind, N, K, M, ws.count, act)) {
+            return launch_gemm_x16(dev, kind, ws, act, N, K, M, out_dtype);
+        }
         return launch_gemm_i8(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }
     const size_t nb = K / QK_K;
