@@ -277,6 +277,10 @@ struct marmot_hip_device {
     // the polls a wavefront may spend (MARMOT_HIP_SPIN_LIMIT, read at creation)
     uint32_t *fault_word = nullptr;
     uint32_t spin_limit = 1u << 26;
+    // Pinned host word in which the MoE route kernel leaves the result of the expert-id check, and the event behind that
+    // kernel (mh_moe.hip; made by the first checked call)
+    int *host_word = nullptr;
+    hipEvent_t host_word_event = nullptr;
     // Timeline build only (-DMH_TIMELINE): device buffer of the caller that instrumented kernels write their marks to
     // (marmot_hip_timeline_attach); nullptr = marks off.
     unsigned long long *timeline = nullptr;
@@ -459,6 +463,12 @@ bool gemm_x16_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K
                       const ActScratch &act);
 int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                     size_t M, int out_dtype);
+// grouped (MoE): work items of up to 64 routes
+bool gemm_x16_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
+                                const void *w1);
+int launch_gemm_x16_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
+                            const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
+                            size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1);
 // Tiled int8 GEMM on Q8_0 activations (mh_gemm_i8.hip): Q8_0 and Q4_0 weights, K a multiple of 256, nine rows and more;
 // `scratch` holds gemm_i8_scratch_bytes for the K-split partial sums
 bool gemm_q23k_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,

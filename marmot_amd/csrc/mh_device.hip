@@ -281,6 +281,12 @@ void marmot_hip_device_destroy(marmot_hip_device_t *dev) {
     if (dev->fault_word != nullptr) {
         (void)hipFree(dev->fault_word);
     }
+    if (dev->host_word_event != nullptr) {
+        (void)hipEventDestroy(dev->host_word_event);
+    }
+    if (dev->host_word != nullptr) {
+        (void)hipHostFree(dev->host_word);
+    }
     branches_destroy(dev);
     (void)hipStreamDestroy(dev->main_stream);
     delete dev;

@@ -772,4 +772,46 @@ int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const
     return MARMOT_HIP_SUCCESS;
 }
 
+// ------------------------------------------------------------------ grouped (MoE)
+bool gemm_x16_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
+                                const void *w1) {
+    const size_t align = kind == MARMOT_HIP_KIND_Q6_K ? 1 : 15;  // (Q6_K rows are loaded from the boundary below)
+    return !dev->knobs.no_gemm_i8 && x16_kind(kind) && K % QK_K == 0 && rows * K < ((size_t)1 << 32) &&
+           32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
+           ((((uintptr_t)w0) | ((uintptr_t)w1)) & align) == 0;
+}
+
+int launch_gemm_x16_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
+                            const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
+                            size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1) {
+    if (max_items > 65535) {
+        return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "grouped tiled GEMM: %zu work items exceed the grid limit",
+                         max_items);
+    }
+    GemmX16Params p = {};
+    p.w[0] = (const uint8_t *)d_w0;
+    p.w[1] = (const uint8_t *)d_w1;
+    p.out[0] = d_out0;
+    p.out[1] = d_out1;
+    p.qs = act.qs;
+    p.ad = act.d;
+    p.sums = act.sums;
+    p.kp = act.kp;
+    p.M = M;
+    p.nb = K / QK_K;
+    p.items = d_items;
+    p.n_items = d_n_items;
+    p.act_index = d_act_index;
+    p.expert_stride = expert_stride;
+    const unsigned weights = d_w1 != nullptr ? 2 : 1;
+    switch (kind) {
+    case MARMOT_HIP_KIND_Q4_K:
+        return x16_launch<MARMOT_HIP_KIND_Q4_K, 2, 4>(dev, p, (unsigned)max_items, weights);
+    case MARMOT_HIP_KIND_Q5_K:
+        return x16_launch<MARMOT_HIP_KIND_Q5_K, 2, 4>(dev, p, (unsigned)max_items, weights);
+    default:
+        return x16_launch<MARMOT_HIP_KIND_Q6_K, 2, 4>(dev, p, (unsigned)max_items, weights);
+    }
+}
+
 } // namespace mh

@@ -10,6 +10,10 @@
 namespace mh {
 
 constexpr int MOE_ITEM_COLS = 8;   // routes per grouped work item (16 or 32 when experts see many routes, see moe_item_cols)
+// Routes per expert from which prompts take the tiled GEMM (mh_gemm_int16.hip, 64 routes per item) instead of passes of
+// 16 or 32 routes, given two of its tiles per compute unit in both projections (us before / tiled, E = 128, top 8, H = 2048,
+// F = 768: Q4_K 512 tokens = 32 routes per expert 248 / 182, 1024 401 / 260, 2048 729 / 429; Q6_K 512 472 / 285)
+constexpr size_t MOE_TILED_ROUTES = 32;
 constexpr int MOE_MAX_EXPERTS = 1024;
 constexpr int MOE_MAX_TOPK = 64;
 
@@ -102,16 +106,20 @@ struct RouteArgs {
     int *route_pos;               // [T, k] position of each (token, slot) in the sorted order
     int4 *items;                  // work items
     int *n_items;
-    int *error_flag;              // set to 1 when an expert id is out of range
+    int *error_flag;              // 1 when an expert id is out of range, else 0: device memory, or pinned host memory
     int T, k, E;
     float weights_scale;
     int renormalize;
     int decode_order;
-    int item_cols;                // routes per work item: 8, 16 or 32
+    int item_cols;                // routes per work item: 8, 16, 32 or 64
+    int id_bits;                  // bits of an expert id
 };
 
 constexpr int MOE_ROUTE_LDS = 4096;    // routes whose ids and positions are kept in LDS
-constexpr int MOE_ROUTE_WAVES = 8;     // wavefronts of the route kernel; each fills one contiguous chunk of routes
+// (16384 routes of 128 experts: 120 -> 22 us with eight loads in flight, ranks by ballots instead of 64 lane reads and the
+// records in a launch of their own, 4.5 us; 512 routes 9.6 -> 5.1 us)
+constexpr int MOE_ROUTE_WAVES = 16;    // wavefronts of the route kernel; each fills one contiguous chunk of routes
+constexpr int MOE_EMIT_ROUTES = 2048;  // from more routes than this on their records are written by a launch of its own
 
 // exclusive prefix sum over the 64 lanes of a wavefront; *total receives the sum over all lanes
 __device__ __forceinline__ int wave_excl_scan(int v, int lane, int *total) {
@@ -127,18 +135,18 @@ __device__ __forceinline__ int wave_excl_scan(int v, int lane, int *total) {
     return incl - v;
 }
 
-// rank = number of lower lanes holding the same id, cnt = number of lanes holding it
-__device__ __forceinline__ void wave_rank(int id, int lane, int *rank, int *cnt) {
-    int rk = 0, c = 0;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) {
-        const int idj = __builtin_amdgcn_readlane(id, j);
-        const bool same = idj == id;
-        c += same ? 1 : 0;
-        rk += (same && j < lane) ? 1 : 0;
+// rank = number of lower lanes holding the same id, cnt = number of lanes holding it. One ballot per bit of the ids (`bits`
+// of them; id -1 counts as an id of its own through its sign bit).
+__device__ __forceinline__ void wave_rank(int id, int lane, int bits, int *rank, int *cnt) {
+    unsigned long long same = __ballot(id < 0);
+    same = id < 0 ? same : ~same;
+    for (int i = 0; i < bits; ++i) {
+        const bool set = (id >> i) & 1;
+        const unsigned long long with = __ballot(set);
+        same &= set ? with : ~with;
     }
-    *rank = rk;
-    *cnt = c;
+    *rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+    *cnt = __builtin_popcountll(same);
 }
 
 __device__ __forceinline__ void route_emit(const RouteArgs &a, int r, int pos) {
@@ -163,6 +171,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
     warm_kernel_arguments<sizeof(RouteArgs), sizeof(RouteArgs)>();
     __shared__ int counts[MOE_MAX_EXPERTS];
     __shared__ int wcount[MOE_ROUTE_WAVES][MOE_MAX_EXPERTS];  // per chunk: routes of each expert, then its cursor
+    __shared__ int bad_id;
     __shared__ int ids_l[MOE_ROUTE_LDS];  // expert id of each route (-1 = invalid), later its sorted position
     const int routes = a.T * a.k;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -183,7 +192,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         }
         const unsigned long long bad = __ballot(lane < routes && id < 0);
         int rank, cnt;
-        wave_rank(id, lane, &rank, &cnt);
+        wave_rank(id, lane, a.id_bits, &rank, &cnt);
         const bool first = id >= 0 && rank == 0;
         int total, n_items;
         const int seg = wave_excl_scan(first ? cnt : 0, lane, &total);
@@ -214,23 +223,35 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         }
     }
     if (tid == 0) {
-        *a.error_flag = 0;
+        bad_id = 0;
     }
     __syncthreads();
     // chunk of wavefront w: routes [w * chunk, (w + 1) * chunk), a multiple of 64
     const int chunk = ((routes + MOE_ROUTE_WAVES * 64 - 1) / (MOE_ROUTE_WAVES * 64)) * 64;
     const int r_begin = wave * chunk;
     const int r_end = r_begin + chunk < routes ? r_begin + chunk : routes;
-    for (int r = r_begin + lane; r < r_end; r += 64) {
-        int id = a.topk_ids[r];
-        if (id < 0 || id >= a.E) {
-            *a.error_flag = 1;
-            id = -1;
-        } else {
-            atomicAdd(&wcount[wave][id], 1);
+    constexpr int BATCH = 8;  // loads in flight per lane: with one, a prompt's counting loop is a chain of memory latencies
+    for (int base = r_begin; base < r_end; base += 64 * BATCH) {
+        int id[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int r = base + 64 * i + lane;
+            id[i] = a.topk_ids[r < r_end ? r : r_end - 1];
         }
-        if (in_lds) {
-            ids_l[r] = id;
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int r = base + 64 * i + lane;
+            if (r < r_end) {
+                if (id[i] < 0 || id[i] >= a.E) {
+                    bad_id = 1;
+                    id[i] = -1;
+                } else {
+                    atomicAdd(&wcount[wave][id[i]], 1);
+                }
+                if (in_lds) {
+                    ids_l[r] = id[i];
+                }
+            }
         }
     }
     __syncthreads();
@@ -268,6 +289,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         }
         if (lane == 0) {
             *a.n_items = n_items;
+            *a.error_flag = bad_id;
         }
     }
     __syncthreads();
@@ -285,21 +307,20 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
     // Stable fill, every wavefront over its own chunk, 64 routes per round in route order: a route's position is its
     // expert's cursor plus the number of earlier lanes of the round with the same expert.
     int *cursor = wcount[wave];
+    auto id_of = [&](int r) {
+        if (in_lds) {
+            return ids_l[r];
+        }
+        const int id = a.topk_ids[r];
+        return id < 0 || id >= a.E ? -1 : id;
+    };
+    int next = r_begin + lane < r_end ? id_of(r_begin + lane) : -1;
     for (int base = r_begin; base < r_end; base += 64) {
         const int r = base + lane;
-        int id = -1;
-        if (r < r_end) {
-            if (in_lds) {
-                id = ids_l[r];
-            } else {
-                id = a.topk_ids[r];
-                if (id < 0 || id >= a.E) {
-                    id = -1;
-                }
-            }
-        }
+        const int id = next;
+        next = r + 64 < r_end ? id_of(r + 64) : -1;
         int rank, cnt;
-        wave_rank(id, lane, &rank, &cnt);
+        wave_rank(id, lane, a.id_bits, &rank, &cnt);
         int pos = -1;
         if (id >= 0) {
             pos = cursor[id] + rank;
@@ -309,57 +330,94 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
             cursor[id] += cnt;
         }
         if (r < r_end) {
-            route_emit(a, r, pos);
+            if (routes > MOE_EMIT_ROUTES) {
+                a.route_pos[r] = pos;  // k_moe_emit writes the rest
+            } else {
+                route_emit(a, r, pos);
+            }
         }
+    }
+}
+
+// The route records of a prompt, after k_moe_route has placed the routes
+__global__ __launch_bounds__(256) void k_moe_emit(const RouteArgs a) {
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r < a.T * a.k) {
+        route_emit(a, r, a.route_pos[r]);
     }
 }
 
 // ------------------------------------------------------------------ weighted combine
 // out[t, :] = sum over the token's routes, in ascending sorted position (moe_ops.c:1034-1042), of
 // weight * down_row; tokens without a valid route get zeros (moe_ops.c:944-947, 984-986).
+// One workgroup per token and 1024 columns (4 per thread, VEC: as one 16-byte access); the rows of COMBINE_BATCH routes are
+// requested before the first is added (2048 tokens, top 8, 2048 columns: 45 -> 24 us, one column per
+// thread and one row at a time before; reading the 134 MB of route rows takes 22).
+constexpr int COMBINE_BATCH = 8;
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_moe_combine(const float *__restrict__ route_down,
                                                      const float *__restrict__ sorted_weights,
                                                      const int *__restrict__ route_pos, int k, size_t H,
                                                      float *__restrict__ out) {
-    __shared__ int pos[MOE_MAX_TOPK];
+    __shared__ int raw[MOE_MAX_TOPK], pos[MOE_MAX_TOPK];
     __shared__ float wts[MOE_MAX_TOPK];
-    __shared__ int npos;
-    __shared__ int raw[MOE_MAX_TOPK];
     const size_t t = blockIdx.x;
-    if ((int)threadIdx.x < k) {
-        raw[threadIdx.x] = route_pos[t * k + threadIdx.x];
+    const int s = threadIdx.x;
+    const int p = s < k ? route_pos[t * k + s] : -1;
+    if (s < k) {
+        raw[s] = p;
+    }
+    const float w = p >= 0 ? sorted_weights[p] : 0.0f;
+    __syncthreads();
+    int n = 0, rank = 0;
+    for (int i = 0; i < k; ++i) {
+        n += raw[i] >= 0 ? 1 : 0;
+        rank += raw[i] >= 0 && raw[i] < p ? 1 : 0;  // (the positions of a token's routes are distinct)
+    }
+    if (p >= 0) {
+        pos[rank] = p;
+        wts[rank] = w;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int n = 0;
-        for (int s = 0; s < k; ++s) {
-            const int p = raw[s];
-            if (p < 0) {
-                continue;
+    const size_t h = (size_t)blockIdx.y * 1024 + 4 * (size_t)threadIdx.x;
+    if (h >= H) {
+        return;
+    }
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int cols = H - h < 4 ? (int)(H - h) : 4;
+    for (int j0 = 0; j0 < n; j0 += COMBINE_BATCH) {
+        float row[COMBINE_BATCH][4];
+#pragma unroll
+        for (int j = 0; j < COMBINE_BATCH; ++j) {
+            const float *src = route_down + (size_t)pos[j0 + j < n ? j0 + j : n - 1] * H + h;
+            if constexpr (VEC) {
+                const float4 v = *(const float4 *)src;
+                row[j][0] = v.x, row[j][1] = v.y, row[j][2] = v.z, row[j][3] = v.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    row[j][e] = src[e < cols ? e : 0];
+                }
             }
-            int j = n++;
-            while (j > 0 && pos[j - 1] > p) {
-                pos[j] = pos[j - 1];
-                --j;
+        }
+#pragma unroll
+        for (int j = 0; j < COMBINE_BATCH; ++j) {
+            if (j0 + j < n) {
+                const float wj = wts[j0 + j];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc[e] += wj * row[j][e];
+                }
             }
-            pos[j] = p;
         }
-        npos = n;
     }
-    __syncthreads();
-    if ((int)threadIdx.x < npos) {
-        wts[threadIdx.x] = sorted_weights[pos[threadIdx.x]];
-    }
-    __syncthreads();
-    const int n = npos;
-    // blockIdx.y selects a slab of 256 columns
-    const size_t h = (size_t)blockIdx.y * blockDim.x + threadIdx.x;
-    if (h < H) {
-        float acc = 0.0f;
-        for (int j = 0; j < n; ++j) {
-            acc += wts[j] * route_down[(size_t)pos[j] * H + h];
+    float *dst = out + t * H + h;
+    if constexpr (VEC) {
+        *(float4 *)dst = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    } else {
+        for (int e = 0; e < cols; ++e) {
+            dst[e] = acc[e];
         }
-        out[t * H + h] = acc;
     }
 }
 
@@ -411,6 +469,18 @@ int marmot_hip_softmax_rows(marmot_hip_device_t *dev, const float *d_x, size_t r
 
 } // extern "C"
 
+// The pinned word and the event of the expert-id check, made by the device object's first checked call
+static int host_word_init(marmot_hip_device *dev) {
+    if (dev->host_word_event != nullptr) {
+        return MARMOT_HIP_SUCCESS;
+    }
+    if (dev->host_word == nullptr) {
+        MH_HIP(hipHostMalloc((void **)&dev->host_word, 64, hipHostMallocDefault));
+    }
+    MH_HIP(hipEventCreateWithFlags(&dev->host_word_event, hipEventDisableTiming));
+    return MARMOT_HIP_SUCCESS;
+}
+
 // One body for marmot_hip_moe_experts and its stage-probing variant. `probe` (may be null) names device buffers that
 // receive the intermediate arrays, and optionally the packed activations the down projection reads instead of the
 // ones this call quantized.
@@ -455,6 +525,15 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     size_t item_cols = MOE_ITEM_COLS;
     if (mmq_gu && mmq_dn && routes >= 12 * E) {
         item_cols = (routes >= 24 * E && q45(kind_gate_up) && q45(kind_down)) ? 32 : 16;
+    }
+    // Prompts with many routes per expert: the tiled GEMM on integer fp16 operands, 64 routes per item
+    const size_t tiled_items = routes / 64 + E / 2, two_per_cu = 2 * (size_t)dev->props.multiProcessorCount;
+    const bool tiled = routes >= MOE_TILED_ROUTES * E && tiled_items * 2 * ((F + 127) / 128) >= two_per_cu &&
+                       tiled_items * ((H + 127) / 128) >= two_per_cu &&
+                       gemm_x16_grouped_supported(dev, kind_gate_up, T, H, F, d_gate, d_up) &&
+                       gemm_x16_grouped_supported(dev, kind_down, routes, F, H, d_down, d_down);
+    if (tiled) {
+        item_cols = 64;
     }
     const size_t max_items = routes < E + routes / item_cols ? routes : E + routes / item_cols;
     const int act_gu = is_k_quant(kind_gate_up) ? MARMOT_HIP_KIND_Q8_K : MARMOT_HIP_KIND_Q8_0;
@@ -503,7 +582,14 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     ra.route_pos = route_pos;
     ra.items = items;
     ra.n_items = flags;
-    ra.error_flag = flags + 1;
+    // Expert ids are validated on the device. The route kernel leaves the answer in pinned host memory and the call waits
+    // for that kernel only, not for the experts; skipped while the stream is being captured into a graph or when the
+    // device object was created with MARMOT_HIP_MOE_NO_VALIDATE set.
+    const bool validate = !dev->capturing && !dev->knobs.moe_no_validate;
+    if (validate) {
+        MH_TRY(host_word_init(dev));
+    }
+    ra.error_flag = validate ? dev->host_word : flags + 1;
     ra.T = (int)T;
     ra.k = (int)k_per_token;
     ra.E = (int)E;
@@ -512,8 +598,19 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     // cpu_moe_should_use_decode_path (moe_ops.c:417-424)
     ra.decode_order = (T <= 4 && routes <= 64) ? 1 : 0;
     ra.item_cols = (int)item_cols;
+    ra.id_bits = 1;
+    while (((size_t)1 << ra.id_bits) < E) {
+        ++ra.id_bits;
+    }
     hipLaunchKernelGGL(k_moe_route, dim3(1), dim3(MOE_ROUTE_WAVES * 64), 0, dev->stream, ra);
     MH_HIP(hipGetLastError());
+    if (validate) {
+        MH_HIP(hipEventRecord(dev->host_word_event, dev->stream));
+    }
+    if (routes > (size_t)MOE_EMIT_ROUTES) {
+        hipLaunchKernelGGL(k_moe_emit, dim3((unsigned)((routes + 255) / 256)), dim3(256), 0, dev->stream, ra);
+        MH_HIP(hipGetLastError());
+    }
 
     // hidden states are quantized once per token; routes refer to them through sorted_tokens
     st = launch_quantize_act_soa(dev, act_gu, d_hidden, MARMOT_HIP_DTYPE_F32, T, H, hidden_q);
@@ -523,7 +620,9 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const size_t gu_stride = F * ((H + bv_gu - 1) / bv_gu) * block_bytes(kind_gate_up);
     const size_t dn_stride = H * ((F + bv_dn - 1) / bv_dn) * block_bytes(kind_down);
     // Q4_K / Q6_K experts run on the int8 matrix cores, the 32-value formats on the dot-product matvec
-    st = mmq_gu ? launch_mmq_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
+    st = tiled  ? launch_gemm_x16_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
+                                          max_items, H, F, gate_out, up_out)
+        : mmq_gu ? launch_mmq_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
                                      max_items, H, F, gate_out, up_out, (int)item_cols)
                 : launch_matvec_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
                                         max_items, H, F, gate_out, up_out);
@@ -557,26 +656,29 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
                                   dev->stream));
         }
     }
-    st = mmq_dn ? launch_mmq_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags, max_items,
+    st = tiled  ? launch_gemm_x16_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags,
+                                          max_items, F, H, route_down, nullptr)
+        : mmq_dn ? launch_mmq_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags, max_items,
                                      F, H, route_down, nullptr, (int)item_cols)
                 : launch_matvec_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags,
                                         max_items, F, H, route_down, nullptr);
     if (st != MARMOT_HIP_SUCCESS) {
         return st;
     }
-    hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)T, (unsigned)((H + 255) / 256)), dim3(256), 0, dev->stream,
-                       route_down, sorted_weights, route_pos, (int)k_per_token, H, d_out);
+    const dim3 combine_grid((unsigned)T, (unsigned)((H + 1023) / 1024));
+    if (H % 4 == 0 && (((uintptr_t)d_out) & 15) == 0) {
+        hipLaunchKernelGGL(k_moe_combine<true>, combine_grid, dim3(256), 0, dev->stream, route_down, sorted_weights,
+                           route_pos, (int)k_per_token, H, d_out);
+    } else {
+        hipLaunchKernelGGL(k_moe_combine<false>, combine_grid, dim3(256), 0, dev->stream, route_down, sorted_weights,
+                           route_pos, (int)k_per_token, H, d_out);
+    }
     MH_HIP(hipGetLastError());
     set_route("moe_experts_grouped");
 
-    // Expert ids are validated on the device; reading the flag needs a stream synchronization, which is skipped
-    // while the stream is being captured into a graph or when the device object was created with
-    // MARMOT_HIP_MOE_NO_VALIDATE set.
-    if (!dev->capturing && !dev->knobs.moe_no_validate) {
-        int host_flag = 0;
-        MH_HIP(hipMemcpyAsync(&host_flag, flags + 1, sizeof(int), hipMemcpyDeviceToHost, dev->stream));
-        MH_HIP(hipStreamSynchronize(dev->stream));
-        if (host_flag != 0) {
+    if (validate) {
+        MH_HIP(hipEventSynchronize(dev->host_word_event));
+        if (*(volatile int *)dev->host_word != 0) {
             return set_error(MARMOT_HIP_ERROR_INVALID_ARGUMENT, "MoE expert id is out of range");
         }
     }

@@ -3,6 +3,7 @@ at the edges of its two tile forms and of the rule that chooses one (x16_form, 2
 import pytest
 
 from oracle.pyoracle import KIND_Q4_K, KIND_Q5_K, KIND_Q6_K
+from tests.test_gpu_moe import check_moe_stages
 from tests.util import assert_matmul_parity, gaussian
 
 pytestmark = pytest.mark.gpu
@@ -37,3 +38,19 @@ def test_integer_operand_gemm_matches_oracle(hip, oracle, name, N, M, K):
     got = hip.linear(x, blocks, kind, M, bias=bias)
     assert hip.last_route() == f"mmq_{name}_q8_k_mfma_tile"
     assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, bias=bias, threads=16), what=f"{name} {N} x {K} x {M}")
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+def test_moe_experts_on_the_tiled_gemm(hip, oracle, name):
+    """Experts that see 333 routes each, in items of 64 with a ragged last one, through the grouped form: two tiles per
+    compute unit in both projections and 32 routes per expert are the line from which the expert layer takes it. Stage by
+    stage with the bounds of the expert tests (the product of gate and up is quantized again in between)."""
+    E, F, H, k, T = 3, 2048, 4096, 2, 500
+    kind = KINDS[name]
+    gate, up = (hip.quantize_weights(kind, gaussian(710 + i, (E * F, H), 0.02)) for i in range(2))
+    down = hip.quantize_weights(kind, gaussian(712, (E * H, F), 0.02))
+    hidden = gaussian(713, (T, H))
+    vals, ids = oracle.topk(gaussian(714, (T, E)), k)
+    w = oracle.softmax_rows(vals)
+    ref = oracle.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind, threads=16)
+    check_moe_stages(hip, oracle, hidden, gate, up, down, ids, w, F, E, kind, ref, f"tiled experts {name}")
