@@ -104,17 +104,22 @@ enum ActSource {
 };
 
 template <int SRC>
+__device__ __forceinline__ float glu_value(float g, float up) {
+    if constexpr (SRC == SRC_SWIGLU) {
+        const float a = g / (1.0f + expf(-g));
+        return a * up;
+    } else {
+        const float a = 0.5f * g * (1.0f + erff(g * 0.70710678118654752440f));
+        return a * up;
+    }
+}
+
+template <int SRC>
 __device__ __forceinline__ float load_act_value(const void *x, const void *x2, size_t i) {
     if constexpr (SRC == SRC_F16) {
         return h2f(((const uint16_t *)x)[i]);
-    } else if constexpr (SRC == SRC_SWIGLU) {
-        const float g = ((const float *)x)[i];
-        const float a = g / (1.0f + expf(-g));
-        return a * ((const float *)x2)[i];
-    } else if constexpr (SRC == SRC_GEGLU) {
-        const float g = ((const float *)x)[i];
-        const float a = 0.5f * g * (1.0f + erff(g * 0.70710678118654752440f));
-        return a * ((const float *)x2)[i];
+    } else if constexpr (SRC == SRC_SWIGLU || SRC == SRC_GEGLU) {
+        return glu_value<SRC>(((const float *)x)[i], ((const float *)x2)[i]);
     } else {
         return ((const float *)x)[i];
     }
@@ -142,15 +147,25 @@ __global__ __launch_bounds__(256) void k_quantize_q8_k(const void *__restrict__ 
         const size_t b = id - row * nb;
         const size_t col0 = b * QK_K + (size_t)lane * 4;
         bool vec = false;
-        if constexpr (SRC == SRC_F32) {
-            // whole 16-byte groups inside the row: one load instead of four
+        if constexpr (SRC != SRC_F16) {
+            // whole 16-byte groups inside the row: one load (two of a gated product) instead of four
             vec = (k & 3) == 0 && ((((uintptr_t)x) & 15) == 0) && col0 + 3 < k;
+            if constexpr (SRC != SRC_F32) {
+                vec = vec && (((uintptr_t)x2) & 15) == 0;
+            }
             if (vec) {
                 const float4 f = *(const float4 *)((const float *)x + row * k + col0);
                 v[w][0] = f.x;
                 v[w][1] = f.y;
                 v[w][2] = f.z;
                 v[w][3] = f.w;
+                if constexpr (SRC != SRC_F32) {
+                    const float4 u = *(const float4 *)((const float *)x2 + row * k + col0);
+                    v[w][0] = glu_value<SRC>(f.x, u.x);
+                    v[w][1] = glu_value<SRC>(f.y, u.y);
+                    v[w][2] = glu_value<SRC>(f.z, u.z);
+                    v[w][3] = glu_value<SRC>(f.w, u.w);
+                }
             }
         }
         if (!vec) {
