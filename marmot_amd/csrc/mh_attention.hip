@@ -46,7 +46,31 @@ struct PaParams {
     uint32_t *claim;                // scratch [blocks][kv heads]: the token whose workgroup rescales the block (~0 = none yet)
     uint32_t splits;    // workgroups along the history of one (token, heads) pair
     float *partial;     // splits > 1: [token][query head][split][2 + head_dim]: maximum, sum, unnormalized output
+    uint32_t tile_tokens;  // tokens per tile of the prompt kernel (k_pa_prompt), 0 = not launched
+    int out_vec;           // prompt kernel: FLOAT32 output rows at 16-byte boundaries
 };
+
+// The prompt kernel takes a token when its tile (tile_tokens consecutive tokens of the call) holds at least this many
+// tokens of the token's sequence; the other kernels of the call take the rest. A pass over a history costs the prompt
+// kernel the same for one token as for the whole tile, so the decode tokens of a mixed call stay where every token has
+// workgroups of its own.
+constexpr uint32_t PA_RUN_MIN = 4;
+
+// Whole wavefront: does the prompt kernel take token t?
+__device__ __forceinline__ bool pa_in_run(const PaParams &p, uint32_t t, uint32_t seq) {
+    if (p.tile_tokens == 0u || seq >= p.max_seqs) {
+        return false;
+    }
+    const uint32_t first = t / p.tile_tokens * p.tile_tokens;
+    uint32_t same = 0;
+    for (uint32_t i = 0; i < p.tile_tokens; i += 64u) {
+        const uint32_t other = first + i + (threadIdx.x & 63u);
+        const bool inside = i + (threadIdx.x & 63u) < p.tile_tokens && other < p.token_count;
+        const uint32_t s = p.meta[(inside ? other : t) * p.meta_stride[0]];
+        same += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(inside && s == seq));
+    }
+    return same >= PA_RUN_MIN;
+}
 
 // marmot_f32_to_bf16_ref / marmot_bf16_to_f32_ref (src/utils/dtype_ref.c:86-104): round to nearest even on the bits
 __device__ __forceinline__ uint16_t pa_f2bf(float v) {
@@ -565,6 +589,9 @@ __global__ __launch_bounds__(16 * PA_GROUPS) void k_pa_attend(const PaParams p) 
     const uint32_t qh0 = blockIdx.y * QH;  // first query head of this workgroup; QH divides the heads per kv head
     const int tid = threadIdx.x, g = tid >> 4, l = tid & 15;
     const uint32_t seq = p.meta[t * p.meta_stride[0]];
+    if (pa_in_run(p, t, seq)) {
+        return;
+    }
     const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
@@ -821,6 +848,9 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
     const uint32_t qh0 = blockIdx.y * QH;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, j = lane >> 4;
     const uint32_t seq = p.meta[t * p.meta_stride[0]];
+    if (pa_in_run(p, t, seq)) {
+        return;
+    }
     const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
@@ -1206,6 +1236,455 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
     }
 }
 
+// ---- prompts: tiles of tokens that share the key / value rows (FLOAT16 or BFLOAT16 cache, rows of 64 or 128 values)
+// One workgroup of four wavefronts per (tile of tokens, key / value head, share of the history). Its 128 rows are the
+// (token, query head) pairs of 128 / group consecutive tokens; wavefront w owns rows 32 w .. + 31, lane l row l % 32.
+// The workgroup walks the histories of the sequences in its tile (one, mostly) in tiles of 64 positions, double-buffered
+// in LDS: keys as rows, values transposed, both requested one tile ahead through registers.
+//   * Scores: S[position][row] = K . q as v_mfma_f32_32x32x16 with the key rows as row operand; lane (row, h = l / 32)
+//     receives positions 8 q + 4 h + e in register 4 q + e, so a row's softmax is 16 registers and one exchange.
+//   * Output: O[dimension][row] += V^T . P with the weights as column operand: registers 8 i .. 8 i + 7 ARE the operand of
+//     instruction i (the k index of lane half h stands for positions 16 i + 4 h + 0..3 and 16 i + 8 + 4 h + 0..3), and the
+//     transposed values are stored in that order, so no weight moves between lanes.
+//   * Precision: query and weights stay fp32 quantities, split into two FLOAT16 parts (rounded to nearest: 2^-23; weights
+//     are scaled by 2^14 first, so that the parts of small ones are normal numbers) or three BFLOAT16 parts (24 bits, exact
+//     for the weights), one instruction per part, fp32 accumulation.
+//   * A value that is not finite would reach rows that may not see it (0 x infinity): a tile that holds one takes the
+//     products of its visible positions one by one.
+// The kernel per token reads a history once per token and head group and uses a quarter of its matrix instructions; this
+// one reads it once per 128 / group tokens. Two sequences x 512 tokens over 2048 cached ones, 32 / 8 heads of 128,
+// BFLOAT16 cache, whole call: 761 -> 249 us.
+typedef float pa_float16v __attribute__((ext_vector_type(16)));
+typedef _Float16 pa_half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 pa_bf8 __attribute__((ext_vector_type(8)));
+typedef uint32_t pa_uint4 __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t PA_PROMPT_ROWS = 128;
+constexpr uint32_t PA_PROMPT_SHARE = 256;  // positions a share of a history has at least
+
+template <int HD>
+struct PaPromptLds {
+    static constexpr uint32_t KROW = 2 * HD + 16;   // bytes; 16 of padding: rows 4 banks apart
+    static constexpr uint32_t K = 64 * KROW, V = HD * 128, STAGE = K + V;
+    static constexpr uint32_t TOKENS = 2 * STAGE;  // sequence, length, longest history: 128 words each; two words
+    static constexpr uint32_t BYTES = TOKENS + (3 * PA_PROMPT_ROWS + 4) * 4;
+};
+
+// byte offset of chunk c (16 bytes: eight positions) of dimension d in the transposed values; the exclusive or spreads
+// eight consecutive dimensions (reads) and dimensions four apart (writes) over the banks
+__device__ __forceinline__ uint32_t pa_vt_chunk(uint32_t d, uint32_t c) {
+    return d * 128u + 16u * (c ^ ((d >> 2) & 7u) ^ ((d & 3u) << 1));
+}
+
+template <bool BF16>
+__device__ __forceinline__ pa_float16v pa_mma32(const uint4 a, const uint4 b, const pa_float16v c) {
+    if constexpr (BF16) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf8, a), __builtin_bit_cast(pa_bf8, b), c, 0, 0, 0);
+    } else {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pa_half8, a), __builtin_bit_cast(pa_half8, b), c, 0, 0,
+                                                      0);
+    }
+}
+
+// (rows of 128 values: 64 or 96 registers of query parts and 64 of output, one wavefront per SIMD)
+template <int HD, bool BF16>
+__global__ __launch_bounds__(256, HD == 128 ? 1 : 2) void k_pa_prompt(const PaParams p) {
+    using L = PaPromptLds<HD>;
+    constexpr int PARTS = BF16 ? 3 : 2, QC = HD / 16, DB = HD / 32;
+    constexpr int KN = HD / 32, VN = HD / 64;  // per thread and tile: 16-byte key chunks, 4 x 4 blocks of values
+    constexpr float UNIT = BF16 ? 1.0f : 16384.0f;
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    uint32_t *s_seq = (uint32_t *)(lds + L::TOKENS), *s_len = s_seq + PA_PROMPT_ROWS, *s_longest = s_len + PA_PROMPT_ROWS;
+    uint32_t *s_odd = s_longest + PA_PROMPT_ROWS;  // per buffer: 1 + number of its tile if that holds a value that is not finite
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u, n = lane & 31u, h = lane >> 5;
+    const uint32_t tt = p.tile_tokens, t0 = (gridDim.x - 1u - blockIdx.x) * tt, kvh = blockIdx.y;  // long histories first
+
+    // the tile's tokens: sequence (NONE: not this kernel's), visible positions, and at the first token of a sequence the
+    // largest number of them
+    if (tid < PA_PROMPT_ROWS) {
+        uint32_t seq = NONE, len = 0;
+        if (tid < tt && t0 + tid < p.token_count) {
+            seq = p.meta[(size_t)(t0 + tid) * p.meta_stride[0]];
+            len = p.meta[(size_t)(t0 + tid) * p.meta_stride[0] + p.meta_stride[1]] + 1u;
+            const uint64_t limit = (uint64_t)p.max_blocks << p.shift;  // no position behind the table's last block
+            len = len < limit ? len : (uint32_t)limit;
+            seq = seq < p.max_seqs ? seq : NONE;
+        }
+        s_seq[tid] = seq;
+        s_len[tid] = len;
+    }
+    if (tid < 2) {
+        s_odd[tid] = 0;
+    }
+    __syncthreads();
+    bool mine = false;
+    if (tid < PA_PROMPT_ROWS) {
+        const uint32_t seq = s_seq[tid];
+        uint32_t same = 0, longest = 0;
+        bool first = true;
+        for (uint32_t i = 0; i < tt; ++i) {
+            const bool eq = s_seq[i] == seq;
+            same += eq ? 1u : 0u;
+            first = first && !(eq && i < tid);
+            longest = eq && s_len[i] > longest ? s_len[i] : longest;
+        }
+        mine = seq != NONE && same >= PA_RUN_MIN;
+        s_longest[tid] = mine && first ? longest : 0u;
+    }
+    __syncthreads();
+    if (tid < PA_PROMPT_ROWS && !mine) {
+        s_seq[tid] = NONE;
+    }
+    __syncthreads();
+
+    const uint32_t row = 32u * wave + n, tl = row / p.group, g = row - tl * p.group;
+    const bool have = tl < tt;
+    const uint32_t row_seq = have ? s_seq[tl] : NONE;
+    const uint32_t full_len = row_seq != NONE ? s_len[tl] : 0u;
+    const uint32_t t = t0 + tl, qh = kvh * p.group + g;
+
+    // the query of this lane's row: dimensions 16 c + 8 h .. + 7, scaled and split. Rows that are not contiguous pass
+    // through LDS (element loads in a loop of their own instead of 64 copies of them here).
+    float *staged = (float *)lds;  // [128][HD]
+    static_assert(L::TOKENS >= PA_PROMPT_ROWS * HD * 4, "the query rows fit the two stages");
+    if (!p.q_vec) {
+        for (uint32_t i = tid; i < PA_PROMPT_ROWS * HD; i += 256u) {
+            const uint32_t r = i / HD, token = r / p.group;
+            if (token < tt && s_seq[token] != NONE) {
+                staged[i] = pa_load(p.q, p.act_dtype, (size_t)(t0 + token) * p.q_stride[0] +
+                                    (size_t)(kvh * p.group + (r - token * p.group)) * p.q_stride[1] + (i % HD) * p.q_stride[2]);
+            }
+        }
+        __syncthreads();
+    }
+    uint4 qpart[PARTS][QC];
+    const size_t q_base = (size_t)t * p.q_stride[0] + (size_t)qh * p.q_stride[1];
+#pragma unroll
+    for (int c = 0; c < QC; ++c) {
+        const uint32_t d = 16u * c + 8u * h;
+        float qv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            qv[e] = 0.0f;
+        }
+        if (row_seq != NONE) {
+            if (!p.q_vec) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    qv[e] = staged[row * HD + d + e];
+                }
+            } else if (p.act_dtype == MARMOT_HIP_DTYPE_F32) {
+                const float4 a = *(const float4 *)((const float *)p.q + q_base + d);
+                const float4 b = *(const float4 *)((const float *)p.q + q_base + d + 4u);
+                qv[0] = a.x, qv[1] = a.y, qv[2] = a.z, qv[3] = a.w, qv[4] = b.x, qv[5] = b.y, qv[6] = b.z, qv[7] = b.w;
+            } else {
+                const uint2 a = *(const uint2 *)((const uint16_t *)p.q + q_base + d);
+                const uint2 b = *(const uint2 *)((const uint16_t *)p.q + q_base + d + 4u);
+                const uint32_t words[4] = {a.x, a.y, b.x, b.y};
+                const bool half = p.act_dtype == MARMOT_HIP_DTYPE_F16;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint16_t bits = (uint16_t)(words[e >> 1] >> (16 * (e & 1)));
+                    qv[e] = half ? h2f(bits) : pa_bf2f(bits);
+                }
+            }
+        }
+        uint32_t w[PARTS][4];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float v = p.scale != 1.0f ? qv[e] * p.scale : qv[e];
+#pragma unroll
+            for (int part = 0; part < PARTS; ++part) {  // each remainder is exact in fp32
+                uint32_t bits;
+                if constexpr (BF16) {
+                    bits = pa_f2bf(v);
+                    v -= pa_bf2f((uint16_t)bits);
+                } else {
+                    bits = f2h(v);
+                    v -= h2f((uint16_t)bits);
+                }
+                w[part][e >> 1] = (e & 1) == 0 ? bits : (w[part][e >> 1] | (bits << 16));
+            }
+        }
+#pragma unroll
+        for (int part = 0; part < PARTS; ++part) {
+            qpart[part][c] = make_uint4(w[part][0], w[part][1], w[part][2], w[part][3]);
+        }
+    }
+
+    if (!p.q_vec) {
+        __syncthreads();
+    }
+
+    const pa_float16v zero = {};
+    pa_float16v out[DB];
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+        out[d] = zero;
+    }
+    float m = -INFINITY, lsum = 0.0f;  // lsum: of this lane's half of the positions
+    const size_t head_base = (size_t)p.layer_idx * p.kv_stride[1] + (size_t)kvh * p.kv_stride[2];
+    const uint16_t *keys = (const uint16_t *)p.kv_k + head_base, *values = (const uint16_t *)p.kv_v + head_base;
+    uint32_t count = 0;  // tiles staged so far, over all sequences: buffer = count & 1
+    pa_uint4 kreg[KN];
+    uint2 vreg[VN][4];
+    uint64_t mask_next = 0;  // positions of the requested tile that exist
+
+    for (uint32_t first = 0; first < tt; ++first) {
+        const uint32_t longest = __builtin_amdgcn_readfirstlane(s_longest[first]);
+        if (longest == 0u) {
+            continue;
+        }
+        const uint32_t seq = __builtin_amdgcn_readfirstlane(s_seq[first]);
+        const uint32_t row_len = row_seq == seq ? full_len : 0u;
+        const uint32_t *table_row = p.table + (size_t)seq * p.table_stride[0];
+        const uint32_t tiles = (longest + 63u) / 64u;
+        const uint32_t per_share = (tiles + p.splits - 1u) / p.splits;
+        const uint32_t begin = blockIdx.z * per_share;
+        const uint32_t end = begin + per_share < tiles ? begin + per_share : tiles;
+        if (begin >= end) {
+            continue;
+        }
+        // lane i locates position i of the tile; rows without a block read block 0
+        auto request = [&](uint32_t tile) {
+            const uint32_t pos = 64u * tile + lane, logical = pos >> p.shift;
+            const uint32_t tb = table_row[(size_t)(logical < p.max_blocks ? logical : p.max_blocks - 1u) * p.table_stride[1]];
+            const bool ok = pos < longest && logical < p.max_blocks && tb != PA_NO_BLOCK && tb < p.kv_blocks;
+            mask_next = __builtin_amdgcn_ballot_w64(ok);
+            const size_t off = ok ? (size_t)tb * p.kv_stride[0] + (size_t)(pos & p.mask) * p.kv_stride[3] : 0u;
+            const int lo = (int)(uint32_t)off, hi = (int)(uint32_t)(off >> 32);
+            auto row_of = [&](uint32_t r) -> size_t {
+                return (size_t)(uint32_t)__shfl(lo, (int)r) | ((size_t)(uint32_t)__shfl(hi, (int)r) << 32);
+            };
+#pragma unroll
+            for (int i = 0; i < KN; ++i) {
+                const uint32_t c = tid + 256u * i, r = c / (HD / 8);
+                kreg[i] = *(const pa_uint4 *)(keys + row_of(r) + 8u * (c % (HD / 8)));
+            }
+#pragma unroll
+            for (int i = 0; i < VN; ++i) {
+                const uint32_t u = tid + 256u * i, pq = u / (HD / 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    vreg[i][e] = *(const uint2 *)(values + row_of(4u * pq + e) + 4u * (u % (HD / 4)));
+                }
+            }
+        };
+        auto store = [&](uint32_t number) {
+            uint8_t *stage = lds + (number & 1u) * L::STAGE;
+#pragma unroll
+            for (int i = 0; i < KN; ++i) {
+                const uint32_t c = tid + 256u * i;
+                *(pa_uint4 *)(stage + c / (HD / 8) * L::KROW + 16u * (c % (HD / 8))) = kreg[i];
+            }
+            uint32_t odd = 0;
+#pragma unroll
+            for (int i = 0; i < VN; ++i) {
+                const uint32_t u = tid + 256u * i, pq = u / (HD / 4), d0 = 4u * (u % (HD / 4));
+                uint2 v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool ok = (mask_next >> (4u * pq + e)) & 1u;
+                    v[e] = ok ? vreg[i][e] : make_uint2(0, 0);
+                    // the top bit of each half: exponent field all ones
+                    constexpr uint32_t ONE = BF16 ? 0x00800080u : 0x04000400u;
+                    odd |= ((v[e].x & 0x7fff7fffu) + ONE) | ((v[e].y & 0x7fff7fffu) + ONE);
+                }
+                const uint32_t chunk = 2u * (pq >> 2) + (pq & 1u), half = 8u * ((pq >> 1) & 1u);
+                uint8_t *vt = stage + L::K + half;
+                constexpr uint32_t LOW = 0x05040100u, HIGH = 0x07060302u;
+                auto pair = [](uint32_t b, uint32_t a, uint32_t sel) { return __builtin_amdgcn_perm(b, a, sel); };
+                *(uint2 *)(vt + pa_vt_chunk(d0, chunk)) = make_uint2(pair(v[1].x, v[0].x, LOW), pair(v[3].x, v[2].x, LOW));
+                *(uint2 *)(vt + pa_vt_chunk(d0 + 1u, chunk)) =
+                    make_uint2(pair(v[1].x, v[0].x, HIGH), pair(v[3].x, v[2].x, HIGH));
+                *(uint2 *)(vt + pa_vt_chunk(d0 + 2u, chunk)) =
+                    make_uint2(pair(v[1].y, v[0].y, LOW), pair(v[3].y, v[2].y, LOW));
+                *(uint2 *)(vt + pa_vt_chunk(d0 + 3u, chunk)) =
+                    make_uint2(pair(v[1].y, v[0].y, HIGH), pair(v[3].y, v[2].y, HIGH));
+            }
+            if ((odd & 0x80008000u) != 0u) {
+                s_odd[number & 1u] = number + 1u;
+            }
+        };
+        auto consume = [&](uint32_t tile, uint32_t number, uint64_t mask) {
+            const uint8_t *stage = lds + (number & 1u) * L::STAGE;
+            const bool odd = __builtin_amdgcn_readfirstlane(s_odd[number & 1u]) == number + 1u;
+#pragma unroll 1
+            for (uint32_t st = 0; st < 2; ++st) {
+                const uint32_t p0 = 64u * tile + 32u * st;
+                if (__builtin_amdgcn_ballot_w64(row_len > p0) == 0) {
+                    continue;
+                }
+                pa_float16v s = zero;
+#pragma unroll
+                for (int c = 0; c < QC; ++c) {
+                    const uint4 k = *(const uint4 *)(stage + (32u * st + n) * L::KROW + 32u * c + 16u * h);
+#pragma unroll
+                    for (int part = PARTS - 1; part >= 0; --part) {
+                        s = pa_mma32<BF16>(k, qpart[part][c], s);
+                    }
+                }
+                const uint32_t there = (uint32_t)(mask >> (32u * st));
+                const uint32_t left = row_len > p0 ? row_len - p0 : 0u;
+                const uint32_t see = there & (left >= 32u ? 0xFFFFFFFFu : (1u << left) - 1u);
+                const uint32_t bits = see >> (4u * h);
+                if (__builtin_amdgcn_ballot_w64(see != 0xFFFFFFFFu) != 0) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        s[r] = (bits >> (8 * (r >> 2) + (r & 3))) & 1u ? s[r] : -INFINITY;
+                    }
+                }
+                float big = s[0];
+#pragma unroll
+                for (int r = 1; r < 16; ++r) {
+                    big = fmaxf(big, s[r]);
+                }
+                big = fmaxf(big, pa_xor32(big));
+                const float m_new = fmaxf(m, big);
+                const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
+                const float m_use = m_new == -INFINITY && see == 0u ? 0.0f : m_new;  // (a row that sees nothing yet)
+                float w[16], sum = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    w[r] = pa_exp(s[r] - m_use) * UNIT;
+                    sum += w[r];
+                }
+                lsum = lsum * corr + sum;
+                if (__builtin_amdgcn_ballot_w64(m_new != m) != 0) {
+#pragma unroll
+                    for (int d = 0; d < DB; ++d) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            out[d][r] *= corr;
+                        }
+                    }
+                }
+                m = m_new;
+                const uint8_t *vt = stage + L::K;
+                if (odd) {
+                    for (uint32_t i = 0; i < 32u; ++i) {
+                        // position i: register 4 (i / 8) + i % 4 of lane half (i / 4) % 2
+                        float mine_w = 0.0f;
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            mine_w = (uint32_t)r == 4u * (i >> 3) + (i & 3u) ? w[r] : mine_w;
+                        }
+                        const float wi = __shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u)));
+                        if ((see >> i) & 1u) {
+                            const uint32_t pos = 32u * st + i, chunk = 2u * (pos >> 4) + ((pos >> 2) & 1u);
+                            const uint32_t in = 8u * ((pos >> 3) & 1u) + 2u * (pos & 3u);
+#pragma unroll
+                            for (int d = 0; d < DB; ++d) {
+#pragma unroll
+                                for (int r = 0; r < 16; ++r) {
+                                    const uint32_t dim = 32u * d + 8u * (r >> 2) + 4u * h + (r & 3);
+                                    const uint16_t v = *(const uint16_t *)(vt + pa_vt_chunk(dim, chunk) + in);
+                                    out[d][r] = __builtin_fmaf(wi, BF16 ? pa_bf2f(v) : h2f(v), out[d][r]);
+                                }
+                            }
+                        }
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    uint32_t wp[PARTS][4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float a = w[8 * i + 2 * e], b = w[8 * i + 2 * e + 1];
+#pragma unroll
+                        for (int part = 0; part < PARTS; ++part) {
+                            if constexpr (BF16) {  // eight bits at a time, cut off: the third part is exact
+                                const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
+                                wp[part][e] = __builtin_amdgcn_perm(bb, ab, 0x07060302u);
+                                a -= __uint_as_float(ab & 0xFFFF0000u);
+                                b -= __uint_as_float(bb & 0xFFFF0000u);
+                            } else {
+                                const uint16_t ah = f2h(a), bh = f2h(b);
+                                wp[part][e] = (uint32_t)ah | ((uint32_t)bh << 16);
+                                a -= h2f(ah);
+                                b -= h2f(bh);
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int d = 0; d < DB; ++d) {
+                        const uint4 v = *(const uint4 *)(vt + pa_vt_chunk(32u * d + n, 4u * st + 2u * i + h));
+#pragma unroll
+                        for (int part = PARTS - 1; part >= 0; --part) {
+                            out[d] = pa_mma32<BF16>(v, make_uint4(wp[part][0], wp[part][1], wp[part][2], wp[part][3]), out[d]);
+                        }
+                    }
+                }
+            }
+        };
+        // A buffer is written after the barrier that follows its last reading: tile k + 1 is stored beside the reading of
+        // tile k, into the buffer that tile k - 1 left before the barrier.
+        request(begin);
+        store(count);
+        uint64_t mask = mask_next;
+        __syncthreads();
+        for (uint32_t tile = begin; tile < end; ++tile, ++count) {
+            const bool more = tile + 1u < end;
+            if (more) {
+                request(tile + 1u);
+            }
+            consume(tile, count, mask);
+            if (more) {
+                store(count + 1u);
+                mask = mask_next;
+            }
+            __syncthreads();
+        }
+    }
+
+    lsum += pa_xor32(lsum);
+    if (row_seq == NONE) {
+        return;
+    }
+    const bool bad = lsum != lsum;
+    if (p.splits > 1u) {
+        float *part = p.partial + (((size_t)t * p.num_q_heads + qh) * p.splits + blockIdx.z) * (HD + 2u);
+        if (h == 0) {
+            part[0] = m;
+            part[1] = lsum;
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float2 *dst = (float2 *)(part + 2 + 32 * d + 8 * q + 4 * h);
+                dst[0] = make_float2(out[d][4 * q], out[d][4 * q + 1]);
+                dst[1] = make_float2(out[d][4 * q + 2], out[d][4 * q + 3]);
+            }
+        }
+        return;
+    }
+    const float inv = bad ? __uint_as_float(0x7fc00000u) : (lsum > 0.0f ? 1.0f / lsum : 0.0f);
+    const size_t base = (size_t)t * p.out_stride[0] + (size_t)qh * p.out_stride[1];
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t dim = 32u * d + 8u * q + 4u * h;
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o[e] = bad || lsum > 0.0f ? out[d][4 * q + e] * inv : 0.0f;
+            }
+            if (p.out_vec) {
+                *(float4 *)((float *)p.out + base + dim) = make_float4(o[0], o[1], o[2], o[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    pa_store(p.out, p.act_dtype, base + (size_t)(dim + e) * p.out_stride[2], o[e]);
+                }
+            }
+        }
+    }
+}
+
 // the shares of a (token, head) pair's history: out = sum_s o_s * exp(M_s - M) / sum_s l_s * exp(M_s - M)
 __global__ __launch_bounds__(256) void k_pa_merge(const PaParams p) {
     __shared__ float s_big[64], s_tot[64];  // splits <= 64
@@ -1243,6 +1722,16 @@ template <int EPL, int QH>
 static void pa_launch(marmot_hip_device *dev, const PaParams &p) {
     hipLaunchKernelGGL((k_pa_attend<EPL, QH>), dim3(p.token_count, p.num_q_heads / QH, p.splits),
                        dim3(16 * PA_GROUPS), 0, dev->stream, p);
+}
+
+template <int HD, bool BF16>
+static int pa_launch_prompt(marmot_hip_device *dev, const PaParams &p) {
+    MH_TRY(allow_large_lds(dev, (const void *)k_pa_prompt<HD, BF16>));
+    const unsigned tiles = (p.token_count + p.tile_tokens - 1) / p.tile_tokens;
+    hipLaunchKernelGGL((k_pa_prompt<HD, BF16>), dim3(tiles, p.num_kv_heads, p.splits), dim3(256), PaPromptLds<HD>::BYTES,
+                       dev->stream, p);
+    MH_HIP(hipGetLastError());
+    return MARMOT_HIP_SUCCESS;
 }
 
 static bool pa_float_dtype(int d) {
@@ -1385,6 +1874,23 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         size_t sp = (want + pairs - 1) / pairs;
         p.splits = (uint32_t)(sp > 64 ? 64 : sp);
     }
+    // Prompts: k_pa_prompt beside the per-token kernel. Two tokens and more per row of the block table on average (a decode
+    // step has at most one, and would pay for an empty launch), 16-byte key rows, 8-byte value rows.
+    const bool prompt = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || kv_bf16) && rows16 && p.kv_vec &&
+                        (a->head_dim == 64 || a->head_dim == 128) && p.group <= 32 && a->token_count >= 16 &&
+                        a->token_count / 2 >= a->max_seqs && !dev->knobs.no_attention_mfma;
+    p.tile_tokens = 0;
+    p.out_vec = 0;
+    if (prompt) {
+        p.tile_tokens = PA_PROMPT_ROWS / p.group;
+        p.out_vec = a->act_dtype == MARMOT_HIP_DTYPE_F32 && a->out_stride[2] == 1 && (((uintptr_t)a->d_out) & 15) == 0 &&
+                    a->out_stride[0] % 4 == 0 && a->out_stride[1] % 4 == 0;
+        const size_t tiles = (a->token_count + p.tile_tokens - 1) / p.tile_tokens * a->num_kv_heads;
+        const size_t most = (p.max_blocks * a->block_size + PA_PROMPT_SHARE - 1) / PA_PROMPT_SHARE;
+        const size_t sp = (2 * (size_t)dev->props.multiProcessorCount + tiles - 1) / tiles;
+        p.splits = (uint32_t)(sp < most ? sp : most);
+        p.splits = p.splits < 1u ? 1u : (p.splits > 16u ? 16u : p.splits);
+    }
     const size_t partial_bytes =
         p.splits > 1u ? (size_t)a->token_count * a->num_q_heads * p.splits * (a->head_dim + 2u) * sizeof(float) : 0;
     if (fp8_bytes + partial_bytes != 0) {
@@ -1416,6 +1922,13 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         hipLaunchKernelGGL(k_pa_write, per_token, dim3(a->head_dim <= 64 ? 64 : 128), 0, dev->stream, p);
     }
     MH_HIP(hipGetLastError());
+    if (prompt) {
+        if (kv_bf16) {
+            MH_TRY((a->head_dim == 64 ? pa_launch_prompt<64, true>(dev, p) : pa_launch_prompt<128, true>(dev, p)));
+        } else {
+            MH_TRY((a->head_dim == 64 ? pa_launch_prompt<64, false>(dev, p) : pa_launch_prompt<128, false>(dev, p)));
+        }
+    }
     if (mfma_scores) {
         const dim3 grid(p.token_count, p.num_q_heads / (uint32_t)qh, p.splits), block(256);
         // FLOAT8_E4M3 decode steps over long contexts (few tokens, a block table of 2048 positions or more): the form

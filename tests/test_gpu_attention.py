@@ -143,6 +143,59 @@ def test_prompt_of_many_tokens_takes_unsplit_histories(hip, oracle):
     check(hip, oracle, case, "prompt chunk")
 
 
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+@pytest.mark.parametrize("head_dim,act", [(64, "f16"), (128, "f32")])
+@pytest.mark.parametrize("hq,hkv,block_size,seqs,shuffle", [
+    (8, 2, 16, [(0, 70)], False),               # group 4: a full tile of 32 tokens, a full and a ragged last one
+    (3, 3, 16, [(63, 66), (64, 63)], False),    # group 1: 128 tokens per tile, two sequences in it, tile edges at 64
+    (14, 2, 64, [(5, 40), (300, 20)], False),   # group 7: 18 tokens per tile, two idle rows
+    (4, 1, 8, [(0, 3), (130, 45), (1, 1), (600, 40), (9, 2)], False),  # runs too short for the tile kernel among others
+    (8, 2, 32, [(31, 40), (200, 33)], True),    # tokens in any order
+])
+def test_prompt_tiles(hip, oracle, hq, hkv, block_size, seqs, shuffle, head_dim, act, kv):
+    """The kernel that shares key / value rows among the tokens of a tile: NaN rows behind the end of a sequence, a hole
+    in the block table, an infinite value that only the later tokens see, split histories, and large queries."""
+    case = make_case(700 + hq + head_dim, seqs, num_q_heads=hq, num_kv_heads=hkv, head_dim=head_dim, block_size=block_size,
+                     act=act, kv=kv, shuffle_tokens=shuffle)
+    assert len(case["token_meta"]) >= 2 * case["block_table"].shape[0]  # the call takes that kernel
+    nan, inf = (np.nan, np.inf) if kv == "f16" else (np.uint16(0x7fc0), np.uint16(0x7f80))
+    table, last = case["block_table"], {}
+    for seq, pos, _, _ in case["token_meta"]:
+        last[int(seq)] = max(last.get(int(seq), -1), int(pos))
+    for seq, end in last.items():
+        for b in range(table.shape[1]):
+            lo = max(0, end + 1 - b * block_size)
+            if table[seq, b] != NO_BLOCK and lo < block_size:
+                case["kv_k"][table[seq, b], :, :, lo:, :] = nan
+                case["kv_v"][table[seq, b], :, :, lo:, :] = nan
+    check(hip, oracle, case, "prompt tiles")
+    longest = max(last, key=last.get)
+    holed = dict(case, block_table=table.copy())
+    holed["block_table"][longest, 1] = NO_BLOCK
+    check(hip, oracle, holed, "prompt tiles, hole")
+    if act == "f32":
+        check(hip, oracle, dict(case, q=(case["q"] * np.float32(40)).astype(np.float32)), "prompt tiles, large queries")
+    # one infinite value in the row of the longest sequence's token in the middle of its new tokens: tokens before it do
+    # not see it, the others' outputs are infinite in that dimension and unchanged in all others
+    mine = [i for i, mt in enumerate(case["token_meta"]) if int(mt[0]) == longest]
+    mine.sort(key=lambda i: int(case["token_meta"][i, 1]))
+    at = mine[len(mine) // 2]
+    odd = dict(case, v_new=case["v_new"].copy())
+    odd["v_new"][at, :, 3] = np.inf if act != "bf16" else inf
+    base, _, _ = run_hip(hip, case)
+    got, _, _ = run_hip(hip, odd)
+    b, g = to_f32(base, act), to_f32(got, act)
+    sees = np.zeros(len(case["token_meta"]), bool)
+    for i in mine:
+        sees[i] = int(case["token_meta"][i, 1]) >= int(case["token_meta"][at, 1])
+    assert np.all(np.isinf(g[sees][:, :, 3])), "infinite value"
+    rest = np.ones(g.shape, bool)
+    rest[sees, :, 3] = False
+    vmax = np.nanmax(np.abs(to_f32(case["v_new"], act))) + np.nanmax(np.abs(to_f32(case["kv_v"], kv)))
+    # (the odd tile's sums run in another order)
+    assert np.max(np.abs(g[rest].astype(np.float64) - b[rest])) <= TOLERANCE[act] * vmax, "rows beside the infinite value"
+
+
 def test_holes_strided_views_token_count_and_errors(hip, oracle):
     case = make_case(13, [(40, 3), (5, 1)], num_q_heads=4, num_kv_heads=2, head_dim=32, block_size=8)
     seq = case["token_meta"][0, 0]
