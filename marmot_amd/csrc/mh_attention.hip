@@ -47,13 +47,14 @@ struct PaParams {
     uint32_t splits;    // workgroups along the history of one (token, heads) pair
     float *partial;     // splits > 1: [token][query head][split][2 + head_dim]: maximum, sum, unnormalized output
     uint32_t tile_tokens;  // tokens per tile of the prompt kernel (k_pa_prompt), 0 = not launched
+    uint32_t long_from;    // prompt kernel: positions a sequence has at least
     int out_vec;           // prompt kernel: FLOAT32 output rows at 16-byte boundaries
 };
 
-// The prompt kernel takes a token when its tile (tile_tokens consecutive tokens of the call) holds at least this many
-// tokens of the token's sequence; the other kernels of the call take the rest. A pass over a history costs the prompt
-// kernel the same for one token as for the whole tile, so the decode tokens of a mixed call stay where every token has
-// workgroups of its own.
+// The prompt kernel takes a token when its tile (tile_tokens consecutive tokens of the call) holds at least PA_RUN_MIN
+// tokens of the token's sequence, one of which sees long_from positions or more; the other kernels of the call take the
+// rest. A pass over a history costs the prompt kernel the same for one token as for the whole tile, so the decode tokens
+// of a mixed call stay where every token has workgroups of its own.
 constexpr uint32_t PA_RUN_MIN = 4;
 
 // Whole wavefront: does the prompt kernel take token t?
@@ -63,13 +64,16 @@ __device__ __forceinline__ bool pa_in_run(const PaParams &p, uint32_t t, uint32_
     }
     const uint32_t first = t / p.tile_tokens * p.tile_tokens;
     uint32_t same = 0;
+    bool any_long = p.long_from == 0u;
     for (uint32_t i = 0; i < p.tile_tokens; i += 64u) {
         const uint32_t other = first + i + (threadIdx.x & 63u);
         const bool inside = i + (threadIdx.x & 63u) < p.tile_tokens && other < p.token_count;
-        const uint32_t s = p.meta[(inside ? other : t) * p.meta_stride[0]];
+        const size_t at = (size_t)(inside ? other : t) * p.meta_stride[0];
+        const uint32_t s = p.meta[at], len = p.meta[at + p.meta_stride[1]] + 1u;
         same += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(inside && s == seq));
+        any_long = any_long || __builtin_amdgcn_ballot_w64(inside && s == seq && len >= p.long_from) != 0;
     }
-    return same >= PA_RUN_MIN;
+    return same >= PA_RUN_MIN && any_long;
 }
 
 // marmot_f32_to_bf16_ref / marmot_bf16_to_f32_ref (src/utils/dtype_ref.c:86-104): round to nearest even on the bits
@@ -1252,8 +1256,10 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 //   * A value that is not finite would reach rows that may not see it (0 x infinity): a tile that holds one takes the
 //     products of its visible positions one by one.
 // The kernel per token reads a history once per token and head group and uses a quarter of its matrix instructions; this
-// one reads it once per 128 / group tokens. Two sequences x 512 tokens over 2048 cached ones, 32 / 8 heads of 128,
-// BFLOAT16 cache, whole call: 761 -> 249 us.
+// one reads it once per 128 / group tokens. Bound by the chain of one wavefront per SIMD (scores, softmax, output): 64
+// positions at a time instead of 32 give it two score chains and half the rescaling. Two sequences x 512 tokens over 2048
+// cached ones, 32 / 8 heads of 128, BFLOAT16 cache, whole call: 756 us per token, 249 with 32 positions at a time and the
+// table entry read in front of each tile, 171 now. Error against 64 bits there: 3.6e-7 per token, 2.2e-7 here.
 typedef float pa_float16v __attribute__((ext_vector_type(16)));
 typedef _Float16 pa_half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 pa_bf8 __attribute__((ext_vector_type(8)));
@@ -1261,6 +1267,8 @@ typedef uint32_t pa_uint4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t PA_PROMPT_ROWS = 128;
 constexpr uint32_t PA_PROMPT_SHARE = 256;  // positions a share of a history has at least
+constexpr uint32_t PA_LONG = 512, PA_MANY = 256;
+constexpr size_t PA_PROMPT_WORK = (size_t)3 << 19;
 
 template <int HD>
 struct PaPromptLds {
@@ -1286,9 +1294,9 @@ __device__ __forceinline__ pa_float16v pa_mma32(const uint4 a, const uint4 b, co
     }
 }
 
-// (rows of 128 values: 64 or 96 registers of query parts and 64 of output, one wavefront per SIMD)
+// (the parts of the query, 64 scores and 64 output registers: one wavefront per SIMD)
 template <int HD, bool BF16>
-__global__ __launch_bounds__(256, HD == 128 ? 1 : 2) void k_pa_prompt(const PaParams p) {
+__global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
     using L = PaPromptLds<HD>;
     constexpr int PARTS = BF16 ? 3 : 2, QC = HD / 16, DB = HD / 32;
     constexpr int KN = HD / 32, VN = HD / 64;  // per thread and tile: 16-byte key chunks, 4 x 4 blocks of values
@@ -1329,7 +1337,7 @@ __global__ __launch_bounds__(256, HD == 128 ? 1 : 2) void k_pa_prompt(const PaPa
             first = first && !(eq && i < tid);
             longest = eq && s_len[i] > longest ? s_len[i] : longest;
         }
-        mine = seq != NONE && same >= PA_RUN_MIN;
+        mine = seq != NONE && same >= PA_RUN_MIN && longest >= p.long_from;  // (no shorter than long_from: the table)
         s_longest[tid] = mine && first ? longest : 0u;
     }
     __syncthreads();
@@ -1447,9 +1455,12 @@ __global__ __launch_bounds__(256, HD == 128 ? 1 : 2) void k_pa_prompt(const PaPa
             continue;
         }
         // lane i locates position i of the tile; rows without a block read block 0
-        auto request = [&](uint32_t tile) {
+        auto table_entry = [&](uint32_t tile) -> uint32_t {
+            const uint32_t logical = (64u * tile + lane) >> p.shift;
+            return table_row[(size_t)(logical < p.max_blocks ? logical : p.max_blocks - 1u) * p.table_stride[1]];
+        };
+        auto request = [&](uint32_t tile, uint32_t tb) {
             const uint32_t pos = 64u * tile + lane, logical = pos >> p.shift;
-            const uint32_t tb = table_row[(size_t)(logical < p.max_blocks ? logical : p.max_blocks - 1u) * p.table_stride[1]];
             const bool ok = pos < longest && logical < p.max_blocks && tb != PA_NO_BLOCK && tb < p.kv_blocks;
             mask_next = __builtin_amdgcn_ballot_w64(ok);
             const size_t off = ok ? (size_t)tb * p.kv_stride[0] + (size_t)(pos & p.mask) * p.kv_stride[3] : 0u;
@@ -1510,125 +1521,144 @@ __global__ __launch_bounds__(256, HD == 128 ? 1 : 2) void k_pa_prompt(const PaPa
         auto consume = [&](uint32_t tile, uint32_t number, uint64_t mask) {
             const uint8_t *stage = lds + (number & 1u) * L::STAGE;
             const bool odd = __builtin_amdgcn_readfirstlane(s_odd[number & 1u]) == number + 1u;
-#pragma unroll 1
-            for (uint32_t st = 0; st < 2; ++st) {
-                const uint32_t p0 = 64u * tile + 32u * st;
-                if (__builtin_amdgcn_ballot_w64(row_len > p0) == 0) {
-                    continue;
-                }
-                pa_float16v s = zero;
+            const uint32_t p0 = 64u * tile;
+            if (__builtin_amdgcn_ballot_w64(row_len > p0) == 0) {
+                return;
+            }
+            pa_float16v s[2] = {zero, zero};
+            uint4 k[2][QC];
+#pragma unroll
+            for (int c = 0; c < QC; ++c) {
+                k[0][c] = *(const uint4 *)(stage + n * L::KROW + 32u * c + 16u * h);
+                k[1][c] = *(const uint4 *)(stage + (32u + n) * L::KROW + 32u * c + 16u * h);
+            }
+#pragma unroll
+            for (int part = PARTS - 1; part >= 0; --part) {  // small parts first
 #pragma unroll
                 for (int c = 0; c < QC; ++c) {
-                    const uint4 k = *(const uint4 *)(stage + (32u * st + n) * L::KROW + 32u * c + 16u * h);
-#pragma unroll
-                    for (int part = PARTS - 1; part >= 0; --part) {
-                        s = pa_mma32<BF16>(k, qpart[part][c], s);
-                    }
+                    s[0] = pa_mma32<BF16>(k[0][c], qpart[part][c], s[0]);
+                    s[1] = pa_mma32<BF16>(k[1][c], qpart[part][c], s[1]);
                 }
-                const uint32_t there = (uint32_t)(mask >> (32u * st));
-                const uint32_t left = row_len > p0 ? row_len - p0 : 0u;
-                const uint32_t see = there & (left >= 32u ? 0xFFFFFFFFu : (1u << left) - 1u);
-                const uint32_t bits = see >> (4u * h);
-                if (__builtin_amdgcn_ballot_w64(see != 0xFFFFFFFFu) != 0) {
+            }
+            const uint32_t left = row_len > p0 ? row_len - p0 : 0u;
+            const uint64_t see = mask & (left >= 64u ? ~0ull : (1ull << left) - 1ull);
+            if (__builtin_amdgcn_ballot_w64(see != ~0ull) != 0) {
+#pragma unroll
+                for (int st = 0; st < 2; ++st) {
+                    const uint32_t bits = (uint32_t)(see >> (32 * st)) >> (4u * h);
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        s[r] = (bits >> (8 * (r >> 2) + (r & 3))) & 1u ? s[r] : -INFINITY;
+                        s[st][r] = (bits >> (8 * (r >> 2) + (r & 3))) & 1u ? s[st][r] : -INFINITY;
                     }
                 }
-                float big = s[0];
+            }
+            float big = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
-                for (int r = 1; r < 16; ++r) {
-                    big = fmaxf(big, s[r]);
+            for (int r = 1; r < 16; ++r) {
+                big = fmaxf(big, fmaxf(s[0][r], s[1][r]));
+            }
+            big = fmaxf(big, pa_xor32(big));
+            const float m_new = fmaxf(m, big);
+            const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
+            const float m_use = m_new == -INFINITY && see == 0u ? 0.0f : m_new;  // (a row that sees nothing yet)
+            m = m_new;
+            float w[32], sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int r = 0; r < 32; ++r) {
+                w[r] = pa_exp(s[r >> 4][r & 15] - m_use) * UNIT;
+                sum[r & 3] += w[r];
+            }
+            lsum = lsum * corr + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
+            const uint8_t *vt = stage + L::K;
+            if (odd) {
+#pragma unroll
+                for (int d = 0; d < DB; ++d) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        out[d][r] *= corr;
+                    }
                 }
-                big = fmaxf(big, pa_xor32(big));
-                const float m_new = fmaxf(m, big);
-                const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
-                const float m_use = m_new == -INFINITY && see == 0u ? 0.0f : m_new;  // (a row that sees nothing yet)
-                float w[16], sum = 0.0f;
+                for (uint32_t i = 0; i < 64u; ++i) {
+                    // position i: register 16 (i / 32) + 4 (i / 8 % 4) + i % 4 of lane half (i / 4) % 2
+                    float mine_w = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 32; ++r) {
+                        mine_w = (uint32_t)r == 4u * (i >> 3) + (i & 3u) ? w[r] : mine_w;
+                    }
+                    const float wi = __shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u)));
+                    if ((see >> i) & 1u) {
+                        const uint32_t chunk = 2u * (i >> 4) + ((i >> 2) & 1u), in = 8u * ((i >> 3) & 1u) + 2u * (i & 3u);
+#pragma unroll
+                        for (int d = 0; d < DB; ++d) {
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) {
+                                const uint32_t dim = 32u * d + 8u * (r >> 2) + 4u * h + (r & 3);
+                                const uint16_t v = *(const uint16_t *)(vt + pa_vt_chunk(dim, chunk) + in);
+                                out[d][r] = __builtin_fmaf(wi, BF16 ? pa_bf2f(v) : h2f(v), out[d][r]);
+                            }
+                        }
+                    }
+                }
+                return;
+            }
+            uint32_t wp[4][PARTS][4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float a = w[8 * i + 2 * e], b = w[8 * i + 2 * e + 1];
+#pragma unroll
+                    for (int part = 0; part < PARTS; ++part) {
+                        if constexpr (BF16) {  // eight bits at a time, cut off: the third part is exact
+                            const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
+                            wp[i][part][e] = __builtin_amdgcn_perm(bb, ab, 0x07060302u);
+                            a -= __uint_as_float(ab & 0xFFFF0000u);
+                            b -= __uint_as_float(bb & 0xFFFF0000u);
+                        } else {
+                            const uint16_t ah = f2h(a), bh = f2h(b);
+                            wp[i][part][e] = (uint32_t)ah | ((uint32_t)bh << 16);
+                            a -= h2f(ah);
+                            b -= h2f(bh);
+                        }
+                    }
+                }
+            }
+            // The tile's products are summed by themselves, small parts first, and join the running output in one rounding
+            // (a third of the error of a chain through the running output, and the rescaling costs nothing)
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+                pa_float16v tile_out = zero;
+                uint4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = *(const uint4 *)(vt + pa_vt_chunk(32u * d + n, 2u * i + h));
+                }
+#pragma unroll
+                for (int part = PARTS - 1; part >= 0; --part) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        tile_out = pa_mma32<BF16>(
+                            v[i], make_uint4(wp[i][part][0], wp[i][part][1], wp[i][part][2], wp[i][part][3]), tile_out);
+                    }
+                }
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    w[r] = pa_exp(s[r] - m_use) * UNIT;
-                    sum += w[r];
-                }
-                lsum = lsum * corr + sum;
-                if (__builtin_amdgcn_ballot_w64(m_new != m) != 0) {
-#pragma unroll
-                    for (int d = 0; d < DB; ++d) {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            out[d][r] *= corr;
-                        }
-                    }
-                }
-                m = m_new;
-                const uint8_t *vt = stage + L::K;
-                if (odd) {
-                    for (uint32_t i = 0; i < 32u; ++i) {
-                        // position i: register 4 (i / 8) + i % 4 of lane half (i / 4) % 2
-                        float mine_w = 0.0f;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            mine_w = (uint32_t)r == 4u * (i >> 3) + (i & 3u) ? w[r] : mine_w;
-                        }
-                        const float wi = __shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u)));
-                        if ((see >> i) & 1u) {
-                            const uint32_t pos = 32u * st + i, chunk = 2u * (pos >> 4) + ((pos >> 2) & 1u);
-                            const uint32_t in = 8u * ((pos >> 3) & 1u) + 2u * (pos & 3u);
-#pragma unroll
-                            for (int d = 0; d < DB; ++d) {
-#pragma unroll
-                                for (int r = 0; r < 16; ++r) {
-                                    const uint32_t dim = 32u * d + 8u * (r >> 2) + 4u * h + (r & 3);
-                                    const uint16_t v = *(const uint16_t *)(vt + pa_vt_chunk(dim, chunk) + in);
-                                    out[d][r] = __builtin_fmaf(wi, BF16 ? pa_bf2f(v) : h2f(v), out[d][r]);
-                                }
-                            }
-                        }
-                    }
-                    continue;
-                }
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    uint32_t wp[PARTS][4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float a = w[8 * i + 2 * e], b = w[8 * i + 2 * e + 1];
-#pragma unroll
-                        for (int part = 0; part < PARTS; ++part) {
-                            if constexpr (BF16) {  // eight bits at a time, cut off: the third part is exact
-                                const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
-                                wp[part][e] = __builtin_amdgcn_perm(bb, ab, 0x07060302u);
-                                a -= __uint_as_float(ab & 0xFFFF0000u);
-                                b -= __uint_as_float(bb & 0xFFFF0000u);
-                            } else {
-                                const uint16_t ah = f2h(a), bh = f2h(b);
-                                wp[part][e] = (uint32_t)ah | ((uint32_t)bh << 16);
-                                a -= h2f(ah);
-                                b -= h2f(bh);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int d = 0; d < DB; ++d) {
-                        const uint4 v = *(const uint4 *)(vt + pa_vt_chunk(32u * d + n, 4u * st + 2u * i + h));
-#pragma unroll
-                        for (int part = PARTS - 1; part >= 0; --part) {
-                            out[d] = pa_mma32<BF16>(v, make_uint4(wp[part][0], wp[part][1], wp[part][2], wp[part][3]), out[d]);
-                        }
-                    }
+                    out[d][r] = __builtin_fmaf(out[d][r], corr, tile_out[r]);
                 }
             }
         };
         // A buffer is written after the barrier that follows its last reading: tile k + 1 is stored beside the reading of
         // tile k, into the buffer that tile k - 1 left before the barrier.
-        request(begin);
+        request(begin, table_entry(begin));
+        uint32_t entry = table_entry(begin + 1u);
         store(count);
         uint64_t mask = mask_next;
         __syncthreads();
         for (uint32_t tile = begin; tile < end; ++tile, ++count) {
             const bool more = tile + 1u < end;
             if (more) {
-                request(tile + 1u);
+                request(tile + 1u, entry);
+                entry = table_entry(tile + 2u);
             }
             consume(tile, count, mask);
             if (more) {
@@ -1874,11 +1904,21 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         size_t sp = (want + pairs - 1) / pairs;
         p.splits = (uint32_t)(sp > 64 ? 64 : sp);
     }
-    // Prompts: k_pa_prompt beside the per-token kernel. Two tokens and more per row of the block table on average (a decode
-    // step has at most one, and would pay for an empty launch), 16-byte key rows, 8-byte value rows.
+    // Prompts: k_pa_prompt beside the kernel per token, from PA_PROMPT_WORK (token, head group, position) triples on, the
+    // positions counted by what the block table has room for, and two tokens and more per row of the table (a decode step
+    // has at most one, and would pay for an empty launch). A call of fewer than PA_MANY tokens gives it the sequences of
+    // PA_LONG positions and more only, and only where the table has room for twice that: a call whose runs go half to one
+    // kernel and half to the other pays for both. 32 / 8 heads of 128, whole call, us per token / tiles: fresh prompts of
+    // 100 tokens 15 / 24, 512 77 / 53, 1024 210 / 82; 64 tokens over 4000 112 / 47; 4 x 8 tokens over 100 15 / 44; eight
+    // heads of 64, 4 x 100 tokens over 500 82 / 57.
+    // 16-byte key rows, 8-byte value rows.
+    const size_t positions = (size_t)p.max_blocks * a->block_size;
+    const bool prompt_size = a->token_count / 2 >= a->max_seqs && pairs * positions >= PA_PROMPT_WORK &&
+                             (a->token_count >= PA_MANY || positions >= 2 * PA_LONG);
     const bool prompt = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || kv_bf16) && rows16 && p.kv_vec &&
-                        (a->head_dim == 64 || a->head_dim == 128) && p.group <= 32 && a->token_count >= 16 &&
-                        a->token_count / 2 >= a->max_seqs && !dev->knobs.no_attention_mfma;
+                        (a->head_dim == 64 || a->head_dim == 128) && p.group <= 32 && !dev->knobs.no_attention_mfma &&
+                        (prompt_size || dev->knobs.attention_prompt_any);
+    p.long_from = a->token_count >= PA_MANY || dev->knobs.attention_prompt_any ? 0u : PA_LONG;
     p.tile_tokens = 0;
     p.out_vec = 0;
     if (prompt) {
@@ -1887,7 +1927,7 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
                     a->out_stride[0] % 4 == 0 && a->out_stride[1] % 4 == 0;
         const size_t tiles = (a->token_count + p.tile_tokens - 1) / p.tile_tokens * a->num_kv_heads;
         const size_t most = (p.max_blocks * a->block_size + PA_PROMPT_SHARE - 1) / PA_PROMPT_SHARE;
-        const size_t sp = (2 * (size_t)dev->props.multiProcessorCount + tiles - 1) / tiles;
+        const size_t sp = (size_t)dev->props.multiProcessorCount / tiles;
         p.splits = (uint32_t)(sp < most ? sp : most);
         p.splits = p.splits < 1u ? 1u : (p.splits > 16u ? 16u : p.splits);
     }

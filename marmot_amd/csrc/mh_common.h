@@ -223,6 +223,7 @@ struct marmot_hip_knobs {
     bool no_row_kernels = false;
     bool no_resident_rows = false;
     bool no_attention_mfma = false;  // MARMOT_HIP_NO_ATTENTION_MFMA: paged attention scores on the vector units
+    bool attention_prompt_any = false;  // MARMOT_HIP_ATTENTION_PROMPT_ANY: the prompt kernel at every size (tests of its edges)
     bool no_fp8_update_fused = false;  // MARMOT_HIP_NO_FP8_UPDATE_FUSED: FLOAT8_E4M3 cache update in four launches
     bool no_lds_ring = false;
     bool no_fused_quant = false;

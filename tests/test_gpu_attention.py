@@ -19,6 +19,18 @@ def hip():
     b.close()
 
 
+@pytest.fixture(scope="module")
+def prompt_hip():
+    """A device object that gives every run of tokens to the kernel for prompts, whatever the size of the call."""
+    from marmot_amd import HipBackend
+
+    with pytest.MonkeyPatch.context() as env:
+        env.setenv("MARMOT_HIP_ATTENTION_PROMPT_ANY", "1")
+        b = HipBackend(0)
+    yield b
+    b.close()
+
+
 def run_hip(hip, case, **kw):
     kv_k, kv_v = case["kv_k"].copy(), case["kv_v"].copy()
     out = hip.paged_attention(case["token_meta"], case["q"], case["k_new"], case["v_new"], kv_k, kv_v,
@@ -152,12 +164,12 @@ def test_prompt_of_many_tokens_takes_unsplit_histories(hip, oracle):
     (4, 1, 8, [(0, 3), (130, 45), (1, 1), (600, 40), (9, 2)], False),  # runs too short for the tile kernel among others
     (8, 2, 32, [(31, 40), (200, 33)], True),    # tokens in any order
 ])
-def test_prompt_tiles(hip, oracle, hq, hkv, block_size, seqs, shuffle, head_dim, act, kv):
+def test_prompt_tiles(prompt_hip, oracle, hq, hkv, block_size, seqs, shuffle, head_dim, act, kv):
     """The kernel that shares key / value rows among the tokens of a tile: NaN rows behind the end of a sequence, a hole
     in the block table, an infinite value that only the later tokens see, split histories, and large queries."""
     case = make_case(700 + hq + head_dim, seqs, num_q_heads=hq, num_kv_heads=hkv, head_dim=head_dim, block_size=block_size,
                      act=act, kv=kv, shuffle_tokens=shuffle)
-    assert len(case["token_meta"]) >= 2 * case["block_table"].shape[0]  # the call takes that kernel
+    hip = prompt_hip
     nan, inf = (np.nan, np.inf) if kv == "f16" else (np.uint16(0x7fc0), np.uint16(0x7f80))
     table, last = case["block_table"], {}
     for seq, pos, _, _ in case["token_meta"]:
@@ -194,6 +206,15 @@ def test_prompt_tiles(hip, oracle, hq, hkv, block_size, seqs, shuffle, head_dim,
     vmax = np.nanmax(np.abs(to_f32(case["v_new"], act))) + np.nanmax(np.abs(to_f32(case["kv_v"], kv)))
     # (the odd tile's sums run in another order)
     assert np.max(np.abs(g[rest].astype(np.float64) - b[rest])) <= TOLERANCE[act] * vmax, "rows beside the infinite value"
+
+
+@pytest.mark.parametrize("seqs", [[(0, 520)], [(1000, 150), (20, 60), (900, 1), (0, 3)]])
+def test_prompt_sizes(hip, oracle, seqs):
+    """By size: a fresh prompt of more than 256 tokens (all of it in tiles), and a call of fewer tokens whose long run goes
+    to tiles while the short sequence, the decode token and the run of three stay on the kernel per token."""
+    case = make_case(790 + len(seqs), seqs, num_q_heads=32, num_kv_heads=8, head_dim=128, block_size=16, act="f32",
+                     kv="bf16", layers=1, layer_idx=0, shuffle_tokens=False)
+    check(hip, oracle, case, "prompt sizes")
 
 
 def test_holes_strided_views_token_count_and_errors(hip, oracle):
