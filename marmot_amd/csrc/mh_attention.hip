@@ -593,10 +593,10 @@ __global__ __launch_bounds__(16 * PA_GROUPS) void k_pa_attend(const PaParams p) 
     const uint32_t qh0 = blockIdx.y * QH;  // first query head of this workgroup; QH divides the heads per kv head
     const int tid = threadIdx.x, g = tid >> 4, l = tid & 15;
     const uint32_t seq = p.meta[t * p.meta_stride[0]];
+    const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
     if (pa_in_run(p, t, seq)) {
         return;
     }
-    const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
     const uint32_t d0 = (uint32_t)l * EPL;  // this lane's first value of the head dimension
@@ -852,10 +852,10 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
     const uint32_t qh0 = blockIdx.y * QH;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, j = lane >> 4;
     const uint32_t seq = p.meta[t * p.meta_stride[0]];
+    const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
     if (pa_in_run(p, t, seq)) {
         return;
     }
-    const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
 
