@@ -170,6 +170,17 @@ __device__ __forceinline__ float pa_exp(float x) {
     return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f);
 }
 
+// A query row is split into FLOAT16 parts after an exact scaling: by the power of two that brings its largest magnitude
+// `most` to 2^14 .. 2^15. Unscaled, values from 65520 on are infinite as FLOAT16, and the second part of a value below
+// 1/8 is subnormal (rms relative error of the split, queries of size 0.09 / 0.01 / 0.001: 2e-7 / 2e-6 / 2e-5). Scaled, the
+// parts leave at most 2^-23 of a value and 2^-40 of the row's largest. (Bounded so that both powers are normal numbers.)
+__device__ __forceinline__ int pa_split_exponent(float most) {
+    int e;
+    (void)frexpf(most, &e);
+    e = 15 - e;
+    return e < -113 ? -113 : (e > 100 ? 100 : e);
+}
+
 // EPL consecutive values starting at element `first` (unit stride, 16-byte aligned start for the storage type)
 template <int EPL>
 __device__ __forceinline__ void pa_load_run(const void *data, int dtype, size_t first, float (&v)[EPL]) {
@@ -1250,9 +1261,9 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 //   * Output: O[dimension][row] += V^T . P with the weights as column operand: registers 8 i .. 8 i + 7 ARE the operand of
 //     instruction i (the k index of lane half h stands for positions 16 i + 4 h + 0..3 and 16 i + 8 + 4 h + 0..3), and the
 //     transposed values are stored in that order, so no weight moves between lanes.
-//   * Precision: query and weights stay fp32 quantities, split into two FLOAT16 parts (rounded to nearest: 2^-23; weights
-//     are scaled by 2^14 first, so that the parts of small ones are normal numbers) or three BFLOAT16 parts (24 bits, exact
-//     for the weights), one instruction per part, fp32 accumulation.
+//   * Precision: query and weights stay fp32 quantities, split into two FLOAT16 parts (rounded to nearest: 2^-23; query rows
+//     are scaled first, see pa_split_exponent, weights by 2^14, so that the parts of small ones are normal numbers) or three
+//     BFLOAT16 parts (24 bits, exact), one instruction per part, fp32 accumulation.
 //   * A value that is not finite would reach rows that may not see it (0 x infinity): a tile that holds one takes the
 //     products of its visible positions one by one.
 // The kernel per token reads a history once per token and head group and uses a quarter of its matrix instructions; this
@@ -1366,26 +1377,29 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         }
         __syncthreads();
     }
-    uint4 qpart[PARTS][QC];
+    float qv[QC][8];
     const size_t q_base = (size_t)t * p.q_stride[0] + (size_t)qh * p.q_stride[1];
 #pragma unroll
     for (int c = 0; c < QC; ++c) {
         const uint32_t d = 16u * c + 8u * h;
-        float qv[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            qv[e] = 0.0f;
+            qv[c][e] = 0.0f;
         }
         if (row_seq != NONE) {
             if (!p.q_vec) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    qv[e] = staged[row * HD + d + e];
+                    qv[c][e] = staged[row * HD + d + e];
                 }
             } else if (p.act_dtype == MARMOT_HIP_DTYPE_F32) {
                 const float4 a = *(const float4 *)((const float *)p.q + q_base + d);
                 const float4 b = *(const float4 *)((const float *)p.q + q_base + d + 4u);
-                qv[0] = a.x, qv[1] = a.y, qv[2] = a.z, qv[3] = a.w, qv[4] = b.x, qv[5] = b.y, qv[6] = b.z, qv[7] = b.w;
+                const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    qv[c][e] = v[e];
+                }
             } else {
                 const uint2 a = *(const uint2 *)((const uint16_t *)p.q + q_base + d);
                 const uint2 b = *(const uint2 *)((const uint16_t *)p.q + q_base + d + 4u);
@@ -1394,19 +1408,43 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const uint16_t bits = (uint16_t)(words[e >> 1] >> (16 * (e & 1)));
-                    qv[e] = half ? h2f(bits) : pa_bf2f(bits);
+                    qv[c][e] = half ? h2f(bits) : pa_bf2f(bits);
                 }
             }
         }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            qv[c][e] = p.scale != 1.0f ? qv[c][e] * p.scale : qv[c][e];
+        }
+    }
+    // FLOAT16 parts: the row times the power of two that brings its largest value to 2^14 .. 2^15; `unit` undoes it on
+    // the scores
+    int up = 0;
+    float unit = 1.0f;
+    if constexpr (!BF16) {
+        float most = 0.0f;
+#pragma unroll
+        for (int c = 0; c < QC; ++c) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                most = fmaxf(most, fabsf(qv[c][e]));
+            }
+        }
+        up = pa_split_exponent(fmaxf(most, pa_xor32(most)));
+        unit = ldexpf(1.0f, -up);
+    }
+    uint4 qpart[PARTS][QC];
+#pragma unroll
+    for (int c = 0; c < QC; ++c) {
         uint32_t w[PARTS][4];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            float v = p.scale != 1.0f ? qv[e] * p.scale : qv[e];
+            float v = BF16 ? qv[c][e] : ldexpf(qv[c][e], up);
 #pragma unroll
             for (int part = 0; part < PARTS; ++part) {  // each remainder is exact in fp32
                 uint32_t bits;
-                if constexpr (BF16) {
-                    bits = pa_f2bf(v);
+                if constexpr (BF16) {  // cut off: rounding up would make infinity of the largest values
+                    bits = __float_as_uint(v) >> 16;
                     v -= pa_bf2f((uint16_t)bits);
                 } else {
                     bits = f2h(v);
@@ -1557,7 +1595,7 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
             for (int r = 1; r < 16; ++r) {
                 big = fmaxf(big, fmaxf(s[0][r], s[1][r]));
             }
-            big = fmaxf(big, pa_xor32(big));
+            big = fmaxf(big, pa_xor32(big)) * unit;
             const float m_new = fmaxf(m, big);
             const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
             const float m_use = m_new == -INFINITY && see == 0u ? 0.0f : m_new;  // (a row that sees nothing yet)
@@ -1565,7 +1603,7 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
             float w[32], sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int r = 0; r < 32; ++r) {
-                w[r] = pa_exp(s[r >> 4][r & 15] - m_use) * UNIT;
+                w[r] = pa_exp(__builtin_fmaf(s[r >> 4][r & 15], unit, -m_use)) * UNIT;
                 sum[r & 3] += w[r];
             }
             lsum = lsum * corr + ((sum[0] + sum[1]) + (sum[2] + sum[3]));

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from marmot_amd import capi
-from tests.attention_cases import NO_BLOCK, TOLERANCE, cache_after_write, dense_reference, make_case, to_f32
+from tests.attention_cases import NO_BLOCK, TOLERANCE, cache_after_write, dense_reference, make_case, to_f32, to_storage
 
 pytestmark = pytest.mark.gpu
 
@@ -206,6 +206,22 @@ def test_prompt_tiles(prompt_hip, oracle, hq, hkv, block_size, seqs, shuffle, he
     vmax = np.nanmax(np.abs(to_f32(case["v_new"], act))) + np.nanmax(np.abs(to_f32(case["kv_v"], kv)))
     # (the odd tile's sums run in another order)
     assert np.max(np.abs(g[rest].astype(np.float64) - b[rest])) <= TOLERANCE[act] * vmax, "rows beside the infinite value"
+
+
+@pytest.mark.parametrize("kv,act", [("f16", "f32"), ("f16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_prompt_tiles_query_magnitudes(prompt_hip, oracle, head_dim, kv, act):
+    """The query is split into parts of the cache's type: one channel far beyond FLOAT16's largest value against keys that
+    bring its products back to size, and rows of tiny queries against large keys, where an error of 2^-25 in a query value
+    would be 3e-4 in the products."""
+    case = make_case(730 + head_dim, [(70, 40), (0, 35)], num_q_heads=8, num_kv_heads=2, head_dim=head_dim, block_size=16,
+                     act=act, kv=kv)
+    for what, gain in (("outlier channel", np.where(np.arange(head_dim) == 5, 2e6, 1.0)), ("tiny", np.full(head_dim, 1e-4))):
+        gain = gain.astype(np.float32)
+        scaled = dict(case, q=to_storage(to_f32(case["q"], act) * gain, act),
+                      k_new=to_storage(to_f32(case["k_new"], act) / gain, act),
+                      kv_k=to_storage(to_f32(case["kv_k"], kv) / gain, kv))
+        check(prompt_hip, oracle, scaled, f"queries, {what}")
 
 
 @pytest.mark.parametrize("seqs", [[(0, 520)], [(1000, 150), (20, 60), (900, 1), (0, 3)]])
