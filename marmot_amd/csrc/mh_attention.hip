@@ -798,8 +798,8 @@ __global__ __launch_bounds__(16 * PA_GROUPS) void k_pa_attend(const PaParams p) 
 //     operand, read from the cache straight into operand registers (lane (r, j) = (lane % 16, lane / 16) reads the 64
 //     contiguous bytes of dimensions 32 j .. 32 j + 31 of position r: the k index of the c-th instruction stands for
 //     dimensions 32 j + 4 c .. + 3, the same in both operands, so no value moves between lanes and none is converted).
-//     The query is the column operand, scaled and split once into a FLOAT16 high part and a FLOAT16 remainder (two
-//     instructions per step: products of FLOAT16 values are exact in fp32, the split leaves 2^-22 of the query); for
+//     The query is the column operand, scaled (see pa_split_exponent) and split once into a FLOAT16 high part and a
+//     FLOAT16 remainder (two instructions per step: products of FLOAT16 values are exact in fp32); for
 //     a BFLOAT16 cache (v_mfma_f32_16x16x16_bf16) into three BFLOAT16 parts of 8 bits each. Columns beyond QH are zero.
 //   * The result layout puts positions 4 j + i (i = 0..3) of head n in lane (n, j): the online softmax of a head runs in
 //     the four lanes n, n + 16, n + 32, n + 48 (two cross-lane exchanges per maximum and per sum).
@@ -870,8 +870,10 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
 
-    // the query: head n (zero beyond QH), dimensions 32 j .. 32 j + 31, scaled, as high part + remainder(s)
+    // the query: head n (zero beyond QH), dimensions 32 j .. 32 j + 31, scaled, as high part + remainder(s); FLOAT16 parts
+    // are those of the row in units of `unit` (see pa_split_exponent)
     constexpr int PARTS = BF16 ? 3 : 2;
+    float unit = 1.0f;
     uint2 qpart[PARTS][8];  // four 16-bit values of the storage type each
     {
         float qv[32];
@@ -899,11 +901,26 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
             }
         }
 #pragma unroll
+        for (int e = 0; e < 32; ++e) {
+            qv[e] = p.scale != 1.0f ? qv[e] * p.scale : qv[e];
+        }
+        int up = 0;
+        if constexpr (!BF16) {
+            float most = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 32; ++e) {
+                most = fmaxf(most, fabsf(qv[e]));
+            }
+            most = fmaxf(most, pa_xor16(most));
+            up = pa_split_exponent(fmaxf(most, pa_xor32(most)));
+            unit = ldexpf(1.0f, -up);
+        }
+#pragma unroll
         for (int c = 0; c < 8; ++c) {
             uint16_t bits[PARTS][4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                float v = p.scale != 1.0f ? qv[4 * c + e] * p.scale : qv[4 * c + e];
+                float v = BF16 ? qv[4 * c + e] : ldexpf(qv[4 * c + e], up);
 #pragma unroll
                 for (int part = 0; part < PARTS; ++part) {  // each remainder is exact in fp32
                     if constexpr (BF16) {
@@ -1102,13 +1119,13 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
             // online softmax of head n over the tile's 16 positions (lanes n, n + 16, n + 32, n + 48)
             float big = fmaxf(fmaxf(s4[0], s4[1]), fmaxf(s4[2], s4[3]));
             big = fmaxf(big, pa_xor16(big));
-            big = fmaxf(big, pa_xor32(big));
+            big = fmaxf(big, pa_xor32(big)) * unit;
             const float m_new = fmaxf(m, big);
             const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
             float w4[4];
     #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                w4[i] = pa_exp(s4[i] - m_new);
+                w4[i] = pa_exp(__builtin_fmaf(s4[i], unit, -m_new));
             }
             float tsum = (w4[0] + w4[1]) + (w4[2] + w4[3]);
             tsum += pa_xor16(tsum);

@@ -210,10 +210,11 @@ def test_prompt_tiles(prompt_hip, oracle, hq, hkv, block_size, seqs, shuffle, he
 
 @pytest.mark.parametrize("kv,act", [("f16", "f32"), ("f16", "bf16"), ("bf16", "f32")])
 @pytest.mark.parametrize("head_dim", [64, 128])
-def test_prompt_tiles_query_magnitudes(prompt_hip, oracle, head_dim, kv, act):
-    """The query is split into parts of the cache's type: one channel far beyond FLOAT16's largest value against keys that
-    bring its products back to size, and rows of tiny queries against large keys, where an error of 2^-25 in a query value
-    would be 3e-4 in the products."""
+@pytest.mark.parametrize("tiles", [True, False])
+def test_query_magnitudes(hip, prompt_hip, oracle, tiles, head_dim, kv, act):
+    """On the matrix cores the query is split into parts of the cache's type: one channel far beyond FLOAT16's largest value
+    against keys that bring its products back to size, and rows of tiny queries against large keys, where an error of
+    2^-25 in a query value would be 3e-4 in the products. In tiles of tokens and one token at a time."""
     case = make_case(730 + head_dim, [(70, 40), (0, 35)], num_q_heads=8, num_kv_heads=2, head_dim=head_dim, block_size=16,
                      act=act, kv=kv)
     for what, gain in (("outlier channel", np.where(np.arange(head_dim) == 5, 2e6, 1.0)), ("tiny", np.full(head_dim, 1e-4))):
@@ -221,7 +222,7 @@ def test_prompt_tiles_query_magnitudes(prompt_hip, oracle, head_dim, kv, act):
         scaled = dict(case, q=to_storage(to_f32(case["q"], act) * gain, act),
                       k_new=to_storage(to_f32(case["k_new"], act) / gain, act),
                       kv_k=to_storage(to_f32(case["kv_k"], kv) / gain, kv))
-        check(prompt_hip, oracle, scaled, f"queries, {what}")
+        check(prompt_hip if tiles else hip, oracle, scaled, f"queries, {what}")
 
 
 @pytest.mark.parametrize("seqs", [[(0, 520)], [(1000, 150), (20, 60), (900, 1), (0, 3)]])
