@@ -383,6 +383,13 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     const uint32_t w_lds = lds_base + (uint32_t)(L::W0 + wave * L::WAVE_W);
     const uint32_t w_first = low4 + w_r * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
     const uint32_t w_last = low4 + last_row * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
+    // Q6_K: the piece that holds the end of the matrix may reach up to 14 bytes behind it (its size need not be a multiple
+    // of 16), and those bytes need not exist. The wavefront of the last row brings the piece before in its place (one
+    // operand more of a minimum that is there anyway) and copies the bytes that exist when the block is read (bring_end).
+    const uint32_t w_end = low4 + (last_row + 1u) * row_bytes;
+    const bool ragged = F::BYTES % 16 != 0 && row0 + 32 >= p.M && (w_end & 15u) != 0;
+    const uint32_t w_most = ragged ? (w_end & ~15u) - 16u : ~0u;
+    const uint32_t end_block = ragged ? (uint32_t)p.nb - 1u : ~0u;
     auto request_weights = [&](uint32_t b, int i) {
         uint32_t at = w_first + (uint32_t)i * (L::ROWS * row_bytes);
         at = at < w_last ? at : w_last;
@@ -392,12 +399,26 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
             const uint32_t last = (at + (uint32_t)F::BYTES - 1u) & ~15u;
             at = (at & ~15u) + w_piece;
             at = at < last ? at : last;
+            at = at < w_most ? at : w_most;
         }
         const uint8_t *base = F::BYTES % 16 != 0 ? wbase : wbase + (size_t)b * F::BYTES;
         // (the launcher checks that rows of whole 16-byte pieces start on 16-byte boundaries)
         // lanes without a row write nothing: the place behind the rows of this load belongs to the next one
         if ((uint32_t)lane < (i + 1 < L::DMA ? L::ROWS : 32 - L::ROWS * (L::DMA - 1)) * F::PIECES) {
             x16_dma(to, base, at);
+        }
+    };
+    // After the loads of block b have arrived: the end of the matrix, two bytes per lane
+    auto bring_end = [&](uint32_t b) {
+        if constexpr (F::BYTES % 16 != 0) {
+            if (b == end_block) {
+                const uint32_t block = low4 + last_row * row_bytes + b * (uint32_t)F::BYTES;
+                const uint32_t from = (w_end & ~15u) + 2u * (uint32_t)lane;
+                if (from < w_end) {
+                    uint8_t *to = lds + L::W0 + wave * L::WAVE_W + last_row * (16 * F::PIECES) + (from - (block & ~15u));
+                    *(uint16_t *)to = *(const uint16_t *)(wbase + from);
+                }
+            }
         }
     };
     const uint32_t my_row = low4 + ((uint32_t)j < last_row ? (uint32_t)j : last_row) * row_bytes;
@@ -524,6 +545,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     store_block(0);
     request_acts(1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    bring_end(0);
     raw.load_head(my_block(0), kh);
     x16_barrier();
     auto walk = [&](auto late_c) {
@@ -620,6 +642,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
                     }
                 }
                 if (hb == 1 && at(24)) {
+                    bring_end(bn);
                     raw.load_head(my_block(bn), kh);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -775,10 +798,10 @@ int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const
 // ------------------------------------------------------------------ grouped (MoE)
 bool gemm_x16_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
                                 const void *w1) {
-    const size_t align = kind == MARMOT_HIP_KIND_Q6_K ? 1 : 15;  // (Q6_K rows are loaded from the boundary below)
+    // (Q6_K rows are loaded from the 16-byte boundary below: the first one must not begin behind it)
     return !dev->knobs.no_gemm_i8 && x16_kind(kind) && K % QK_K == 0 && rows * K < ((size_t)1 << 32) &&
            32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
-           ((((uintptr_t)w0) | ((uintptr_t)w1)) & align) == 0;
+           ((((uintptr_t)w0) | ((uintptr_t)w1)) & 15) == 0;
 }
 
 int launch_gemm_x16_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,

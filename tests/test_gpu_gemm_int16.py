@@ -1,7 +1,9 @@
 """Tiled GEMM of K-quant weights and Q8_K activations with integer fp16 operands (mh_gemm_int16.hip) against the CPU oracle,
 at the edges of its two tile forms and of the rule that chooses one (x16_form, 256 compute units)."""
+import numpy as np
 import pytest
 
+from marmot_amd.capi import DT_F32
 from oracle.pyoracle import KIND_Q4_K, KIND_Q5_K, KIND_Q6_K
 from tests.test_gpu_moe import check_moe_stages
 from tests.util import assert_matmul_parity, gaussian
@@ -54,3 +56,27 @@ def test_moe_experts_on_the_tiled_gemm(hip, oracle, name):
     w = oracle.softmax_rows(vals)
     ref = oracle.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind, threads=16)
     check_moe_stages(hip, oracle, hidden, gate, up, down, ids, w, F, E, kind, ref, f"tiled experts {name}")
+
+
+@pytest.mark.parametrize("N,M,K", [
+    (130, 8225, 256),   # 2 bytes; one block per row: the end arrives with the first block; one row in the last wavefront
+    (130, 8229, 768),   # the matrix ends 14 bytes into a 16-byte piece
+    (193, 6333, 1536),  # 12 bytes; 29 rows in the last wavefront
+    (130, 8232, 256),   # whole 16-byte pieces
+])
+def test_end_of_a_q6_k_matrix(hip, oracle, N, M, K):
+    """210-byte blocks: the last 16-byte piece may hold bytes that are not the matrix's. They are left alone (here NaN scales
+    follow at once), and the bytes in front of them arrive."""
+    blocks = hip.quantize_weights(KIND_Q6_K, gaussian(720 + M, (M, K), 0.02))
+    x = gaussian(721 + M, (N, K))
+    size = blocks.nbytes
+    d_w, d_x, d_out = hip.alloc(size + 64), hip.to_device(x), hip.alloc(4 * N * M)
+    try:
+        d_w.upload(np.concatenate([blocks.reshape(-1), np.full(64, 0xFF, np.uint8)]))
+        hip.linear_d(KIND_Q6_K, d_w, d_x, DT_F32, N, K, M, d_out, DT_F32)
+        assert hip.last_route() == "mmq_q6_k_q8_k_mfma_tile"
+        got = d_out.download(np.float32, (N, M))
+    finally:
+        for b in (d_w, d_x, d_out):
+            b.free()
+    assert_matmul_parity(got, oracle.matmul(KIND_Q6_K, blocks, x, M, threads=16), what=f"q6_k end {N} x {K} x {M}")
