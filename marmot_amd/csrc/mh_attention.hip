@@ -45,35 +45,59 @@ struct PaParams {
     uint32_t *min_off;              // scratch [blocks]: first offset this call writes (block_size = untouched)
     uint32_t *claim;                // scratch [blocks][kv heads]: the token whose workgroup rescales the block (~0 = none yet)
     uint32_t splits;    // workgroups along the history of one (token, heads) pair
-    float *partial;     // splits > 1: [token][query head][split][2 + head_dim]: maximum, sum, unnormalized output
+    float *partial;     // splits > 1: [token][query head][partial_splits][2 + head_dim]: maximum, sum, unnormalized output
+    uint32_t partial_splits;  // the largest split count of the call: every (token, head) pair has room for any kernel
     uint32_t tile_tokens;  // tokens per tile of the prompt kernel (k_pa_prompt), 0 = not launched
-    uint32_t long_from;    // prompt kernel: positions a sequence has at least
+    uint32_t tile_splits;  // prompt kernel: workgroups along a history
+    uint32_t long_from;    // prompt kernel: positions the longest history of the call has at least
+    uint32_t *tiled;       // scratch [token_count]: 1 = the prompt kernel takes the token, 2 = a token in share_splits shares
+    uint32_t share_splits; // workgroups along the history of a token by itself in a call whose runs are in tiles
     int out_vec;           // prompt kernel: FLOAT32 output rows at 16-byte boundaries
 };
 
 // The prompt kernel takes a token when its tile (tile_tokens consecutive tokens of the call) holds at least PA_RUN_MIN
-// tokens of the token's sequence, one of which sees long_from positions or more; the other kernels of the call take the
-// rest. A pass over a history costs the prompt kernel the same for one token as for the whole tile, so the decode tokens
-// of a mixed call stay where every token has workgroups of its own.
+// tokens of the token's sequence, that sequence has long_from / 2 positions or more and some sequence of the call has
+// long_from; the other kernels of the call take the rest. A pass over a history costs the prompt kernel the same for one
+// token as for the whole tile, so the decode tokens of a mixed call stay where every token has workgroups of its own.
+// The lengths are those of the tile's tokens and of 64 probes, tokens spread evenly over the call (its last one among
+// them): what the block table has room for says nothing about a call. The launch that writes the cache finds the answer
+// and leaves it in p.tiled (in the workgroups of the other kernels it cost 12 - 20 us of 256-token calls).
 constexpr uint32_t PA_RUN_MIN = 4;
 
-// Whole wavefront: does the prompt kernel take token t?
-__device__ __forceinline__ bool pa_in_run(const PaParams &p, uint32_t t, uint32_t seq) {
-    if (p.tile_tokens == 0u || seq >= p.max_seqs) {
-        return false;
-    }
-    const uint32_t first = t / p.tile_tokens * p.tile_tokens;
+// positions that token t sees, none behind the table's last block
+__device__ __forceinline__ uint32_t pa_visible(const PaParams &p, uint32_t position) {
+    const uint64_t limit = (uint64_t)p.max_blocks << p.shift;
+    const uint32_t len = position + 1u;
+    return len < limit ? len : (uint32_t)limit;
+}
+__device__ __forceinline__ uint32_t pa_probe(const PaParams &p, uint32_t i) {
+    const uint32_t step = (p.token_count + 63u) / 64u, t = (i + 1u) * step - 1u;
+    return t < p.token_count ? t : p.token_count - 1u;
+}
+
+// Whole wavefront: 1 = the prompt kernel takes token t. 2 = not a run, beside one that it takes, and a long history: the
+// few tokens that are left do not fill the chip, so their histories are split (100 tokens over 4000 positions and 16 decode
+// tokens over 2000: 110 us unsplit). Else 0.
+__device__ __forceinline__ uint32_t pa_in_run(const PaParams &p, uint32_t t, uint32_t seq) {
+    const uint32_t first = t / p.tile_tokens * p.tile_tokens, lane = threadIdx.x & 63u;
+    const size_t probe = (size_t)pa_probe(p, lane) * p.meta_stride[0];
+    const uint32_t probe_seq = p.meta[probe], probe_len = pa_visible(p, p.meta[probe + p.meta_stride[1]]);
+    bool far = probe_seq < p.max_seqs && probe_len >= p.long_from;
+    bool own = probe_seq == seq && probe_len >= p.long_from / 2u;
     uint32_t same = 0;
-    bool any_long = p.long_from == 0u;
     for (uint32_t i = 0; i < p.tile_tokens; i += 64u) {
-        const uint32_t other = first + i + (threadIdx.x & 63u);
-        const bool inside = i + (threadIdx.x & 63u) < p.tile_tokens && other < p.token_count;
+        const uint32_t other = first + i + lane;
+        const bool inside = i + lane < p.tile_tokens && other < p.token_count;
         const size_t at = (size_t)(inside ? other : t) * p.meta_stride[0];
-        const uint32_t s = p.meta[at], len = p.meta[at + p.meta_stride[1]] + 1u;
+        const uint32_t s = p.meta[at], len = pa_visible(p, p.meta[at + p.meta_stride[1]]);
         same += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(inside && s == seq));
-        any_long = any_long || __builtin_amdgcn_ballot_w64(inside && s == seq && len >= p.long_from) != 0;
+        far = far || (s < p.max_seqs && len >= p.long_from);
+        own = own || (s == seq && len >= p.long_from / 2u);
     }
-    return same >= PA_RUN_MIN && any_long;
+    if (seq >= p.max_seqs || __builtin_amdgcn_ballot_w64(far) == 0 || __builtin_amdgcn_ballot_w64(own) == 0) {
+        return 0u;
+    }
+    return same >= PA_RUN_MIN ? 1u : 2u;
 }
 
 // marmot_f32_to_bf16_ref / marmot_bf16_to_f32_ref (src/utils/dtype_ref.c:86-104): round to nearest even on the bits
@@ -261,6 +285,12 @@ __global__ __launch_bounds__(128) void k_pa_write(const PaParams p) {
     const uint32_t t = blockIdx.x, h = blockIdx.y;
     const uint32_t slot = p.meta[t * p.meta_stride[0] + 2 * p.meta_stride[1]];
     const uint32_t block = slot >> p.shift;
+    if (p.tile_tokens != 0u && h == 0 && threadIdx.x < 64u) {
+        const uint32_t tiled = pa_in_run(p, t, p.meta[t * p.meta_stride[0]]);
+        if (threadIdx.x == 0) {
+            p.tiled[t] = tiled;
+        }
+    }
     if (block >= p.kv_blocks) {
         return;
     }
@@ -605,8 +635,13 @@ __global__ __launch_bounds__(16 * PA_GROUPS) void k_pa_attend(const PaParams p) 
     const int tid = threadIdx.x, g = tid >> 4, l = tid & 15;
     const uint32_t seq = p.meta[t * p.meta_stride[0]];
     const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
-    if (pa_in_run(p, t, seq)) {
-        return;
+    uint32_t splits = p.splits;
+    if (p.tile_tokens != 0u) {
+        const uint32_t tiled = __builtin_amdgcn_readfirstlane(p.tiled[t]);  // (the loop over the shares stays scalar)
+        splits = tiled == 2u ? p.share_splits : splits;
+        if (tiled == 1u || blockIdx.z >= splits) {
+            return;
+        }
     }
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
@@ -713,7 +748,7 @@ __global__ __launch_bounds__(16 * PA_GROUPS) void k_pa_attend(const PaParams p) 
         }
     };
     // this workgroup's share of the history (the whole of it without a split)
-    const uint32_t chunk = (kv_len + p.splits - 1u) / p.splits;
+    const uint32_t chunk = (kv_len + splits - 1u) / splits;
     const uint32_t first = blockIdx.z * chunk;
     const uint32_t stop = first + chunk < kv_len ? first + chunk : kv_len;
     for (uint32_t pp = first + (uint32_t)g; pp < stop; pp += 2u * PA_GROUPS) {
@@ -775,8 +810,8 @@ __global__ __launch_bounds__(16 * PA_GROUPS) void k_pa_attend(const PaParams p) 
                 o = __builtin_fmaf(s_acc[gg][h][d], f, o);
             }
         }
-        if (p.splits > 1u) {  // the shares of the history meet in k_pa_merge
-            float *part = p.partial + (((size_t)t * p.num_q_heads + qh0 + h) * p.splits + blockIdx.z) * (p.head_dim + 2u);
+        if (splits > 1u) {  // the shares of the history meet in k_pa_merge
+            float *part = p.partial + (((size_t)t * p.num_q_heads + qh0 + h) * p.partial_splits + blockIdx.z) * (p.head_dim + 2u);
             if (d == 0) {
                 part[0] = big;
                 part[1] = bad ? __uint_as_float(0x7fc00000u) : total;
@@ -864,8 +899,13 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, j = lane >> 4;
     const uint32_t seq = p.meta[t * p.meta_stride[0]];
     const uint32_t pos = p.meta[t * p.meta_stride[0] + p.meta_stride[1]];
-    if (pa_in_run(p, t, seq)) {
-        return;
+    uint32_t splits = p.splits;
+    if (p.tile_tokens != 0u) {
+        const uint32_t tiled = __builtin_amdgcn_readfirstlane(p.tiled[t]);  // (the loop over the shares stays scalar)
+        splits = tiled == 2u ? p.share_splits : splits;
+        if (tiled == 1u || blockIdx.z >= splits) {
+            return;
+        }
     }
     const uint32_t kv_len = seq < p.max_seqs ? pos + 1u : 0u;
     const uint32_t kvh = qh0 / p.group;
@@ -962,7 +1002,7 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
     const uint32_t *table_row = p.table + (size_t)seq * p.table_stride[0];
     // this workgroup's share of the history, in whole tiles of 16 positions
     const uint32_t tiles = (kv_len + 15u) >> 4;
-    const uint32_t tiles_per_split = (tiles + p.splits - 1u) / p.splits;
+    const uint32_t tiles_per_split = (tiles + splits - 1u) / splits;
     const uint32_t tile_first = blockIdx.z * tiles_per_split;
     const uint32_t tile_stop = tile_first + tiles_per_split < tiles ? tile_first + tiles_per_split : tiles;
     // Tiles of this wavefront: tile_first + wave, + 4, ... Two memory latencies lie in front of a tile's arithmetic, the
@@ -1253,8 +1293,8 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
                 o = __builtin_fmaf(s_acc[gg][h][d], f, o);
             }
         }
-        if (p.splits > 1u) {
-            float *part = p.partial + (((size_t)t * p.num_q_heads + qh0 + h) * p.splits + blockIdx.z) * (p.head_dim + 2u);
+        if (splits > 1u) {
+            float *part = p.partial + (((size_t)t * p.num_q_heads + qh0 + h) * p.partial_splits + blockIdx.z) * (p.head_dim + 2u);
             if (d == 0) {
                 part[0] = top;
                 part[1] = bad ? __uint_as_float(0x7fc00000u) : total;
@@ -1295,14 +1335,15 @@ typedef uint32_t pa_uint4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t PA_PROMPT_ROWS = 128;
 constexpr uint32_t PA_PROMPT_SHARE = 256;  // positions a share of a history has at least
-constexpr uint32_t PA_LONG = 512, PA_MANY = 256;
-constexpr size_t PA_PROMPT_WORK = (size_t)3 << 19;
+constexpr uint32_t PA_LONG = 512, PA_MANY = 256, PA_ANY_TABLE = 512;
+constexpr size_t PA_PROMPT_WORK = (size_t)1 << 20;
+constexpr uint32_t PA_SHARES = 4;  // of the history of a token that is left over
 
 template <int HD>
 struct PaPromptLds {
     static constexpr uint32_t KROW = 2 * HD + 16;   // bytes; 16 of padding: rows 4 banks apart
     static constexpr uint32_t K = 64 * KROW, V = HD * 128, STAGE = K + V;
-    static constexpr uint32_t TOKENS = 2 * STAGE;  // sequence, length, longest history: 128 words each; two words
+    static constexpr uint32_t TOKENS = 2 * STAGE;  // sequence, length, longest history: 128 words each; four words
     static constexpr uint32_t BYTES = TOKENS + (3 * PA_PROMPT_ROWS + 4) * 4;
 };
 
@@ -1338,39 +1379,36 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
 
     // the tile's tokens: sequence (NONE: not this kernel's), visible positions, and at the first token of a sequence the
     // largest number of them
+    const bool mine = tid < tt && t0 + tid < p.token_count && p.tiled[t0 + tid] == 1u;
+    static_assert(PA_PROMPT_ROWS == 2 * 64, "tokens of a tile: in the first two wavefronts");
+    const unsigned long long any_mine = __builtin_amdgcn_ballot_w64(mine);
+    if (lane == 0 && wave < 2u) {
+        s_odd[2 + wave] = any_mine != 0 ? 1u : 0u;
+    }
+    __syncthreads();
+    if ((s_odd[2] | s_odd[3]) == 0u) {
+        return;
+    }
     if (tid < PA_PROMPT_ROWS) {
-        uint32_t seq = NONE, len = 0;
-        if (tid < tt && t0 + tid < p.token_count) {
-            seq = p.meta[(size_t)(t0 + tid) * p.meta_stride[0]];
-            len = p.meta[(size_t)(t0 + tid) * p.meta_stride[0] + p.meta_stride[1]] + 1u;
-            const uint64_t limit = (uint64_t)p.max_blocks << p.shift;  // no position behind the table's last block
-            len = len < limit ? len : (uint32_t)limit;
-            seq = seq < p.max_seqs ? seq : NONE;
-        }
-        s_seq[tid] = seq;
-        s_len[tid] = len;
+        const size_t at = (size_t)(t0 + tid) * p.meta_stride[0];
+        s_seq[tid] = mine ? p.meta[at] : NONE;
+        s_len[tid] = mine ? pa_visible(p, p.meta[at + p.meta_stride[1]]) : 0u;
     }
     if (tid < 2) {
         s_odd[tid] = 0;
     }
     __syncthreads();
-    bool mine = false;
     if (tid < PA_PROMPT_ROWS) {
         const uint32_t seq = s_seq[tid];
-        uint32_t same = 0, longest = 0;
+        uint32_t longest = 0;
         bool first = true;
         for (uint32_t i = 0; i < tt; ++i) {
+            const uint32_t len = s_len[i];
             const bool eq = s_seq[i] == seq;
-            same += eq ? 1u : 0u;
             first = first && !(eq && i < tid);
-            longest = eq && s_len[i] > longest ? s_len[i] : longest;
+            longest = eq && len > longest ? len : longest;
         }
-        mine = seq != NONE && same >= PA_RUN_MIN && longest >= p.long_from;  // (no shorter than long_from: the table)
         s_longest[tid] = mine && first ? longest : 0u;
-    }
-    __syncthreads();
-    if (tid < PA_PROMPT_ROWS && !mine) {
-        s_seq[tid] = NONE;
     }
     __syncthreads();
 
@@ -1503,7 +1541,9 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         const uint32_t row_len = row_seq == seq ? full_len : 0u;
         const uint32_t *table_row = p.table + (size_t)seq * p.table_stride[0];
         const uint32_t tiles = (longest + 63u) / 64u;
-        const uint32_t per_share = (tiles + p.splits - 1u) / p.splits;
+        // shares of PA_PROMPT_SHARE positions at least; the others hold nothing
+        const uint32_t most = (longest + PA_PROMPT_SHARE - 1u) / PA_PROMPT_SHARE, shares = p.tile_splits < most ? p.tile_splits : most;
+        const uint32_t per_share = (tiles + shares - 1u) / shares;
         const uint32_t begin = blockIdx.z * per_share;
         const uint32_t end = begin + per_share < tiles ? begin + per_share : tiles;
         if (begin >= end) {
@@ -1729,11 +1769,14 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         return;
     }
     const bool bad = lsum != lsum;
-    if (p.splits > 1u) {
-        float *part = p.partial + (((size_t)t * p.num_q_heads + qh) * p.splits + blockIdx.z) * (HD + 2u);
+    if (p.tile_splits > 1u) {
+        float *part = p.partial + (((size_t)t * p.num_q_heads + qh) * p.partial_splits + blockIdx.z) * (HD + 2u);
         if (h == 0) {
             part[0] = m;
             part[1] = lsum;
+        }
+        if (m == -INFINITY && !bad) {  // a share that holds nothing: k_pa_merge leaves its sums alone
+            return;
         }
 #pragma unroll
         for (int d = 0; d < DB; ++d) {
@@ -1771,31 +1814,44 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
 }
 
 // the shares of a (token, head) pair's history: out = sum_s o_s * exp(M_s - M) / sum_s l_s * exp(M_s - M)
+// (TILES: beside the prompt kernel, whose tokens have a split count of their own; without it the look at p.tiled costs a
+// decode step 0.9 us)
+template <bool TILES>
 __global__ __launch_bounds__(256) void k_pa_merge(const PaParams p) {
     __shared__ float s_big[64], s_tot[64];  // splits <= 64
     const uint32_t t = blockIdx.x, qh = blockIdx.y;
-    const float *part = p.partial + ((size_t)t * p.num_q_heads + qh) * p.splits * (p.head_dim + 2u);
-    if (threadIdx.x < p.splits) {
+    uint32_t splits = p.splits;
+    if constexpr (TILES) {
+        const uint32_t tiled = __builtin_amdgcn_readfirstlane(p.tiled[t]);
+        splits = tiled == 1u ? p.tile_splits : (tiled == 2u ? p.share_splits : splits);
+        if (splits <= 1u) {
+            return;  // the token's own kernel has written its output
+        }
+    }
+    const float *part = p.partial + ((size_t)t * p.num_q_heads + qh) * (TILES ? p.partial_splits : splits) * (p.head_dim + 2u);
+    if (threadIdx.x < splits) {
         s_big[threadIdx.x] = part[(size_t)threadIdx.x * (p.head_dim + 2u)];
         s_tot[threadIdx.x] = part[(size_t)threadIdx.x * (p.head_dim + 2u) + 1];
     }
     __syncthreads();
     float big = -INFINITY;
-    for (uint32_t z = 0; z < p.splits; ++z) {
+    for (uint32_t z = 0; z < splits; ++z) {
         big = fmaxf(big, s_big[z]);
     }
     const size_t out_base = (size_t)t * p.out_stride[0] + (size_t)qh * p.out_stride[1];
     for (uint32_t d = threadIdx.x; d < p.head_dim; d += blockDim.x) {
         float o = 0.0f, total = 0.0f;
         bool bad = false;  // a share saw a NaN score
-        for (uint32_t z = 0; z < p.splits; ++z) {
+        for (uint32_t z = 0; z < splits; ++z) {
             bad = bad || s_tot[z] != s_tot[z];
         }
         if (big != -INFINITY) {
-            for (uint32_t z = 0; z < p.splits; ++z) {
+            for (uint32_t z = 0; z < splits; ++z) {
+                const bool empty = TILES && s_big[z] == -INFINITY;  // (k_pa_prompt leaves the sums of such a share unwritten)
                 const float f = s_big[z] == -INFINITY ? 0.0f : pa_exp(s_big[z] - big);
                 total = __builtin_fmaf(s_tot[z], f, total);
-                o = __builtin_fmaf(part[(size_t)z * (p.head_dim + 2u) + 2 + d], f, o);
+                const float v = part[(size_t)z * (p.head_dim + 2u) + 2 + d];
+                o = empty ? o : __builtin_fmaf(v, f, o);
             }
         }
         o = bad ? __uint_as_float(0x7fc00000u) : (total > 0.0f ? o * (1.0f / total) : 0.0f);
@@ -1805,7 +1861,7 @@ __global__ __launch_bounds__(256) void k_pa_merge(const PaParams p) {
 
 template <int EPL, int QH>
 static void pa_launch(marmot_hip_device *dev, const PaParams &p) {
-    hipLaunchKernelGGL((k_pa_attend<EPL, QH>), dim3(p.token_count, p.num_q_heads / QH, p.splits),
+    hipLaunchKernelGGL((k_pa_attend<EPL, QH>), dim3(p.token_count, p.num_q_heads / QH, p.share_splits),
                        dim3(16 * PA_GROUPS), 0, dev->stream, p);
 }
 
@@ -1813,7 +1869,7 @@ template <int HD, bool BF16>
 static int pa_launch_prompt(marmot_hip_device *dev, const PaParams &p) {
     MH_TRY(allow_large_lds(dev, (const void *)k_pa_prompt<HD, BF16>));
     const unsigned tiles = (p.token_count + p.tile_tokens - 1) / p.tile_tokens;
-    hipLaunchKernelGGL((k_pa_prompt<HD, BF16>), dim3(tiles, p.num_kv_heads, p.splits), dim3(256), PaPromptLds<HD>::BYTES,
+    hipLaunchKernelGGL((k_pa_prompt<HD, BF16>), dim3(tiles, p.num_kv_heads, p.tile_splits), dim3(256), PaPromptLds<HD>::BYTES,
                        dev->stream, p);
     MH_HIP(hipGetLastError());
     return MARMOT_HIP_SUCCESS;
@@ -1933,7 +1989,7 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
                              a->token_count - (uint32_t)host_flag);
         }
     }
-    // workspace: [fp8 scratch][partial results of split histories]
+    // workspace: [fp8 scratch][the tokens in tiles][partial results of split histories]
     const size_t fp8_words = fp8 ? 3 * a->kv_blocks * a->num_kv_heads + a->kv_blocks : 0;
     const size_t fp8_bytes = (fp8_words * sizeof(uint32_t) + 255) & ~(size_t)255;
     // query heads per workgroup: as many heads of one key / value head as the LDS tile of the final merge allows
@@ -1959,45 +2015,55 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         size_t sp = (want + pairs - 1) / pairs;
         p.splits = (uint32_t)(sp > 64 ? 64 : sp);
     }
-    // Prompts: k_pa_prompt beside the kernel per token, from PA_PROMPT_WORK (token, head group, position) triples on, the
-    // positions counted by what the block table has room for, and two tokens and more per row of the table (a decode step
-    // has at most one, and would pay for an empty launch). A call of fewer than PA_MANY tokens gives it the sequences of
-    // PA_LONG positions and more only, and only where the table has room for twice that: a call whose runs go half to one
-    // kernel and half to the other pays for both. 32 / 8 heads of 128, whole call, us per token / tiles: fresh prompts of
-    // 100 tokens 15 / 24, 512 77 / 53, 1024 210 / 82; 64 tokens over 4000 112 / 47; 4 x 8 tokens over 100 15 / 44; eight
-    // heads of 64, 4 x 100 tokens over 500 82 / 57.
-    // 16-byte key rows, 8-byte value rows.
-    const size_t positions = (size_t)p.max_blocks * a->block_size;
-    const bool prompt_size = a->token_count / 2 >= a->max_seqs && pairs * positions >= PA_PROMPT_WORK &&
-                             (a->token_count >= PA_MANY || positions >= 2 * PA_LONG);
+    // Prompts: k_pa_prompt beside the kernel per token. Which tokens it takes is found on the device (pa_in_run): those of
+    // calls with PA_PROMPT_WORK (token, head group, position) triples and more, counted with the longest history; a call of
+    // fewer than PA_MANY tokens needs 2 PA_LONG positions too. 32 / 8 heads of 128, whole call, us per token / tiles: fresh
+    // prompts of 100 tokens 15 / 24, 300 41 / 42, 440 63 / 50, 512 77 / 51, 1024 210 / 78; 64 tokens over 4000 112 / 45;
+    // 4 x 8 tokens over 100 15 / 44; 32 / 8 heads of 64, 4 x 100 tokens over 500 151 / 50. It is launched where that can be:
+    // two tokens and more per row of the block table, or PA_ANY_TABLE tokens (a decode step has one token per row at most
+    // and would pay for an empty launch), and room for such a history in the table. A table with more room than the call
+    // needs costs the empty launch: 100 fresh tokens 15.2 / 18.9, 256 in 32 short runs 34.3 / 39.6, 512 decode tokens over
+    // 100 57.5 / 61.0. 16-byte key rows, 8-byte value rows.
+    const bool any = dev->knobs.attention_prompt_any, many = a->token_count >= PA_MANY;
+    const size_t enough = (PA_PROMPT_WORK + pairs - 1) / pairs, least = many || enough > 2 * PA_LONG ? enough : 2 * PA_LONG;
+    const bool runs = a->token_count / 2 >= a->max_seqs;
+    const bool prompt_size = (runs || a->token_count >= PA_ANY_TABLE) && (size_t)p.max_blocks * a->block_size >= least;
     const bool prompt = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || kv_bf16) && rows16 && p.kv_vec &&
                         (a->head_dim == 64 || a->head_dim == 128) && p.group <= 32 && !dev->knobs.no_attention_mfma &&
-                        (prompt_size || dev->knobs.attention_prompt_any);
-    p.long_from = a->token_count >= PA_MANY || dev->knobs.attention_prompt_any ? 0u : PA_LONG;
+                        (prompt_size || any);
+    p.long_from = any ? 0u : (uint32_t)least;
     p.tile_tokens = 0;
+    p.tile_splits = 1, p.share_splits = p.splits;
     p.out_vec = 0;
     if (prompt) {
         p.tile_tokens = PA_PROMPT_ROWS / p.group;
         p.out_vec = a->act_dtype == MARMOT_HIP_DTYPE_F32 && a->out_stride[2] == 1 && (((uintptr_t)a->d_out) & 15) == 0 &&
                     a->out_stride[0] % 4 == 0 && a->out_stride[1] % 4 == 0;
         const size_t tiles = (a->token_count + p.tile_tokens - 1) / p.tile_tokens * a->num_kv_heads;
-        const size_t most = (p.max_blocks * a->block_size + PA_PROMPT_SHARE - 1) / PA_PROMPT_SHARE;
-        const size_t sp = (size_t)dev->props.multiProcessorCount / tiles;
-        p.splits = (uint32_t)(sp < most ? sp : most);
-        p.splits = p.splits < 1u ? 1u : (p.splits > 16u ? 16u : p.splits);
+        // (what may be a decode step of many sequences is spared the launch that joins two shares: 512 x 100 positions
+        // 57.9 us without tiles, 65.3 with both launches)
+        const size_t cus = (size_t)dev->props.multiProcessorCount, sp = !runs && 2 * tiles >= cus ? 1 : cus / tiles;
+        p.tile_splits = (uint32_t)(sp < 1 ? 1 : (sp > 16 ? 16 : sp));
+        const uint32_t shares = p.tile_splits < PA_SHARES ? p.tile_splits : PA_SHARES;
+        p.share_splits = runs && shares > p.splits ? shares : p.splits;
     }
-    const size_t partial_bytes =
-        p.splits > 1u ? (size_t)a->token_count * a->num_q_heads * p.splits * (a->head_dim + 2u) * sizeof(float) : 0;
-    if (fp8_bytes + partial_bytes != 0) {
+    p.partial_splits = p.share_splits > p.tile_splits ? p.share_splits : p.tile_splits;
+    const size_t partial_bytes = p.partial_splits > 1u ? (size_t)a->token_count * a->num_q_heads * p.partial_splits *
+                                                             (a->head_dim + 2u) * sizeof(float)
+                                                       : 0;
+    const size_t tiled_bytes = prompt ? ((size_t)a->token_count * sizeof(uint32_t) + 255) & ~(size_t)255 : 0;
+    p.tiled = nullptr;
+    if (fp8_bytes + tiled_bytes + partial_bytes != 0) {
         void *ws = nullptr;
-        MH_TRY(workspace_reserve(dev, fp8_bytes + partial_bytes, &ws));
+        MH_TRY(workspace_reserve(dev, fp8_bytes + tiled_bytes + partial_bytes, &ws));
         if (fp8) {
             p.new_kmax = (uint32_t *)ws;
             p.new_vmax = p.new_kmax + a->kv_blocks * a->num_kv_heads;
             p.min_off = p.new_vmax + a->kv_blocks * a->num_kv_heads;
             p.claim = p.min_off + a->kv_blocks;
         }
-        p.partial = p.splits > 1u ? (float *)((uint8_t *)ws + fp8_bytes) : nullptr;
+        p.tiled = prompt ? (uint32_t *)((uint8_t *)ws + fp8_bytes) : nullptr;
+        p.partial = p.partial_splits > 1u ? (float *)((uint8_t *)ws + fp8_bytes + tiled_bytes) : nullptr;
     }
     const dim3 per_token(a->token_count, a->num_kv_heads);
     if (fp8) {
@@ -2025,7 +2091,7 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         }
     }
     if (mfma_scores) {
-        const dim3 grid(p.token_count, p.num_q_heads / (uint32_t)qh, p.splits), block(256);
+        const dim3 grid(p.token_count, p.num_q_heads / (uint32_t)qh, p.share_splits), block(256);
         // FLOAT8_E4M3 decode steps over long contexts (few tokens, a block table of 2048 positions or more): the form
         // whose tile loop is pipelined (16 x 4096 positions 60.7 -> 48.7 us). It needs the registers of a third
         // resident wavefront per SIMD, which short histories and prompts miss more than they gain (FLOAT16, pipeline
@@ -2071,11 +2137,17 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         qh == 2 ? pa_launch<16, 2>(dev, p) : pa_launch<16, 1>(dev, p);
     }
     MH_HIP(hipGetLastError());
-    if (p.splits > 1u) {
-        hipLaunchKernelGGL(k_pa_merge, dim3(a->token_count, a->num_q_heads), dim3(a->head_dim <= 64 ? 64 : 128), 0,
-                           dev->stream, p);
+    if (p.partial_splits > 1u) {
+        const dim3 grid(a->token_count, a->num_q_heads), block(a->head_dim <= 64 ? 64 : 128);
+        if (prompt) {
+            hipLaunchKernelGGL(k_pa_merge<true>, grid, block, 0, dev->stream, p);
+        } else {
+            hipLaunchKernelGGL(k_pa_merge<false>, grid, block, 0, dev->stream, p);
+        }
         MH_HIP(hipGetLastError());
     }
-    set_route(mfma_scores ? "paged_attention_mfma_scores" : "paged_attention");
+    set_route(prompt        ? "paged_attention_tiles"
+              : mfma_scores ? "paged_attention_mfma_scores"
+                            : "paged_attention");
     return MARMOT_HIP_SUCCESS;
 }

@@ -48,12 +48,13 @@ def run_oracle(oracle, case, **kw):
     return out, kv_k, kv_v
 
 
-def check(hip, oracle, case, what):
+def check(hip, oracle, case, what, tiles=False):
     got, kv_k, kv_v = run_hip(hip, case)
     # FLOAT16 caches with rows of 128 values in blocks of 16 positions or more take the kernel whose scores run on the
     # matrix cores (BFLOAT16 caches likewise); everything else the kernel that works on the vector units
     mfma = case["kv"] in ("f16", "bf16") and case["q"].shape[-1] == 128 and case["block_size"] >= 16
-    assert hip.last_route() == ("paged_attention_mfma_scores" if mfma else "paged_attention"), what
+    assert hip.last_route() == ("paged_attention_tiles" if tiles else "paged_attention_mfma_scores" if mfma else
+                                "paged_attention"), what
     ref, ref_k, ref_v = run_oracle(oracle, case)
     assert np.array_equal(kv_k.view(np.uint8), ref_k.view(np.uint8)), f"{what}: key cache"
     assert np.array_equal(kv_v.view(np.uint8), ref_v.view(np.uint8)), f"{what}: value cache"
@@ -63,6 +64,7 @@ def check(hip, oracle, case, what):
     assert np.max(np.abs(g32 - r32)) <= TOLERANCE[act] * vmax, f"{what}: against the oracle"
     dense = dense_reference(case, ref_k, ref_v)
     assert np.max(np.abs(g32 - dense)) <= TOLERANCE[act] * vmax, f"{what}: against dense float64 attention"
+    return got
 
 
 def test_reference_closed_form_case(hip):
@@ -180,13 +182,14 @@ def test_prompt_tiles(prompt_hip, oracle, hq, hkv, block_size, seqs, shuffle, he
             if table[seq, b] != NO_BLOCK and lo < block_size:
                 case["kv_k"][table[seq, b], :, :, lo:, :] = nan
                 case["kv_v"][table[seq, b], :, :, lo:, :] = nan
-    check(hip, oracle, case, "prompt tiles")
+    check(hip, oracle, case, "prompt tiles", tiles=True)
     longest = max(last, key=last.get)
     holed = dict(case, block_table=table.copy())
     holed["block_table"][longest, 1] = NO_BLOCK
-    check(hip, oracle, holed, "prompt tiles, hole")
+    check(hip, oracle, holed, "prompt tiles, hole", tiles=True)
     if act == "f32":
-        check(hip, oracle, dict(case, q=(case["q"] * np.float32(40)).astype(np.float32)), "prompt tiles, large queries")
+        check(hip, oracle, dict(case, q=(case["q"] * np.float32(40)).astype(np.float32)), "prompt tiles, large queries",
+              tiles=True)
     # one infinite value in the row of the longest sequence's token in the middle of its new tokens: tokens before it do
     # not see it, the others' outputs are infinite in that dimension and unchanged in all others
     mine = [i for i, mt in enumerate(case["token_meta"]) if int(mt[0]) == longest]
@@ -222,7 +225,7 @@ def test_query_magnitudes(hip, prompt_hip, oracle, tiles, head_dim, kv, act):
         scaled = dict(case, q=to_storage(to_f32(case["q"], act) * gain, act),
                       k_new=to_storage(to_f32(case["k_new"], act) / gain, act),
                       kv_k=to_storage(to_f32(case["kv_k"], kv) / gain, kv))
-        check(prompt_hip if tiles else hip, oracle, scaled, f"queries, {what}")
+        check(prompt_hip if tiles else hip, oracle, scaled, f"queries, {what}", tiles=tiles)
 
 
 @pytest.mark.parametrize("seqs", [[(0, 520)], [(1000, 150), (20, 60), (900, 1), (0, 3)]])
@@ -231,7 +234,48 @@ def test_prompt_sizes(hip, oracle, seqs):
     to tiles while the short sequence, the decode token and the run of three stay on the kernel per token."""
     case = make_case(790 + len(seqs), seqs, num_q_heads=32, num_kv_heads=8, head_dim=128, block_size=16, act="f32",
                      kv="bf16", layers=1, layer_idx=0, shuffle_tokens=False)
-    check(hip, oracle, case, "prompt sizes")
+    check(hip, oracle, case, "prompt sizes", tiles=True)
+
+
+@pytest.fixture(scope="module")
+def token_hip():
+    """A device object without the matrix-core attention kernels: every token by itself."""
+    from marmot_amd import HipBackend
+
+    with pytest.MonkeyPatch.context() as env:
+        env.setenv("MARMOT_HIP_NO_ATTENTION_MFMA", "1")
+        b = HipBackend(0)
+    yield b
+    b.close()
+
+
+@pytest.mark.parametrize("seqs,tiled", [
+    ([(0, 900)], [True]),                               # a long prompt in a table of many rows
+    ([(30, 8)] * 31 + [(0, 8)], [False] * 32),          # many short runs in a table of long rows
+    ([(0, 100)], [False]),                              # a short prompt in a table of long rows
+    ([(0, 850), (0, 200), (700, 1)], [True, False, True]),  # by the length of each sequence; shares of a decode token's history
+])
+def test_tiles_are_chosen_by_the_call(hip, prompt_hip, token_hip, oracle, seqs, tiled):
+    """Which kernel takes a sequence depends on its tokens and their histories, not on what the block table has room for:
+    with spare rows and columns the outputs have the bits of the kernel that the sequence belongs to. (Rows of 64 values:
+    there the kernel per token is the same with and without matrix cores. 8 / 2 heads: the longest history has to
+    reach 499 at 1051 tokens, a sequence half of it; the decode token is split like beside any other run in tiles.)"""
+    case = make_case(830 + len(seqs), seqs, num_q_heads=8, num_kv_heads=2, head_dim=64, block_size=16, act="f32", kv="f16",
+                     layers=1, layer_idx=0, shuffle_tokens=False)
+    table = case["block_table"]
+    roomy = np.full((600 if len(seqs) == 1 and tiled[0] else table.shape[0], 4096), NO_BLOCK, np.uint32)
+    roomy[:table.shape[0], :table.shape[1]] = table
+    case["block_table"] = roomy
+    launched = sum(n for _, n in seqs) >= 2 * roomy.shape[0]
+    got = check(hip, oracle, case, "roomy table", tiles=launched or tiled[0])
+    in_tiles, per_token = run_hip(prompt_hip, case)[0], run_hip(token_hip, case)[0]
+    at = 0
+    for (_, new), own in zip(seqs, tiled):
+        rows = slice(at, at + new)
+        at += new
+        if new >= 4:
+            assert not np.array_equal(in_tiles[rows], per_token[rows])
+        assert np.array_equal(got[rows], in_tiles[rows] if own else per_token[rows])
 
 
 def test_holes_strided_views_token_count_and_errors(hip, oracle):
