@@ -2028,7 +2028,7 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
     const size_t enough = (PA_PROMPT_WORK + pairs - 1) / pairs, least = many || enough > 2 * PA_LONG ? enough : 2 * PA_LONG;
     const bool runs = a->token_count / 2 >= a->max_seqs;
     const bool prompt_size = (runs || a->token_count >= PA_ANY_TABLE) && (size_t)p.max_blocks * a->block_size >= least;
-    const bool prompt = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || kv_bf16) && rows16 && p.kv_vec &&
+    bool prompt = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || kv_bf16) && rows16 && p.kv_vec &&
                         (a->head_dim == 64 || a->head_dim == 128) && p.group <= 32 && !dev->knobs.no_attention_mfma &&
                         (prompt_size || any);
     p.long_from = any ? 0u : (uint32_t)least;
@@ -2047,11 +2047,20 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
         const uint32_t shares = p.tile_splits < PA_SHARES ? p.tile_splits : PA_SHARES;
         p.share_splits = runs && shares > p.splits ? shares : p.splits;
     }
-    p.partial_splits = p.share_splits > p.tile_splits ? p.share_splits : p.tile_splits;
-    const size_t partial_bytes = p.partial_splits > 1u ? (size_t)a->token_count * a->num_q_heads * p.partial_splits *
-                                                             (a->head_dim + 2u) * sizeof(float)
-                                                       : 0;
-    const size_t tiled_bytes = prompt ? ((size_t)a->token_count * sizeof(uint32_t) + 255) & ~(size_t)255 : 0;
+    size_t tiled_bytes = 0, partial_bytes = 0;
+    auto scratch = [&]() {
+        p.partial_splits = p.share_splits > p.tile_splits ? p.share_splits : p.tile_splits;
+        tiled_bytes = prompt ? ((size_t)a->token_count * sizeof(uint32_t) + 255) & ~(size_t)255 : 0;
+        partial_bytes = p.partial_splits > 1u ? (size_t)a->token_count * a->num_q_heads * p.partial_splits *
+                                                    (a->head_dim + 2u) * sizeof(float)
+                                              : 0;
+        return fp8_bytes + tiled_bytes + partial_bytes;
+    };
+    if (scratch() > workspace_room(dev) && prompt) {  // captured without an eager run before: the kernel per token needs less
+        prompt = false;
+        p.tile_tokens = 0, p.tile_splits = 1, p.share_splits = p.splits;
+        (void)scratch();
+    }
     p.tiled = nullptr;
     if (fp8_bytes + tiled_bytes + partial_bytes != 0) {
         void *ws = nullptr;

@@ -393,6 +393,8 @@ int allow_large_lds(marmot_hip_device *dev, const void *kernel);
 
 // Returns a workspace of at least `bytes` (256-byte aligned). Growing it synchronizes the stream first.
 int workspace_reserve(marmot_hip_device *dev, size_t bytes, void **out);
+// Bytes that workspace_reserve grants without an error: all there are, unless it must not allocate
+size_t workspace_room(const marmot_hip_device *dev);
 
 // Carves the activation scratch for `rows` x `k` out of `base`; returns bytes consumed (256-byte rounded).
 size_t act_scratch_layout(int act_kind, size_t rows, size_t k, void *base, ActScratch *out);

@@ -34,6 +34,10 @@ int check_hip(hipError_t e, const char *what) {
     return set_error(code, "HIP error %d (%s) in %s", (int)e, hipGetErrorString(e), what);
 }
 
+size_t workspace_room(const marmot_hip_device *dev) {
+    return dev->use_static_scratch ? dev->static_scratch_bytes : (dev->capturing ? dev->workspace_bytes : ~(size_t)0);
+}
+
 int workspace_reserve(marmot_hip_device *dev, size_t bytes, void **out) {
     if (dev->use_static_scratch) {
         if (bytes > dev->static_scratch_bytes) {

@@ -278,6 +278,36 @@ def test_tiles_are_chosen_by_the_call(hip, prompt_hip, token_hip, oracle, seqs, 
         assert np.array_equal(got[rows], in_tiles[rows] if own else per_token[rows])
 
 
+def test_prompt_captured_without_an_eager_run(oracle):
+    """A prompt whose histories need no split fits no workspace: a fresh device object captures it (on the kernel per token,
+    whose results need no scratch memory), and an eager call on the same object takes the tiles."""
+    from marmot_amd import HipBackend
+
+    case = make_case(840, [(0, 600)], num_q_heads=32, num_kv_heads=8, head_dim=128, block_size=16, act="f32", kv="f16",
+                     layers=1, layer_idx=0)
+    names = ("token_meta", "q", "k_new", "v_new", "kv_k", "kv_v", "block_table")
+    hip = HipBackend(0)
+    out = np.zeros_like(case["q"])
+    bufs = {id(a): hip.to_device(a.reshape(-1).view(np.uint8)) for a in [case[n] for n in names] + [out]}
+    try:
+        p = hip.paged_attention_args(lambda a: bufs[id(a)].ptr, *(case[n] for n in names), out, 0, case["scale"])
+        graph = hip.graph_capture(lambda: capi.check(hip.lib.marmot_hip_paged_attention(hip.dev, p, 0)))
+        assert hip.last_route() == "paged_attention_mfma_scores"
+        ref, _, _ = run_oracle(oracle, case)
+        for _ in range(2):
+            hip.graph_launch(graph)
+            hip.synchronize()
+            got = bufs[id(out)].download(np.float32, out.shape)
+            assert np.max(np.abs(got.astype(np.float64) - ref)) <= TOLERANCE["f32"] * np.abs(case["v_new"]).max()
+            capi.check(hip.lib.marmot_hip_paged_attention(hip.dev, p, 0))
+            assert hip.last_route() == "paged_attention_tiles"
+        hip.graph_destroy(graph)
+    finally:
+        for b in bufs.values():
+            b.free()
+        hip.close()
+
+
 def test_holes_strided_views_token_count_and_errors(hip, oracle):
     case = make_case(13, [(40, 3), (5, 1)], num_q_heads=4, num_kv_heads=2, head_dim=32, block_size=8)
     seq = case["token_meta"][0, 0]
