@@ -44,7 +44,7 @@ def test_mirror_header_matches_reference_layout(tmp_path, golden_layout):
     assert len(mine) > 150
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="reference tree not present")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "include")), reason="reference tree not present")
 def test_layout_fixture_is_current(golden_layout):
     import importlib.util
     spec = importlib.util.spec_from_file_location("make_abi_layout", os.path.join(GOLDEN, "make_abi_layout.py"))
