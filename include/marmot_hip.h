@@ -507,8 +507,8 @@ int marmot_hip_softmax_rows(marmot_hip_device_t *dev, const float *d_x, size_t r
  *   d_down: E slices of [H rows, F] blocks of kind_down; d_topk_ids int32 [T,k]; d_topk_weights fp32 [T,k];
  *   d_out [T,H] fp32 (fully overwritten).
  * An expert id out of range returns MARMOT_HIP_ERROR_INVALID_ARGUMENT: the call waits for the kernel that sorts the routes
- * (not for the experts: d_out is complete in stream order, like every output). No wait and no check while a graph is being
- * captured. */
+ * (not for the experts: d_out is complete in stream order, like every output; with the error it has waited for the experts
+ * too, and the buffers are the caller's again). No wait and no check while a graph is being captured. */
 int marmot_hip_moe_experts(marmot_hip_device_t *dev, const float *d_hidden, size_t T, size_t H, size_t F, size_t E,
                            size_t k_per_token, int kind_gate_up, int kind_down, const void *d_gate, const void *d_up,
                            const void *d_down, const int32_t *d_topk_ids, const float *d_topk_weights,

@@ -679,6 +679,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     if (validate) {
         MH_HIP(hipEventSynchronize(dev->host_word_event));
         if (*(volatile int *)dev->host_word != 0) {
+            // the caller takes the call for refused: its buffers are its own again
+            MH_HIP(hipStreamSynchronize(dev->stream));
             return set_error(MARMOT_HIP_ERROR_INVALID_ARGUMENT, "MoE expert id is out of range");
         }
     }

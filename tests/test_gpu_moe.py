@@ -211,6 +211,32 @@ def check_moe_stages(hip, oracle, hidden, gate, up, down, ids, w, F, E, kind, re
             "down_combine": m_down}
 
 
+def test_moe_bad_expert_id_leaves_no_work_behind(hip):
+    """With the error the buffers are the caller's again: nothing of the call is still running."""
+    import ctypes as C
+
+    from marmot_amd import MarmotHipError
+
+    E, F, H, k, T = 8, 1024, 1024, 8, 2048
+    gate, up, down = (hip.to_device(hip.quantize_weights(KIND_Q4_K, gaussian(900 + i, shape, 0.02)))
+                      for i, shape in enumerate(((E * F, H), (E * F, H), (E * H, F))))
+    ids = np.tile(np.arange(k, dtype=np.int32), (T, 1))
+    ids[T // 2, 3] = E
+    d_x, d_ids = hip.to_device(gaussian(903, (T, H))), hip.to_device(ids)
+    d_w, d_out = hip.to_device(np.full((T, k), 1.0 / k, np.float32)), hip.alloc(4 * T * H)
+    query = hip.lib.hipStreamQuery  # (the runtime that the library is linked with)
+    query.argtypes, query.restype = [C.c_void_p], C.c_int
+    try:
+        for _ in range(3):
+            with pytest.raises(MarmotHipError) as e:
+                hip.moe_experts_d(d_x, T, H, F, E, k, KIND_Q4_K, KIND_Q4_K, gate, up, down, d_ids, d_w, d_out)
+            assert query(hip.lib.marmot_hip_stream(hip.dev)) == 0, "work of the refused call is still running"
+            assert e.value.code == -1
+    finally:
+        for b in (gate, up, down, d_x, d_ids, d_w, d_out):
+            b.free()
+
+
 def test_moe_stages_small(hip, oracle):
     """The stage-wise comparison on a small layer, grouped and decode-order routing."""
     E, F, H, k = 6, 512, 512, 3
