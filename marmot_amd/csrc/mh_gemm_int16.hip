@@ -5,8 +5,9 @@
 // vec_dot_impl.h:689-860) y += a.d * (w.d * isum - w.dmin * msum) with isum = sum_j sc_j * (q_j . a_j) and msum = sum_j mn_j *
 // (sum of a over sub-block j). Here the sub-block scale goes into the weight operand: sc * q is at most 63 * 15 = 945 (Q4_K)
 // or 63 * 31 = 1953 (Q5_K), below 2048, so it is exact in fp16, and the activation codes (-127 .. 127) are too: ONE chain of
-// v_mfma_f32_32x32x16_f16 per block gives isum in fp32 (exact below 2^24, where the reference's own conversion of isum to
-// float starts to round), and one more instruction on the stored sums of 16 codes (at most 2032, exact) and the mins gives
+// v_mfma_f32_32x32x16_f16 per block gives isum in fp32 (exact below 2^24; from there on, up to 2^24.9 for Q4_K, 2^25.9 for
+// Q5_K and 2^27 for Q6_K, where the reference rounds isum once, every instruction of the chain may round: at most 16 (Q6_K 32) units
+// in the last place), and one more instruction on the stored sums of 16 codes (at most 2032, exact) and the mins gives
 // msum. Q6_K: sc * q reaches 127 * 32 = 4064, so q = 8 * qh + ql (qh = -4 .. 3, ql = 0 .. 7) and both sc * ql and
 // 8 * sc * qh (in units of a quarter) are exact: two operands on one accumulator. fp32 work per output and block: three
 // multiply(-add)s, two for Q6_K.
@@ -33,7 +34,7 @@
 //                    1000 x 4096 x 14336   1024 x 14336 x 4096   2048 x 4096 x 4096   512 x 4096 x 4096
 //   Q4_K before / now    186 / 155             174 / -               107 / 85             30 / -
 //   Q5_K before / now    237 / 173             223 / 190             135 / 93             36 / -
-//   Q6_K before / now    428 / 290             414 / 288             246 / 170            63 / 59
+//   Q6_K before / now    428 / 290             414 / 315             246 / 170            63 / 59
 // 155 us are 760 TOP/s. What is left: waits for LDS operands (a step reads its A operand three steps ahead, all the
 // registers allow at C = 4) and the conversion of the activations, which every row tile repeats.
 #include "mh_rows.h"
@@ -750,10 +751,12 @@ template <int KIND>
 static int x16_launch_kind(marmot_hip_device *dev, const GemmX16Params &p, unsigned weights) {
     if constexpr (KIND != MARMOT_HIP_KIND_Q6_K) {
         if (x16_form(dev, KIND, p.N, p.M, weights) == 4) {
+            set_route(KIND == MARMOT_HIP_KIND_Q4_K ? "mmq_q4_k_q8_k_fp16_tile_256x128" : "mmq_q5_k_q8_k_fp16_tile_256x128");
             return x16_launch<KIND, 4, 8>(dev, p, (unsigned)((p.N + 127) / 128), weights);
         }
     }
     if constexpr (KIND != MARMOT_HIP_KIND_Q4_K) {
+        set_route(KIND == MARMOT_HIP_KIND_Q5_K ? "mmq_q5_k_q8_k_fp16_tile_128x64" : "mmq_q6_k_q8_k_fp16_tile_128x64");
         return x16_launch<KIND, 2, 4>(dev, p, (unsigned)((p.N + 63) / 64), weights);
     }
     return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "fp16-operand GEMM: no form for this shape");
@@ -780,19 +783,12 @@ int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const
     const unsigned weights = (unsigned)ws.count;
     switch (kind) {
     case MARMOT_HIP_KIND_Q4_K:
-        MH_TRY(x16_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights));
-        set_route("mmq_q4_k_q8_k_mfma_tile");
-        break;
+        return x16_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights);
     case MARMOT_HIP_KIND_Q5_K:
-        MH_TRY(x16_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights));
-        set_route("mmq_q5_k_q8_k_mfma_tile");
-        break;
+        return x16_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights);
     default:
-        MH_TRY(x16_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights));
-        set_route("mmq_q6_k_q8_k_mfma_tile");
-        break;
+        return x16_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights);
     }
-    return MARMOT_HIP_SUCCESS;
 }
 
 // ------------------------------------------------------------------ grouped (MoE)

@@ -619,7 +619,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     }
     const size_t gu_stride = F * ((H + bv_gu - 1) / bv_gu) * block_bytes(kind_gate_up);
     const size_t dn_stride = H * ((F + bv_dn - 1) / bv_dn) * block_bytes(kind_down);
-    // Q4_K / Q6_K experts run on the int8 matrix cores, the 32-value formats on the dot-product matvec
+    // K-quant experts run on the matrix cores (long prompts on the tiled GEMM with integer fp16 operands, else passes on
+    // int8), the 32-value formats on the dot-product matvec
     st = tiled  ? launch_gemm_x16_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
                                           max_items, H, F, gate_out, up_out)
         : mmq_gu ? launch_mmq_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
@@ -674,7 +675,7 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
                            route_pos, (int)k_per_token, H, d_out);
     }
     MH_HIP(hipGetLastError());
-    set_route("moe_experts_grouped");
+    set_route(tiled ? "moe_experts_tiled" : "moe_experts_grouped");
 
     if (validate) {
         MH_HIP(hipEventSynchronize(dev->host_word_event));
