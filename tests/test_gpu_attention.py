@@ -158,7 +158,7 @@ def test_prompt_of_many_tokens_takes_unsplit_histories(hip, oracle):
 
 
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
-@pytest.mark.parametrize("head_dim,act", [(64, "f16"), (128, "f32")])
+@pytest.mark.parametrize("head_dim,act", [(64, "f16"), (128, "f32"), (128, "bf16")])
 @pytest.mark.parametrize("hq,hkv,block_size,seqs,shuffle", [
     (8, 2, 16, [(0, 70)], False),               # group 4: a full tile of 32 tokens, a full and a ragged last one
     (3, 3, 16, [(63, 66), (64, 63)], False),    # group 1: 128 tokens per tile, two sequences in it, tile edges at 64
@@ -196,7 +196,7 @@ def test_prompt_tiles(prompt_hip, oracle, hq, hkv, block_size, seqs, shuffle, he
     mine.sort(key=lambda i: int(case["token_meta"][i, 1]))
     at = mine[len(mine) // 2]
     odd = dict(case, v_new=case["v_new"].copy())
-    odd["v_new"][at, :, 3] = np.inf if act != "bf16" else inf
+    odd["v_new"][at, :, 3] = np.inf if act != "bf16" else np.uint16(0x7f80)
     base, _, _ = run_hip(hip, case)
     got, _, _ = run_hip(hip, odd)
     b, g = to_f32(base, act), to_f32(got, act)
@@ -276,6 +276,36 @@ def test_tiles_are_chosen_by_the_call(hip, prompt_hip, token_hip, oracle, seqs, 
         if new >= 4:
             assert not np.array_equal(in_tiles[rows], per_token[rows])
         assert np.array_equal(got[rows], in_tiles[rows] if own else per_token[rows])
+
+
+@pytest.mark.parametrize("hq,hkv,head_dim,act,kv", [(14, 2, 64, "f32", "f16"), (14, 2, 128, "f16", "bf16"),
+                                                    (8, 2, 128, "bf16", "bf16"), (8, 2, 64, "f32", "bf16")])
+def test_prompt_tiles_strided_views(prompt_hip, hq, hkv, head_dim, act, kv):
+    """Queries that are not contiguous pass through LDS, and output rows off 16-byte boundaries are stored value by value:
+    the same bits as from dense tensors. Split histories; groups of 7 leave rows of a tile idle."""
+    case = make_case(850 + hq + head_dim, [(300, 60), (0, 40)], num_q_heads=hq, num_kv_heads=hkv, head_dim=head_dim,
+                     block_size=16, act=act, kv=kv)
+    plain, _, _ = run_hip(prompt_hip, case)
+    wide = np.zeros(case["q"].shape[:2] + (2 * head_dim,), case["q"].dtype)
+    wide[..., ::2] = case["q"]
+    view, _, _ = run_hip(prompt_hip, dict(case, q=wide[..., ::2]))
+    assert prompt_hip.last_route() == "paged_attention_tiles"
+    assert np.array_equal(view.view(np.uint8), plain.view(np.uint8)), "queries"
+    room = np.zeros(case["q"].shape[:2] + (head_dim + 1,), case["q"].dtype)
+    names = ("token_meta", "q", "k_new", "v_new", "kv_k", "kv_v", "block_table")
+    bufs = {id(a): prompt_hip.to_device(a.reshape(-1).view(np.uint8)) for a in [case[n] for n in names] + [room]}
+    try:
+        def dev_ptr(a):
+            return bufs[id(a)].ptr if id(a) in bufs else bufs[id(room)].ptr + room.itemsize
+        p = prompt_hip.paged_attention_args(dev_ptr, *(case[n] for n in names), room[..., 1:], case["layer_idx"], case["scale"],
+                                            act == "bf16", kv == "bf16")
+        capi.check(prompt_hip.lib.marmot_hip_paged_attention(prompt_hip.dev, p, 0))
+        got = bufs[id(room)].download(room.dtype, room.shape)
+    finally:
+        for b in bufs.values():
+            b.free()
+    assert np.array_equal(np.ascontiguousarray(got[..., 1:]).view(np.uint8), plain.view(np.uint8)), "output"
+    assert not got[..., 0].any(), "values beside the rows"
 
 
 def test_prompt_captured_without_an_eager_run(oracle):
