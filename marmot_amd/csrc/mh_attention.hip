@@ -1336,7 +1336,7 @@ typedef uint32_t pa_uint4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t PA_PROMPT_ROWS = 128;
 constexpr uint32_t PA_PROMPT_SHARE = 256;  // positions a share of a history has at least
 constexpr uint32_t PA_LONG = 512, PA_MANY = 256, PA_ANY_TABLE = 512;
-constexpr size_t PA_PROMPT_WORK = (size_t)1 << 20;
+constexpr size_t PA_PROMPT_WORK = (size_t)3 << 19;
 constexpr uint32_t PA_SHARES = 4;  // of the history of a token that is left over
 
 template <int HD>
@@ -2031,7 +2031,8 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
     bool prompt = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || kv_bf16) && rows16 && p.kv_vec &&
                         (a->head_dim == 64 || a->head_dim == 128) && p.group <= 32 && !dev->knobs.no_attention_mfma &&
                         (prompt_size || any);
-    p.long_from = any ? 0u : (uint32_t)least;
+    // (a history counts in whole blocks, like the room for it)
+    p.long_from = any ? 0u : (uint32_t)(least > p.mask ? least - p.mask : 1u);
     p.tile_tokens = 0;
     p.tile_splits = 1, p.share_splits = p.splits;
     p.out_vec = 0;

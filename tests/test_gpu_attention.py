@@ -259,7 +259,7 @@ def test_tiles_are_chosen_by_the_call(hip, prompt_hip, token_hip, oracle, seqs, 
     """Which kernel takes a sequence depends on its tokens and their histories, not on what the block table has room for:
     with spare rows and columns the outputs have the bits of the kernel that the sequence belongs to. (Rows of 64 values:
     there the kernel per token is the same with and without matrix cores. 8 / 2 heads: the longest history has to
-    reach 499 at 1051 tokens, a sequence half of it; the decode token is split like beside any other run in tiles.)"""
+    reach 734 at 1051 tokens, a sequence half of it; the decode token is split like beside any other run in tiles.)"""
     case = make_case(830 + len(seqs), seqs, num_q_heads=8, num_kv_heads=2, head_dim=64, block_size=16, act="f32", kv="f16",
                      layers=1, layer_idx=0, shuffle_tokens=False)
     table = case["block_table"]
