@@ -32,11 +32,13 @@
 //                    independent, so one computes while another waits.
 // Measured (us; before = k_gemm_q{4,5,6}k_q8k_tile of mh_gemm_i8.hip; tokens x K x M):
 //                    1000 x 4096 x 14336   1024 x 14336 x 4096   2048 x 4096 x 4096   512 x 4096 x 4096
-//   Q4_K before / now    186 / 155             174 / -               107 / 85             30 / -
-//   Q5_K before / now    237 / 173             223 / 190             135 / 93             36 / -
-//   Q6_K before / now    428 / 290             414 / 315             246 / 170            63 / 59
-// 155 us are 760 TOP/s. What is left: waits for LDS operands (a step reads its A operand three steps ahead, all the
-// registers allow at C = 4) and the conversion of the activations, which every row tile repeats.
+//   Q4_K before / now    186 / 145             174 / -               107 / 85             30 / -
+//   Q5_K before / now    237 / 160             223 / 190             135 / 93             36 / -
+//   Q6_K before / now    428 / 290             414 / 310             246 / 170            63 / 59
+// 145 us are 810 TOP/s. (At 155 the activation loads were flat loads, which count as LDS accesses too: an operand read
+// then waited for memory.) Of the 145, the matrix instructions alone take about 75 at the clock the chip holds under
+// them (1.7 - 1.9 GHz), the stores of the 57 MB of output 12, waits for the weights 12; what is left is unpacking and
+// the conversion of the activations, which every row tile repeats.
 #include "mh_rows.h"
 
 #include <type_traits>
@@ -46,6 +48,8 @@ namespace mh {
 typedef _Float16 x_half2 __attribute__((ext_vector_type(2)));
 typedef _Float16 x_half8 __attribute__((ext_vector_type(8)));
 typedef float x_float16 __attribute__((ext_vector_type(16)));
+typedef uint32_t x_u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) x_u32x4 glb_u32x4_t;
 
 struct GemmX16Params {
     const uint8_t *w[3];   // weights: M rows of nb blocks each
@@ -392,7 +396,11 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     const uint32_t w_most = ragged ? (w_end & ~15u) - 16u : ~0u;
     const uint32_t end_block = ragged ? (uint32_t)p.nb - 1u : ~0u;
     auto request_weights = [&](uint32_t b, int i) {
-        uint32_t at = w_first + (uint32_t)i * (L::ROWS * row_bytes);
+        uint32_t at = w_first;
+        if (C == 4) {  // formed at each load: kept in registers, the L::DMA offsets would be spilled
+            asm volatile("" : "+v"(at));
+        }
+        at += (uint32_t)i * (L::ROWS * row_bytes);
         at = at < w_last ? at : w_last;
         const uint32_t to = w_lds + (uint32_t)(i * L::ROWS * 16 * F::PIECES);
         if constexpr (F::BYTES % 16 != 0) {
@@ -417,7 +425,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
                 const uint32_t from = (w_end & ~15u) + 2u * (uint32_t)lane;
                 if (from < w_end) {
                     uint8_t *to = lds + L::W0 + wave * L::WAVE_W + last_row * (16 * F::PIECES) + (from - (block & ~15u));
-                    *(uint16_t *)to = *(const uint16_t *)(wbase + from);
+                    *(uint16_t *)to = *(const __attribute__((address_space(1))) uint16_t *)(wbase + from);
                 }
             }
         }
@@ -425,26 +433,28 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     const uint32_t my_row = low4 + ((uint32_t)j < last_row ? (uint32_t)j : last_row) * row_bytes;
     const uint8_t *my_w = lds + L::W0 + wave * L::WAVE_W + j * (16 * F::PIECES);
 
-    uint4 a_next[APT];
-    uint4 s_next;
+    x_u32x4 a_next[APT];
+    x_u32x4 s_next;
     float d_next = 0.0f;
     auto request_acts = [&](uint32_t stage) {
-        const int8_t *base = p.qs + (size_t)stage * 128u;
-        asm("" : "+s"(base));  // stays a scalar base + 32-bit lane offsets, not a 64-bit address per lane and load
+        // The asm keeps a scalar base + 32-bit lane offsets, not a 64-bit address per lane and load; the pointer says that
+        // it is global memory, since a flat load also counts as an LDS access and every operand read then waits for it.
+        glb_u8_t *base = (glb_u8_t *)p.qs + (size_t)stage * 128u;
+        asm("" : "+s"(base));
 #pragma unroll
         for (int i = 0; i < APT; ++i) {
-            a_next[i] = *(const uint4 *)(base + (size_t)a_row[i]);
+            a_next[i] = *(const glb_u32x4_t *)(base + (size_t)a_row[i]);
         }
     };
     auto request_block = [&](uint32_t b) {
         if constexpr (F::MIN) {
-            const uint8_t *sums = (const uint8_t *)p.sums + (size_t)b * 32u;
+            glb_u8_t *sums = (glb_u8_t *)p.sums + (size_t)b * 32u;
             asm("" : "+s"(sums));
-            s_next = *(const uint4 *)(sums + (size_t)s_off);
+            s_next = *(const glb_u32x4_t *)(sums + (size_t)s_off);
         }
-        const uint8_t *ad = (const uint8_t *)p.ad + (size_t)b * 4u;
+        glb_u8_t *ad = (glb_u8_t *)p.ad + (size_t)b * 4u;
         asm("" : "+s"(ad));
-        d_next = *(const float *)(ad + (size_t)d_off);
+        d_next = *(const __attribute__((address_space(1))) float *)(ad + (size_t)d_off);
     };
     auto store_acts = [&](int buffer, int i) {
         uint8_t *stage = lds + buffer * L::ACT;
@@ -487,7 +497,9 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     // A operand of (g, kh, i): chunk 4 g + 2 kh + i of token 32 t + j. One address register: the others differ from it in
     // bits 4 .. 7 and are formed where they are used (kept out of registers by the volatile asm).
     const uint32_t a_at = lds_base + (uint32_t)(j * 256 + 16 * ((2 * kh) ^ (j & 15)));
-    auto my_block = [&](uint32_t b) { return my_w + ((my_row + b * (uint32_t)F::BYTES) & 15u); };
+    auto my_block = [&](uint32_t b) {  // (blocks of whole pieces start at the beginning of their place)
+        return F::BYTES % 16 != 0 ? my_w + ((my_row + b * (uint32_t)F::BYTES) & 15u) : my_w;
+    };
 
     // fp32 step of a block, token tile t: y += a.d * (w.d * isum - w.dmin * msum)
     x_float16 P[C];
@@ -555,18 +567,20 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
         const uint32_t bn = b + 1 < nb ? b + 1 : b;  // (the last block is requested again rather than branched around)
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
-            // Steps (g, t, i): one matrix instruction per plane each. The A operand of a step is read AHEAD steps before
-            // it, the weight operands of group g + 1 are unpacked, a quarter at a time, between the steps of group g.
-            constexpr int STEPS = 8 * C, AHEAD = 3;
+            // Steps (g, i, t): one matrix instruction per plane each, consecutive ones on different accumulators. The A operand
+            // of a step is read AHEAD steps before it, the weight operands of group g + 1 are unpacked, a quarter at a time,
+            // between the steps of group g. AHEAD is what the register budget carries without spills; with 3 in place of 4
+            // the C = 2 form takes 425 in place of 400 us (the whole call of 2048 tokens, 128 experts of 768 x 2048).
+            constexpr int STEPS = 8 * C, AHEAD = C == 4 ? 3 : 4;
             x_half8 ring[AHEAD];
             uint32_t a_addr[2];
             auto read_a = [&](int s) {
-                const int g = s / (2 * C), t = (s / 2) % C, i = s & 1;
+                const int g = s / (2 * C), t = s % C, i = (s / C) & 1;
                 if (t == 0) {
-                    asm volatile("v_xor_b32 %0, %1, %2" : "=v"(a_addr[s & 1]) : "s"(16 * (4 * g + i)), "v"(a_at));
+                    asm volatile("v_xor_b32 %0, %1, %2" : "=v"(a_addr[i]) : "s"(16 * (4 * g + i)), "v"(a_at));
                 }
                 ring[s % AHEAD] = *(const __attribute__((address_space(3))) x_half8 *)(
-                    (const lds_u8_t *)(uintptr_t)a_addr[s & 1] + hb * L::ACT + t * 8192);
+                    (const lds_u8_t *)(uintptr_t)a_addr[i] + hb * L::ACT + t * 8192);
             };
             x_half8 op[2][X16Raw<KIND>::PLANES][2];
             if (hb == 0 && LATE && b != 0) {
@@ -593,7 +607,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < STEPS; ++s) {
-                const int g = s / (2 * C), t = (s / 2) % C, i = s & 1;
+                const int g = s / (2 * C), t = s % C, i = (s / C) & 1;
                 const x_half8 a = ring[s % AHEAD];
 #pragma unroll
                 for (int pl = 0; pl < X16Raw<KIND>::PLANES; ++pl) {
