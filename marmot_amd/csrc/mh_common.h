@@ -460,7 +460,7 @@ int launch_mmq(marmot_hip_device *dev, int kind, const void *d_w0, const void *d
 // Tiled int8 GEMM on Q8_K activations (mh_gemm_i8.hip): Q4_K, Q5_K and Q6_K weights; 33 activation rows and more
 bool gemm_i8_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,
                      const ActScratch &act);
-size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, size_t N, size_t K, size_t M, int weights);
+size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights);
 int launch_gemm_i8(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                    size_t M, int out_dtype, void *scratch);
 // Tiled GEMM of K-quant weights and Q8_K activations on the fp16 matrix cores with integer operands (mh_gemm_int16.hip)

@@ -28,6 +28,8 @@ namespace mh {
 
 typedef int i8_intx4 __attribute__((ext_vector_type(4)));
 typedef int i8_intx16 __attribute__((ext_vector_type(16)));
+typedef float i8_floatx16 __attribute__((ext_vector_type(16)));
+typedef _Float16 i8_half8 __attribute__((ext_vector_type(8)));
 typedef unsigned short i8_u16x2 __attribute__((ext_vector_type(2)));
 
 struct GemmI8Params {
@@ -1026,9 +1028,13 @@ __global__ __launch_bounds__(I8_THREADS) void k_gemm_q6k_q8k_tile(const GemmI8Pa
 // unsigned and add w.min * a.d * sum(a) per block: a.d * sum(a) depends on the token alone and is formed once per
 // round and token into LDS ([block][token], beside the scales), so the term costs one more multiply-add per output.
 // integer dot exact, one fp32 multiply-add per block in block order. Here a block of 32 weight rows x 32 tokens is one
-// v_mfma_i32_32x32x32_i8, and every output takes its block's product of the two scales with three vector
-// instructions (convert, scale product, multiply-add): the formats have one scale per 32 values and nothing to fold,
-// so the kernel is bound by these, at about an eighth of the int8 peak.
+// v_mfma_i32_32x32x32_i8, and every output takes its block's product of the two scales: the formats have one scale per 32
+// values and nothing to fold. The products of the scales come from a second matrix instruction (one value of K, halves:
+// exact), which leaves two vector instructions per output and block, convert and multiply-add (three with the scale product
+// on the vector unit). What bounds the kernel is latency: every product waits for operands from LDS. Two wavefronts per
+// SIMD, with two stages of a 34-byte format, keep its vector unit busy for half the time; two workgroups of one stage each
+// do better (Q8_0, 1024 tokens x 4096 x 14336: 283 us -> 256 with the scales from the matrix core -> 207 with one stage;
+// Q4_0, which always had room for two workgroups: 216 -> 205). Prefetching operands by hand at two wavefronts gave 4 %.
 // Same tile and wavefront roles as the Q6_K kernel: a round is 256 values of K (eight blocks), K group kg takes blocks
 // 4 kg .. 4 kg + 3 of every round. Weight rows must be a multiple of eight blocks (K % 256 == 0: rows and rounds start
 // on 16-byte boundaries); the stage holds each row's 272 (Q8_0) / 144 (Q4_0) bytes of the round at a pitch of 304 / 144
@@ -1051,17 +1057,65 @@ struct Q80Tile {
     static constexpr int STAGE_S = HAS_MIN ? I8_TOK * 16 : 0;       // the round's 8 code sums of every token
     static constexpr int STAGE_M = HAS_MIN ? 8 * I8_TOK * 4 : 0;    // scale x sum as [block][token]
     static constexpr int STAGE = STAGE_W + I8_STAGE_A + STAGE_D + STAGE_S + STAGE_M;
-    static constexpr int LDS_BYTES = 2 * STAGE;
+    // Two workgroups of two stages each fit a compute unit (Q4_0, Q5_0). The others have a form with one stage besides,
+    // for calls with more workgroups than compute units.
+    static constexpr bool SHARES = 4 * STAGE <= 160 * 1024;
     static constexpr int W_INSTR = (I8_WROWS * PITCH_P + 63) / 64;
     static constexpr int W_PER_WAVE = (W_INSTR + I8_WAVES - 1) / I8_WAVES;
     static_assert(CHUNK % 16 == 0 && STAGE % 16 == 0, "16-byte pieces");
     static_assert(PITCH_P >= PIECES, "a row's pieces fit its pitch");
-    static_assert(I8_OUT_TILE_BYTES <= LDS_BYTES, "the output tile reuses the stages");
+    static_assert(I8_OUT_TILE_BYTES <= STAGE, "the output tile reuses the stages");
+};
+
+// What lane (j, kh) needs of its row's block: the 16 values 16 kh .. + 15 of it as they are stored, scale and minimum
+template <int KIND>
+struct Q80Raw {
+    uint4 q;
+    uint32_t qh;
+    uint16_t d, m;
+    __device__ __forceinline__ void load(const uint8_t *block, int kh) {
+        using T = Q80Tile<KIND>;
+        __builtin_memcpy(&d, block, 2);
+        if constexpr (T::HAS_MIN) {
+            __builtin_memcpy(&m, block + 2, 2);
+        }
+        __builtin_memcpy(&q, block + T::QS_AT + (KIND == MARMOT_HIP_KIND_Q8_0 ? 16 * kh : 0), 16);
+        if constexpr (T::FIFTH) {
+            __builtin_memcpy(&qh, block + T::QS_AT - 4, 4);
+        }
+    }
+    // Byte i of a nibble block: value i in the low nibble, value 16 + i in the high nibble; Q5_0 / Q5_1: bit i (16 + i) of
+    // the 32-bit word before them is the value's fifth bit. Q4_0: (n + 0x78) ^ 0x80 is n - 8 as a signed byte, Q5_0:
+    // (v + 0x70) ^ 0x80 is v - 16, both without carries between bytes.
+    __device__ __forceinline__ i8_intx4 values(int kh) const {
+        using T = Q80Tile<KIND>;
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        i8_intx4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (KIND == MARMOT_HIP_KIND_Q8_0) {
+                r[e] = (int)w[e];
+            } else {
+                uint32_t v = (kh ? (w[e] >> 4) : w[e]) & 0x0f0f0f0fu;
+                if constexpr (T::FIFTH) {  // bits 4 e .. 4 e + 3 to bit 4 of bytes 0 .. 3
+                    const uint32_t bits = kh ? qh >> 16 : qh;
+                    v |= ((((bits >> (4 * e)) & 0xfu) * 0x00204081u) & 0x01010101u) << 4;
+                }
+                if constexpr (KIND == MARMOT_HIP_KIND_Q4_0) {
+                    v = (v + 0x78787878u) ^ 0x80808080u;
+                } else if constexpr (KIND == MARMOT_HIP_KIND_Q5_0) {
+                    v = (v + 0x70707070u) ^ 0x80808080u;
+                }
+                r[e] = (int)v;
+            }
+        }
+        return r;
+    }
 };
 
 // p.nb counts rounds (K / 256); p.ad holds 8 p.nb scales per token
-template <int KIND, int NA>
-__global__ __launch_bounds__(I8_THREADS) void k_gemm_q80_tile(const GemmI8Params p) {
+template <int KIND, int NA, int STAGES>
+__global__ __launch_bounds__(I8_THREADS, 4) void k_gemm_q80_tile(const GemmI8Params p) {
     using T = Q80Tile<KIND>;
     constexpr int TOK = 32 * NA;  // tokens per workgroup: 64, or 32 for at most 32 activation rows
     warm_kernel_arguments<sizeof(GemmI8Params)>();
@@ -1128,7 +1182,7 @@ __global__ __launch_bounds__(I8_THREADS) void k_gemm_q80_tile(const GemmI8Params
     const uint32_t s_voff = (uint32_t)(((uint32_t)lane < last_tok ? (uint32_t)lane : last_tok) * 16u * p.nb);
     auto issue = [&](int ri) {
         const size_t b = b0 + (size_t)ri;
-        const uint32_t s0 = lds_base + (uint32_t)((ri & 1) * T::STAGE);
+        const uint32_t s0 = lds_base + (uint32_t)((ri % STAGES) * T::STAGE);
         const uint8_t *qb = tile_q + b * QK_K;
 #pragma unroll
         for (int c = 0; c < NA; ++c) {
@@ -1157,7 +1211,7 @@ __global__ __launch_bounds__(I8_THREADS) void k_gemm_q80_tile(const GemmI8Params
     // scale x sum of a landed round, one (block, token) per thread
     auto fold_sums = [&](int ri) {
         if constexpr (T::HAS_MIN) {
-            uint8_t *stage = lds + (size_t)(ri & 1) * T::STAGE;
+            uint8_t *stage = lds + (size_t)(ri % STAGES) * T::STAGE;
             const int blk = tid >> 6, tok = tid & 63;
             const float da = *(const float *)(stage + T::STAGE_W + I8_STAGE_A + 4 * tid);
             const int16_t sum = *(const int16_t *)(stage + T::STAGE_W + I8_STAGE_A + T::STAGE_D + 16 * tok + 2 * blk);
@@ -1176,91 +1230,81 @@ __global__ __launch_bounds__(I8_THREADS) void k_gemm_q80_tile(const GemmI8Params
     i8_lds_barrier();
     fold_sums(0);
     for (int ri = 0; ri < nrounds; ++ri) {
-        if (ri + 1 < nrounds) {
+        if (STAGES == 2 && ri + 1 < nrounds) {
             issue(ri + 1);  // into the other buffer, which the barrier that closed the previous round has released
         }
-        {
-            const uint8_t *stage = lds + (size_t)(ri & 1) * T::STAGE;
-            const uint8_t *wrow = stage + w_off;
-            const i8_intx16 zero = {0};
+        const uint8_t *stage = lds + (size_t)(ri % STAGES) * T::STAGE;
+        const uint8_t *wrow = stage + w_off;
+        // The product of the two scales of every output comes from a matrix instruction with one value of K (exact: both are
+        // halves, the format's scales). Lane (j, kh) holds the scale of token 32 a + j. Scales that are no halves, as only
+        // a scratch filled by hand can hold them, are multiplied on the vector unit.
+        bool halves = true;
+        uint32_t ah[4][NA];
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi) {
-                const int blk = 4 * kg + bi;
-                uint16_t dh;
-                __builtin_memcpy(&dh, wrow + T::BLK * blk, 2);
-                float dw = h2f(dh);
-                asm volatile("" : "+v"(dw));  // a conversion of its own (not folded into mixed-precision multiplies)
-                float mw = 0.0f;
-                if constexpr (T::HAS_MIN) {
-                    uint16_t mh;
-                    __builtin_memcpy(&mh, wrow + T::BLK * blk + 2, 2);
-                    mw = h2f(mh);
-                    asm volatile("" : "+v"(mw));
-                }
-                i8_intx4 wv;
-                if constexpr (KIND == MARMOT_HIP_KIND_Q8_0) {
-                    __builtin_memcpy(&wv, wrow + T::BLK * blk + 2 + 16 * kh, 16);
-                } else {
-                    // byte i of the block: value i in the low nibble, value 16 + i in the high nibble; Q5_0 / Q5_1: bit
-                    // i (16 + i) of the 32-bit word before them is the value's fifth bit. Q4_0: (n + 0x78) ^ 0x80 is
-                    // n - 8 as a signed byte, Q5_0: (v + 0x70) ^ 0x80 is v - 16, both without carries between bytes.
-                    uint4 raw;
-                    __builtin_memcpy(&raw, wrow + T::BLK * blk + T::QS_AT, 16);
-                    const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
-                    uint32_t qh = 0u;
-                    if constexpr (T::FIFTH) {
-                        __builtin_memcpy(&qh, wrow + T::BLK * blk + T::QS_AT - 4, 4);
-                        qh = kh ? qh >> 16 : qh;
+        for (int bi = 0; bi < 4; ++bi) {
+#pragma unroll
+            for (int a = 0; a < NA; ++a) {
+                const float da = *(const float *)(stage + T::STAGE_W + I8_STAGE_A + 256 * (4 * kg + bi) + 4 * (32 * a + j));
+                const uint16_t h = f2h(da);
+                halves = halves && h2f(h) == da;
+                ah[bi][a] = kh != 0 ? 0u : (uint32_t)h;
+            }
+        }
+        const bool outer = __builtin_amdgcn_ballot_w64(!halves) == 0;
+#pragma unroll
+        for (int bi = 0; bi < 4; ++bi) {
+            const int blk = 4 * kg + bi;
+            Q80Raw<KIND> raw;
+            raw.load(wrow + T::BLK * blk, kh);
+            const i8_intx4 wv = raw.values(kh);
+            const float mw = T::HAS_MIN ? h2f(raw.m) : 0.0f;
+            const i8_intx4 wscale = {kh != 0 ? 0 : (int)raw.d, 0, 0, 0};
+            const i8_intx16 zero = {0};
+            const i8_floatx16 fzero = {0.0f};
+#pragma unroll
+            for (int a = 0; a < NA; ++a) {
+                const i8_intx4 av = *(const i8_intx4 *)(stage + a_base + a * (32 * QK_K) + 16 * ((2 * blk + kh) ^ (j & 15)));
+                const i8_intx16 dq = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, wv, zero, 0, 0, 0);
+                const i8_intx4 ascale = {(int)ah[bi][a], 0, 0, 0};
+                i8_floatx16 scales = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                    __builtin_bit_cast(i8_half8, ascale), __builtin_bit_cast(i8_half8, wscale), fzero, 0, 0, 0);
+                if (!outer) {
+                    float dw = h2f(raw.d);
+                    asm volatile("" : "+v"(dw));  // a conversion of its own (not folded into mixed-precision multiplies)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        scales[r] = dw * *(const float *)(stage + d_off + 256 * blk + 4 * (32 * a + 8 * (r >> 2) + (r & 3)));
                     }
+                }
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        uint32_t v = (kh ? (rw[e] >> 4) : rw[e]) & 0x0f0f0f0fu;
-                        if constexpr (T::FIFTH) {  // bits 4 e .. 4 e + 3 to bit 4 of bytes 0 .. 3
-                            v |= ((((qh >> (4 * e)) & 0xfu) * 0x00204081u) & 0x01010101u) << 4;
-                        }
-                        if constexpr (KIND == MARMOT_HIP_KIND_Q4_0) {
-                            v = (v + 0x78787878u) ^ 0x80808080u;
-                        } else if constexpr (KIND == MARMOT_HIP_KIND_Q5_0) {
-                            v = (v + 0x70707070u) ^ 0x80808080u;
-                        }
-                        wv[e] = (int)v;
+                        const int r = 4 * q4 + e;
+                        total[a][r] = __builtin_fmaf((float)dq[r], scales[r], total[a][r]);
                     }
-                }
-#pragma unroll
-                for (int a = 0; a < NA; ++a) {
-                    const i8_intx4 av = *(const i8_intx4 *)(stage + a_base + a * (32 * QK_K) +
-                                                           16 * ((2 * blk + kh) ^ (j & 15)));
-                    const i8_intx16 dq = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, wv, zero, 0, 0, 0);
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4) {
-                        const float4 d4 = *(const float4 *)(stage + d_off + 256 * blk + 4 * (32 * a + 8 * q4));
-                        const float da[4] = {d4.x, d4.y, d4.z, d4.w};
+                    if constexpr (T::HAS_MIN) {
+                        const float4 m4 = *(const float4 *)(stage + d_off + T::STAGE_D + T::STAGE_S + 256 * blk +
+                                                            4 * (32 * a + 8 * q4));
+                        const float ms[4] = {m4.x, m4.y, m4.z, m4.w};
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const int r = 4 * q4 + e;
-                            total[a][r] = __builtin_fmaf((float)dq[r], dw * da[e], total[a][r]);
-                        }
-                        if constexpr (T::HAS_MIN) {
-                            const float4 m4 = *(const float4 *)(stage + d_off + T::STAGE_D + T::STAGE_S + 256 * blk +
-                                                                4 * (32 * a + 8 * q4));
-                            const float ms[4] = {m4.x, m4.y, m4.z, m4.w};
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const int r = 4 * q4 + e;
-                                total[a][r] = __builtin_fmaf(mw, ms[e], total[a][r]);
-                            }
-                        }
-                    }
-                    if constexpr (T::HAS_MIN) {
-                        // one matrix product and its 16 outputs at a time (left alone, the compiler forms all eight
-                        // products of the round first and spills their 128 results)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            asm volatile("" : "+v"(total[a][r]));
+                            total[a][r] = __builtin_fmaf(mw, ms[e], total[a][r]);
                         }
                     }
                 }
+                // one product and its 16 outputs at a time (left alone, the compiler forms several products first, and
+                // their results are more registers than four wavefronts per SIMD have)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    asm volatile("" : "+v"(total[a][r]));
+                }
             }
+        }
+        if (STAGES == 1 && ri + 1 < nrounds) {
+            i8_lds_barrier();  // every wavefront has read this round
+            issue(ri + 1);
         }
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wavefront's share of the next round has landed
         i8_lds_barrier();
@@ -1532,9 +1576,28 @@ bool gemm_i8_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K,
     return true;
 }
 
-size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, size_t N, size_t K, size_t M, int weights) {
+static bool q80_format(int kind) {
+    return kind == MARMOT_HIP_KIND_Q8_0 || kind == MARMOT_HIP_KIND_Q4_0 || kind == MARMOT_HIP_KIND_Q4_1 ||
+           kind == MARMOT_HIP_KIND_Q5_0 || kind == MARMOT_HIP_KIND_Q5_1;
+}
+// The 32-value formats: two workgroups share a compute unit, so from half a chip to a chip of tiles K is split until the
+// second places are taken too (300 x 4096 x 4096, 160 tiles, whole call: Q8_0 46 us unsplit, 39 in three; Q4_0 44 / 40;
+// Q8_0 300 x 14336 x 4096 161 / 82). The partial sums cost about 6 us: not below 3072 values of K (300 x 1024 x 4096: 18 us
+// unsplit, 24 in two or three).
+static size_t gemm_q80_splits(const marmot_hip_device *dev, size_t N, size_t M, size_t nb, size_t *blocks_per_split) {
+    const size_t tiles = ((N + I8_TOK - 1) / I8_TOK) * ((M + I8_WROWS - 1) / I8_WROWS);
+    const size_t cus = (size_t)dev->props.multiProcessorCount;
+    if (tiles * 2 <= cus || tiles > cus || nb < 12) {
+        return gemm_i8_splits(dev, N, M, nb, blocks_per_split);
+    }
+    const size_t bps = (nb + 2 * cus / tiles - 1) / (2 * cus / tiles);
+    *blocks_per_split = bps;
+    return (nb + bps - 1) / bps;
+}
+
+size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights) {
     size_t bps = 0;
-    const size_t splits = gemm_i8_splits(dev, N, M, K / QK_K, &bps);
+    const size_t splits = q80_format(kind) ? gemm_q80_splits(dev, N, M, K / QK_K, &bps) : gemm_i8_splits(dev, N, M, K / QK_K, &bps);
     return splits > 1 ? splits * N * M * sizeof(float) * (size_t)weights : 0;
 }
 
@@ -1547,7 +1610,7 @@ int launch_gemm_i8(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
     float *partial = (float *)scratch;
     if (splits > 1 && partial == nullptr) {
         void *wsp = nullptr;
-        MH_TRY(workspace_reserve(dev, gemm_i8_scratch_bytes(dev, N, K, M, ws.count), &wsp));
+        MH_TRY(workspace_reserve(dev, gemm_i8_scratch_bytes(dev, kind, N, K, M, ws.count), &wsp));
         partial = (float *)wsp;
     }
     MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q4k_q8k_tile));
@@ -1598,10 +1661,6 @@ constexpr size_t Q23K_MIN_ROWS = 5;
 size_t gemm_q80_min_rows(int kind) {
     return (kind == MARMOT_HIP_KIND_Q2_K || kind == MARMOT_HIP_KIND_Q3_K) ? Q23K_MIN_ROWS : Q80_MIN_ROWS;
 }
-static bool q80_format(int kind) {
-    return kind == MARMOT_HIP_KIND_Q8_0 || kind == MARMOT_HIP_KIND_Q4_0 || kind == MARMOT_HIP_KIND_Q4_1 ||
-           kind == MARMOT_HIP_KIND_Q5_0 || kind == MARMOT_HIP_KIND_Q5_1;
-}
 static bool q23k_format(int kind) {
     return kind == MARMOT_HIP_KIND_Q2_K || kind == MARMOT_HIP_KIND_Q3_K;
 }
@@ -1633,16 +1692,23 @@ bool gemm_q80_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K
 
 // at most 32 activation rows: the form with one token tile of 32 per workgroup (half the matrix instructions and
 // epilogue of the 64-token form, whose second tile would hold no token)
+template <int KIND, int NA, int STAGES>
+static int launch_gemm_q80_form(marmot_hip_device *dev, const GemmI8Params &p, dim3 grid) {
+    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q80_tile<KIND, NA, STAGES>));
+    hipLaunchKernelGGL((k_gemm_q80_tile<KIND, NA, STAGES>), grid, dim3(I8_THREADS), STAGES * Q80Tile<KIND>::STAGE, dev->stream, p);
+    return MARMOT_HIP_SUCCESS;
+}
 template <int KIND>
 static int launch_gemm_q80_kind(marmot_hip_device *dev, const GemmI8Params &p, dim3 grid) {
-    if (p.N <= 32) {
-        MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q80_tile<KIND, 1>));
-        hipLaunchKernelGGL((k_gemm_q80_tile<KIND, 1>), grid, dim3(I8_THREADS), Q80Tile<KIND>::LDS_BYTES, dev->stream, p);
-    } else {
-        MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q80_tile<KIND, 2>));
-        hipLaunchKernelGGL((k_gemm_q80_tile<KIND, 2>), grid, dim3(I8_THREADS), Q80Tile<KIND>::LDS_BYTES, dev->stream, p);
+    if constexpr (!Q80Tile<KIND>::SHARES) {
+        // More workgroups than compute units: with one stage two of them share a compute unit, and one computes while the
+        // other's loads are on their way (Q8_0, 1024 tokens x 4096 x 14336: 283 us with two stages, 207 with one). At most
+        // one workgroup per compute unit: two stages (300 x 4096 x 4096 unsplit: 46 us, with one stage 54).
+        if ((size_t)grid.x * grid.y * grid.z > (size_t)dev->props.multiProcessorCount) {
+            return p.N <= 32 ? launch_gemm_q80_form<KIND, 1, 1>(dev, p, grid) : launch_gemm_q80_form<KIND, 2, 1>(dev, p, grid);
+        }
     }
-    return MARMOT_HIP_SUCCESS;
+    return p.N <= 32 ? launch_gemm_q80_form<KIND, 1, 2>(dev, p, grid) : launch_gemm_q80_form<KIND, 2, 2>(dev, p, grid);
 }
 
 int launch_gemm_q80(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
@@ -1652,7 +1718,7 @@ int launch_gemm_q80(marmot_hip_device *dev, int kind, const WeightSet &ws, const
     }
     const size_t nb = K / QK_K;
     size_t bps = 0;
-    const size_t splits = gemm_i8_splits(dev, N, M, nb, &bps);
+    const size_t splits = gemm_q80_splits(dev, N, M, nb, &bps);
     float *partial = (float *)scratch;
     if (splits > 1 && partial == nullptr) {
         return set_error(MARMOT_HIP_ERROR_INVALID_ARGUMENT, "tiled Q8_0 GEMM: no room for the K-split partial sums");

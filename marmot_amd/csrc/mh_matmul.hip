@@ -273,7 +273,7 @@ static int matmul_impl(marmot_hip_device *dev, int kind, const void *d_w0, const
     // sums behind the activations)
     const bool q80_kind = gemm_q80_kind(kind) && N >= gemm_q80_min_rows(kind) && K % QK_K == 0;
     const size_t need = act_bytes + (mmq ? mmq_scratch_bytes(dev, kind, N, K, M, d_w1 != nullptr ? 2 : 1) : 0) +
-                        (q80_kind ? gemm_i8_scratch_bytes(dev, N, K, M, d_w1 != nullptr ? 2 : 1) : 0);
+                        (q80_kind ? gemm_i8_scratch_bytes(dev, kind, N, K, M, d_w1 != nullptr ? 2 : 1) : 0);
     void *ws = nullptr;
     int st = workspace_reserve(dev, need, &ws);
     if (st != MARMOT_HIP_SUCCESS) {
@@ -537,7 +537,7 @@ int marmot_hip_matmul_prepacked(marmot_hip_device_t *dev, int kind, const void *
         ws.bias_dtype = bias_dtype;
         if (gemm_q80_applies(dev, kind, N, K, ws.w, 1, act)) {
             MH_HIP(hipSetDevice(dev->device_index));
-            const size_t partial_bytes = gemm_i8_scratch_bytes(dev, N, K, M, 1);
+            const size_t partial_bytes = gemm_i8_scratch_bytes(dev, kind, N, K, M, 1);
             void *scratch = nullptr;
             if (partial_bytes != 0) {
                 MH_TRY(workspace_reserve(dev, partial_bytes, &scratch));
@@ -734,7 +734,7 @@ int marmot_hip_matmul_qkv_rope_quantized(marmot_hip_device_t *dev, int kind, con
     // sums where the mmq scratch would be
     const bool q80_kind = !fuse_quant && gemm_q80_kind(kind) && N >= gemm_q80_min_rows(kind) && K % QK_K == 0;
     const size_t mmq_bytes = mmq ? ((mmq_scratch_bytes(dev, kind, N, K, M, 3) + 255) & ~(size_t)255)
-        : q80_kind               ? ((gemm_i8_scratch_bytes(dev, N, K, M, 3) + 255) & ~(size_t)255)
+        : q80_kind               ? ((gemm_i8_scratch_bytes(dev, kind, N, K, M, 3) + 255) & ~(size_t)255)
                                  : 0;
     void *wsp = nullptr;
     int st = MARMOT_HIP_SUCCESS;

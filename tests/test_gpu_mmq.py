@@ -527,6 +527,69 @@ def test_tiled_int8_gemm_32_value_formats_random_blocks_routes_and_epilogues(hip
     assert_matmul_parity(pre, oracle.matmul(kind, w3, x3, m3, bias=b3), what=f"{name} prepacked, K split")
 
 
+@pytest.mark.parametrize("N,M,K", [(290, 4000, 3072), (300, 4096, 2816), (1100, 2001, 256)])
+@pytest.mark.parametrize("name", ["q8_0", "q4_0", "q4_1"])
+def test_tiled_int8_gemm_32_value_formats_two_workgroups_per_unit(hip, oracle, name, N, M, K):
+    """160 tiles with K split over the second places of the compute units (12 rounds of 256 values), the same unsplit
+    (11 rounds), and more tiles than compute units (the form with one stage); ragged rows and tokens."""
+    kind = Q80_KINDS[name]
+    blocks = oracle.quantize(kind, gaussian(460 + N, (M, K), 0.02))
+    x = gaussian(461 + N, (N, K))
+    got = hip.linear(x, blocks, kind, M)
+    assert hip.last_route() == f"gemm_{name}_q8_0_mfma_tile"
+    some = np.unique(np.r_[0, 1, 31, 32, 63, 64, N // 2, N - 45:N])  # rows of the first tiles, a middle and the last ones
+    assert_matmul_parity(got[some], oracle.matmul(kind, blocks, np.ascontiguousarray(x[some]), M), what=f"{name} {M}x{K} N={N}")
+
+
+@pytest.mark.parametrize("scales", ["subnormal", "not_halves"])
+@pytest.mark.parametrize("name", ["q8_0", "q4_0"])
+def test_tiled_int8_gemm_32_value_formats_scale_products(hip, name, scales):
+    """The product of the two block scales: exact where both are halves, the smallest subnormals included (powers of two:
+    every output then equals the chain of one rounding per block), and correctly rounded where a scratch filled by hand
+    holds scales that no half has (three roundings of at most 2^-24 of a term per block, 8 blocks)."""
+    kind, bb = Q80_KINDS[name], {"q8_0": 34, "q4_0": 18}[name]
+    N, M, K = 70, 200, 256
+    nb = K // 32
+    rng = np.random.default_rng(470)
+    blocks = random_valid_blocks(rng, kind, M, K).reshape(M, nb, bb).copy()
+    d = np.ldexp(1.0, rng.integers(-24, -12, size=(M, nb)))
+    blocks[:, :, 0:2] = d.astype(np.float16).view(np.uint8).reshape(M, nb, 2)
+    q = rng.integers(-127, 128, size=(N, K)).astype(np.int8)
+    ad = np.ldexp(1.0, rng.integers(-24, -12, size=(N, nb))).astype(np.float32)
+    if scales == "not_halves":
+        ad = (ad * rng.uniform(1.0, 2.0, size=ad.shape)).astype(np.float32)
+    lay = hip.packed_activation_layout(kind, N, K)
+    image = np.zeros(lay.total_bytes, np.uint8)
+    vals = np.zeros((N, lay.values_per_row), np.int8)
+    vals[:, :K] = q
+    image[lay.values_offset:lay.values_offset + vals.size] = vals.view(np.uint8).reshape(-1)
+    image[lay.scales_offset:lay.scales_offset + ad.nbytes] = ad.view(np.uint8).reshape(-1)
+    if name == "q8_0":
+        wq = blocks[:, :, 2:].view(np.int8).astype(np.int64)
+    else:
+        qs = blocks[:, :, 2:].astype(np.int64)
+        wq = np.concatenate([(qs & 15) - 8, (qs >> 4) - 8], axis=2)
+    dots = np.einsum("nbk,mbk->nmb", q.reshape(N, nb, 32).astype(np.int64), wq)
+    terms = dots * (ad.astype(np.float64)[:, None, :] * d[None, :, :])
+    d_w, d_p, d_out = hip.to_device(blocks.reshape(M, nb * bb)), hip.to_device(image), hip.alloc(N * M * 4)
+    hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out)
+    assert hip.last_route() == f"gemm_{name}_q8_0_mfma_tile"
+    got = d_out.download(np.float32, (N, M))
+    for b_ in (d_w, d_p, d_out):
+        b_.free()
+    if scales == "subnormal":
+        halves = []
+        for first in (0, 4):
+            acc = np.zeros((N, M), np.float32)
+            for b in range(first, first + 4):
+                acc = (acc.astype(np.float64) + terms[:, :, b]).astype(np.float32)
+            halves.append(acc)
+        assert np.array_equal(bits(got), bits(halves[0] + halves[1]))
+    else:
+        bound = 8 * 3 * 2.0 ** -24 * np.abs(terms).sum(axis=2)
+        assert np.all(np.abs(got.astype(np.float64) - terms.sum(axis=2)) <= bound)
+
+
 Q23K_KINDS = {"q2_k": 7, "q3_k": 8}
 
 
