@@ -443,6 +443,10 @@ int launch_matvec_rows2_q4k(marmot_hip_device *dev, const WeightSet &ws, const f
 bool mmq_rows_supported(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int nw, bool packed);
 int launch_mmq_rows_q4k(marmot_hip_device *dev, const WeightSet &ws, const float *d_x_f32, const ActScratch *act,
                         size_t N, size_t K, size_t M, int out_dtype);
+// The same for Q6_K, packed rows only
+bool mmq_rows_q6k_supported(const marmot_hip_device *dev, size_t N, size_t K, size_t M);
+int launch_mmq_rows_q6k(marmot_hip_device *dev, const WeightSet &ws, const ActScratch &act, size_t N, size_t K, size_t M,
+                        int out_dtype);
 // quantizes act(gate) * up (SwiGLU or GeGLU) of two fp32 [rows, k] arrays into the activation scratch
 int launch_quantize_glu_soa(marmot_hip_device *dev, int act_kind, const float *d_gate, const float *d_up, bool geglu,
                             size_t rows, size_t k, const ActScratch &dst);

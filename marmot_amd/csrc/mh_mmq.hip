@@ -1074,6 +1074,15 @@ int launch_mmq_set(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
         }
         return launch_gemm_i8(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }
+    if (kind == MARMOT_HIP_KIND_Q6_K) {
+        const int st = launch_mmq_rows_q6k(dev, ws, act, N, K, M, out_dtype);
+        if (st != MARMOT_HIP_ERROR_NOT_IMPLEMENTED) {
+            if (st == MARMOT_HIP_SUCCESS) {
+                set_route("mmq_q6_k_q8_k_mfma");
+            }
+            return st;
+        }
+    }
     const size_t nb = K / QK_K;
     const MmqPlan pl = mmq_plan(dev, kind, N, M, nb, ws.count);
     float *partial = (float *)scratch;

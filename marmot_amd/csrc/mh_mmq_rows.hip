@@ -66,24 +66,29 @@ __host__ __device__ constexpr uint32_t mr_ctrl_words(uint32_t nslots, uint32_t g
     return (MR_CTRL_SLOTS + 2u * nslots + groups + 3u) & ~3u;
 }
 
-__device__ __forceinline__ void mr_store(const MmqRowsParams &p, void *out, const void *bias, size_t n, size_t row,
-                                         float v) {
+template <class P>
+__device__ __forceinline__ void mr_put(const P &p, void *out, bool has_bias, float bv, size_t n, size_t row, float v) {
     const size_t o = n * p.M + row;
-    float bv = 0.0f;
-    if (bias != nullptr) {
-        bv = p.bias_is_f16 ? h2f(((const uint16_t *)bias)[row]) : ((const float *)bias)[row];
-    }
     if (!p.out_is_f16) {
-        ((float *)out)[o] = bias != nullptr ? v + bv : v;
+        ((float *)out)[o] = has_bias ? v + bv : v;
     } else if (p.bias_first) {
-        ((uint16_t *)out)[o] = f2h(bias != nullptr ? v + bv : v);
+        ((uint16_t *)out)[o] = f2h(has_bias ? v + bv : v);
     } else {
         uint16_t h = f2h(v);
-        if (bias != nullptr) {
+        if (has_bias) {
             h = f2h(h2f(h) + bv);
         }
         ((uint16_t *)out)[o] = h;
     }
+}
+template <class P>
+__device__ __forceinline__ float mr_bias(const P &p, const void *bias, size_t row) {
+    return p.bias_is_f16 ? h2f(((const uint16_t *)bias)[row]) : ((const float *)bias)[row];
+}
+__device__ __forceinline__ void mr_store(const MmqRowsParams &p, void *out, const void *bias, size_t n, size_t row,
+                                         float v) {
+    const float bv = bias != nullptr ? mr_bias(p, bias, row) : 0.0f;
+    mr_put(p, out, bias != nullptr, bv, n, row, v);
 }
 
 // direct-to-LDS load of 64 x 4 bytes: lane l's 4 bytes at base + voff land at LDS byte address M0 + 4 l
@@ -757,6 +762,363 @@ int launch_mmq_rows_q4k(marmot_hip_device *dev, const WeightSet &ws, const float
     return pl.NT == 4   ? launch_mmq_rows_nt<4, false>(dev, p, pl, nw)
            : pl.NT == 8 ? launch_mmq_rows_nt<8, false>(dev, p, pl, nw)
                         : launch_mmq_rows_nt<16, false>(dev, p, pl, nw);
+}
+
+// ------------------------------------------------------------------ Q6_K x Q8_K, up to 16 activation rows
+// The integer products are those of k_mmq_q6k_ls (mh_mmq.hip); the split of a block over the lanes is another one. A
+// wavefront multiplies 16 weight rows x 256 values. Lane (row r, g) unpacks what one half h = g / 2 and one 16-value
+// column s = g % 2 of the block hold of ITS row: two 16-byte pieces of low nibbles and one of high bits, 16 values for
+// each of the four scale groups 8 h + 2 q + s (q = 0 .. 3). The four lanes of a row thus work on four different scale
+// groups in one v_mfma_i32_16x16x64_i8; the products are kept apart by the token operand: its 16 rows are four tokens
+// x four groups, row 4 g + i holding token i's codes in k group g and zeros elsewhere. Lane (r, g) gets four tokens of
+// exactly its own scale group, so a lane decodes four scales instead of sixteen, and no product of two tokens is
+// computed twice with up to four of them. q - 32 comes as 4 (q - 32), a signed byte: the value in bits 2 .. 7 with its
+// top bit inverted (one xor per four high-bit bytes, a quarter in the block scale).
+//
+// A workgroup takes row groups of 16; its wavefronts split K, each with a ring of its own (two stages: one block of 16
+// rows, of the tokens' codes and of their scales, direct-to-LDS loads), no barrier but one per row group, where the
+// partial sums meet in LDS; the ring runs on into the next row group. Row slots of 240 bytes: the 14 pieces from the
+// 16-byte boundary below the block's start, an odd number of pieces so that 16 rows lie in different banks.
+//
+// What bounds it: per task and compute unit 450 clocks (N = 8), of which the LDS pipe takes about 200 and the vector units
+// 240 (230 instructions per SIMD and task); memory would allow 350. Three stages or twelve wavefronts change nothing.
+// Measured against k_mmq_q6k_ls (us with the quantization launch and, there, the reduction launch; N = 8 / 16):
+//   K x M      14336 x 4096   4096 x 14336   4096 x 4096    4096 x 1024   8192 x 16384   4096 x 128256
+//   before     27.9 / 29.6    29.1 / 31.2    17.5 / 18.4    15.6 / 16.5   45.9 / 49.4    155.4 / 179.7
+//   now        17.7 / 21.8    18.4 / 22.2     9.7 / 11.4     8.8 / 10.2   29.4 / 37.0    104.4 / 129.6
+struct MmqRowsQ6Params {
+    const uint8_t *w[3];
+    void *out[3];
+    const void *bias[3];
+    const int8_t *qs;  // packed activations: rows of kp bytes
+    const float *ad;   // their block scales [row][nb]
+    uint32_t kp, N, M, nb;
+    uint32_t row_bytes;
+    uint32_t groups;         // row groups of a workgroup
+    int bias_is_f16, bias_first, out_is_f16;
+};
+
+template <int NQ>
+struct MmqRowsQ6Lds {
+    static constexpr int ROWB = 240, A_OFF = 16 * ROWB, D_OFF = A_OFF + NQ * 1024, STAGE = D_OFF + 64;
+    static constexpr int STAGES = 2;
+    static constexpr int ZERO = NQ * 1024;              // what the lanes of the token operand's zeros read
+    static constexpr int PART = NQ * 256;               // partial sums of one wavefront: [token / 4][row][token % 4]
+    static constexpr int bytes(int waves) { return ZERO + waves * (2 * PART + STAGES * STAGE); }
+};
+
+template <int NQ>
+__global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
+    using L = MmqRowsQ6Lds<NQ>;
+    constexpr int S = L::STAGES, LOADS = 4 + NQ + 1;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int waves = (int)(blockDim.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const uint8_t *wbase = p.w[blockIdx.y];
+    void *out = p.out[blockIdx.y];
+    const void *bias = p.bias[blockIdx.y];
+
+    uint8_t *ring = lds + L::ZERO + waves * 2 * L::PART + wave * (S * L::STAGE);
+    float *parts = (float *)(lds + L::ZERO);
+    const uint32_t ring_addr = (uint32_t)(uintptr_t)(lds_u8_t *)ring;
+    for (int i = tid; i < L::ZERO / 16; i += (int)blockDim.x) {
+        ((uint4 *)lds)[i] = uint4{0, 0, 0, 0};
+    }
+
+    const uint32_t all_groups = (p.M + 15u) / 16u;
+    const uint32_t group0 = blockIdx.x * p.groups;
+    const uint32_t groups = all_groups - group0 < p.groups ? all_groups - group0 : p.groups;
+    // wavefront w takes blocks w, w + waves, ...: what the workgroup reads of a row at a time is one run
+    const uint32_t b0 = (uint32_t)wave, blocks = (p.nb - b0 + (uint32_t)waves - 1u) / (uint32_t)waves;
+    const uint32_t b1 = b0 + blocks * (uint32_t)waves, tasks = groups * blocks;
+    // the tensor's size need not be a multiple of 16: a piece that would end behind it comes two bytes at a time through
+    // registers, and the loads in flight are then not whole stages
+    const bool ragged = group0 + groups == all_groups && (((uint64_t)p.M * p.row_bytes) & 15u) != 0;
+
+    // loads: piece `idx` of a stage is piece idx % 15 (the 15th repeats the 14th) of row idx / 15
+    uint32_t piece[4], row_of[4], a_off[NQ], d_off;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint32_t idx = (uint32_t)(c * 64 + lane);
+        row_of[c] = idx / 15u;
+        const uint32_t pc = idx - row_of[c] * 15u;
+        piece[c] = 16u * (pc < 14u ? pc : 13u);
+    }
+    // token codes, four tokens per load: unit [q / 2][h][token][q % 2, inverted for h = 1][s] of 16 bytes. Four lanes of a
+    // load read 64 bytes in a row, and the 16 lanes that read one q of four tokens hit different banks.
+#pragma unroll
+    for (int a = 0; a < NQ; ++a) {
+        const uint32_t tk = 4u * a + (((uint32_t)lane >> 2) & 3u), h = ((uint32_t)lane >> 4) & 1u;
+        a_off[a] = (tk < p.N ? tk : 0u) * p.kp + 128u * h + 64u * ((uint32_t)lane >> 5) + 32u * ((((uint32_t)lane >> 1) & 1u) ^ h) +
+                   16u * ((uint32_t)lane & 1u);
+    }
+    d_off = ((uint32_t)lane < p.N ? (uint32_t)lane : 0u) * p.nb * 4u;
+
+    // the row group that loads are issued for
+    uint32_t is_group = 0, is_block = b0, w_row[4], w_end = 0;
+    const uint8_t *wgroup = nullptr;
+    auto issue_group = [&](uint32_t i) {
+        const uint32_t row0 = (group0 + i) * 16u, last = p.M - 1u - row0;
+        const uint64_t at = (uint64_t)row0 * p.row_bytes;
+        const uint32_t lead = (uint32_t)at & 15u;
+        wgroup = uniform_pointer(wbase + (at - lead));
+        const uint64_t end = (uint64_t)(p.M - row0) * p.row_bytes + lead;
+        w_end = end > 0xffffffffull ? 0xffffffffu : (uint32_t)end;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            w_row[c] = lead + (row_of[c] < last ? row_of[c] : last) * p.row_bytes;
+        }
+    };
+    auto issue = [&](uint32_t slot) {
+        const uint32_t dst = ring_addr + slot * L::STAGE;
+        const uint32_t boff = is_block * Q6_K_BYTES;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t voff = ((w_row[c] + boff) & ~15u) + piece[c];
+            const bool past = ragged && voff + 16u > w_end;
+            dma_set_lds_base(dst + c * 1024);
+            if ((c < 3 || lane < 48) && !past) {
+                dma16_to_lds<0>(wgroup, voff);
+            }
+            if ((c < 3 || lane < 48) && past) {
+                // (in assembly with its wait: a load the compiler knows of would put a wait for all of them into the loop)
+                uint8_t *d = ring + slot * L::STAGE + c * 1024 + 16 * lane;
+#pragma unroll 1
+                for (uint32_t e = 0; e < 16u && voff + e < w_end; e += 2u) {
+                    uint32_t v;
+                    asm volatile("global_load_ushort %0, %1, %2\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(voff + e), "s"(wgroup) : "memory");
+                    *(uint16_t *)(d + e) = (uint16_t)v;
+                }
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < NQ; ++a) {
+            dma_set_lds_base(dst + L::A_OFF + a * 1024);
+            dma16_to_lds<0>((const uint8_t *)p.qs, a_off[a] + is_block * QK_K);
+        }
+        dma_set_lds_base(dst + L::D_OFF);
+        if (lane < 4 * NQ) {
+            mr_dma4_to_lds(p.ad, d_off + is_block * 4u);
+        }
+        if ((is_block += (uint32_t)waves) == b1) {
+            is_block = b0;
+            if (++is_group < groups) {
+                issue_group(is_group);
+            }
+        }
+    };
+
+    float acc[NQ][4];
+    uint32_t own = 0;  // where this lane's weight row begins, modulo 16
+    auto work_group = [&](uint32_t i) {
+        const uint32_t row0 = (group0 + i) * 16u, last = p.M - 1u - row0;
+        own = (uint32_t)(((uint64_t)row0 + ((uint32_t)r < last ? (uint32_t)r : last)) * p.row_bytes) & 15u;
+#pragma unroll
+        for (int a = 0; a < NQ; ++a) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                acc[a][k] = 0.0f;
+            }
+        }
+    };
+
+    issue_group(0);
+    work_group(0);
+    for (uint32_t s = 0; s + 1 < (uint32_t)S && s < tasks; ++s) {
+        issue(s);
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // the zeros
+    __builtin_amdgcn_s_barrier();
+    const int code_off = (g >> 1) * 288 + (r & 3) * 64 + (g & 1) * 16;  // h = 1: 256 on, the other half of 64 bytes first
+    uint32_t group = 0, block = b0, slot = 0, free_slot = S - 1;
+    for (uint32_t t = 0; t < tasks; ++t) {
+        if (t + S - 1 < tasks) {
+            issue(free_slot);
+        }
+        const uint32_t newer = tasks - 1 - t < (uint32_t)S - 1 ? tasks - 1 - t : (uint32_t)S - 1;
+        if (newer == (uint32_t)S - 1 && !ragged) {
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"((S - 1) * LOADS) : "memory");
+        } else {
+            wait_vmcnt_at_most(ragged ? 0 : (int)newer * LOADS);
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // pieces at the tensor's end
+        }
+        const uint8_t *stage = ring + slot * L::STAGE;
+        // a block begins at any even byte; reads off a 4-byte boundary hold the LDS pipe (in 16-byte reads at the block's own
+        // offsets a third of the kernel's time), so the words around a piece are read and shifted
+        const uint32_t at = (own + block * Q6_K_BYTES) & 15u, shift = 8u * (at & 2u);
+        const uint8_t *wrow = stage + r * L::ROWB + (at & 12u) + 16 * (g & 1);
+        auto words = [&](const uint8_t *from, uint32_t (&v)[4]) {
+            const uint32_t *src = (const uint32_t *)from;
+            uint32_t raw[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                raw[k] = src[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v[k] = __builtin_amdgcn_alignbit(raw[k + 1], raw[k], shift);
+            }
+        };
+        const uint8_t *codes[2];
+        codes[0] = (r >> 2) == g ? stage + L::A_OFF + code_off : lds;
+        codes[1] = (r >> 2) == g ? stage + L::A_OFF + (code_off ^ 32) : lds;
+        uint32_t ql[2][4], qh[4], sc[2];
+        words(wrow + 64 * (g >> 1), ql[0]);
+        words(wrow + 64 * (g >> 1) + 32, ql[1]);
+        words(wrow + 128 + 32 * (g >> 1), qh);
+        const uint32_t *tail = (const uint32_t *)(wrow - 16 * (g & 1) + 192);  // scales, then d
+        sc[0] = __builtin_amdgcn_alignbit(tail[1 + 2 * (g >> 1)], tail[2 * (g >> 1)], shift);
+        sc[1] = __builtin_amdgcn_alignbit(tail[2 + 2 * (g >> 1)], tail[1 + 2 * (g >> 1)], shift);
+        const uint16_t dh = (uint16_t)(tail[4] >> shift);
+        int sums[NQ][4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            qh[k] ^= 0xaaaaaaaau;
+        }
+        sc[0] >>= 8 * (g & 1);
+        sc[1] >>= 8 * (g & 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            mr_intx4 wv;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t lo = ql[q & 1][k], hi = qh[k];
+                wv[k] = (int)(((q < 2 ? lo << 2 : lo >> 2) & 0x3c3c3c3cu) | ((hi << (6 - 2 * q)) & 0xc0c0c0c0u));
+            }
+            const int scale = (int)(int8_t)(sc[q >> 1] >> (16 * (q & 1)));
+#pragma unroll
+            for (int a = 0; a < NQ; ++a) {
+                const mr_intx4 zero = {0, 0, 0, 0};
+                const mr_intx4 av = *(const mr_intx4 *)(codes[q & 1] + a * 1024 + (q >> 1) * 512);
+                const mr_intx4 dot = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, zero, 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    sums[a][k] = q == 0 ? __mul24(dot[k], scale) : sums[a][k] + __mul24(dot[k], scale);
+                }
+            }
+        }
+        const float d = h2f(dh) * 0.25f;
+#pragma unroll
+        for (int a = 0; a < NQ; ++a) {
+            const float4 ad = *(const float4 *)(stage + L::D_OFF + 16 * a);
+            acc[a][0] += (ad.x * d) * (float)sums[a][0];
+            acc[a][1] += (ad.y * d) * (float)sums[a][1];
+            acc[a][2] += (ad.z * d) * (float)sums[a][2];
+            acc[a][3] += (ad.w * d) * (float)sums[a][3];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // the stage is read before it is written again
+        free_slot = slot;
+        slot = slot + 1 == (uint32_t)S ? 0 : slot + 1;
+        if ((block += (uint32_t)waves) == b1) {
+            // the four lanes of a row hold the sums of four scale groups; then the wavefronts' partial sums in K order.
+            // Two buffers: a wavefront writes the next group's while others still read this one's
+            uint8_t *part = (uint8_t *)parts + (group & 1u) * (uint32_t)(waves * L::PART);
+#pragma unroll
+            for (int a = 0; a < NQ; ++a) {
+                float4 v;
+                float *f = (float *)&v;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float s = acc[a][k];
+                    s += __shfl_xor(s, 16);
+                    s += __shfl_xor(s, 32);
+                    f[k] = s;
+                }
+                if (g == a) {
+                    *(float4 *)(part + wave * L::PART + a * 256 + r * 16) = v;
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+            __builtin_amdgcn_s_barrier();
+            compiler_memory_fence();
+            for (int i = tid; i < 64 * NQ; i += (int)blockDim.x) {
+                const uint32_t row = (group0 + group) * 16u + ((uint32_t)i & 15u), tk = (uint32_t)i >> 4;
+                if (tk < p.N && row < p.M) {
+                    const float *src = (const float *)(part + (tk >> 2) * 256 + (i & 15) * 16) + (tk & 3u);
+                    float s = src[0];
+                    for (int w = 1; w < waves; ++w) {
+                        s += src[w * (L::PART / 4)];
+                    }
+                    float bv = 0.0f;
+                    if (bias != nullptr) {
+                        bv = mr_bias(p, bias, row);
+                        asm volatile("" : "+v"(bv));  // its wait belongs here, not into the loop over the blocks
+                    }
+                    mr_put(p, out, bias != nullptr, bv, tk, row, s);
+                }
+            }
+            block = b0;
+            if (++group < groups) {
+                work_group(group);
+            }
+        }
+    }
+}
+
+// Rows of one block stay on the streaming kernel: there is no K to split, and its sum of a block is one integer.
+bool mmq_rows_q6k_supported(const marmot_hip_device *dev, size_t N, size_t K, size_t M) {
+    const size_t row_bytes = K / QK_K * Q6_K_BYTES;
+    return !dev->knobs.no_row_kernels && N >= 1 && N <= 16 && K % QK_K == 0 && K >= 2 * QK_K && M >= 1 &&
+           M <= 0x7fffffffull && 17 * row_bytes <= 0x7fffffffull && N * K <= 0x7fffffffull;
+}
+
+template <int NQ>
+static int launch_mmq_rows_q6k_nq(marmot_hip_device *dev, const MmqRowsQ6Params &p, const dim3 grid, int waves) {
+    MH_TRY(allow_large_lds(dev, (const void *)k_mmq_rows_q6k<NQ>));
+    hipLaunchKernelGGL((k_mmq_rows_q6k<NQ>), grid, dim3(64 * waves), MmqRowsQ6Lds<NQ>::bytes(waves), dev->stream, p);
+    MH_HIP(hipGetLastError());
+    return MARMOT_HIP_SUCCESS;
+}
+
+// Q6_K weight set x up to 16 packed activation rows. Returns MARMOT_HIP_ERROR_NOT_IMPLEMENTED (error text untouched)
+// when the shape or the alignment is not covered.
+int launch_mmq_rows_q6k(marmot_hip_device *dev, const WeightSet &ws, const ActScratch &act, size_t N, size_t K, size_t M,
+                        int out_dtype) {
+    if (!mmq_rows_q6k_supported(dev, N, K, M) || (((uintptr_t)act.qs) & 15) != 0 || (((uintptr_t)act.d) & 3) != 0 ||
+        (act.kp & 15) != 0 || act.kp < K || N * act.kp > 0x7fffffffull || act.nb != K / QK_K) {
+        return MARMOT_HIP_ERROR_NOT_IMPLEMENTED;
+    }
+    for (int i = 0; i < ws.count; ++i) {
+        if ((((uintptr_t)ws.w[i]) & 15) != 0) {
+            return MARMOT_HIP_ERROR_NOT_IMPLEMENTED;
+        }
+    }
+    MmqRowsQ6Params p;
+    for (int i = 0; i < 3; ++i) {
+        const int src = i < ws.count ? i : 0;
+        p.w[i] = (const uint8_t *)ws.w[src];
+        p.out[i] = ws.out[src];
+        p.bias[i] = ws.bias[src];
+    }
+    p.qs = act.qs;
+    p.ad = act.d;
+    p.kp = (uint32_t)act.kp;
+    p.N = (uint32_t)N;
+    p.M = (uint32_t)M;
+    p.nb = (uint32_t)(K / QK_K);
+    p.row_bytes = p.nb * Q6_K_BYTES;
+    p.bias_is_f16 = ws.bias_dtype == MARMOT_HIP_DTYPE_F16;
+    p.bias_first = ws.bias_first ? 1 : 0;
+    p.out_is_f16 = out_dtype == MARMOT_HIP_DTYPE_F16;
+    const uint32_t cus = (uint32_t)dev->props.multiProcessorCount;
+    const uint32_t slots = cus / (uint32_t)ws.count > 0 ? cus / (uint32_t)ws.count : 1;
+    const uint32_t all = (p.M + 15u) / 16u;
+    // Eight wavefronts per compute unit, as workgroups of 8 / 4 / 2 (parts of K) by the number of row groups: a part more
+    // is a barrier and a sum more per row group (K 4096, 128256 rows, N = 8: 8 parts 116.6 us, 4: 109.2, 2: 104.4;
+    // 14336 rows 20.4, 19.1, 18.4), too few leave compute units idle (4096 rows, K 14336: 17.7, 21.5, 32.3).
+    uint32_t parts = 8u * slots / all;
+    parts = parts > 8 ? 8 : parts < 2 ? 2 : parts;
+    const uint32_t resident = slots * (8u / parts);
+    // Workgroups that stay for several row groups save their start-up; up to two rounds, the second fills in behind the
+    // first as it finishes.
+    p.groups = all <= 2 * resident ? 1 : (all + resident - 1) / resident;
+    const int waves = (int)(p.nb < parts ? p.nb : parts);
+    const dim3 grid((all + p.groups - 1) / p.groups, (unsigned)ws.count);
+    return N <= 4    ? launch_mmq_rows_q6k_nq<1>(dev, p, grid, waves)
+           : N <= 8  ? launch_mmq_rows_q6k_nq<2>(dev, p, grid, waves)
+           : N <= 12 ? launch_mmq_rows_q6k_nq<3>(dev, p, grid, waves)
+                     : launch_mmq_rows_q6k_nq<4>(dev, p, grid, waves);
 }
 
 } // namespace mh

@@ -702,3 +702,18 @@ def test_tiled_int8_gemm_32_value_formats_integers_are_exact(hip, name):
     for b_ in (d_w, d_p, d_out):
         b_.free()
     assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("M,K", [(1, 512), (15, 256 * 3), (16, 2048), (70, 1280), (1031, 256 * 9), (5000, 768), (16400, 512)])
+def test_q6k_up_to_16_rows_by_row_groups(hip, oracle, M, K):
+    """Row groups of 16 with K split over 2 to 8 wavefronts (fewer with fewer blocks), several row groups per workgroup,
+    row counts that end inside a group, tensors that do not end on a 16-byte boundary, every count of four-token steps;
+    bias. Random blocks: negative and extreme scales, all 6-bit values."""
+    rng = np.random.default_rng(390 + M)
+    blocks = random_valid_blocks(rng, KIND_Q6_K, M, K)
+    for N in (5, 8, 9, 12, 13, 16):
+        x = gaussian(391 + N, (N, K))
+        bias = gaussian(392, (M,)) if N % 2 else None
+        got = hip.linear(x, blocks, KIND_Q6_K, M, bias=bias)
+        assert hip.last_route() == "mmq_q6_k_q8_k_mfma"
+        assert_matmul_parity(got, oracle.matmul(KIND_Q6_K, blocks, x, M, threads=8, bias=bias), what=f"Q6_K {M}x{K} N={N}")
