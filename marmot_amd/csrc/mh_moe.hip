@@ -100,26 +100,28 @@ __global__ __launch_bounds__(64) void k_softmax_rows(const float *__restrict__ x
 // work items of up to MOE_ITEM_COLS routes for the grouped matvec.
 struct RouteArgs {
     const int32_t *topk_ids;      // [T, k]
-    const float *topk_weights;    // [T, k]
     uint32_t *sorted_tokens;      // [routes]
-    float *sorted_weights;        // [routes]
     int *route_pos;               // [T, k] position of each (token, slot) in the sorted order
     int4 *items;                  // work items
     int *n_items;
     int *error_flag;              // 1 when an expert id is out of range, else 0: device memory, or pinned host memory
     int T, k, E;
-    float weights_scale;
-    int renormalize;
     int decode_order;
     int item_cols;                // routes per work item: 8, 16, 32 or 64
     int id_bits;                  // bits of an expert id
+    int span;                     // routes per workgroup
+    int *table;                   // [workgroups, E + 1] routes per expert, and whether an id is bad; null for one workgroup
 };
 
-constexpr int MOE_ROUTE_LDS = 4096;    // routes whose ids and positions are kept in LDS
-// (16384 routes of 128 experts: 120 -> 22 us with eight loads in flight, ranks by ballots instead of 64 lane reads and the
-// records in a launch of their own, 4.5 us; 512 routes 9.6 -> 5.1 us)
+constexpr int MOE_ROUTE_LDS = 4096;    // routes of a workgroup whose expert ids are kept in LDS
 constexpr int MOE_ROUTE_WAVES = 16;    // wavefronts of the route kernel; each fills one contiguous chunk of routes
-constexpr int MOE_EMIT_ROUTES = 2048;  // from more routes than this on their records are written by a launch of its own
+// From more routes than this on the sort is spread over workgroups: one launch counts every workgroup's routes, in the next
+// each places its own. One compute unit alone is bound by its atomics in LDS and by stores to scattered addresses
+// (128 experts, us of one workgroup and the launch that wrote its records / of these two: 2240 routes 10.1 / 9.7, 4096
+// 11.6 / 9.8, 8192 15.7 / 9.8, 16384 24.4 / 11.4; the ids of 16384 routes kept in LDS left the one workgroup at 23).
+constexpr int MOE_SPLIT_ROUTES = 2048;
+constexpr int MOE_SPLIT_SPAN = 1024;   // routes per workgroup: one round of every wavefront
+constexpr int MOE_SPLIT_GROUPS = 64;   // at most, as each reads every one's counts; with more routes the spans grow
 
 // exclusive prefix sum over the 64 lanes of a wavefront; *total receives the sum over all lanes
 __device__ __forceinline__ int wave_excl_scan(int v, int lane, int *total) {
@@ -151,28 +153,54 @@ __device__ __forceinline__ void wave_rank(int id, int lane, int bits, int *rank,
 
 __device__ __forceinline__ void route_emit(const RouteArgs &a, int r, int pos) {
     a.route_pos[r] = pos;
-    if (pos < 0) {
-        return;
+    if (pos >= 0) {
+        a.sorted_tokens[pos] = (uint32_t)r / (uint32_t)a.k;
     }
-    const int t = r / a.k;
-    float norm = a.weights_scale;
-    if (a.renormalize) {
-        float wsum = 0.0f;
-        for (int s = 0; s < a.k; ++s) {
-            wsum += a.topk_weights[t * a.k + s];
-        }
-        norm = wsum > FLT_MIN ? a.weights_scale / wsum : 0.0f;
-    }
-    a.sorted_tokens[pos] = (uint32_t)t;
-    a.sorted_weights[pos] = a.topk_weights[r] * norm;
 }
 
+// Routes per expert of every workgroup's span, for k_moe_route
+__global__ __launch_bounds__(256) void k_moe_count(const RouteArgs a) {
+    __shared__ int counts[MOE_MAX_EXPERTS + 1];
+    for (int e = threadIdx.x; e <= a.E; e += blockDim.x) {
+        counts[e] = 0;
+    }
+    __syncthreads();
+    const int routes = a.T * a.k;
+    const int first = (int)blockIdx.x * a.span;
+    const int last = routes - first < a.span ? routes : first + a.span;
+    for (int base = first; base < last; base += 1024) {
+        int id[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = base + 256 * i + (int)threadIdx.x;
+            id[i] = a.topk_ids[r < last ? r : last - 1];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (base + 256 * i + (int)threadIdx.x < last) {
+                if (id[i] < 0 || id[i] >= a.E) {
+                    counts[a.E] = 1;
+                } else {
+                    atomicAdd(&counts[id[i]], 1);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e <= a.E; e += blockDim.x) {
+        a.table[(size_t)blockIdx.x * (a.E + 1) + e] = counts[e];
+    }
+}
+
+// Bound by latencies: loads of the ids are batched and ranks come from ballots. The weights of the routes are left to the
+// combine, which reads them by token.
 __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteArgs a) {
     warm_kernel_arguments<sizeof(RouteArgs), sizeof(RouteArgs)>();
     __shared__ int counts[MOE_MAX_EXPERTS];
     __shared__ int wcount[MOE_ROUTE_WAVES][MOE_MAX_EXPERTS];  // per chunk: routes of each expert, then its cursor
+    __shared__ int before[MOE_MAX_EXPERTS];  // routes of each expert in the spans of earlier workgroups
     __shared__ int bad_id;
-    __shared__ int ids_l[MOE_ROUTE_LDS];  // expert id of each route (-1 = invalid), later its sorted position
+    __shared__ int ids_l[MOE_ROUTE_LDS];  // expert id of each route of this workgroup (-1 = invalid)
     const int routes = a.T * a.k;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
@@ -215,7 +243,9 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         return;
     }
 
-    const bool in_lds = routes <= MOE_ROUTE_LDS;
+    const int first = (int)blockIdx.x * a.span;
+    const int last = routes - first < a.span ? routes : first + a.span;
+    const bool in_lds = last - first <= MOE_ROUTE_LDS;
     for (int e = tid; e < a.E; e += blockDim.x) {
 #pragma unroll
         for (int w = 0; w < MOE_ROUTE_WAVES; ++w) {
@@ -226,10 +256,10 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         bad_id = 0;
     }
     __syncthreads();
-    // chunk of wavefront w: routes [w * chunk, (w + 1) * chunk), a multiple of 64
-    const int chunk = ((routes + MOE_ROUTE_WAVES * 64 - 1) / (MOE_ROUTE_WAVES * 64)) * 64;
-    const int r_begin = wave * chunk;
-    const int r_end = r_begin + chunk < routes ? r_begin + chunk : routes;
+    // chunk of wavefront w: routes [first + w * chunk, first + (w + 1) * chunk), a multiple of 64
+    const int chunk = ((last - first + MOE_ROUTE_WAVES * 64 - 1) / (MOE_ROUTE_WAVES * 64)) * 64;
+    const int r_begin = first + wave * chunk;
+    const int r_end = r_begin + chunk < last ? r_begin + chunk : last;
     constexpr int BATCH = 8;  // loads in flight per lane: with one, a prompt's counting loop is a chain of memory latencies
     for (int base = r_begin; base < r_end; base += 64 * BATCH) {
         int id[BATCH];
@@ -249,19 +279,36 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
                     atomicAdd(&wcount[wave][id[i]], 1);
                 }
                 if (in_lds) {
-                    ids_l[r] = id[i];
+                    ids_l[r - first] = id[i];
                 }
             }
         }
     }
     __syncthreads();
     for (int e = tid; e < a.E; e += blockDim.x) {
-        int c = 0;
+        int c = 0, b = 0;
+        if (a.table != nullptr) {
+            const int groups = (int)gridDim.x;
+            for (int g0 = 0; g0 < groups; g0 += 16) {
+                int n[16];
 #pragma unroll
-        for (int w = 0; w < MOE_ROUTE_WAVES; ++w) {
-            c += wcount[w][e];
+                for (int g = 0; g < 16; ++g) {
+                    n[g] = a.table[(size_t)(g0 + g < groups ? g0 + g : groups - 1) * (a.E + 1) + e];
+                }
+#pragma unroll
+                for (int g = 0; g < 16; ++g) {
+                    c += g0 + g < groups ? n[g] : 0;
+                    b += g0 + g < (int)blockIdx.x ? n[g] : 0;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int w = 0; w < MOE_ROUTE_WAVES; ++w) {
+                c += wcount[w][e];
+            }
         }
         counts[e] = c;
+        before[e] = b;
     }
     __syncthreads();
     // exclusive prefix over experts in ascending id and the work items of every expert: lane l of the first
@@ -282,20 +329,26 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         for (int e = e0; e < e1; ++e) {
             const int c = counts[e];
             counts[e] = prefix;  // from here on: start of the expert's segment
-            for (int j = 0; j < c; j += a.item_cols) {
+            for (int j = 0; blockIdx.x == 0 && j < c; j += a.item_cols) {
                 a.items[n++] = make_int4(e, prefix + j, (c - j) < a.item_cols ? (c - j) : a.item_cols, 0);
             }
             prefix += c;
         }
-        if (lane == 0) {
-            *a.n_items = n_items;
-            *a.error_flag = bad_id;
+        if (blockIdx.x == 0) {
+            int bad = bad_id;
+            if (a.table != nullptr) {  // (at most one workgroup per lane)
+                bad = __ballot(lane < (int)gridDim.x && a.table[(size_t)lane * (a.E + 1) + a.E] != 0) != 0 ? 1 : 0;
+            }
+            if (lane == 0) {
+                *a.n_items = n_items;
+                *a.error_flag = bad;
+            }
         }
     }
     __syncthreads();
     // cursor of chunk w for expert e: segment start + routes of e in earlier chunks
     for (int e = tid; e < a.E; e += blockDim.x) {
-        int run = counts[e];
+        int run = counts[e] + before[e];
 #pragma unroll
         for (int w = 0; w < MOE_ROUTE_WAVES; ++w) {
             const int c = wcount[w][e];
@@ -309,7 +362,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
     int *cursor = wcount[wave];
     auto id_of = [&](int r) {
         if (in_lds) {
-            return ids_l[r];
+            return ids_l[r - first];
         }
         const int id = a.topk_ids[r];
         return id < 0 || id >= a.E ? -1 : id;
@@ -330,20 +383,8 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
             cursor[id] += cnt;
         }
         if (r < r_end) {
-            if (routes > MOE_EMIT_ROUTES) {
-                a.route_pos[r] = pos;  // k_moe_emit writes the rest
-            } else {
-                route_emit(a, r, pos);
-            }
+            route_emit(a, r, pos);
         }
-    }
-}
-
-// The route records of a prompt, after k_moe_route has placed the routes
-__global__ __launch_bounds__(256) void k_moe_emit(const RouteArgs a) {
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r < a.T * a.k) {
-        route_emit(a, r, a.route_pos[r]);
     }
 }
 
@@ -356,27 +397,31 @@ __global__ __launch_bounds__(256) void k_moe_emit(const RouteArgs a) {
 constexpr int COMBINE_BATCH = 8;
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_moe_combine(const float *__restrict__ route_down,
-                                                     const float *__restrict__ sorted_weights,
-                                                     const int *__restrict__ route_pos, int k, size_t H,
+                                                     const float *__restrict__ topk_weights, float weights_scale,
+                                                     int renormalize, const int *__restrict__ route_pos, int k, size_t H,
                                                      float *__restrict__ out) {
     __shared__ int raw[MOE_MAX_TOPK], pos[MOE_MAX_TOPK];
-    __shared__ float wts[MOE_MAX_TOPK];
+    __shared__ float raw_w[MOE_MAX_TOPK], wts[MOE_MAX_TOPK];
     const size_t t = blockIdx.x;
     const int s = threadIdx.x;
     const int p = s < k ? route_pos[t * k + s] : -1;
+    const float w = s < k ? topk_weights[t * k + s] : 0.0f;
     if (s < k) {
         raw[s] = p;
+        raw_w[s] = w;
     }
-    const float w = p >= 0 ? sorted_weights[p] : 0.0f;
     __syncthreads();
     int n = 0, rank = 0;
+    float wsum = 0.0f;  // of every slot, in slot order, those of an invalid id too
     for (int i = 0; i < k; ++i) {
+        wsum += raw_w[i];
         n += raw[i] >= 0 ? 1 : 0;
         rank += raw[i] >= 0 && raw[i] < p ? 1 : 0;  // (the positions of a token's routes are distinct)
     }
     if (p >= 0) {
         pos[rank] = p;
-        wts[rank] = w;
+        const float norm = !renormalize ? weights_scale : wsum > FLT_MIN ? weights_scale / wsum : 0.0f;
+        wts[rank] = w * norm;
     }
     __syncthreads();
     const size_t h = (size_t)blockIdx.y * 1024 + 4 * (size_t)threadIdx.x;
@@ -549,10 +594,13 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const size_t o_hidden_q = take(act_scratch_layout(act_gu, T, H, nullptr, nullptr));
     const size_t o_fused_q = take(act_scratch_layout(act_dn, routes, F, nullptr, nullptr));
     const size_t o_tokens = take(routes * sizeof(uint32_t));
-    const size_t o_weights = take(routes * sizeof(float));
     const size_t o_pos = take(routes * sizeof(int));
     const size_t o_items = take((max_items + 1) * sizeof(int4));
     const size_t o_flags = take(2 * sizeof(int));
+    const size_t split_span = (routes + (size_t)MOE_SPLIT_GROUPS * MOE_SPLIT_SPAN - 1) /
+                              ((size_t)MOE_SPLIT_GROUPS * MOE_SPLIT_SPAN) * MOE_SPLIT_SPAN;
+    const size_t route_groups = routes > (size_t)MOE_SPLIT_ROUTES ? (routes + split_span - 1) / split_span : 1;
+    const size_t o_table = take(route_groups > 1 ? route_groups * (E + 1) * sizeof(int) : 0);
     const size_t o_gate = take(routes * F * sizeof(float));
     const size_t o_up = take(routes * F * sizeof(float));
     const size_t o_down = take(routes * H * sizeof(float));
@@ -566,7 +614,6 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     act_scratch_layout(act_gu, T, H, base + o_hidden_q, &hidden_q);
     act_scratch_layout(act_dn, routes, F, base + o_fused_q, &fused_q);
     uint32_t *sorted_tokens = (uint32_t *)(base + o_tokens);
-    float *sorted_weights = (float *)(base + o_weights);
     int *route_pos = (int *)(base + o_pos);
     int4 *items = (int4 *)(base + o_items);
     int *flags = (int *)(base + o_flags);  // [0] = number of items, [1] = error flag; both set by the route kernel
@@ -576,9 +623,7 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
 
     RouteArgs ra;
     ra.topk_ids = d_topk_ids;
-    ra.topk_weights = d_topk_weights;
     ra.sorted_tokens = sorted_tokens;
-    ra.sorted_weights = sorted_weights;
     ra.route_pos = route_pos;
     ra.items = items;
     ra.n_items = flags;
@@ -593,8 +638,6 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     ra.T = (int)T;
     ra.k = (int)k_per_token;
     ra.E = (int)E;
-    ra.weights_scale = weights_scale;
-    ra.renormalize = router_weight_policy == MARMOT_HIP_ROUTER_RENORMALIZE_SELECTED;
     // cpu_moe_should_use_decode_path (moe_ops.c:417-424)
     ra.decode_order = (T <= 4 && routes <= 64) ? 1 : 0;
     ra.item_cols = (int)item_cols;
@@ -602,14 +645,16 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     while (((size_t)1 << ra.id_bits) < E) {
         ++ra.id_bits;
     }
-    hipLaunchKernelGGL(k_moe_route, dim3(1), dim3(MOE_ROUTE_WAVES * 64), 0, dev->stream, ra);
+    ra.span = (int)(route_groups > 1 ? split_span : routes);
+    ra.table = route_groups > 1 ? (int *)(base + o_table) : nullptr;
+    if (route_groups > 1) {
+        hipLaunchKernelGGL(k_moe_count, dim3((unsigned)route_groups), dim3(256), 0, dev->stream, ra);
+        MH_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_moe_route, dim3((unsigned)route_groups), dim3(MOE_ROUTE_WAVES * 64), 0, dev->stream, ra);
     MH_HIP(hipGetLastError());
     if (validate) {
         MH_HIP(hipEventRecord(dev->host_word_event, dev->stream));
-    }
-    if (routes > (size_t)MOE_EMIT_ROUTES) {
-        hipLaunchKernelGGL(k_moe_emit, dim3((unsigned)((routes + 255) / 256)), dim3(256), 0, dev->stream, ra);
-        MH_HIP(hipGetLastError());
     }
 
     // hidden states are quantized once per token; routes refer to them through sorted_tokens
@@ -666,13 +711,14 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     if (st != MARMOT_HIP_SUCCESS) {
         return st;
     }
+    const int renormalize = router_weight_policy == MARMOT_HIP_ROUTER_RENORMALIZE_SELECTED;
     const dim3 combine_grid((unsigned)T, (unsigned)((H + 1023) / 1024));
     if (H % 4 == 0 && (((uintptr_t)d_out) & 15) == 0) {
-        hipLaunchKernelGGL(k_moe_combine<true>, combine_grid, dim3(256), 0, dev->stream, route_down, sorted_weights,
-                           route_pos, (int)k_per_token, H, d_out);
+        hipLaunchKernelGGL(k_moe_combine<true>, combine_grid, dim3(256), 0, dev->stream, route_down, d_topk_weights,
+                           weights_scale, renormalize, route_pos, (int)k_per_token, H, d_out);
     } else {
-        hipLaunchKernelGGL(k_moe_combine<false>, combine_grid, dim3(256), 0, dev->stream, route_down, sorted_weights,
-                           route_pos, (int)k_per_token, H, d_out);
+        hipLaunchKernelGGL(k_moe_combine<false>, combine_grid, dim3(256), 0, dev->stream, route_down, d_topk_weights,
+                           weights_scale, renormalize, route_pos, (int)k_per_token, H, d_out);
     }
     MH_HIP(hipGetLastError());
     set_route(tiled ? "moe_experts_tiled" : "moe_experts_grouped");

@@ -5,7 +5,7 @@ import pytest
 from oracle.pyoracle import KIND_Q2_K, KIND_Q3_K, KIND_Q4_1, KIND_Q4_K, KIND_Q5_0, KIND_Q5_1, KIND_Q5_K, KIND_Q6_K, KIND_Q8_0
 from tests.test_oracle_moe import make_experts
 from oracle.pyoracle import KIND_Q8_K
-from tests.util import assert_matmul_parity, assert_moe_parity, gaussian, parity_metrics, quantize_weights
+from tests.util import assert_matmul_parity, assert_moe_parity, gaussian, parity_metrics, quantize_weights, random_valid_blocks
 
 pytestmark = pytest.mark.gpu
 
@@ -81,8 +81,8 @@ def test_moe_small(hip, oracle, kind_gu, kind_dn, T):
 
 @pytest.mark.parametrize("T", [200, 1400])
 def test_moe_many_routes(hip, oracle, T):
-    """Route sort over several chunks of routes (one per wavefront), below and above the number of routes whose ids
-    fit in LDS (4096); every expert gets many work items."""
+    """Route sort over several chunks of routes (one per wavefront), of few rounds and of more than one batch of id
+    loads each; every expert gets many work items."""
     print(f"moe many routes T={T}", flush=True)
     E, F, H, k = 7, 256, 256, 3
     kind = KIND_Q4_K
@@ -93,6 +93,38 @@ def test_moe_many_routes(hip, oracle, T):
     ref = oracle.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind, threads=8)
     got = hip.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind)
     assert_moe_parity(got, ref, what=f"moe many routes T={T}")
+
+
+@pytest.mark.parametrize("T,k,E", [(33, 1, 1), (1023, 1, 1000), (256, 8, 7), (2049, 1, 1024), (2048, 8, 128),
+                                   (8192, 8, 5), (8193, 8, 1024), (4097, 64, 7)])
+def test_moe_route_order(hip, T, k, E):
+    """Every route's place at both sides of the count from which workgroups share the sort (2048), of the one from which
+    their spans grow (65536) and beyond the ids LDS holds (64 x 4096), with chunks that end inside a round, the largest
+    expert id and a single expert: a stable sort by expert, exactly."""
+    rng = np.random.default_rng(T + E)
+    H = F = 256
+    gate, up, down = (random_valid_blocks(rng, KIND_Q4_K, E * n, m) for n, m in ((F, H), (F, H), (H, F)))
+    ids = rng.integers(0, E, (T, k), dtype=np.int32)
+    ids[T // 2, 0] = E - 1
+    st = hip.moe_experts_probe(gaussian(77, (T, H)), gate, up, down, ids, np.full((T, k), 1.0 / k, np.float32), F, E,
+                               KIND_Q4_K, KIND_Q4_K)
+    order = np.argsort(ids.ravel(), kind="stable")
+    pos = np.empty(T * k, np.int64)
+    pos[order] = np.arange(T * k)
+    assert np.array_equal(np.asarray(st["route_pos"]).ravel(), pos)
+    assert np.array_equal(np.asarray(st["sorted_tokens"]).ravel(), order // k)
+
+
+@pytest.mark.parametrize("bad", [-1, 7])
+def test_moe_bad_expert_id_of_a_late_workgroup(hip, bad):
+    """The sort is shared by workgroups and only the last one's routes hold an id out of range: the call is refused."""
+    rng = np.random.default_rng(5)
+    T, k, E, H = 1025, 3, 7, 256
+    gate, up, down = (random_valid_blocks(rng, KIND_Q4_K, E * H, H) for _ in range(3))
+    ids = rng.integers(0, E, (T, k), dtype=np.int32)
+    ids[T - 1, k - 1] = bad
+    with pytest.raises(Exception, match="out of range"):
+        hip.moe_experts(gaussian(78, (T, H)), gate, up, down, ids, np.ones((T, k), np.float32), H, E, KIND_Q4_K, KIND_Q4_K)
 
 
 def test_moe_q6k_experts_with_aligned_rows(hip, oracle):
