@@ -397,6 +397,11 @@ int allow_large_lds(marmot_hip_device *dev, const void *kernel);
 int workspace_reserve(marmot_hip_device *dev, size_t bytes, void **out);
 // Bytes that workspace_reserve grants without an error: all there are, unless it must not allocate
 size_t workspace_room(const marmot_hip_device *dev);
+// What is left of it, in whole 256 bytes, behind `used` bytes
+inline size_t workspace_room_behind(const marmot_hip_device *dev, size_t used) {
+    const size_t room = workspace_room(dev);
+    return room > used ? (room - used) & ~(size_t)255 : 0;
+}
 
 // Carves the activation scratch for `rows` x `k` out of `base`; returns bytes consumed (256-byte rounded).
 size_t act_scratch_layout(int act_kind, size_t rows, size_t k, void *base, ActScratch *out);
@@ -464,7 +469,7 @@ int launch_mmq(marmot_hip_device *dev, int kind, const void *d_w0, const void *d
 // Tiled int8 GEMM on Q8_K activations (mh_gemm_i8.hip): Q4_K, Q5_K and Q6_K weights; 33 activation rows and more
 bool gemm_i8_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,
                      const ActScratch &act);
-size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights);
+size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights, size_t room);
 int launch_gemm_i8(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                    size_t M, int out_dtype, void *scratch);
 // Tiled GEMM of K-quant weights and Q8_K activations on the fp16 matrix cores with integer operands (mh_gemm_int16.hip)
@@ -479,7 +484,7 @@ int launch_gemm_x16_grouped(marmot_hip_device *dev, int kind, const void *d_w0, 
                             const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
                             size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1);
 // Tiled int8 GEMM on Q8_0 activations (mh_gemm_i8.hip): Q8_0 and Q4_0 weights, K a multiple of 256, nine rows and more;
-// `scratch` holds gemm_i8_scratch_bytes for the K-split partial sums
+// `scratch` holds the gemm_i8_scratch_bytes of the call for the K-split partial sums
 bool gemm_q23k_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,
                        const ActScratch &act);
 int launch_gemm_q23k(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
@@ -489,7 +494,7 @@ bool gemm_q80_kind(int kind);  // Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, Q2_K, Q3_K: form
 bool gemm_q80_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,
                       const ActScratch &act);
 int launch_gemm_q80(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
-                    size_t M, int out_dtype, void *scratch);
+                    size_t M, int out_dtype, void *scratch, size_t scratch_bytes);
 int launch_mmq_set(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                    size_t M, int out_dtype, void *scratch);
 bool mmq_grouped_supported(const marmot_hip_device *dev, int kind, size_t K);

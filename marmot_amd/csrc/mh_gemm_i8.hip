@@ -42,6 +42,7 @@ struct GemmI8Params {
     void *out;          // [N][M] of the output type, or fp32 partials [splits][N][M] when splits > 1
     int splits;
     int blocks_per_split;
+    int part = 0;       // k_gemm_q80_tile: rounds of a part of K where one workgroup adds up all parts, else 0
     const void *bias;
     int bias_is_f16;
     int bias_first;     // fp16 output: f16(dot + bias) instead of f16(f16(dot) + bias)
@@ -78,6 +79,9 @@ __device__ __forceinline__ int i8_scale_bytes(uint32_t nib, uint32_t s16) {
     return __builtin_bit_cast(int, r);
 }
 
+template <int NA>
+__device__ __forceinline__ void i8_store(const GemmI8Params &p, const float *tile, int tid, size_t tt, size_t row0, int split);
+
 // The two K groups of a workgroup meet in LDS as one [token][weight row] tile, then every thread stores 16 bytes per
 // step. Lane (j, kh) of wavefront (rg, kg) holds weight row 32 rg + j for tokens 32 a + 8 (r / 4) + 4 kh + r % 4. Every
 // wavefront of the workgroup calls this after its last read of the stages (the function contains barriers).
@@ -108,7 +112,12 @@ __device__ __forceinline__ void i8_merge_and_store(const GemmI8Params &p, uint8_
         }
     }
     i8_lds_barrier();
+    i8_store<NA>(p, tile, tid, tt, row0, split);
+}
 
+// The output tile in LDS to the output
+template <int NA>
+__device__ __forceinline__ void i8_store(const GemmI8Params &p, const float *tile, int tid, size_t tt, size_t row0, int split) {
     const bool partials = p.splits > 1;
     const bool has_bias = !partials && p.bias != nullptr;
     const bool out_f16 = !partials && p.out_is_f16;
@@ -1113,9 +1122,34 @@ struct Q80Raw {
     }
 };
 
-// p.nb counts rounds (K / 256); p.ad holds 8 p.nb scales per token
-template <int KIND, int NA, int STAGES>
-__global__ __launch_bounds__(I8_THREADS, 4) void k_gemm_q80_tile(const GemmI8Params p) {
+// Adds the sums of a part of K, and clears them: the K groups (the same lanes of both hold the same outputs) exchange halves
+// through LDS, and each keeps the sums of its half. Every wavefront of the workgroup calls this; `x` is free before and after.
+template <int NA>
+__device__ __forceinline__ void q80_end_part(float *x, float (&total)[NA][16], float (&sums)[8 * NA], int tid, int kg) {
+    constexpr int H = 8 * NA;  // outputs of a half
+    float *theirs = x + (tid & 255) + (kg == 0 ? H : 0) * 256, *ours = x + (tid & 255) + (kg == 0 ? 0 : H) * 256;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+        const int o = H + i;
+        theirs[i * 256] = kg == 0 ? total[o >> 4][o & 15] : total[i >> 4][i & 15];
+    }
+    i8_lds_barrier();
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+        const int o = H + i;
+        sums[i] += (kg == 0 ? total[i >> 4][i & 15] : total[o >> 4][o & 15]) + ours[i * 256];
+    }
+    i8_lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 16 * NA; ++i) {
+        total[i >> 4][i & 15] = 0.0f;
+    }
+}
+
+// p.nb counts rounds (K / 256); p.ad holds 8 p.nb scales per token. PARTS: the workgroup takes all parts of K, of p.part rounds
+// each, and adds up their sums.
+template <int KIND, int NA, int STAGES, bool PARTS>
+__global__ __launch_bounds__(I8_THREADS, PARTS ? 2 : 4) void k_gemm_q80_tile(const GemmI8Params p) {
     using T = Q80Tile<KIND>;
     constexpr int TOK = 32 * NA;  // tokens per workgroup: 64, or 32 for at most 32 activation rows
     warm_kernel_arguments<sizeof(GemmI8Params)>();
@@ -1225,10 +1259,18 @@ __global__ __launch_bounds__(I8_THREADS, 4) void k_gemm_q80_tile(const GemmI8Par
     const uint32_t a_base = (uint32_t)(T::STAGE_W + j * QK_K);
     const uint32_t d_off = (uint32_t)(T::STAGE_W + I8_STAGE_A + 16 * kh);
 
+    float sums[8 * NA];
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int i = 0; i < 8 * NA; ++i) {
+            sums[i] = 0.0f;
+        }
+    }
     issue(0);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     i8_lds_barrier();
     fold_sums(0);
+    int part_end = PARTS ? p.part : 0;
     for (int ri = 0; ri < nrounds; ++ri) {
         if (STAGES == 2 && ri + 1 < nrounds) {
             issue(ri + 1);  // into the other buffer, which the barrier that closed the previous round has released
@@ -1308,11 +1350,30 @@ __global__ __launch_bounds__(I8_THREADS, 4) void k_gemm_q80_tile(const GemmI8Par
         }
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wavefront's share of the next round has landed
         i8_lds_barrier();
+        if constexpr (PARTS) {
+            static_assert(STAGES == 2, "the stage read last is free until the next round's loads");
+            if (ri + 1 == part_end && ri + 1 < nrounds) {
+                q80_end_part<NA>((float *)(lds + (size_t)(ri & 1) * T::STAGE), total, sums, tid, kg);
+                part_end += p.part;
+            }
+        }
         if (ri + 1 < nrounds) {
             fold_sums(ri + 1);
         }
     }
-    i8_merge_and_store<NA>(p, lds, total, tid, rg, kg, j, kh, tt, row0, split);
+    if constexpr (PARTS) {
+        float *tile = (float *)lds;
+        q80_end_part<NA>(tile, total, sums, tid, kg);
+#pragma unroll
+        for (int i = 0; i < 8 * NA; ++i) {
+            const int o = 8 * NA * kg + i;
+            tile[(32 * (o >> 4) + 8 * ((o & 15) >> 2) + 4 * kh + (o & 3)) * I8_OUT_PITCH + 32 * rg + j] = sums[i];
+        }
+        i8_lds_barrier();
+        i8_store<NA>(p, tile, tid, tt, row0, split);
+    } else {
+        i8_merge_and_store<NA>(p, lds, total, tid, rg, kg, j, kh, tt, row0, split);
+    }
 }
 
 // ------------------------------------------------------------------ Q2_K / Q3_K x Q8_K
@@ -1584,20 +1645,36 @@ static bool q80_format(int kind) {
 // second places are taken too (300 x 4096 x 4096, 160 tiles, whole call: Q8_0 46 us unsplit, 39 in three; Q4_0 44 / 40;
 // Q8_0 300 x 14336 x 4096 161 / 82). The partial sums cost about 6 us: not below 3072 values of K (300 x 1024 x 4096: 18 us
 // unsplit, 24 in two or three).
-static size_t gemm_q80_splits(const marmot_hip_device *dev, size_t N, size_t M, size_t nb, size_t *blocks_per_split) {
+// This split is a choice (gemm_i8_splits leaves such calls unsplit) and may not cost a call its scratch: without room for
+// the partial sums one workgroup takes the parts one after another and adds them up in the same order, to the same bits (the
+// entry point that does not allocate promises them). It takes the time of an unsplit call.
+struct Q80Plan {
+    size_t splits, bps;  // parts of K, rounds per part
+    bool optional;
+};
+static Q80Plan gemm_q80_plan(const marmot_hip_device *dev, size_t N, size_t M, size_t nb) {
     const size_t tiles = ((N + I8_TOK - 1) / I8_TOK) * ((M + I8_WROWS - 1) / I8_WROWS);
     const size_t cus = (size_t)dev->props.multiProcessorCount;
-    if (tiles * 2 <= cus || tiles > cus || nb < 12) {
-        return gemm_i8_splits(dev, N, M, nb, blocks_per_split);
+    Q80Plan pl;
+    pl.optional = tiles * 2 > cus && tiles <= cus && nb >= 12;
+    if (pl.optional) {
+        pl.bps = (nb + 2 * cus / tiles - 1) / (2 * cus / tiles);
+        pl.splits = (nb + pl.bps - 1) / pl.bps;
+    } else {
+        pl.splits = gemm_i8_splits(dev, N, M, nb, &pl.bps);
     }
-    const size_t bps = (nb + 2 * cus / tiles - 1) / (2 * cus / tiles);
-    *blocks_per_split = bps;
-    return (nb + bps - 1) / bps;
+    return pl;
 }
 
-size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights) {
+// Bytes of partial sums of a call that may use `room` bytes for them; more than that only where it cannot do without them
+size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights, size_t room) {
+    if (q80_format(kind)) {
+        const Q80Plan pl = gemm_q80_plan(dev, N, M, K / QK_K);
+        const size_t bytes = pl.splits > 1 ? pl.splits * N * M * sizeof(float) * (size_t)weights : 0;
+        return pl.optional && bytes > room ? 0 : bytes;
+    }
     size_t bps = 0;
-    const size_t splits = q80_format(kind) ? gemm_q80_splits(dev, N, M, K / QK_K, &bps) : gemm_i8_splits(dev, N, M, K / QK_K, &bps);
+    const size_t splits = gemm_i8_splits(dev, N, M, K / QK_K, &bps);
     return splits > 1 ? splits * N * M * sizeof(float) * (size_t)weights : 0;
 }
 
@@ -1610,7 +1687,7 @@ int launch_gemm_i8(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
     float *partial = (float *)scratch;
     if (splits > 1 && partial == nullptr) {
         void *wsp = nullptr;
-        MH_TRY(workspace_reserve(dev, gemm_i8_scratch_bytes(dev, kind, N, K, M, ws.count), &wsp));
+        MH_TRY(workspace_reserve(dev, gemm_i8_scratch_bytes(dev, kind, N, K, M, ws.count, 0), &wsp));
         partial = (float *)wsp;
     }
     MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q4k_q8k_tile));
@@ -1692,14 +1769,18 @@ bool gemm_q80_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K
 
 // at most 32 activation rows: the form with one token tile of 32 per workgroup (half the matrix instructions and
 // epilogue of the 64-token form, whose second tile would hold no token)
-template <int KIND, int NA, int STAGES>
+template <int KIND, int NA, int STAGES, bool PARTS = false>
 static int launch_gemm_q80_form(marmot_hip_device *dev, const GemmI8Params &p, dim3 grid) {
-    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q80_tile<KIND, NA, STAGES>));
-    hipLaunchKernelGGL((k_gemm_q80_tile<KIND, NA, STAGES>), grid, dim3(I8_THREADS), STAGES * Q80Tile<KIND>::STAGE, dev->stream, p);
+    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_q80_tile<KIND, NA, STAGES, PARTS>));
+    hipLaunchKernelGGL((k_gemm_q80_tile<KIND, NA, STAGES, PARTS>), grid, dim3(I8_THREADS), STAGES * Q80Tile<KIND>::STAGE,
+                       dev->stream, p);
     return MARMOT_HIP_SUCCESS;
 }
 template <int KIND>
 static int launch_gemm_q80_kind(marmot_hip_device *dev, const GemmI8Params &p, dim3 grid) {
+    if (p.part != 0) {  // (at most one workgroup per compute unit)
+        return p.N <= 32 ? launch_gemm_q80_form<KIND, 1, 2, true>(dev, p, grid) : launch_gemm_q80_form<KIND, 2, 2, true>(dev, p, grid);
+    }
     if constexpr (!Q80Tile<KIND>::SHARES) {
         // More workgroups than compute units: with one stage two of them share a compute unit, and one computes while the
         // other's loads are on their way (Q8_0, 1024 tokens x 4096 x 14336: 283 us with two stages, 207 with one). At most
@@ -1712,15 +1793,16 @@ static int launch_gemm_q80_kind(marmot_hip_device *dev, const GemmI8Params &p, d
 }
 
 int launch_gemm_q80(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
-                    size_t M, int out_dtype, void *scratch) {
+                    size_t M, int out_dtype, void *scratch, size_t scratch_bytes) {
     if (q23k_format(kind)) {
         return launch_gemm_q23k(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }
     const size_t nb = K / QK_K;
-    size_t bps = 0;
-    const size_t splits = gemm_q80_splits(dev, N, M, nb, &bps);
+    const Q80Plan pl = gemm_q80_plan(dev, N, M, nb);
+    const bool room = scratch != nullptr && pl.splits * N * M * sizeof(float) * (size_t)ws.count <= scratch_bytes;
+    const size_t splits = pl.splits > 1 && pl.optional && !room ? 1 : pl.splits;
     float *partial = (float *)scratch;
-    if (splits > 1 && partial == nullptr) {
+    if (splits > 1 && !room) {
         return set_error(MARMOT_HIP_ERROR_INVALID_ARGUMENT, "tiled Q8_0 GEMM: no room for the K-split partial sums");
     }
     const dim3 grid((unsigned)((M + I8_WROWS - 1) / I8_WROWS), (unsigned)((N + I8_TOK - 1) / I8_TOK), (unsigned)splits);
@@ -1737,7 +1819,8 @@ int launch_gemm_q80(marmot_hip_device *dev, int kind, const WeightSet &ws, const
         float *part = splits > 1 ? partial + (size_t)which * splits * N * M : nullptr;
         p.out = splits > 1 ? (void *)part : ws.out[which];
         p.splits = (int)splits;
-        p.blocks_per_split = (int)bps;
+        p.blocks_per_split = (int)(splits < pl.splits ? nb : pl.bps);
+        p.part = splits < pl.splits ? (int)pl.bps : 0;
         p.bias = ws.bias[which];
         p.bias_is_f16 = ws.bias_dtype == MARMOT_HIP_DTYPE_F16;
         p.bias_first = ws.bias_first ? 1 : 0;

@@ -272,8 +272,9 @@ static int matmul_impl(marmot_hip_device *dev, int kind, const void *d_w0, const
     // Q2_K, Q3_K (from five rows on) and the 32-value formats but Q8_1 (from nine): the tiled int8 GEMMs (their K-split partial
     // sums behind the activations)
     const bool q80_kind = gemm_q80_kind(kind) && N >= gemm_q80_min_rows(kind) && K % QK_K == 0;
-    const size_t need = act_bytes + (mmq ? mmq_scratch_bytes(dev, kind, N, K, M, d_w1 != nullptr ? 2 : 1) : 0) +
-                        (q80_kind ? gemm_i8_scratch_bytes(dev, kind, N, K, M, d_w1 != nullptr ? 2 : 1) : 0);
+    const size_t q80_bytes =
+        q80_kind ? gemm_i8_scratch_bytes(dev, kind, N, K, M, rows_ws.count, workspace_room_behind(dev, act_bytes)) : 0;
+    const size_t need = act_bytes + (mmq ? mmq_scratch_bytes(dev, kind, N, K, M, rows_ws.count) : 0) + q80_bytes;
     void *ws = nullptr;
     int st = workspace_reserve(dev, need, &ws);
     if (st != MARMOT_HIP_SUCCESS) {
@@ -286,7 +287,7 @@ static int matmul_impl(marmot_hip_device *dev, int kind, const void *d_w0, const
         return st;
     }
     if (q80_kind && gemm_q80_applies(dev, kind, N, K, rows_ws.w, rows_ws.count, act)) {
-        return launch_gemm_q80(dev, kind, rows_ws, act, N, K, M, out_dtype, (uint8_t *)ws + act_bytes);
+        return launch_gemm_q80(dev, kind, rows_ws, act, N, K, M, out_dtype, (uint8_t *)ws + act_bytes, q80_bytes);
     }
     if (rows_kernel) {
         st = launch_mmq_rows_q4k(dev, rows_ws, nullptr, &act, N, K, M, out_dtype);
@@ -537,12 +538,12 @@ int marmot_hip_matmul_prepacked(marmot_hip_device_t *dev, int kind, const void *
         ws.bias_dtype = bias_dtype;
         if (gemm_q80_applies(dev, kind, N, K, ws.w, 1, act)) {
             MH_HIP(hipSetDevice(dev->device_index));
-            const size_t partial_bytes = gemm_i8_scratch_bytes(dev, kind, N, K, M, 1);
+            const size_t partial_bytes = gemm_i8_scratch_bytes(dev, kind, N, K, M, 1, workspace_room_behind(dev, 0));
             void *scratch = nullptr;
             if (partial_bytes != 0) {
                 MH_TRY(workspace_reserve(dev, partial_bytes, &scratch));
             }
-            return launch_gemm_q80(dev, kind, ws, act, N, K, M, out_dtype, scratch);
+            return launch_gemm_q80(dev, kind, ws, act, N, K, M, out_dtype, scratch, partial_bytes);
         }
     }
     return launch_matvec_packed(dev, kind, d_weight, nullptr, &act, nullptr, N, K, M, d_bias, bias_dtype, d_out,
@@ -733,9 +734,9 @@ int marmot_hip_matmul_qkv_rope_quantized(marmot_hip_device_t *dev, int kind, con
     // Q2_K, Q3_K (from five rows on) and the 32-value formats but Q8_1 (from nine): the tiled int8 GEMMs, their K-split partial
     // sums where the mmq scratch would be
     const bool q80_kind = !fuse_quant && gemm_q80_kind(kind) && N >= gemm_q80_min_rows(kind) && K % QK_K == 0;
-    const size_t mmq_bytes = mmq ? ((mmq_scratch_bytes(dev, kind, N, K, M, 3) + 255) & ~(size_t)255)
-        : q80_kind               ? ((gemm_i8_scratch_bytes(dev, kind, N, K, M, 3) + 255) & ~(size_t)255)
-                                 : 0;
+    const size_t q80_bytes =
+        q80_kind ? gemm_i8_scratch_bytes(dev, kind, N, K, M, 3, workspace_room_behind(dev, act_bytes + stage_bytes)) : 0;
+    const size_t mmq_bytes = ((mmq ? mmq_scratch_bytes(dev, kind, N, K, M, 3) : q80_bytes) + 255) & ~(size_t)255;
     void *wsp = nullptr;
     int st = MARMOT_HIP_SUCCESS;
     if (act_bytes + mmq_bytes + stage_bytes != 0) {
@@ -768,7 +769,7 @@ int marmot_hip_matmul_qkv_rope_quantized(marmot_hip_device_t *dev, int kind, con
         } else if (mmq) {
             st = launch_mmq_set(dev, kind, ws, act, N, K, M, mm_out_dtype, (uint8_t *)wsp + act_bytes);
         } else if (q80_kind && gemm_q80_applies(dev, kind, N, K, ws.w, ws.count, act)) {
-            st = launch_gemm_q80(dev, kind, ws, act, N, K, M, mm_out_dtype, (uint8_t *)wsp + act_bytes);
+            st = launch_gemm_q80(dev, kind, ws, act, N, K, M, mm_out_dtype, (uint8_t *)wsp + act_bytes, q80_bytes);
         } else {
             st = launch_matvec_set(dev, kind, ws, &act, nullptr, N, K, M, mm_out_dtype);
         }

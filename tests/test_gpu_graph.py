@@ -4,8 +4,8 @@ import numpy as np
 import pytest
 
 from marmot_amd import capi
-from oracle.pyoracle import KIND_Q4_K
-from tests.util import bits, gaussian
+from oracle.pyoracle import KIND_Q4_0, KIND_Q4_1, KIND_Q4_K, KIND_Q8_0
+from tests.util import assert_matmul_parity, bits, gaussian
 
 pytestmark = pytest.mark.gpu
 
@@ -73,4 +73,51 @@ def test_graph_survives_workspace_growth(hip, oracle):
     finally:
         hip.graph_destroy(g)
         for b in (d_w, d_x, d_out):
+            b.free()
+
+
+@pytest.mark.parametrize("kind", [KIND_Q8_0, KIND_Q4_0, KIND_Q4_1])
+def test_prepacked_prompt_is_captured_whatever_the_workspace(hip, oracle, kind):
+    """A 32-value format at 160 tiles splits K where the workspace holds the partial sums (14.7 MB). A call that cannot grow
+    the workspace gives the same bits without them: on a fresh device object, which has none, with a workspace too small for
+    them, and with one that holds them."""
+    N, K, M = 300, 4096, 4096
+    blocks = oracle.quantize(kind, gaussian(810, (M, K), 0.02))
+    x = gaussian(811, (N, K))
+    some = np.r_[0, 1, 63, 64, 127, 128, 255, 256, 298, 299]
+    ref = oracle.matmul(kind, blocks, np.ascontiguousarray(x[some]), M)
+    d_w, d_x, d_out = hip.to_device(blocks), hip.to_device(x), hip.alloc(N * M * 4)
+    d_p = hip.alloc(hip.packed_activation_bytes(kind, N, K))
+    hip.pack_activations_d(kind, d_x, capi.DT_F32, N, K, d_p)
+    hip.synchronize()
+
+    def captured():
+        """The captured call's output, the same on every one of three replays."""
+        g = hip.graph_capture(lambda: hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out))
+        outs = []
+        try:
+            for _ in range(3):
+                d_out.upload(np.full(N * M * 4, 0xFF, dtype=np.uint8))
+                hip.graph_launch(g)
+                hip.synchronize()
+                outs.append(d_out.download(np.float32, (N, M)))
+        finally:
+            hip.graph_destroy(g)
+        assert all(np.array_equal(bits(o), bits(outs[0])) for o in outs)
+        return outs[0]
+
+    try:
+        no_room = captured()
+        # an eager call that needs between 4 and 8 MB of it: 600 packed rows
+        small = oracle.quantize(kind, gaussian(812, (64, 8192), 0.02))
+        hip.linear(gaussian(813, (600, 8192)), small, kind, 64)
+        some_room = captured()
+        hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out)
+        eager = d_out.download(np.float32, (N, M))
+        assert_matmul_parity(eager[some], ref, what="eager")
+        assert np.array_equal(bits(no_room), bits(eager))
+        assert np.array_equal(bits(some_room), bits(eager))
+        assert np.array_equal(bits(captured()), bits(eager))
+    finally:
+        for b in (d_w, d_x, d_p, d_out):
             b.free()

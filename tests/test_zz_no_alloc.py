@@ -65,6 +65,33 @@ def test_packed_matvec_and_fused_routes(hip, oracle):
     list(run_pair(hip, oracle, KIND_Q8_0, [(8, 2048, 640), (1, 1024, 128)], capi.DT_F32))
 
 
+@pytest.mark.parametrize("name", ["q8_0", "q4_0", "q4_1", "q5_0", "q5_1"])
+def test_k_split_of_the_32_value_formats(hip, oracle, name):
+    """Tiles for more than half of the chip: the partial sums of the K split are more than the static array holds (300 rows:
+    14.7 MB), and one workgroup adds up the parts to the same bits, three or two, whole or with a short last one, tokens in
+    tiles of 64 or 32; calls whose partial sums fit; FLOAT16 outputs."""
+    from oracle import pyoracle
+
+    kind = getattr(pyoracle, "KIND_" + name.upper())
+    for route in run_pair(hip, oracle, kind, [(300, 4096, 4096), (1000, 5120, 2047), (200, 3072, 4224), (32, 3584, 21700)], capi.DT_F32):
+        assert route == f"gemm_{name}_q8_0_mfma_tile"
+    N, K, M = 290, 3072, 4001
+    d_w = hip.to_device(oracle.quantize(kind, gaussian(960, (M, K), 0.02)))
+    d_x = hip.to_device(gaussian(961, (N, K)).astype(np.float16))
+    d_out = hip.alloc(N * M * 2)
+    try:
+        hip.linear_d(kind, d_w, d_x, capi.DT_F16, N, K, M, d_out, capi.DT_F16, flags=capi.FLAG_FORCE_PACK)
+        ref = d_out.download(np.uint16, (N, M))
+        d_out.upload(np.full(N * M * 2, 0xFF, dtype=np.uint8))
+        hip.linear_noalloc_d(kind, d_w, d_x, capi.DT_F16, N, K, M, d_out, capi.DT_F16, flags=capi.FLAG_FORCE_PACK)
+        assert hip.last_route() == f"gemm_{name}_q8_0_mfma_tile"
+        got = d_out.download(np.uint16, (N, M))
+        assert np.array_equal(got, ref) and np.all(np.isfinite(got.view(np.float16)))
+    finally:
+        for b in (d_w, d_x, d_out):
+            b.free()
+
+
 def test_oversized_request_is_refused(hip, oracle):
     kind = KIND_Q4_K
     N, K, M = 1024, 8192, 64  # 1024 rows of 8192 int8 values alone exceed the 8 MiB array
