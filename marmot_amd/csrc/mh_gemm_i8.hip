@@ -1642,9 +1642,12 @@ static bool q80_format(int kind) {
            kind == MARMOT_HIP_KIND_Q5_0 || kind == MARMOT_HIP_KIND_Q5_1;
 }
 // The 32-value formats: two workgroups share a compute unit, so from half a chip to a chip of tiles K is split until the
-// second places are taken too (300 x 4096 x 4096, 160 tiles, whole call: Q8_0 46 us unsplit, 39 in three; Q4_0 44 / 40;
-// Q8_0 300 x 14336 x 4096 161 / 82). The partial sums cost about 6 us: not below 3072 values of K (300 x 1024 x 4096: 18 us
-// unsplit, 24 in two or three).
+// second places are taken too: in three up to a third of the places (170 tiles of 256 compute units), else in two. The
+// partial sums cost about 6 us, so the line is a length of K (whole call, us unsplit / split, of Q8_0, Q4_0 and Q5_1):
+//   160 tiles, 300 x K x 4096, three   K = 2048: 25 / 29, 25 / 30, 32 / 33   3072: 34 / 30, 34 / 33, 44 / 38
+//   200 tiles, 200 x K x 6400, two     K = 4096: 43 / 43, 43 / 42, 57 / 55   5120: 52 / 51, 52 / 49, 69 / 64
+// Up to 32 tokens of Q8_0 gain nothing from two below 8192 (256 tiles, 16 x 6144 x 32768: 41 / 47; 8192: 58 / 58; Q4_0 41 / 39,
+// 53 / 47).
 // This split is a choice (gemm_i8_splits leaves such calls unsplit) and may not cost a call its scratch: without room for
 // the partial sums one workgroup takes the parts one after another and adds them up in the same order, to the same bits (the
 // entry point that does not allocate promises them). It takes the time of an unsplit call.
@@ -1652,13 +1655,15 @@ struct Q80Plan {
     size_t splits, bps;  // parts of K, rounds per part
     bool optional;
 };
-static Q80Plan gemm_q80_plan(const marmot_hip_device *dev, size_t N, size_t M, size_t nb) {
+static Q80Plan gemm_q80_plan(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t nb) {
     const size_t tiles = ((N + I8_TOK - 1) / I8_TOK) * ((M + I8_WROWS - 1) / I8_WROWS);
     const size_t cus = (size_t)dev->props.multiProcessorCount;
+    const size_t parts = 2 * cus / tiles;
     Q80Plan pl;
-    pl.optional = tiles * 2 > cus && tiles <= cus && nb >= 12;
+    pl.optional = tiles * 2 > cus && tiles <= cus &&
+                  nb >= (size_t)(parts > 2 ? 12 : kind == MARMOT_HIP_KIND_Q8_0 && N <= 32 ? 32 : 20);
     if (pl.optional) {
-        pl.bps = (nb + 2 * cus / tiles - 1) / (2 * cus / tiles);
+        pl.bps = (nb + parts - 1) / parts;
         pl.splits = (nb + pl.bps - 1) / pl.bps;
     } else {
         pl.splits = gemm_i8_splits(dev, N, M, nb, &pl.bps);
@@ -1669,7 +1674,7 @@ static Q80Plan gemm_q80_plan(const marmot_hip_device *dev, size_t N, size_t M, s
 // Bytes of partial sums of a call that may use `room` bytes for them; more than that only where it cannot do without them
 size_t gemm_i8_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights, size_t room) {
     if (q80_format(kind)) {
-        const Q80Plan pl = gemm_q80_plan(dev, N, M, K / QK_K);
+        const Q80Plan pl = gemm_q80_plan(dev, kind, N, M, K / QK_K);
         const size_t bytes = pl.splits > 1 ? pl.splits * N * M * sizeof(float) * (size_t)weights : 0;
         return pl.optional && bytes > room ? 0 : bytes;
     }
@@ -1798,7 +1803,7 @@ int launch_gemm_q80(marmot_hip_device *dev, int kind, const WeightSet &ws, const
         return launch_gemm_q23k(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }
     const size_t nb = K / QK_K;
-    const Q80Plan pl = gemm_q80_plan(dev, N, M, nb);
+    const Q80Plan pl = gemm_q80_plan(dev, kind, N, M, nb);
     const bool room = scratch != nullptr && pl.splits * N * M * sizeof(float) * (size_t)ws.count <= scratch_bytes;
     const size_t splits = pl.splits > 1 && pl.optional && !room ? 1 : pl.splits;
     float *partial = (float *)scratch;
