@@ -780,12 +780,19 @@ int launch_mmq_rows_q4k(marmot_hip_device *dev, const WeightSet &ws, const float
 // partial sums meet in LDS; the ring runs on into the next row group. Row slots of 240 bytes: the 14 pieces from the
 // 16-byte boundary below the block's start, an odd number of pieces so that 16 rows lie in different banks.
 //
-// What bounds it: per task and compute unit 450 clocks (N = 8), of which the LDS pipe takes about 200 and the vector units
-// 240 (230 instructions per SIMD and task); memory would allow 350. Three stages or twelve wavefronts change nothing.
-// Measured against k_mmq_q6k_ls (us with the quantization launch and, there, the reduction launch; N = 8 / 16):
+// A block's sum is one integer, rounded once, as in k_mmq_q6k_ls: the four lanes of a row add theirs up before the conversion
+// (three exchanges and three additions for four tokens, after which every lane has one token's). Chains of four blocks, those
+// of a wavefront, and the wavefronts in pairs: the rounding error against 64 bits is 0.71 (4096 x 14336) to 1.00 (one block per
+// wavefront) times that kernel's. (Each lane's part converted and summed for itself was up to 1.3 times it, and slower: 8 rows
+// 14336 x 4096 17.6 us, 16 rows 8192 x 16384 37.7.)
+//
+// What bounds it: LDS and the vector units, at about half of what a task takes (N = 8) each; memory would allow three
+// quarters of it. Three stages or twelve wavefronts change nothing.
+// Measured against k_mmq_q6k_ls (us with the quantization launch and, there, the reduction launch; weights from memory;
+// N = 8 / 16):
 //   K x M      14336 x 4096   4096 x 14336   4096 x 4096    4096 x 1024   8192 x 16384   4096 x 128256
-//   before     27.9 / 29.6    29.1 / 31.2    17.5 / 18.4    15.6 / 16.5   45.9 / 49.4    155.4 / 179.7
-//   now        17.7 / 21.8    18.4 / 22.2     9.7 / 11.4     8.8 / 10.2   29.4 / 37.0    104.4 / 129.6
+//   before     28.3 / 29.3    28.8 / 30.8    18.2 / 18.2    16.1 / 17.0   47.3 / 48.8    152.8 / 176.9
+//   now        16.9 / 20.6    17.5 / 21.1     9.8 / 11.3     9.1 / 9.6    29.4 / 35.8    101.2 / 120.7
 struct MmqRowsQ6Params {
     const uint8_t *w[3];
     void *out[3];
@@ -806,6 +813,14 @@ struct MmqRowsQ6Lds {
     static constexpr int PART = NQ * 256;               // partial sums of one wavefront: [token / 4][row][token % 4]
     static constexpr int bytes(int waves) { return ZERO + waves * (2 * PART + STAGES * STAGE); }
 };
+
+// Sums over the four lanes of a weight row: lane (r, g) gets that of v[g]. Two exchanges of half a wavefront, one of rows of 16.
+__device__ __forceinline__ int q6_join_rows(const int (&v)[4]) {
+    const auto a = __builtin_amdgcn_permlane32_swap((unsigned)v[0], (unsigned)v[2], false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap((unsigned)v[1], (unsigned)v[3], false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[0] + a[1], b[0] + b[1], false, false);
+    return (int)(c[0] + c[1]);
+}
 
 template <int NQ>
 __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
@@ -909,18 +924,17 @@ __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
         }
     };
 
-    float acc[NQ][4];
+    float acc[NQ], total[NQ];  // token 4 a + g of row r: the last blocks' chain and those before it
+    uint32_t chain = 0;
     uint32_t own = 0;  // where this lane's weight row begins, modulo 16
     auto work_group = [&](uint32_t i) {
         const uint32_t row0 = (group0 + i) * 16u, last = p.M - 1u - row0;
         own = (uint32_t)(((uint64_t)row0 + ((uint32_t)r < last ? (uint32_t)r : last)) * p.row_bytes) & 15u;
 #pragma unroll
         for (int a = 0; a < NQ; ++a) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                acc[a][k] = 0.0f;
-            }
+            acc[a] = total[a] = 0.0f;
         }
+        chain = 0;
     };
 
     issue_group(0);
@@ -971,6 +985,18 @@ __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
         sc[0] = __builtin_amdgcn_alignbit(tail[1 + 2 * (g >> 1)], tail[2 * (g >> 1)], shift);
         sc[1] = __builtin_amdgcn_alignbit(tail[2 + 2 * (g >> 1)], tail[1 + 2 * (g >> 1)], shift);
         const uint16_t dh = (uint16_t)(tail[4] >> shift);
+        // every LDS read of the task before its first use (left alone, the compiler reads an operand where it is used and waits)
+        mr_intx4 av[4][NQ];
+        float ad[NQ];
+#pragma unroll
+        for (int a = 0; a < NQ; ++a) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                av[q][a] = *(const mr_intx4 *)(codes[q & 1] + a * 1024 + (q >> 1) * 512);
+            }
+            ad[a] = *(const float *)(stage + L::D_OFF + 16 * a + 4 * g);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         int sums[NQ][4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -990,44 +1016,35 @@ __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
 #pragma unroll
             for (int a = 0; a < NQ; ++a) {
                 const mr_intx4 zero = {0, 0, 0, 0};
-                const mr_intx4 av = *(const mr_intx4 *)(codes[q & 1] + a * 1024 + (q >> 1) * 512);
-                const mr_intx4 dot = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, wv, zero, 0, 0, 0);
+                const mr_intx4 dot = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[q][a], wv, zero, 0, 0, 0);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     sums[a][k] = q == 0 ? __mul24(dot[k], scale) : sums[a][k] + __mul24(dot[k], scale);
                 }
             }
         }
-        const float d = h2f(dh) * 0.25f;
+        const float d = h2f(dh);
 #pragma unroll
         for (int a = 0; a < NQ; ++a) {
-            const float4 ad = *(const float4 *)(stage + L::D_OFF + 16 * a);
-            acc[a][0] += (ad.x * d) * (float)sums[a][0];
-            acc[a][1] += (ad.y * d) * (float)sums[a][1];
-            acc[a][2] += (ad.z * d) * (float)sums[a][2];
-            acc[a][3] += (ad.w * d) * (float)sums[a][3];
+            acc[a] += (ad[a] * d) * (float)(q6_join_rows(sums[a]) >> 2);
+        }
+        if (++chain == 4) {
+            chain = 0;
+#pragma unroll
+            for (int a = 0; a < NQ; ++a) {
+                total[a] += acc[a];
+                acc[a] = 0.0f;
+            }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // the stage is read before it is written again
         free_slot = slot;
         slot = slot + 1 == (uint32_t)S ? 0 : slot + 1;
         if ((block += (uint32_t)waves) == b1) {
-            // the four lanes of a row hold the sums of four scale groups; then the wavefronts' partial sums in K order.
-            // Two buffers: a wavefront writes the next group's while others still read this one's
+            // the wavefronts' partial sums; two buffers: a wavefront writes the next group's while others still read this one's
             uint8_t *part = (uint8_t *)parts + (group & 1u) * (uint32_t)(waves * L::PART);
 #pragma unroll
             for (int a = 0; a < NQ; ++a) {
-                float4 v;
-                float *f = (float *)&v;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    float s = acc[a][k];
-                    s += __shfl_xor(s, 16);
-                    s += __shfl_xor(s, 32);
-                    f[k] = s;
-                }
-                if (g == a) {
-                    *(float4 *)(part + wave * L::PART + a * 256 + r * 16) = v;
-                }
+                *(float *)(part + wave * L::PART + a * 256 + r * 16 + 4 * g) = total[a] + acc[a];
             }
             asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
             __builtin_amdgcn_s_barrier();
@@ -1036,10 +1053,16 @@ __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
                 const uint32_t row = (group0 + group) * 16u + ((uint32_t)i & 15u), tk = (uint32_t)i >> 4;
                 if (tk < p.N && row < p.M) {
                     const float *src = (const float *)(part + (tk >> 2) * 256 + (i & 15) * 16) + (tk & 3u);
-                    float s = src[0];
-                    for (int w = 1; w < waves; ++w) {
-                        s += src[w * (L::PART / 4)];
+                    float v[8];
+#pragma unroll
+                    for (int w = 0; w < 8; ++w) {
+                        v[w] = src[(w < waves ? w : 0) * (L::PART / 4)];
                     }
+#pragma unroll
+                    for (int w = 2; w < 8; ++w) {  // (there are two wavefronts at least)
+                        v[w] = w < waves ? v[w] : 0.0f;
+                    }
+                    const float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
                     float bv = 0.0f;
                     if (bias != nullptr) {
                         bv = mr_bias(p, bias, row);
@@ -1056,7 +1079,7 @@ __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
     }
 }
 
-// Rows of one block stay on the streaming kernel: there is no K to split, and its sum of a block is one integer.
+// Rows of one block stay on the streaming kernel: there is no K to split over the wavefronts.
 bool mmq_rows_q6k_supported(const marmot_hip_device *dev, size_t N, size_t K, size_t M) {
     const size_t row_bytes = K / QK_K * Q6_K_BYTES;
     return !dev->knobs.no_row_kernels && N >= 1 && N <= 16 && K % QK_K == 0 && K >= 2 * QK_K && M >= 1 &&

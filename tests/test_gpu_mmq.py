@@ -717,3 +717,62 @@ def test_q6k_up_to_16_rows_by_row_groups(hip, oracle, M, K):
         got = hip.linear(x, blocks, KIND_Q6_K, M, bias=bias)
         assert hip.last_route() == "mmq_q6_k_q8_k_mfma"
         assert_matmul_parity(got, oracle.matmul(KIND_Q6_K, blocks, x, M, threads=8, bias=bias), what=f"Q6_K {M}x{K} N={N}")
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 512, 5), (70, 2048, 16), (1024, 4096, 9), (4096, 4096, 8), (4096, 14336, 8),
+                                   (7000, 14336, 8), (14336, 4096, 12), (32785, 768, 8)])
+def test_q6k_up_to_16_rows_rounds_a_block_once(hip, oracle, monkeypatch, M, K, N):
+    """Block sums of more than 24 bits (large codes and scales) are integers up to the one conversion. One block with a scale:
+    the output is the product of three rounded factors, bit for bit. All blocks: the error against 64 bits is no larger than
+    that of the streaming kernel, which a device object without the row kernels keeps (sum of 16 scale groups and block
+    products in the same roundings, K split into other parts)."""
+    from marmot_amd import HipBackend
+
+    rng = np.random.default_rng(480 + M)
+    nb = K // 256
+    blocks = random_valid_blocks(rng, KIND_Q6_K, M, K).reshape(M, nb, 210).copy()
+    blocks[:, :, 192:208] = rng.choice(np.array([-128, -127, -100, 90, 127], np.int8), size=(M, nb, 16)).view(np.uint8)
+    blocks[::2, :, 128:192] = 0  # every other row: values of -32 .. -17 with negative scales
+    blocks[::2, :, 192:208] = rng.choice(np.array([-128, -127, -100], np.int8), size=blocks[::2, :, 192:208].shape).view(np.uint8)
+    d = (rng.uniform(0.5, 1.0, (M, nb)) * 1e-4).astype(np.float16)
+    ones = blocks.copy()
+    ones[:, :, 208:210] = np.ones((M, nb), np.float16).view(np.uint8).reshape(M, nb, 2)
+    w = oracle.dequantize(KIND_Q6_K, ones.reshape(M, nb * 210), K).reshape(M, nb, 256)  # code times scale, exact
+    q = rng.choice(np.array([-127, -120, 100, 127], np.int8), size=(N, nb, 256))
+    q[::2] = np.abs(q[::2])
+    ad = rng.uniform(0.01, 0.03, (N, nb)).astype(np.float32)
+    lay = hip.packed_activation_layout(KIND_Q6_K, N, K)
+    image = np.zeros(lay.total_bytes, np.uint8)
+    image[lay.values_offset:lay.values_offset + q.size] = q.view(np.uint8).reshape(-1)
+    image[lay.scales_offset:lay.scales_offset + ad.nbytes] = ad.view(np.uint8).reshape(-1)
+    dots = np.stack([q[:, b].astype(np.float64) @ w[:, b].astype(np.float64).T for b in range(nb)])  # [nb, N, M], exact
+    assert np.max(np.abs(dots)) > 2.0 ** 24
+
+    def run(backend, d_now):
+        now = blocks.copy()
+        now[:, :, 208:210] = d_now.view(np.uint8).reshape(M, nb, 2)
+        d_w, d_p, d_out = backend.to_device(now.reshape(M, nb * 210)), backend.to_device(image), backend.alloc(N * M * 4)
+        backend.linear_prepacked_d(KIND_Q6_K, d_w, d_p, N, K, M, d_out)
+        out = d_out.download(np.float32, (N, M))
+        for b_ in (d_w, d_p, d_out):
+            b_.free()
+        return out
+
+    one = int(rng.integers(nb))
+    only = np.zeros_like(d)
+    only[:, one] = d[:, one]
+    factor = (ad[:, one][:, None] * d[:, one].astype(np.float32)[None, :]).astype(np.float32)
+    assert np.array_equal(bits(run(hip, only)), bits(factor * dots[one].astype(np.float32)))
+
+    exact = np.einsum("bnm,nb,mb->nm", dots, ad.astype(np.float64), d.astype(np.float64))
+    monkeypatch.setenv("MARMOT_HIP_NO_ROW_KERNELS", "1")
+    plain = HipBackend(0)
+    monkeypatch.delenv("MARMOT_HIP_NO_ROW_KERNELS")
+    try:
+        before = run(plain, d)
+    finally:
+        plain.close()
+    error = lambda got: np.sqrt(np.mean((got.astype(np.float64) - exact) ** 2))
+    print(f"M={M} K={K} N={N}: error ratio {error(run(hip, d)) / error(before):.3f}", flush=True)
+    # (two samples of N * M roundings each: a tenth over 165 outputs is noise, a hundredth over 30000)
+    assert error(run(hip, d)) <= (1.0 + 1.5 / np.sqrt(N * M)) * error(before)
