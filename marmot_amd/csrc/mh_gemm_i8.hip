@@ -1645,9 +1645,9 @@ static bool q80_format(int kind) {
 // second places are taken too: in three up to a third of the places (170 tiles of 256 compute units), else in two. The
 // partial sums cost about 6 us, so the line is a length of K (whole call, us unsplit / split, of Q8_0, Q4_0 and Q5_1):
 //   160 tiles, 300 x K x 4096, three   K = 2048: 25 / 29, 25 / 30, 32 / 33   3072: 34 / 30, 34 / 33, 44 / 38
-//   200 tiles, 200 x K x 6400, two     K = 4096: 43 / 43, 43 / 42, 57 / 55   5120: 52 / 51, 52 / 49, 69 / 64
-// Up to 32 tokens of Q8_0 gain nothing from two below 8192 (256 tiles, 16 x 6144 x 32768: 41 / 47; 8192: 58 / 58; Q4_0 41 / 39,
-// 53 / 47).
+//   200 tiles, 200 x K x 6400, two     K = 3072: 35 / 36, 34 / 36, 45 / 44   4096: 43 / 43, 43 / 42, 57 / 55
+//                                      K = 5120: 52 / 51, 52 / 49, 69 / 64
+//   256 tiles, 16 x K x 32768, two     K = 6144: 41 / 47, 41 / 39, 53 / 51   8192: 58 / 58, 53 / 47, 69 / 64
 // This split is a choice (gemm_i8_splits leaves such calls unsplit) and may not cost a call its scratch: without room for
 // the partial sums one workgroup takes the parts one after another and adds them up in the same order, to the same bits (the
 // entry point that does not allocate promises them). It takes the time of an unsplit call.
@@ -1661,7 +1661,7 @@ static Q80Plan gemm_q80_plan(const marmot_hip_device *dev, int kind, size_t N, s
     const size_t parts = 2 * cus / tiles;
     Q80Plan pl;
     pl.optional = tiles * 2 > cus && tiles <= cus &&
-                  nb >= (size_t)(parts > 2 ? 12 : kind == MARMOT_HIP_KIND_Q8_0 && N <= 32 ? 32 : 20);
+                  nb >= (size_t)(parts > 2 ? 12 : kind != MARMOT_HIP_KIND_Q8_0 ? 16 : N > 32 ? 20 : 32);
     if (pl.optional) {
         pl.bps = (nb + parts - 1) / parts;
         pl.splits = (nb + pl.bps - 1) / pl.bps;
