@@ -508,7 +508,9 @@ int marmot_hip_softmax_rows(marmot_hip_device_t *dev, const float *d_x, size_t r
  *   d_out [T,H] fp32 (fully overwritten).
  * An expert id out of range returns MARMOT_HIP_ERROR_INVALID_ARGUMENT: the call waits for the kernel that sorts the routes
  * (not for the experts: d_out is complete in stream order, like every output; with the error it has waited for the experts
- * too, and the buffers are the caller's again). No wait and no check while a graph is being captured. */
+ * too, and the buffers are the caller's again). No wait and no check while a graph is being captured. That kernel is the last
+ * to read d_topk_ids and d_topk_weights: after a call that waited they may be written from any stream, and d_out may overlap
+ * them. */
 int marmot_hip_moe_experts(marmot_hip_device_t *dev, const float *d_hidden, size_t T, size_t H, size_t F, size_t E,
                            size_t k_per_token, int kind_gate_up, int kind_down, const void *d_gate, const void *d_up,
                            const void *d_down, const int32_t *d_topk_ids, const float *d_topk_weights,

@@ -100,6 +100,8 @@ __global__ __launch_bounds__(64) void k_softmax_rows(const float *__restrict__ x
 // work items of up to MOE_ITEM_COLS routes for the grouped matvec.
 struct RouteArgs {
     const int32_t *topk_ids;      // [T, k]
+    const float *topk_weights;    // [T, k]
+    float *weights;               // [T, k] a copy: the combine runs when the caller's may already be overwritten (by d_out)
     uint32_t *sorted_tokens;      // [routes]
     int *route_pos;               // [T, k] position of each (token, slot) in the sorted order
     int4 *items;                  // work items
@@ -151,8 +153,9 @@ __device__ __forceinline__ void wave_rank(int id, int lane, int bits, int *rank,
     *cnt = __builtin_popcountll(same);
 }
 
-__device__ __forceinline__ void route_emit(const RouteArgs &a, int r, int pos) {
+__device__ __forceinline__ void route_emit(const RouteArgs &a, int r, int pos, float weight) {
     a.route_pos[r] = pos;
+    a.weights[r] = weight;
     if (pos >= 0) {
         a.sorted_tokens[pos] = (uint32_t)r / (uint32_t)a.k;
     }
@@ -192,8 +195,8 @@ __global__ __launch_bounds__(256) void k_moe_count(const RouteArgs a) {
     }
 }
 
-// Bound by latencies: loads of the ids are batched and ranks come from ballots. The weights of the routes are left to the
-// combine, which reads them by token.
+// Bound by latencies: loads of the ids are batched and ranks come from ballots. The weights of the routes are copied as they
+// are; the combine scales them, by token.
 __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteArgs a) {
     warm_kernel_arguments<sizeof(RouteArgs), sizeof(RouteArgs)>();
     __shared__ int counts[MOE_MAX_EXPERTS];
@@ -212,8 +215,10 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
             return;
         }
         int id = -1;
+        float weight = 0.0f;
         if (lane < routes) {
             id = a.topk_ids[lane];
+            weight = a.topk_weights[lane];
             if (id < 0 || id >= a.E) {
                 id = -1;
             }
@@ -234,7 +239,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the segment starts are in LDS (same wavefront)
         if (lane < routes) {
-            route_emit(a, lane, id >= 0 ? counts[id] + rank : -1);
+            route_emit(a, lane, id >= 0 ? counts[id] + rank : -1, weight);
         }
         if (lane == 0) {
             *a.n_items = n_items;
@@ -260,6 +265,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
     const int chunk = ((last - first + MOE_ROUTE_WAVES * 64 - 1) / (MOE_ROUTE_WAVES * 64)) * 64;
     const int r_begin = first + wave * chunk;
     const int r_end = r_begin + chunk < last ? r_begin + chunk : last;
+    float next_weight = r_begin + lane < r_end ? a.topk_weights[r_begin + lane] : 0.0f;  // requested before the ids are waited for
     constexpr int BATCH = 8;  // loads in flight per lane: with one, a prompt's counting loop is a chain of memory latencies
     for (int base = r_begin; base < r_end; base += 64 * BATCH) {
         int id[BATCH];
@@ -371,7 +377,9 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
     for (int base = r_begin; base < r_end; base += 64) {
         const int r = base + lane;
         const int id = next;
+        const float weight = next_weight;
         next = r + 64 < r_end ? id_of(r + 64) : -1;
+        next_weight = r + 64 < r_end ? a.topk_weights[r + 64] : 0.0f;
         int rank, cnt;
         wave_rank(id, lane, a.id_bits, &rank, &cnt);
         int pos = -1;
@@ -383,7 +391,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
             cursor[id] += cnt;
         }
         if (r < r_end) {
-            route_emit(a, r, pos);
+            route_emit(a, r, pos, weight);
         }
     }
 }
@@ -397,7 +405,7 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * 64) void k_moe_route(const RouteA
 constexpr int COMBINE_BATCH = 8;
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_moe_combine(const float *__restrict__ route_down,
-                                                     const float *__restrict__ topk_weights, float weights_scale,
+                                                     const float *__restrict__ weights, float weights_scale,
                                                      int renormalize, const int *__restrict__ route_pos, int k, size_t H,
                                                      float *__restrict__ out) {
     __shared__ int raw[MOE_MAX_TOPK], pos[MOE_MAX_TOPK];
@@ -405,7 +413,7 @@ __global__ __launch_bounds__(256) void k_moe_combine(const float *__restrict__ r
     const size_t t = blockIdx.x;
     const int s = threadIdx.x;
     const int p = s < k ? route_pos[t * k + s] : -1;
-    const float w = s < k ? topk_weights[t * k + s] : 0.0f;
+    const float w = s < k ? weights[t * k + s] : 0.0f;
     if (s < k) {
         raw[s] = p;
         raw_w[s] = w;
@@ -594,14 +602,16 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const size_t o_hidden_q = take(act_scratch_layout(act_gu, T, H, nullptr, nullptr));
     const size_t o_fused_q = take(act_scratch_layout(act_dn, routes, F, nullptr, nullptr));
     const size_t o_tokens = take(routes * sizeof(uint32_t));
+    const size_t o_weights = take(routes * sizeof(float));
     const size_t o_pos = take(routes * sizeof(int));
     const size_t o_items = take((max_items + 1) * sizeof(int4));
     const size_t o_flags = take(2 * sizeof(int));
     const size_t split_span = (routes + (size_t)MOE_SPLIT_GROUPS * MOE_SPLIT_SPAN - 1) /
                               ((size_t)MOE_SPLIT_GROUPS * MOE_SPLIT_SPAN) * MOE_SPLIT_SPAN;
     const size_t route_groups = routes > (size_t)MOE_SPLIT_ROUTES ? (routes + split_span - 1) / split_span : 1;
-    const size_t o_table = take(route_groups > 1 ? route_groups * (E + 1) * sizeof(int) : 0);
-    const size_t o_gate = take(routes * F * sizeof(float));
+    const size_t table_bytes = route_groups > 1 ? route_groups * (E + 1) * sizeof(int) : 0;
+    const size_t gate_bytes = routes * F * sizeof(float);
+    const size_t o_gate = take(gate_bytes > table_bytes ? gate_bytes : table_bytes);  // the counts lie where gate comes later
     const size_t o_up = take(routes * F * sizeof(float));
     const size_t o_down = take(routes * H * sizeof(float));
     void *ws = nullptr;
@@ -614,6 +624,7 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     act_scratch_layout(act_gu, T, H, base + o_hidden_q, &hidden_q);
     act_scratch_layout(act_dn, routes, F, base + o_fused_q, &fused_q);
     uint32_t *sorted_tokens = (uint32_t *)(base + o_tokens);
+    float *weights = (float *)(base + o_weights);
     int *route_pos = (int *)(base + o_pos);
     int4 *items = (int4 *)(base + o_items);
     int *flags = (int *)(base + o_flags);  // [0] = number of items, [1] = error flag; both set by the route kernel
@@ -623,6 +634,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
 
     RouteArgs ra;
     ra.topk_ids = d_topk_ids;
+    ra.topk_weights = d_topk_weights;
+    ra.weights = weights;
     ra.sorted_tokens = sorted_tokens;
     ra.route_pos = route_pos;
     ra.items = items;
@@ -646,7 +659,7 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
         ++ra.id_bits;
     }
     ra.span = (int)(route_groups > 1 ? split_span : routes);
-    ra.table = route_groups > 1 ? (int *)(base + o_table) : nullptr;
+    ra.table = route_groups > 1 ? (int *)(base + o_gate) : nullptr;
     if (route_groups > 1) {
         hipLaunchKernelGGL(k_moe_count, dim3((unsigned)route_groups), dim3(256), 0, dev->stream, ra);
         MH_HIP(hipGetLastError());
@@ -714,11 +727,11 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const int renormalize = router_weight_policy == MARMOT_HIP_ROUTER_RENORMALIZE_SELECTED;
     const dim3 combine_grid((unsigned)T, (unsigned)((H + 1023) / 1024));
     if (H % 4 == 0 && (((uintptr_t)d_out) & 15) == 0) {
-        hipLaunchKernelGGL(k_moe_combine<true>, combine_grid, dim3(256), 0, dev->stream, route_down, d_topk_weights,
-                           weights_scale, renormalize, route_pos, (int)k_per_token, H, d_out);
+        hipLaunchKernelGGL(k_moe_combine<true>, combine_grid, dim3(256), 0, dev->stream, route_down, weights, weights_scale,
+                           renormalize, route_pos, (int)k_per_token, H, d_out);
     } else {
-        hipLaunchKernelGGL(k_moe_combine<false>, combine_grid, dim3(256), 0, dev->stream, route_down, d_topk_weights,
-                           weights_scale, renormalize, route_pos, (int)k_per_token, H, d_out);
+        hipLaunchKernelGGL(k_moe_combine<false>, combine_grid, dim3(256), 0, dev->stream, route_down, weights, weights_scale,
+                           renormalize, route_pos, (int)k_per_token, H, d_out);
     }
     MH_HIP(hipGetLastError());
     set_route(tiled ? "moe_experts_tiled" : "moe_experts_grouped");

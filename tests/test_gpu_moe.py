@@ -127,6 +127,39 @@ def test_moe_bad_expert_id_of_a_late_workgroup(hip, bad):
         hip.moe_experts(gaussian(78, (T, H)), gate, up, down, ids, np.ones((T, k), np.float32), H, E, KIND_Q4_K, KIND_Q4_K)
 
 
+@pytest.mark.parametrize("T,k", [(2, 8), (40, 8), (1025, 1), (1300, 8)])
+def test_moe_output_over_the_router_buffers(hip, T, k):
+    """The sort has read expert ids and router weights when the output is written: both may lie inside it, at its first rows
+    or its last, for one wavefront, one workgroup (of one and of several rounds) and several."""
+    import ctypes as C
+
+    from marmot_amd.capi import check
+
+    rng = np.random.default_rng(T)
+    E, F, H = 11, 256, 512
+    gate, up, down = (random_valid_blocks(rng, KIND_Q4_K, E * n, m) for n, m in ((F, H), (F, H), (H, F)))
+    hidden = gaussian(79, (T, H))
+    ids = rng.integers(0, E, (T, k), dtype=np.int32)
+    w = rng.uniform(0.05, 1.0, (T, k)).astype(np.float32)
+    ref = hip.moe_experts(hidden, gate, up, down, ids, w, F, E, KIND_Q4_K, KIND_Q4_K, policy=2)
+    bufs = [hip.to_device(a) for a in (hidden, gate, up, down)]
+    d_out = hip.alloc(T * H * 4)
+    vp = lambda b, at=0: C.c_void_p(b.ptr + at)
+    try:
+        for at in (0, (T * H * 4 - 2 * ids.nbytes) // 16 * 16):
+            image = np.zeros(T * H * 4, np.uint8)
+            image[at:at + ids.nbytes] = ids.view(np.uint8).reshape(-1)
+            image[at + ids.nbytes:at + 2 * ids.nbytes] = w.view(np.uint8).reshape(-1)
+            d_out.upload(image)
+            check(hip.lib.marmot_hip_moe_experts(hip.dev, vp(bufs[0]), T, H, F, E, k, KIND_Q4_K, KIND_Q4_K, vp(bufs[1]),
+                                                 vp(bufs[2]), vp(bufs[3]), vp(d_out, at), vp(d_out, at + ids.nbytes), 1.0, 2, 0,
+                                                 vp(d_out)))
+            assert np.array_equal(d_out.download(np.float32, (T, H)).view(np.uint32), ref.view(np.uint32)), at
+    finally:
+        for b in bufs + [d_out]:
+            b.free()
+
+
 def test_moe_q6k_experts_with_aligned_rows(hip, oracle):
     """Q6_K experts whose rows hold a multiple of 8 blocks (K = 2048): the grouped matmuls take the loader/consumer
     kernel with its 16-byte aligned row copies, both the dual gate/up launch and the down launch."""
