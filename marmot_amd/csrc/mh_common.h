@@ -449,7 +449,7 @@ bool mmq_rows_supported(const marmot_hip_device *dev, int kind, size_t N, size_t
 int launch_mmq_rows_q4k(marmot_hip_device *dev, const WeightSet &ws, const float *d_x_f32, const ActScratch *act,
                         size_t N, size_t K, size_t M, int out_dtype);
 // The same for Q6_K, packed rows only
-bool mmq_rows_q6k_supported(const marmot_hip_device *dev, size_t N, size_t K, size_t M);
+bool mmq_rows_q6k_applies(const marmot_hip_device *dev, const WeightSet &ws, size_t N, size_t K, size_t M);
 int launch_mmq_rows_q6k(marmot_hip_device *dev, const WeightSet &ws, const ActScratch &act, size_t N, size_t K, size_t M,
                         int out_dtype);
 // quantizes act(gate) * up (SwiGLU or GeGLU) of two fp32 [rows, k] arrays into the activation scratch
@@ -462,7 +462,7 @@ int launch_matvec_f16(marmot_hip_device *dev, int kind, const void *d_w, const v
                       const void *d_bias, int bias_dtype, void *d_out, int out_dtype);
 // small-batch int8-MFMA matmul (mh_mmq.hip)
 bool mmq_supported(const marmot_hip_device *dev, int kind, size_t N, size_t K, int weights = 1);
-size_t mmq_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights);
+size_t mmq_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, const WeightSet &ws);
 int launch_mmq(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, const ActScratch &act, size_t N,
                size_t K, size_t M, const void *d_bias, int bias_dtype, void *d_out0, void *d_out1, int out_dtype,
                void *scratch);

@@ -274,7 +274,7 @@ static int matmul_impl(marmot_hip_device *dev, int kind, const void *d_w0, const
     const bool q80_kind = gemm_q80_kind(kind) && N >= gemm_q80_min_rows(kind) && K % QK_K == 0;
     const size_t q80_bytes =
         q80_kind ? gemm_i8_scratch_bytes(dev, kind, N, K, M, rows_ws.count, workspace_room_behind(dev, act_bytes)) : 0;
-    const size_t need = act_bytes + (mmq ? mmq_scratch_bytes(dev, kind, N, K, M, rows_ws.count) : 0) + q80_bytes;
+    const size_t need = act_bytes + (mmq ? mmq_scratch_bytes(dev, kind, N, K, M, rows_ws) : 0) + q80_bytes;
     void *ws = nullptr;
     int st = workspace_reserve(dev, need, &ws);
     if (st != MARMOT_HIP_SUCCESS) {
@@ -736,7 +736,7 @@ int marmot_hip_matmul_qkv_rope_quantized(marmot_hip_device_t *dev, int kind, con
     const bool q80_kind = !fuse_quant && gemm_q80_kind(kind) && N >= gemm_q80_min_rows(kind) && K % QK_K == 0;
     const size_t q80_bytes =
         q80_kind ? gemm_i8_scratch_bytes(dev, kind, N, K, M, 3, workspace_room_behind(dev, act_bytes + stage_bytes)) : 0;
-    const size_t mmq_bytes = ((mmq ? mmq_scratch_bytes(dev, kind, N, K, M, 3) : q80_bytes) + 255) & ~(size_t)255;
+    const size_t mmq_bytes = ((mmq ? mmq_scratch_bytes(dev, kind, N, K, M, ws) : q80_bytes) + 255) & ~(size_t)255;
     void *wsp = nullptr;
     int st = MARMOT_HIP_SUCCESS;
     if (act_bytes + mmq_bytes + stage_bytes != 0) {

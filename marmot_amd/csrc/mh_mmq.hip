@@ -932,7 +932,11 @@ static MmqPlan mmq_plan(const marmot_hip_device *dev, int kind, size_t N, size_t
 }
 
 // bytes of fp32 partials launch_mmq needs for this shape (0 when K is not split across workgroups)
-size_t mmq_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights) {
+size_t mmq_scratch_bytes(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, const WeightSet &ws) {
+    const int weights = ws.count;
+    if (kind == MARMOT_HIP_KIND_Q6_K && mmq_rows_q6k_applies(dev, ws, N, K, M)) {
+        return 0;  // (17 rows and more are the tiled GEMM's)
+    }
     const MmqPlan pl = mmq_plan(dev, kind, N, M, K / QK_K, weights);
     const size_t passes = pl.S > 1 ? (size_t)pl.S * N * M * sizeof(float) * (size_t)weights : 0;
     // the tiled GEMM may take the call instead (decided at launch, when the operands' alignment is known)
@@ -1074,21 +1078,19 @@ int launch_mmq_set(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
         }
         return launch_gemm_i8(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }
-    if (kind == MARMOT_HIP_KIND_Q6_K) {
+    if (kind == MARMOT_HIP_KIND_Q6_K && mmq_rows_q6k_applies(dev, ws, N, K, M)) {
         const int st = launch_mmq_rows_q6k(dev, ws, act, N, K, M, out_dtype);
-        if (st != MARMOT_HIP_ERROR_NOT_IMPLEMENTED) {
-            if (st == MARMOT_HIP_SUCCESS) {
-                set_route("mmq_q6_k_q8_k_mfma");
-            }
-            return st;
+        if (st == MARMOT_HIP_SUCCESS) {
+            set_route("mmq_q6_k_q8_k_mfma");
         }
+        return st;
     }
     const size_t nb = K / QK_K;
     const MmqPlan pl = mmq_plan(dev, kind, N, M, nb, ws.count);
     float *partial = (float *)scratch;
     if (pl.S > 1 && partial == nullptr) {
         void *wsp = nullptr;
-        int st = workspace_reserve(dev, mmq_scratch_bytes(dev, kind, N, K, M, ws.count), &wsp);
+        int st = workspace_reserve(dev, mmq_scratch_bytes(dev, kind, N, K, M, ws), &wsp);
         if (st != MARMOT_HIP_SUCCESS) {
             return st;
         }

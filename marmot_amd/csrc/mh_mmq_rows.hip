@@ -1080,8 +1080,13 @@ __global__ __launch_bounds__(512) void k_mmq_rows_q6k(const MmqRowsQ6Params p) {
 }
 
 // Rows of one block stay on the streaming kernel: there is no K to split over the wavefronts.
-bool mmq_rows_q6k_supported(const marmot_hip_device *dev, size_t N, size_t K, size_t M) {
+bool mmq_rows_q6k_applies(const marmot_hip_device *dev, const WeightSet &ws, size_t N, size_t K, size_t M) {
     const size_t row_bytes = K / QK_K * Q6_K_BYTES;
+    for (int i = 0; i < ws.count; ++i) {
+        if ((((uintptr_t)ws.w[i]) & 15) != 0) {
+            return false;
+        }
+    }
     return !dev->knobs.no_row_kernels && N >= 1 && N <= 16 && K % QK_K == 0 && K >= 2 * QK_K && M >= 1 &&
            M <= 0x7fffffffull && 17 * row_bytes <= 0x7fffffffull && N * K <= 0x7fffffffull;
 }
@@ -1094,18 +1099,11 @@ static int launch_mmq_rows_q6k_nq(marmot_hip_device *dev, const MmqRowsQ6Params 
     return MARMOT_HIP_SUCCESS;
 }
 
-// Q6_K weight set x up to 16 packed activation rows. Returns MARMOT_HIP_ERROR_NOT_IMPLEMENTED (error text untouched)
-// when the shape or the alignment is not covered.
+// Q6_K weight set x up to 16 packed activation rows, where mmq_rows_q6k_applies
 int launch_mmq_rows_q6k(marmot_hip_device *dev, const WeightSet &ws, const ActScratch &act, size_t N, size_t K, size_t M,
                         int out_dtype) {
-    if (!mmq_rows_q6k_supported(dev, N, K, M) || (((uintptr_t)act.qs) & 15) != 0 || (((uintptr_t)act.d) & 3) != 0 ||
-        (act.kp & 15) != 0 || act.kp < K || N * act.kp > 0x7fffffffull || act.nb != K / QK_K) {
-        return MARMOT_HIP_ERROR_NOT_IMPLEMENTED;
-    }
-    for (int i = 0; i < ws.count; ++i) {
-        if ((((uintptr_t)ws.w[i]) & 15) != 0) {
-            return MARMOT_HIP_ERROR_NOT_IMPLEMENTED;
-        }
+    if ((((uintptr_t)act.qs) & 15) != 0 || (((uintptr_t)act.d) & 3) != 0 || act.kp != K || act.nb != K / QK_K) {
+        return set_error(MARMOT_HIP_ERROR_INVALID_OPERATION, "Q6_K row groups: activations not in the packed layout");
     }
     MmqRowsQ6Params p;
     for (int i = 0; i < 3; ++i) {

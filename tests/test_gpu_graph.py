@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from marmot_amd import capi
-from oracle.pyoracle import KIND_Q4_0, KIND_Q4_1, KIND_Q4_K, KIND_Q8_0
+from oracle.pyoracle import KIND_Q4_0, KIND_Q4_1, KIND_Q4_K, KIND_Q6_K, KIND_Q8_0
 from tests.util import assert_matmul_parity, bits, gaussian
 
 pytestmark = pytest.mark.gpu
@@ -120,4 +120,29 @@ def test_prepacked_prompt_is_captured_whatever_the_workspace(hip, oracle, kind):
         assert np.array_equal(bits(captured()), bits(eager))
     finally:
         for b in (d_w, d_x, d_p, d_out):
+            b.free()
+
+
+def test_q6k_small_batch_needs_no_room_for_partial_sums(hip, oracle):
+    """16 rows x 14336: the packed activations fit a workspace of 1 MiB, K-split partial sums (2 MB) would not. The row-group
+    kernel has none, so the call is captured without an eager run of its own."""
+    kind = KIND_Q6_K
+    N, K, M = 16, 14336, 4096
+    hip.linear(gaussian(820, (5, 512)), oracle.quantize(kind, gaussian(821, (16, 512), 0.02)), kind, 16)
+    d_w, d_x = hip.to_device(oracle.quantize(kind, gaussian(822, (M, K), 0.02))), hip.to_device(gaussian(823, (N, K)))
+    d_out = hip.alloc(N * M * 4)
+    g = None
+    try:
+        g = hip.graph_capture(lambda: hip.linear_d(kind, d_w, d_x, capi.DT_F32, N, K, M, d_out, capi.DT_F32))
+        hip.linear_d(kind, d_w, d_x, capi.DT_F32, N, K, M, d_out, capi.DT_F32)
+        eager = d_out.download(np.float32, (N, M))
+        for rep in range(3):
+            d_out.upload(np.full(N * M * 4, 0xFF, dtype=np.uint8))
+            hip.graph_launch(g)
+            hip.synchronize()
+            assert np.array_equal(bits(d_out.download(np.float32, (N, M))), bits(eager)), f"replay {rep}"
+    finally:
+        if g is not None:
+            hip.graph_destroy(g)
+        for b in (d_w, d_x, d_out):
             b.free()
