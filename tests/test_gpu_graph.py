@@ -91,9 +91,10 @@ def test_prepacked_prompt_is_captured_whatever_the_workspace(hip, oracle, kind):
     hip.pack_activations_d(kind, d_x, capi.DT_F32, N, K, d_p)
     hip.synchronize()
 
-    def captured():
-        """The captured call's output, the same on every one of three replays."""
+    def captured(kernels):
+        """The captured call's output, the same on every one of three replays. Without partial sums it is one kernel."""
         g = hip.graph_capture(lambda: hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out))
+        assert hip.graph_last_capture_nodes() == kernels
         outs = []
         try:
             for _ in range(3):
@@ -107,17 +108,17 @@ def test_prepacked_prompt_is_captured_whatever_the_workspace(hip, oracle, kind):
         return outs[0]
 
     try:
-        no_room = captured()
+        no_room = captured(1)
         # an eager call that needs between 4 and 8 MB of it: 600 packed rows
         small = oracle.quantize(kind, gaussian(812, (64, 8192), 0.02))
         hip.linear(gaussian(813, (600, 8192)), small, kind, 64)
-        some_room = captured()
+        some_room = captured(1)
         hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out)
         eager = d_out.download(np.float32, (N, M))
         assert_matmul_parity(eager[some], ref, what="eager")
         assert np.array_equal(bits(no_room), bits(eager))
         assert np.array_equal(bits(some_room), bits(eager))
-        assert np.array_equal(bits(captured()), bits(eager))
+        assert np.array_equal(bits(captured(2)), bits(eager))
     finally:
         for b in (d_w, d_x, d_p, d_out):
             b.free()

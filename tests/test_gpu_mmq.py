@@ -527,17 +527,20 @@ def test_tiled_int8_gemm_32_value_formats_random_blocks_routes_and_epilogues(hip
     assert_matmul_parity(pre, oracle.matmul(kind, w3, x3, m3, bias=b3), what=f"{name} prepacked, K split")
 
 
-@pytest.mark.parametrize("N,M,K", [(290, 4000, 3072), (300, 4096, 2816), (1100, 2001, 256)])
-@pytest.mark.parametrize("name", ["q8_0", "q4_0", "q4_1"])
+@pytest.mark.parametrize("N,M,K", [(290, 4000, 3072), (300, 4096, 2816), (1100, 2001, 256), (1100, 2001, 768),
+                                   (200, 6300, 5120), (16, 16520, 3072), (20, 33000, 512)])
+@pytest.mark.parametrize("name", ["q8_0", "q4_0", "q4_1", "q5_0", "q5_1"])
 def test_tiled_int8_gemm_32_value_formats_two_workgroups_per_unit(hip, oracle, name, N, M, K):
-    """160 tiles with K split over the second places of the compute units (12 rounds of 256 values), the same unsplit
-    (11 rounds), and more tiles than compute units (the form with one stage); ragged rows and tokens."""
+    """160 tiles with K split in three over the second places of the compute units (12 rounds of 256 values), the same unsplit
+    (11 rounds), 200 tiles in two; more workgroups than compute units (the form with one stage) by their tiles, of one and of
+    several rounds, and by the split; tiles of 32 tokens with one stage, split and not; ragged rows and tokens."""
     kind = Q80_KINDS[name]
     blocks = oracle.quantize(kind, gaussian(460 + N, (M, K), 0.02))
     x = gaussian(461 + N, (N, K))
     got = hip.linear(x, blocks, kind, M)
     assert hip.last_route() == f"gemm_{name}_q8_0_mfma_tile"
-    some = np.unique(np.r_[0, 1, 31, 32, 63, 64, N // 2, N - 45:N])  # rows of the first tiles, a middle and the last ones
+    some = np.unique(np.r_[0, 1, 31, 32, 63, 64, N // 2, max(N - 45, 0):N])  # rows of the first tiles, a middle and the last ones
+    some = some[some < N]
     assert_matmul_parity(got[some], oracle.matmul(kind, blocks, np.ascontiguousarray(x[some]), M), what=f"{name} {M}x{K} N={N}")
 
 
@@ -704,11 +707,30 @@ def test_tiled_int8_gemm_32_value_formats_integers_are_exact(hip, name):
     assert np.array_equal(bits(got), bits(want))
 
 
-@pytest.mark.parametrize("M,K", [(1, 512), (15, 256 * 3), (16, 2048), (70, 1280), (1031, 256 * 9), (5000, 768), (16400, 512)])
-def test_q6k_up_to_16_rows_by_row_groups(hip, oracle, M, K):
-    """Row groups of 16 with K split over 2 to 8 wavefronts (fewer with fewer blocks), several row groups per workgroup,
-    row counts that end inside a group, tensors that do not end on a 16-byte boundary, every count of four-token steps;
-    bias. Random blocks: negative and extreme scales, all 6-bit values."""
+@pytest.fixture(scope="module")
+def streaming():
+    """A device object without the row-owning kernels: small Q6_K batches take the loader / consumer kernel."""
+    import os
+
+    from marmot_amd import HipBackend
+
+    os.environ["MARMOT_HIP_NO_ROW_KERNELS"] = "1"
+    try:
+        b = HipBackend(0)
+    finally:
+        del os.environ["MARMOT_HIP_NO_ROW_KERNELS"]
+    yield b
+    b.close()
+
+
+@pytest.mark.parametrize("M,K", [(1, 512), (15, 256 * 3), (16, 2048), (70, 1280), (1031, 256 * 9), (5000, 768), (16400, 512),
+                                 (32785, 512), (32785, 768)])
+def test_q6k_up_to_16_rows_by_row_groups(hip, streaming, oracle, M, K):
+    """Row groups of 16 with K split over 2 to 8 wavefronts (fewer with fewer blocks), three row groups per workgroup and a
+    last workgroup of one (32785 rows on 256 compute units), row counts that end inside a group, tensors that do not end on
+    a 16-byte boundary, two to four steps of four tokens; bias. Random blocks: negative and extreme scales, all 6-bit values.
+    The streaming kernel goes by the same route name; it adds the blocks in another order (not told apart by sums of two or
+    three blocks in a row)."""
     rng = np.random.default_rng(390 + M)
     blocks = random_valid_blocks(rng, KIND_Q6_K, M, K)
     for N in (5, 8, 9, 12, 13, 16):
@@ -717,17 +739,55 @@ def test_q6k_up_to_16_rows_by_row_groups(hip, oracle, M, K):
         got = hip.linear(x, blocks, KIND_Q6_K, M, bias=bias)
         assert hip.last_route() == "mmq_q6_k_q8_k_mfma"
         assert_matmul_parity(got, oracle.matmul(KIND_Q6_K, blocks, x, M, threads=8, bias=bias), what=f"Q6_K {M}x{K} N={N}")
+        if K >= 1280 or (M, K) == (32785, 768):
+            assert not np.array_equal(bits(got), bits(streaming.linear(x, blocks, KIND_Q6_K, M, bias=bias)))
+
+
+@pytest.mark.parametrize("K", [768, 1280])
+def test_q6k_sets_by_row_groups(hip, streaming, oracle, K):
+    """Two and three weights in one launch, one step of four tokens (sets of three from three rows on) to four; 11003 and
+    16501 rows are three row groups per workgroup, with ragged ends."""
+    rng = np.random.default_rng(395)
+    for M in (90, 11003):
+        ws = [random_valid_blocks(rng, KIND_Q6_K, M, K) for _ in range(3)]
+        bias = [gaussian(396, (M,)), None, gaussian(397, (M,))]
+        for N in (3, 4, 7, 16):
+            x = gaussian(398 + N, (N, K))
+            got = hip.linear_qkv(x, *ws, KIND_Q6_K, M, *bias)
+            assert hip.last_route() == "mmq_q6_k_q8_k_mfma"
+            for g, w, b in zip(got, ws, bias):
+                assert_matmul_parity(g, oracle.matmul(KIND_Q6_K, w, x, M, threads=8, bias=b), what=f"q/k/v {M}x{K} N={N}")
+            if K >= 1280 or M == 11003:
+                assert not np.array_equal(bits(got[1]), bits(streaming.linear_qkv(x, *ws, KIND_Q6_K, M, *bias)[1]))
+    for M in (90, 16501):
+        ws = [random_valid_blocks(rng, KIND_Q6_K, M, K) for _ in range(2)]
+        for N in (5, 16):
+            x = gaussian(399 + N, (N, K))
+            got = hip.linear_dual(x, *ws, KIND_Q6_K, M)
+            assert hip.last_route() == "mmq_q6_k_q8_k_mfma"
+            for g, w in zip(got, ws):
+                assert_matmul_parity(g, oracle.matmul(KIND_Q6_K, w, x, M, threads=8), what=f"dual {M}x{K} N={N}")
+
+
+@pytest.mark.parametrize("K", [256, 1280, 3584])
+def test_q6k_streaming_kernel_off_16_byte_boundaries(streaming, oracle, K):
+    """The loader / consumer kernel at the row lengths of test_q6k_rows_off_16_byte_boundaries, which the row groups have taken
+    over; rows of one block are still its own."""
+    for M in (70, 1031):
+        blocks = oracle.quantize(KIND_Q6_K, gaussian(345, (M, K), 0.02))
+        for N in (5, 8, 16):
+            x = gaussian(346 + N, (N, K))
+            got = streaming.linear(x, blocks, KIND_Q6_K, M)
+            assert streaming.last_route() == "mmq_q6_k_q8_k_mfma"
+            assert_matmul_parity(got, oracle.matmul(KIND_Q6_K, blocks, x, M, threads=8), what=f"Q6_K {M}x{K} N={N}")
 
 
 @pytest.mark.parametrize("M,K,N", [(33, 512, 5), (70, 2048, 16), (1024, 4096, 9), (4096, 4096, 8), (4096, 14336, 8),
                                    (7000, 14336, 8), (14336, 4096, 12), (32785, 768, 8)])
-def test_q6k_up_to_16_rows_rounds_a_block_once(hip, oracle, monkeypatch, M, K, N):
+def test_q6k_up_to_16_rows_rounds_a_block_once(hip, streaming, oracle, M, K, N):
     """Block sums of more than 24 bits (large codes and scales) are integers up to the one conversion. One block with a scale:
     the output is the product of three rounded factors, bit for bit. All blocks: the error against 64 bits is no larger than
-    that of the streaming kernel, which a device object without the row kernels keeps (sum of 16 scale groups and block
-    products in the same roundings, K split into other parts)."""
-    from marmot_amd import HipBackend
-
+    that of the streaming kernel (block products in the same roundings, K split into other parts)."""
     rng = np.random.default_rng(480 + M)
     nb = K // 256
     blocks = random_valid_blocks(rng, KIND_Q6_K, M, K).reshape(M, nb, 210).copy()
@@ -765,13 +825,7 @@ def test_q6k_up_to_16_rows_rounds_a_block_once(hip, oracle, monkeypatch, M, K, N
     assert np.array_equal(bits(run(hip, only)), bits(factor * dots[one].astype(np.float32)))
 
     exact = np.einsum("bnm,nb,mb->nm", dots, ad.astype(np.float64), d.astype(np.float64))
-    monkeypatch.setenv("MARMOT_HIP_NO_ROW_KERNELS", "1")
-    plain = HipBackend(0)
-    monkeypatch.delenv("MARMOT_HIP_NO_ROW_KERNELS")
-    try:
-        before = run(plain, d)
-    finally:
-        plain.close()
+    before = run(streaming, d)
     error = lambda got: np.sqrt(np.mean((got.astype(np.float64) - exact) ** 2))
     print(f"M={M} K={K} N={N}: error ratio {error(run(hip, d)) / error(before):.3f}", flush=True)
     # (two samples of N * M roundings each: a tenth over 165 outputs is noise, a hundredth over 30000)
