@@ -1042,8 +1042,8 @@ __global__ __launch_bounds__(I8_THREADS) void k_gemm_q6k_q8k_tile(const GemmI8Pa
 // exact), which leaves two vector instructions per output and block, convert and multiply-add (three with the scale product
 // on the vector unit). What bounds the kernel is latency: every product waits for operands from LDS. Two wavefronts per
 // SIMD, with two stages of a 34-byte format, keep its vector unit busy for half the time; two workgroups of one stage each
-// do better (Q8_0, 1024 tokens x 4096 x 14336: 283 us -> 256 with the scales from the matrix core -> 207 with one stage;
-// Q4_0, which always had room for two workgroups: 216 -> 205). Prefetching operands by hand at two wavefronts gave 4 %.
+// do better (Q8_0, whole call of 1024 tokens x 4096 x 14336: 283 us -> 262 with the scales from the matrix core -> 205 with one
+// stage; Q4_0, which always had room for two workgroups: 208 -> 198). Prefetching operands by hand at two wavefronts gave 4 %.
 // Same tile and wavefront roles as the Q6_K kernel: a round is 256 values of K (eight blocks), K group kg takes blocks
 // 4 kg .. 4 kg + 3 of every round. Weight rows must be a multiple of eight blocks (K % 256 == 0: rows and rounds start
 // on 16-byte boundaries); the stage holds each row's 272 (Q8_0) / 144 (Q4_0) bytes of the round at a pitch of 304 / 144
@@ -1611,8 +1611,8 @@ static size_t gemm_i8_splits(const marmot_hip_device *dev, size_t N, size_t M, s
 
 bool gemm_i8_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,
                      const ActScratch &act) {
-    // Q6_K: the small-batch kernel holds 16 rows per pass, and from the second pass on the tile is faster (14336 x 4096
-    // at 17 .. 32 rows: 48 us in two passes, the tile 41 us at 33 rows; 18944 x 3584: 87 - 94 against 63 us)
+    // Q6_K: the small-batch kernels hold 16 rows per pass; the tile takes over from the second pass on (14336 x 4096: one pass
+    // of 16 rows 20.5 us with the quantization of 4.5, the tile 39.0 at 17 rows and 39.8 at 32; 4096 x 4096: 11.4, 20.2, 21.5)
     const size_t min_rows = kind == MARMOT_HIP_KIND_Q6_K ? 17 : I8_MIN_ROWS;
     if (dev->knobs.no_gemm_i8 || N < min_rows || K % QK_K != 0) {
         return false;
@@ -1643,14 +1643,16 @@ static bool q80_format(int kind) {
 }
 // The 32-value formats: two workgroups share a compute unit, so from half a chip to a chip of tiles K is split until the
 // second places are taken too: in three up to a third of the places (170 tiles of 256 compute units), else in two. The
-// partial sums cost about 6 us, so the line is a length of K (whole call, us unsplit / split, of Q8_0, Q4_0 and Q5_1):
+// partial sums cost about 6 us, so the line is a length of K (whole call, us unsplit / split, of Q8_0, Q4_0 and Q5_1; Q4_1 and
+// Q5_0 lie between the last two):
 //   160 tiles, 300 x K x 4096, three   K = 2048: 25 / 29, 25 / 30, 32 / 33   3072: 34 / 30, 34 / 33, 44 / 38
+//                                      K = 4096: 42 / 36, 43 / 38, 57 / 45   14336: 128 / 78, 130 / 80, 179 / 109
 //   200 tiles, 200 x K x 6400, two     K = 3072: 35 / 36, 34 / 36, 45 / 44   4096: 43 / 43, 43 / 42, 57 / 55
 //                                      K = 5120: 52 / 51, 52 / 49, 69 / 64
 //   256 tiles, 16 x K x 32768, two     K = 6144: 41 / 47, 41 / 39, 53 / 51   8192: 58 / 58, 53 / 47, 69 / 64
 // This split is a choice (gemm_i8_splits leaves such calls unsplit) and may not cost a call its scratch: without room for
 // the partial sums one workgroup takes the parts one after another and adds them up in the same order, to the same bits (the
-// entry point that does not allocate promises them). It takes the time of an unsplit call.
+// entry point that does not allocate promises them), in about the time of an unsplit call (300 x 4096 x 4096: 44, 44, 58).
 struct Q80Plan {
     size_t splits, bps;  // parts of K, rounds per part
     bool optional;
@@ -1788,8 +1790,9 @@ static int launch_gemm_q80_kind(marmot_hip_device *dev, const GemmI8Params &p, d
     }
     if constexpr (!Q80Tile<KIND>::SHARES) {
         // More workgroups than compute units: with one stage two of them share a compute unit, and one computes while the
-        // other's loads are on their way (Q8_0, 1024 tokens x 4096 x 14336: 283 us with two stages, 207 with one). At most
-        // one workgroup per compute unit: two stages (300 x 4096 x 4096 unsplit: 46 us, with one stage 54).
+        // other's loads are on their way (whole calls, us with two stages / one: 1024 tokens x 4096 x 14336 Q8_0 262 / 205,
+        // Q4_1 337 / 258, Q5_1 363 / 281; 300 x 4096 x 4096 split in three 43 / 36, 51 / 43, 54 / 45). At most one workgroup
+        // per compute unit: two stages (300 x 4096 x 4096 unsplit: 42 / 51, 53 / 61, 57 / 65).
         if ((size_t)grid.x * grid.y * grid.z > (size_t)dev->props.multiProcessorCount) {
             return p.N <= 32 ? launch_gemm_q80_form<KIND, 1, 1>(dev, p, grid) : launch_gemm_q80_form<KIND, 2, 1>(dev, p, grid);
         }

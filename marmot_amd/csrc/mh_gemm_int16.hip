@@ -30,15 +30,17 @@
 //                    at once and the matrix core idles meanwhile.
 //   <2, 4>           128 rows x 64 tokens, four wavefronts, two or three workgroups per compute unit: their barriers are
 //                    independent, so one computes while another waits.
-// Measured (us; before = k_gemm_q{4,5,6}k_q8k_tile of mh_gemm_i8.hip; tokens x K x M):
-//                    1000 x 4096 x 14336   1024 x 14336 x 4096   2048 x 4096 x 4096   512 x 4096 x 4096
-//   Q4_K before / now    186 / 145             174 / -               107 / 85             30 / -
-//   Q5_K before / now    237 / 160             223 / 190             135 / 93             36 / -
-//   Q6_K before / now    428 / 290             414 / 310             246 / 170            63 / 59
-// 145 us are 810 TOP/s. (At 155 the activation loads were flat loads, which count as LDS accesses too: an operand read
-// then waited for memory.) Of the 145, the matrix instructions alone take about 75 at the clock the chip holds under
-// them (1.7 - 1.9 GHz), the stores of the 57 MB of output 12, waits for the weights 12; what is left is unpacking and
-// the conversion of the activations, which every row tile repeats.
+// Measured (us of whole calls in a row, the quantization of 6 - 17 included; tile = k_gemm_q{4,5,6}k_q8k_tile of
+// mh_gemm_i8.hip, flat = this kernel with flat loads of the activations; tokens x K x M):
+//                          1000 x 4096 x 14336   1024 x 14336 x 4096   2048 x 4096 x 4096   512 x 4096 x 4096
+//   Q4_K tile / flat / now   193 / 163 / 155       188 / - / -           118 / 94 / 88        34 / - / -
+//   Q5_K tile / flat / now   247 / 178 / 162       238 / 203 / 200       146 / 101 / 92       41 / - / -
+//   Q6_K tile / flat / now   437 / 307 / 301       432 / 309 / 307       257 / 185 / 181      69 / 66 / 64
+// (Flat loads count as LDS accesses too: an operand read then waited for memory. Among the other kernels of a layer, where the
+// chip's clock is lower, the Q6_K call of 1024 x 14336 x 4096 takes 331, with either loads, and Q4_K 1024 x 4096 x 14336 164
+// after 182.) 155 us with 7 of quantization are 790 TOP/s. The matrix instructions alone are about half of it at the
+// clock the chip holds under them (1.7 - 1.9 GHz), the stores of the 57 MB of output 12, waits for the weights 12; what is
+// left is unpacking and the conversion of the activations, which every row tile repeats.
 #include "mh_rows.h"
 
 #include <type_traits>

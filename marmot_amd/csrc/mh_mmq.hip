@@ -866,8 +866,10 @@ bool mmq_supported(const marmot_hip_device *dev, int kind, size_t N, size_t K, i
     if (dev->knobs.no_mmq) {
         return false;
     }
-    // below these row counts the fused-quantization matvec is faster (no separate quantization pass)
-    // (a Q6_K set of three weights crosses over earlier: the matvec streams every weight per column tile)
+    // Below these row counts the fused-quantization matvec is faster than the streaming kernels (no separate quantization
+    // pass; a Q6_K set of three weights crosses over earlier: the matvec streams every weight per column tile). The row groups
+    // of Q6_K, which take over at the same counts, would pay from two rows on (us, matvec / row groups at 1, 2, 3 and 4 rows:
+    // 14336 x 4096 16.5 / 15.4, 19.4 / 15.1, 32.2 / 15.0, 26.5 / 15.1; 4096 x 4096 7.9 / 9.5, 10.5 / 9.9, 17.8 / 9.9, 15.8 / 9.6).
     const size_t q6_set_min = 3;
     const size_t min_rows = mmq_is_q4k_family(kind) ? 3 : (weights >= 3 ? q6_set_min : 5);
     return (mmq_is_q4k_family(kind) || kind == MARMOT_HIP_KIND_Q6_K) && N >= min_rows && K % QK_K == 0;

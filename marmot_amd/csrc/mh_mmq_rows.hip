@@ -786,8 +786,9 @@ int launch_mmq_rows_q4k(marmot_hip_device *dev, const WeightSet &ws, const float
 // wavefront) times that kernel's. (Each lane's part converted and summed for itself was up to 1.3 times it, and slower: 8 rows
 // 14336 x 4096 17.6 us, 16 rows 8192 x 16384 37.7.)
 //
-// What bounds it: LDS and the vector units, at about half of what a task takes (N = 8) each; memory would allow three
-// quarters of it. Three stages or twelve wavefronts change nothing.
+// What bounds it: per task and compute unit about 400 clocks (N = 8, 128256 rows), of which the LDS pipe takes about 190 and
+// the vector units as many (170 instructions beside the 8 matrix instructions); memory would allow 340. Three stages or twelve
+// wavefronts change nothing.
 // Measured against k_mmq_q6k_ls (us with the quantization launch and, there, the reduction launch; weights from memory;
 // N = 8 / 16):
 //   K x M      14336 x 4096   4096 x 14336   4096 x 4096    4096 x 1024   8192 x 16384   4096 x 128256
@@ -1125,9 +1126,10 @@ int launch_mmq_rows_q6k(marmot_hip_device *dev, const WeightSet &ws, const ActSc
     const uint32_t cus = (uint32_t)dev->props.multiProcessorCount;
     const uint32_t slots = cus / (uint32_t)ws.count > 0 ? cus / (uint32_t)ws.count : 1;
     const uint32_t all = (p.M + 15u) / 16u;
-    // Eight wavefronts per compute unit, as workgroups of 8 / 4 / 2 (parts of K) by the number of row groups: a part more
-    // is a barrier and a sum more per row group (K 4096, 128256 rows, N = 8: 8 parts 116.6 us, 4: 109.2, 2: 104.4;
-    // 14336 rows 20.4, 19.1, 18.4), too few leave compute units idle (4096 rows, K 14336: 17.7, 21.5, 32.3).
+    // Eight wavefronts per compute unit, as workgroups of 2 to 8 (parts of K) by the number of row groups: a part more is a
+    // barrier and a sum more per row group (K 4096, 128256 rows, N = 8, before the four lanes of a row added up their integers:
+    // 8 parts 116.6 us, 4: 109.2, 2: 104.4; 14336 rows 20.4, 19.1, 18.4), too few leave compute units idle (4096 rows, K 14336:
+    // 17.7, 21.5, 32.3). Numbers between that do not divide 8 leave wavefronts' places empty.
     uint32_t parts = 8u * slots / all;
     parts = parts > 8 ? 8 : parts < 2 ? 2 : parts;
     const uint32_t resident = slots * (8u / parts);
