@@ -1,46 +1,38 @@
-// Prompts with packed (Q8_K) activations: K-quant weights x activation codes as a tiled GEMM on the fp16 matrix cores,
+// Long prompts with packed (Q8_K) activations: Q4_K / Q5_K weights x activation codes as a tiled GEMM on the fp16 matrix cores,
 // both operands integers that fp16 holds exactly.
 //
-// Per 256-value block the reference forms (cpu_vec_dot_q{4,5,6}_k_q8_k, src/backends/cpu/ops/matmul/quantized/
-// vec_dot_impl.h:689-860) y += a.d * (w.d * isum - w.dmin * msum) with isum = sum_j sc_j * (q_j . a_j) and msum = sum_j mn_j *
+// Per 256-value block the reference forms (cpu_vec_dot_q{4,5}_k_q8_k, src/backends/cpu/ops/matmul/quantized/
+// vec_dot_impl.h:689-787) y += a.d * (w.d * isum - w.dmin * msum) with isum = sum_j sc_j * (q_j . a_j) and msum = sum_j mn_j *
 // (sum of a over sub-block j). Here the sub-block scale goes into the weight operand: sc * q is at most 63 * 15 = 945 (Q4_K)
 // or 63 * 31 = 1953 (Q5_K), below 2048, so it is exact in fp16, and the activation codes (-127 .. 127) are too: ONE chain of
-// v_mfma_f32_32x32x16_f16 per block gives isum in fp32 (exact below 2^24; from there on, up to 2^24.9 for Q4_K, 2^25.9 for
-// Q5_K and 2^27 for Q6_K, where the reference rounds isum once, every instruction of the chain may round: at most 16 (Q6_K 32) units
-// in the last place), and one more instruction on the stored sums of 16 codes (at most 2032, exact) and the mins gives
-// msum. Q6_K: sc * q reaches 127 * 32 = 4064, so q = 8 * qh + ql (qh = -4 .. 3, ql = 0 .. 7) and both sc * ql and
-// 8 * sc * qh (in units of a quarter) are exact: two operands on one accumulator. fp32 work per output and block: three
-// multiply(-add)s, two for Q6_K.
+// v_mfma_f32_32x32x16_f16 per block gives isum in fp32 (exact below 2^24; from there on, up to 2^24.9 for Q4_K and 2^25.9 for
+// Q5_K, where the reference rounds isum once, every instruction of the chain may round: at most 16 units in the last place),
+// and one more instruction on the stored sums of 16 codes (at most 2032, exact) and the mins gives msum. fp32 work per output
+// and block: three multiply(-add)s.
 //
 // What bounds it: vector instructions. A SIMD issues one per 4.2 clocks, a matrix instruction holds the issue port for 8 of
-// its 32 clocks (measured with two wavefronts per SIMD), and per 32 x 32 outputs and block this kernel issues 17 (Q4_K,
-// Q5_K) or 32 (Q6_K) matrix instructions beside 48 (32) vector instructions of the fp32 step and its share of the unpacking
-// (190 / 250 / 500 per 32 rows and block) and of the conversion of the activations. The int8 instructions (twice the rate)
-// hold sc * q only as two planes for Q4_K, three for Q5_K and four for Q6_K, so they cost the same matrix time or more,
-// and their result takes a shift-add and a conversion per output and plane pair on the vector unit; Q6_K on int8 takes a
-// multiply-add per output and 16 values. Hence the tile: every unpacked weight operand meets C token tiles.
+// its 32 clocks (measured with two wavefronts per SIMD), and per 32 x 32 outputs and block this kernel issues 17 matrix
+// instructions beside 48 vector instructions of the fp32 step and its share of the unpacking (190 / 250 per 32 rows and block)
+// and of the conversion of the activations. The int8 planes of mh_gemm_planes.hip take the same matrix time and as many
+// vector instructions; what this kernel has is one workgroup of 256 x 128 outputs per compute unit, so it is taken where
+// such tiles fill the chip well (x16_form).
 //
-// A wavefront owns 32 weight rows x 32 C tokens: its lane (row j, half kh) unpacks, in registers, the bytes only it reads.
+// A wavefront owns 32 weight rows x 128 tokens: its lane (row j, half kh) unpacks, in registers, the bytes only it reads.
 // Activations pass through LDS as fp16 (converted once per workgroup on the way from memory: code -> byte under the
 // exponent of 1024 -> minus 1152), half a block (128 values) per stage, two stages, one barrier per stage; raw weight
 // blocks go through a private LDS area of the wavefront (direct-to-LDS loads in whole 16-byte pieces, a block ahead).
-// Everything that is not a matrix instruction is spread between them, a few instructions per step. Two forms:
-//   <C = 4, RG = 8>  256 rows x 128 tokens, eight wavefronts, one workgroup per compute unit. All of them meet at the same
-//                    barriers, so the second wavefront of a SIMD does its fp32 step one stage late: without that both do it
-//                    at once and the matrix core idles meanwhile.
-//   <2, 4>           128 rows x 64 tokens, four wavefronts, two or three workgroups per compute unit: their barriers are
-//                    independent, so one computes while another waits.
-// Measured (us of whole calls in a row, the quantization of 6 - 17 included; tile = k_gemm_q{4,5,6}k_q8k_tile of
-// mh_gemm_i8.hip, flat = this kernel with flat loads of the activations; tokens x K x M):
-//                          1000 x 4096 x 14336   1024 x 14336 x 4096   2048 x 4096 x 4096   512 x 4096 x 4096
-//   Q4_K tile / flat / now   193 / 163 / 155       188 / - / -           118 / 94 / 88        34 / - / -
-//   Q5_K tile / flat / now   247 / 178 / 162       238 / 203 / 200       146 / 101 / 92       41 / - / -
-//   Q6_K tile / flat / now   437 / 307 / 301       432 / 309 / 307       257 / 185 / 181      69 / 66 / 64
-// (Flat loads count as LDS accesses too: an operand read then waited for memory. Among the other kernels of a layer, where the
-// chip's clock is lower, the Q6_K call of 1024 x 14336 x 4096 takes 331, with either loads, and Q4_K 1024 x 4096 x 14336 164
-// after 182.) 155 us with 7 of quantization are 790 TOP/s. The matrix instructions alone are about half of it at the
-// clock the chip holds under them (1.7 - 1.9 GHz), the stores of the 57 MB of output 12, waits for the weights 12; what is
-// left is unpacking and the conversion of the activations, which every row tile repeats.
+// Everything that is not a matrix instruction is spread between them, a few instructions per step. The eight wavefronts of
+// the workgroup meet at the same barriers, so the second wavefront of a SIMD does its fp32 step one stage late: without that
+// both do it at once and the matrix core idles meanwhile.
+// Measured (us of whole calls in a row, the quantization of 6 - 17 included; tile = k_gemm_q{4,5}k_q8k_tile of
+// mh_gemm_i8.hip, flat = this kernel with flat loads of the activations, which count as LDS accesses too: an operand read then
+// waited for memory; tokens x K x M):
+//                          1000 x 4096 x 14336   2048 x 4096 x 4096
+//   Q4_K tile / flat / now   193 / 163 / 155       118 / 94 / 88
+//   Q5_K tile / flat / now   247 / 178 / 162       146 / 101 / 92
+// 155 us with 7 of quantization are 790 TOP/s. The matrix instructions alone are about half of it at the clock the chip holds
+// under them (1.7 - 1.9 GHz), the stores of the 57 MB of output 12, waits for the weights 12; what is left is unpacking and the
+// conversion of the activations, which every row tile repeats.
 #include "mh_rows.h"
 
 #include <type_traits>
@@ -62,45 +54,34 @@ struct GemmX16Params {
     void *out[3];
     const void *bias[3];
     int bias_is_f16, bias_first, out_is_f16;
-    // grouped (MoE): blockIdx.y selects a work item (expert, first route, routes); activation row of a route through
-    // act_index (null: the route itself), output row = route
-    const int4 *items;
-    const int *n_items;
-    const uint32_t *act_index;
-    size_t expert_stride;
 };
 
-// Per format: 16-byte pieces that cover a row's block from the boundary below its start, and whether a minimum exists
+// Per format: bytes of a block, in whole 16-byte pieces
 template <int KIND>
 struct X16Format;
 template <>
 struct X16Format<MARMOT_HIP_KIND_Q4_K> {
     static constexpr int BYTES = Q4_K_BYTES, PIECES = 9;
-    static constexpr bool MIN = true;
 };
 template <>
 struct X16Format<MARMOT_HIP_KIND_Q5_K> {
     static constexpr int BYTES = Q5_K_BYTES, PIECES = 11;
-    static constexpr bool MIN = true;
-};
-template <>
-struct X16Format<MARMOT_HIP_KIND_Q6_K> {
-    static constexpr int BYTES = Q6_K_BYTES, PIECES = 14;  // 14 + 210 bytes at most
-    static constexpr bool MIN = false;
 };
 
-template <int KIND, int C, int RG>
+constexpr int X16_TILES = 4, X16_ROWS = 8;  // token tiles of a wavefront, wavefronts along the rows
+
+template <int KIND>
 struct X16Lds {
+    static constexpr int C = X16_TILES, RG = X16_ROWS;
     static constexpr int ROWS = 64 / X16Format<KIND>::PIECES;             // whole rows per direct-to-LDS load
     static constexpr int DMA = (32 + ROWS - 1) / ROWS;                    // such loads of a wavefront per block
     static constexpr int ACT = 32 * C * 256;                              // one stage: 32 C tokens x 128 fp16
     static constexpr int W0 = 2 * ACT;
     static constexpr int WAVE_W = 32 * 16 * X16Format<KIND>::PIECES;
     static constexpr int S0 = W0 + RG * WAVE_W;                           // sums of the block as fp16: [token][16]
-    static constexpr int SUMS = X16Format<KIND>::MIN ? 32 * C * 32 : 0;
+    static constexpr int SUMS = 32 * C * 32;
     static constexpr int SD = SUMS + 32 * C * 4;                          // then the activation scales [token]; two blocks
-    static constexpr int SD_BUFFERS = RG == 8 ? 2 : 1;
-    static constexpr int BYTES = S0 + SD_BUFFERS * SD;
+    static constexpr int BYTES = S0 + 2 * SD;
 };
 
 __device__ __forceinline__ x_half2 x_h2(uint32_t v) {
@@ -114,9 +95,9 @@ __device__ __forceinline__ x_half2 x_splat(_Float16 v) {
 }
 // (v & mask) | magic in one instruction: two 32-bit literals do not fit one, so both sit in registers
 struct X16Masks {
-    uint32_t magic, low, high, low3, high3;
-    __device__ __forceinline__ X16Masks() : magic(0x64006400u), low(0x000f000fu), high(0x00f000f0u), low3(0x00070007u), high3(0x00380038u) {
-        asm volatile("" : "+v"(magic), "+v"(low), "+v"(high), "+v"(low3), "+v"(high3));
+    uint32_t magic, low, high;
+    __device__ __forceinline__ X16Masks() : magic(0x64006400u), low(0x000f000fu), high(0x00f000f0u) {
+        asm volatile("" : "+v"(magic), "+v"(low), "+v"(high));
     }
 };
 __device__ __forceinline__ x_half2 x_and_or(uint32_t v, uint32_t mask, uint32_t magic) {
@@ -145,7 +126,6 @@ struct X16Raw;
 
 template <>
 struct X16Raw<MARMOT_HIP_KIND_Q4_K> {
-    static constexpr int PLANES = 1;
     uint32_t sc_lo, sc_hi, mn_lo, mn_hi;
     float d, ndmin;
     uint4 q[4];
@@ -195,7 +175,7 @@ struct X16Raw<MARMOT_HIP_KIND_Q4_K> {
         return x_splat((sub & 2) ? pair[1] : pair[0]);
     }
     __device__ __forceinline__ void operands(int hb, int g, int, int piece, const X16Masks &mk,
-                                             x_half8 (&op)[1][2]) const {
+                                             x_half8 (&op)[2]) const {
         const int sub = 4 * hb + g;
         const uint4 &v = q[2 * hb + (g >> 1)];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -205,14 +185,13 @@ struct X16Raw<MARMOT_HIP_KIND_Q4_K> {
         const x_half2 c = m * x_splat((_Float16)-1024.0f);
         const uint32_t mask = (g & 1) ? mk.high : mk.low;
         const uint32_t x = w[piece];
-        x_put(op[0][piece >> 1], piece & 1, __builtin_elementwise_fma(x_and_or(x, mask, mk.magic), m, c),
+        x_put(op[piece >> 1], piece & 1, __builtin_elementwise_fma(x_and_or(x, mask, mk.magic), m, c),
               __builtin_elementwise_fma(x_and_or(x >> 8, mask, mk.magic), m, c));
     }
 };
 
 template <>
 struct X16Raw<MARMOT_HIP_KIND_Q5_K> {
-    static constexpr int PLANES = 1;
     X16Raw<MARMOT_HIP_KIND_Q4_K> k4;
     float d, ndmin;
     uint4 h;  // fifth bits of this lane's 16 positions of every group: bit 4 hb + g
@@ -237,7 +216,7 @@ struct X16Raw<MARMOT_HIP_KIND_Q5_K> {
         return k4.mins(kh);
     }
     __device__ __forceinline__ void operands(int hb, int g, int, int piece, const X16Masks &mk,
-                                             x_half8 (&op)[1][2]) const {
+                                             x_half8 (&op)[2]) const {
         const int sub = 4 * hb + g;
         const uint4 &v = k4.q[2 * hb + (g >> 1)];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -247,66 +226,8 @@ struct X16Raw<MARMOT_HIP_KIND_Q5_K> {
         // four 5-bit values as bytes
         const uint32_t nib = (g & 1) ? (w[piece] >> 4) & 0x0f0f0f0fu : w[piece] & 0x0f0f0f0fu;
         const uint32_t b = nib | (((hw[piece] >> sub) & 0x01010101u) << 4);
-        x_put(op[0][piece >> 1], piece & 1, __builtin_elementwise_fma(x_bytes<0>(b), m, c),
+        x_put(op[piece >> 1], piece & 1, __builtin_elementwise_fma(x_bytes<0>(b), m, c),
               __builtin_elementwise_fma(x_bytes<1>(b), m, c));
-    }
-};
-
-template <>
-struct X16Raw<MARMOT_HIP_KIND_Q6_K> {
-    static constexpr int PLANES = 2;
-    uint4 ql[4];  // [hb][g & 1]: low four bits of values 32 (g & 1) + 16 kh .. (low nibbles), 64 more (high nibbles)
-    uint4 qh[2];  // [hb]
-    uint32_t scw[4];
-    float d, ndmin;
-    uint32_t scw_next[4];
-    uint16_t d_next;
-    __device__ __forceinline__ void load_head(const uint8_t *at, int kh) {
-        __builtin_memcpy(&ql[0], at + 16 * kh, 16);
-        __builtin_memcpy(&ql[1], at + 32 + 16 * kh, 16);
-        __builtin_memcpy(&qh[0], at + 128 + 16 * kh, 16);
-        __builtin_memcpy(scw_next, at + 192, 16);
-        __builtin_memcpy(&d_next, at + 208, 2);
-    }
-    __device__ __forceinline__ void load_tail(const uint8_t *at, int kh) {
-        __builtin_memcpy(&ql[2], at + 64 + 16 * kh, 16);
-        __builtin_memcpy(&ql[3], at + 96 + 16 * kh, 16);
-        __builtin_memcpy(&qh[1], at + 160 + 16 * kh, 16);
-    }
-    __device__ __forceinline__ void decode_head(int kh) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            scw[i] = scw_next[i] >> (8 * kh);  // bytes 0 and 2: this lane's groups
-        }
-        d = 4.0f * h2f(d_next);  // the operands are in units of a quarter
-        asm volatile("" : "+v"(d));
-        ndmin = 0.0f;
-    }
-    __device__ __forceinline__ x_half8 mins(int) const {
-        return x_half8{};
-    }
-    __device__ __forceinline__ void operands(int hb, int g, int, int piece, const X16Masks &mk,
-                                             x_half8 (&op)[2][2]) const {
-        // the group of 16 values of this lane: scale 8 hb + 2 g + kh
-        const uint32_t word = scw[2 * hb + (g >> 1)];
-        const int sc = (int)(int8_t)((word >> (16 * (g & 1))) & 0xffu);
-        const x_half2 m = x_splat((_Float16)(0.25f * (float)sc));
-        const x_half2 c = m * x_splat((_Float16)-1024.0f);
-        const uint4 &lv = ql[2 * hb + (g & 1)];
-        const uint4 &hv = qh[hb];
-        const uint32_t lw[4] = {lv.x, lv.y, lv.z, lv.w};
-        const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w};
-        const uint32_t nib = (g >> 1) ? (lw[piece] >> 4) & 0x0f0f0f0fu : lw[piece] & 0x0f0f0f0fu;
-        const uint32_t two = g == 0 ? (hw[piece] << 4) & 0x30303030u
-            : g == 1               ? (hw[piece] << 2) & 0x30303030u
-            : g == 2               ? hw[piece] & 0x30303030u
-                                   : (hw[piece] >> 2) & 0x30303030u;
-        const uint32_t b = nib | two, b1 = b >> 8;
-        const x_half2 bias = x_splat((_Float16)1056.0f);  // 1024 + 8 * 4
-        x_put(op[0][piece >> 1], piece & 1, __builtin_elementwise_fma(x_and_or(b, mk.low3, mk.magic), m, c),
-              __builtin_elementwise_fma(x_and_or(b1, mk.low3, mk.magic), m, c));
-        x_put(op[1][piece >> 1], piece & 1, (x_and_or(b, mk.high3, mk.magic) - bias) * m,
-              (x_and_or(b1, mk.high3, mk.magic) - bias) * m);
     }
 };
 
@@ -324,10 +245,11 @@ __device__ __forceinline__ void x16_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int KIND, int C, int RG>
-__global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3 : 2) void k_gemm_x16(const GemmX16Params p) {
+template <int KIND>
+__global__ __launch_bounds__(64 * X16_ROWS, 2) void k_gemm_x16(const GemmX16Params p) {
     using F = X16Format<KIND>;
-    using L = X16Lds<KIND, C, RG>;
+    using L = X16Lds<KIND>;
+    constexpr int C = X16_TILES, RG = X16_ROWS;
     constexpr int THREADS = 64 * RG, TOK = 32 * C;
     constexpr int APT = 8 * TOK / THREADS;  // 16-byte pieces of codes per thread and stage
     static_assert(8 * TOK % THREADS == 0, "whole pieces per thread");
@@ -338,18 +260,8 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     const int which = blockIdx.z;
     const size_t row0 = (size_t)blockIdx.x * (32 * RG) + 32 * wave;  // this wavefront's first weight row
     const uint8_t *w = p.w[which];
-    size_t tok0 = (size_t)blockIdx.y * TOK;  // first output row
-    uint32_t toks = (uint32_t)(p.N - tok0 < (size_t)TOK ? p.N - tok0 : (size_t)TOK);
-    if (p.items != nullptr) {
-        if ((int)blockIdx.y >= *p.n_items) {
-            return;
-        }
-        const int4 it = p.items[blockIdx.y];
-        w += (size_t)it.x * p.expert_stride;
-        tok0 = (size_t)it.y;
-        toks = (uint32_t)it.z;
-    }
-
+    const size_t tok0 = (size_t)blockIdx.y * TOK;  // first output row
+    const uint32_t toks = (uint32_t)(p.N - tok0 < (size_t)TOK ? p.N - tok0 : (size_t)TOK);
     // ---- activations: piece `tid + THREADS i` of a stage is 16 codes (part q % 8) of token q / 8; rows beyond the last
     // token re-read it and are never stored
     uint32_t a_row[APT];
@@ -357,82 +269,43 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
 #pragma unroll
     for (int i = 0; i < APT; ++i) {
         const uint32_t q = (uint32_t)(tid + THREADS * i), t = q >> 3, part = q & 7u;
-        uint32_t row = (uint32_t)tok0 + (t < toks ? t : toks - 1u);
-        if (p.act_index != nullptr) {
-            row = p.act_index[row];
-        }
+        const uint32_t row = (uint32_t)tok0 + (t < toks ? t : toks - 1u);
         a_row[i] = row * (uint32_t)p.kp + 16u * part;
         a_lds[i] = t * 256u + 16u * ((2u * part) ^ (t & 15u));
     }
     // sums and scales of a block: thread's piece (tokens wrap around: several threads then write the same bytes)
     const uint32_t s_tok = (uint32_t)(tid >> 1) % TOK, d_tok = (uint32_t)tid % TOK;
-    uint32_t s_row = (uint32_t)tok0 + (s_tok < toks ? s_tok : toks - 1u);
-    uint32_t d_row = (uint32_t)tok0 + (d_tok < toks ? d_tok : toks - 1u);
-    if (p.act_index != nullptr) {
-        s_row = p.act_index[s_row];
-        d_row = p.act_index[d_row];
-    }
+    const uint32_t s_row = (uint32_t)tok0 + (s_tok < toks ? s_tok : toks - 1u);
+    const uint32_t d_row = (uint32_t)tok0 + (d_tok < toks ? d_tok : toks - 1u);
     const uint32_t s_off = s_row * (uint32_t)p.nb * 32u + 16u * (tid & 1);
     const uint32_t d_off = d_row * (uint32_t)p.nb * 4u;
 
     // ---- weights: load i of a block brings rows ROWS i .. + ROWS - 1 of the wavefront: lane l the 16-byte piece l % PIECES
-    // of row l / PIECES, counted from the 16-byte boundary at or below the row's block; a piece that holds no byte of the
-    // block re-reads the last one that does, lanes behind the last row and rows behind the matrix re-read a row before.
+    // of row l / PIECES; lanes behind the last row and rows behind the matrix re-read a row before.
     const uint32_t row_bytes = (uint32_t)p.nb * F::BYTES;
     const uint32_t rows = (uint32_t)(row0 < p.M ? (p.M - row0 < 32 ? p.M - row0 : 32) : 0);
     const uint8_t *wbase = w + (row0 < p.M ? row0 : p.M - 1) * row_bytes;
-    const uint32_t low4 = (uint32_t)((uintptr_t)wbase & 15u);
-    wbase = uniform_pointer(wbase - low4);
+    wbase = uniform_pointer(wbase);
     const uint32_t last_row = rows == 0 ? 0 : rows - 1u;
     const uint32_t w_r = (uint32_t)lane / F::PIECES < L::ROWS ? (uint32_t)lane / F::PIECES : L::ROWS - 1u;
     const uint32_t w_piece = 16u * ((uint32_t)lane - F::PIECES * w_r < F::PIECES ? (uint32_t)lane - F::PIECES * w_r : F::PIECES - 1u);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_u8_t *)lds;
     const uint32_t w_lds = lds_base + (uint32_t)(L::W0 + wave * L::WAVE_W);
-    const uint32_t w_first = low4 + w_r * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
-    const uint32_t w_last = low4 + last_row * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
-    // Q6_K: the piece that holds the end of the matrix may reach up to 14 bytes behind it (its size need not be a multiple
-    // of 16), and those bytes need not exist. The wavefront of the last row brings the piece before in its place (one
-    // operand more of a minimum that is there anyway) and copies the bytes that exist when the block is read (bring_end).
-    const uint32_t w_end = low4 + (last_row + 1u) * row_bytes;
-    const bool ragged = F::BYTES % 16 != 0 && row0 + 32 >= p.M && (w_end & 15u) != 0;
-    const uint32_t w_most = ragged ? (w_end & ~15u) - 16u : ~0u;
-    const uint32_t end_block = ragged ? (uint32_t)p.nb - 1u : ~0u;
+    const uint32_t w_first = w_r * row_bytes + w_piece;
+    const uint32_t w_last = last_row * row_bytes + w_piece;
     auto request_weights = [&](uint32_t b, int i) {
         uint32_t at = w_first;
-        if (C == 4) {  // formed at each load: kept in registers, the L::DMA offsets would be spilled
-            asm volatile("" : "+v"(at));
-        }
+        asm volatile("" : "+v"(at));  // formed at each load: kept in registers, the L::DMA offsets would be spilled
         at += (uint32_t)i * (L::ROWS * row_bytes);
         at = at < w_last ? at : w_last;
         const uint32_t to = w_lds + (uint32_t)(i * L::ROWS * 16 * F::PIECES);
-        if constexpr (F::BYTES % 16 != 0) {
-            at += b * (uint32_t)F::BYTES;
-            const uint32_t last = (at + (uint32_t)F::BYTES - 1u) & ~15u;
-            at = (at & ~15u) + w_piece;
-            at = at < last ? at : last;
-            at = at < w_most ? at : w_most;
-        }
-        const uint8_t *base = F::BYTES % 16 != 0 ? wbase : wbase + (size_t)b * F::BYTES;
+        const uint8_t *base = wbase + (size_t)b * F::BYTES;
         // (the launcher checks that rows of whole 16-byte pieces start on 16-byte boundaries)
         // lanes without a row write nothing: the place behind the rows of this load belongs to the next one
         if ((uint32_t)lane < (i + 1 < L::DMA ? L::ROWS : 32 - L::ROWS * (L::DMA - 1)) * F::PIECES) {
             x16_dma(to, base, at);
         }
     };
-    // After the loads of block b have arrived: the end of the matrix, two bytes per lane
-    auto bring_end = [&](uint32_t b) {
-        if constexpr (F::BYTES % 16 != 0) {
-            if (b == end_block) {
-                const uint32_t block = low4 + last_row * row_bytes + b * (uint32_t)F::BYTES;
-                const uint32_t from = (w_end & ~15u) + 2u * (uint32_t)lane;
-                if (from < w_end) {
-                    uint8_t *to = lds + L::W0 + wave * L::WAVE_W + last_row * (16 * F::PIECES) + (from - (block & ~15u));
-                    *(uint16_t *)to = *(const __attribute__((address_space(1))) uint16_t *)(wbase + from);
-                }
-            }
-        }
-    };
-    const uint32_t my_row = low4 + ((uint32_t)j < last_row ? (uint32_t)j : last_row) * row_bytes;
     const uint8_t *my_w = lds + L::W0 + wave * L::WAVE_W + j * (16 * F::PIECES);
 
     x_u32x4 a_next[APT];
@@ -449,7 +322,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
         }
     };
     auto request_block = [&](uint32_t b) {
-        if constexpr (F::MIN) {
+        {
             glb_u8_t *sums = (glb_u8_t *)p.sums + (size_t)b * 32u;
             asm("" : "+s"(sums));
             s_next = *(const glb_u32x4_t *)(sums + (size_t)s_off);
@@ -473,8 +346,8 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
         *(uint4 *)(stage + (a_lds[i] ^ 16u)) = make_uint4(e[4], e[5], e[6], e[7]);
     };
     auto store_block = [&](uint32_t b) {
-        uint8_t *sd = lds + L::S0 + (b & (L::SD_BUFFERS - 1u)) * L::SD;
-        if constexpr (F::MIN) {
+        uint8_t *sd = lds + L::S0 + (b & 1u) * L::SD;
+        {
             const uint32_t v[4] = {s_next.x, s_next.y, s_next.z, s_next.w};
             uint32_t e[4];
 #pragma unroll
@@ -499,28 +372,19 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     // A operand of (g, kh, i): chunk 4 g + 2 kh + i of token 32 t + j. One address register: the others differ from it in
     // bits 4 .. 7 and are formed where they are used (kept out of registers by the volatile asm).
     const uint32_t a_at = lds_base + (uint32_t)(j * 256 + 16 * ((2 * kh) ^ (j & 15)));
-    auto my_block = [&](uint32_t b) {  // (blocks of whole pieces start at the beginning of their place)
-        return F::BYTES % 16 != 0 ? my_w + ((my_row + b * (uint32_t)F::BYTES) & 15u) : my_w;
-    };
-
     // fp32 step of a block, token tile t: y += a.d * (w.d * isum - w.dmin * msum)
     x_float16 P[C];
     float d = 0.0f, ndmin = 0.0f;
     x_half8 mins = {};
     auto finish = [&](uint32_t b) {
-        const uint8_t *sd = lds + L::S0 + (b & (L::SD_BUFFERS - 1u)) * L::SD;
-        x_half8 sums = {};
-        if constexpr (F::MIN) {
-            sums = *(const x_half8 *)(sd + j * 32 + 16 * kh);
-        }
+        const uint8_t *sd = lds + L::S0 + (b & 1u) * L::SD;
+        x_half8 sums = *(const x_half8 *)(sd + j * 32 + 16 * kh);
 #pragma unroll
         for (int t = 0; t < C; ++t) {
             x_float16 T = {};
-            if constexpr (F::MIN) {
-                T = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, mins, T, 0, 0, 0);
-                if (t + 1 < C) {
-                    sums = *(const x_half8 *)(sd + (32 * (t + 1) + j) * 32 + 16 * kh);
-                }
+            T = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, mins, T, 0, 0, 0);
+            if (t + 1 < C) {
+                sums = *(const x_half8 *)(sd + (32 * (t + 1) + j) * 32 + 16 * kh);
             }
             float4 da4[4];
 #pragma unroll
@@ -533,10 +397,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int r = 4 * q + e;
-                    float v = d * P[t][r];
-                    if constexpr (F::MIN) {
-                        v = __builtin_fmaf(ndmin, T[r], v);
-                    }
+                    const float v = __builtin_fmaf(ndmin, T[r], d * P[t][r]);
                     total[t][r] = __builtin_fmaf(da[e], v, total[t][r]);
                 }
             }
@@ -560,8 +421,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     store_block(0);
     request_acts(1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    bring_end(0);
-    raw.load_head(my_block(0), kh);
+    raw.load_head(my_w, kh);
     x16_barrier();
     auto walk = [&](auto late_c) {
     constexpr bool LATE = decltype(late_c)::value;
@@ -569,11 +429,10 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
         const uint32_t bn = b + 1 < nb ? b + 1 : b;  // (the last block is requested again rather than branched around)
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
-            // Steps (g, i, t): one matrix instruction per plane each, consecutive ones on different accumulators. The A operand
+            // Steps (g, i, t): one matrix instruction each, consecutive ones on different accumulators. The A operand
             // of a step is read AHEAD steps before it, the weight operands of group g + 1 are unpacked, a quarter at a time,
-            // between the steps of group g. AHEAD is what the register budget carries without spills; with 3 in place of 4
-            // the C = 2 form takes 425 in place of 400 us (the whole call of 2048 tokens, 128 experts of 768 x 2048).
-            constexpr int STEPS = 8 * C, AHEAD = C == 4 ? 3 : 4;
+            // between the steps of group g. AHEAD is what the register budget carries without spills.
+            constexpr int STEPS = 8 * C, AHEAD = 3;
             x_half8 ring[AHEAD];
             uint32_t a_addr[2];
             auto read_a = [&](int s) {
@@ -584,12 +443,12 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
                 ring[s % AHEAD] = *(const __attribute__((address_space(3))) x_half8 *)(
                     (const lds_u8_t *)(uintptr_t)a_addr[i] + hb * L::ACT + t * 8192);
             };
-            x_half8 op[2][X16Raw<KIND>::PLANES][2];
+            x_half8 op[2][2];
             if (hb == 0 && LATE && b != 0) {
                 finish(b - 1);
             }
             if (hb == 0) {
-                raw.load_tail(my_block(b), kh);
+                raw.load_tail(my_w, kh);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -611,12 +470,8 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
             for (int s = 0; s < STEPS; ++s) {
                 const int g = s / (2 * C), t = s % C, i = (s / C) & 1;
                 const x_half8 a = ring[s % AHEAD];
-#pragma unroll
-                for (int pl = 0; pl < X16Raw<KIND>::PLANES; ++pl) {
-                    const x_float16 zero = {};
-                    P[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                        a, op[g & 1][pl][i], hb == 0 && g == 0 && i == 0 && pl == 0 ? zero : P[t], 0, 0, 0);
-                }
+                const x_float16 zero = {};
+                P[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, op[g & 1][i], hb == 0 && g == 0 && i == 0 ? zero : P[t], 0, 0, 0);
                 if (s + AHEAD < STEPS) {
                     read_a(s + AHEAD);
                 }
@@ -659,8 +514,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
                     }
                 }
                 if (hb == 1 && at(24)) {
-                    bring_end(bn);
-                    raw.load_head(my_block(bn), kh);
+                    raw.load_head(my_w, kh);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -674,7 +528,7 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
         finish(nb - 1);
     }
     };
-    if (RG == 8 && wave >= 4) {
+    if (wave >= 4) {
         walk(std::true_type{});
     } else {
         walk(std::false_type{});
@@ -718,64 +572,36 @@ __global__ __launch_bounds__(64 * RG, KIND == MARMOT_HIP_KIND_Q4_K && C == 2 ? 3
     }
 }
 
-template <int KIND, int C, int RG>
-static int x16_launch(marmot_hip_device *dev, const GemmX16Params &p, unsigned col_tiles, unsigned weights) {
-    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_x16<KIND, C, RG>));
-    const dim3 grid((unsigned)((p.M + 32 * RG - 1) / (32 * RG)), col_tiles, weights);
-    hipLaunchKernelGGL((k_gemm_x16<KIND, C, RG>), grid, dim3(64 * RG), (X16Lds<KIND, C, RG>::BYTES), dev->stream, p);
-    MH_HIP(hipGetLastError());
-    return MARMOT_HIP_SUCCESS;
-}
-
-static bool x16_kind(int kind) {
-    return kind == MARMOT_HIP_KIND_Q4_K || kind == MARMOT_HIP_KIND_Q5_K || kind == MARMOT_HIP_KIND_Q6_K;
-}
-
-// Which form (C), or none (0) where the tiles of mh_gemm_i8.hip are as fast or faster. A compute unit takes as long for one
-// 256 x 128 tile as for three rounds of 128 x 64 tiles (2048 x 4096 x 4096, one large tile per compute unit: 85 us; four
-// rounds of small ones: 107 us in mh_gemm_i8.hip, 101 us here), so the large tile has to save a round. The small tile
-// needs company on its compute unit: with one workgroup per compute unit (256 tiles, 512 x 4096 x 4096) Q4_K takes 39 us
-// against 30 and Q5_K 44 against 36, with two (1024 x 4096 x 4096) 54 against 54 and 60 against 68; so from one and a half
-// on for Q5_K, never for Q4_K. Q6_K is faster from half a chip of tiles on (128 tokens x 14336 rows: 61 against 63 us,
-// 256 x 4096 x 4096 43 against 41) and has no large form (it needs more registers than there are).
-static int x16_form(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t weights) {
+// Whether a call takes this kernel. A compute unit takes as long for one 256 x 128 tile as for three rounds of 128 x 64 tiles
+// (2048 x 4096 x 4096, one large tile per compute unit: 85 us; four rounds of small ones: 107 us in mh_gemm_i8.hip, 101 us in
+// mh_gemm_planes.hip), so the large tile has to save a round.
+static bool x16_form(const marmot_hip_device *dev, size_t N, size_t M, size_t weights) {
     const size_t cus = (size_t)dev->props.multiProcessorCount;
     const size_t small = ((N + 63) / 64) * ((M + 127) / 128) * weights;
-    if (kind == MARMOT_HIP_KIND_Q6_K) {
-        return small > cus / 2 ? 2 : 0;
-    }
     const size_t large = ((N + 127) / 128) * ((M + 255) / 256) * weights;
-    if (3 * ((large + cus - 1) / cus) < (small + cus - 1) / cus) {
-        return 4;
-    }
-    return kind == MARMOT_HIP_KIND_Q5_K && 2 * small > 3 * cus ? 2 : 0;
+    return 3 * ((large + cus - 1) / cus) < (small + cus - 1) / cus;
 }
 
 bool gemm_x16_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights,
                       const ActScratch &act) {
-    if (dev->knobs.no_gemm_i8 || !x16_kind(kind) || K % QK_K != 0) {
+    if (dev->knobs.no_gemm_i8 || (kind != MARMOT_HIP_KIND_Q4_K && kind != MARMOT_HIP_KIND_Q5_K) || K % QK_K != 0) {
         return false;
     }
     if ((((uintptr_t)act.qs) & 15) != 0 || act.kp % 16 != 0 || N * act.kp >= ((size_t)1 << 32) ||
         32 * (K / QK_K) * block_bytes(kind) >= ((size_t)1 << 31) || N > (size_t)65535 * 64) {
         return false;  // 32-bit lane offsets
     }
-    return x16_form(dev, kind, N, M, (size_t)weights) != 0;
+    return x16_form(dev, N, M, (size_t)weights);
 }
 
 template <int KIND>
-static int x16_launch_kind(marmot_hip_device *dev, const GemmX16Params &p, unsigned weights) {
-    if constexpr (KIND != MARMOT_HIP_KIND_Q6_K) {
-        if (x16_form(dev, KIND, p.N, p.M, weights) == 4) {
-            set_route(KIND == MARMOT_HIP_KIND_Q4_K ? "mmq_q4_k_q8_k_fp16_tile_256x128" : "mmq_q5_k_q8_k_fp16_tile_256x128");
-            return x16_launch<KIND, 4, 8>(dev, p, (unsigned)((p.N + 127) / 128), weights);
-        }
-    }
-    if constexpr (KIND != MARMOT_HIP_KIND_Q4_K) {
-        set_route(KIND == MARMOT_HIP_KIND_Q5_K ? "mmq_q5_k_q8_k_fp16_tile_128x64" : "mmq_q6_k_q8_k_fp16_tile_128x64");
-        return x16_launch<KIND, 2, 4>(dev, p, (unsigned)((p.N + 63) / 64), weights);
-    }
-    return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "fp16-operand GEMM: no form for this shape");
+static int x16_launch(marmot_hip_device *dev, const GemmX16Params &p, unsigned weights) {
+    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_x16<KIND>));
+    const dim3 grid((unsigned)((p.M + 32 * X16_ROWS - 1) / (32 * X16_ROWS)), (unsigned)((p.N + 127) / 128), weights);
+    hipLaunchKernelGGL((k_gemm_x16<KIND>), grid, dim3(64 * X16_ROWS), X16Lds<KIND>::BYTES, dev->stream, p);
+    MH_HIP(hipGetLastError());
+    set_route(KIND == MARMOT_HIP_KIND_Q4_K ? "mmq_q4_k_q8_k_fp16_tile_256x128" : "mmq_q5_k_q8_k_fp16_tile_256x128");
+    return MARMOT_HIP_SUCCESS;
 }
 
 int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
@@ -797,56 +623,8 @@ int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const
     p.bias_first = ws.bias_first ? 1 : 0;
     p.out_is_f16 = out_dtype == MARMOT_HIP_DTYPE_F16;
     const unsigned weights = (unsigned)ws.count;
-    switch (kind) {
-    case MARMOT_HIP_KIND_Q4_K:
-        return x16_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights);
-    case MARMOT_HIP_KIND_Q5_K:
-        return x16_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights);
-    default:
-        return x16_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights);
-    }
-}
-
-// ------------------------------------------------------------------ grouped (MoE)
-bool gemm_x16_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
-                                const void *w1) {
-    // (Q6_K rows are loaded from the 16-byte boundary below: the first one must not begin behind it)
-    return !dev->knobs.no_gemm_i8 && x16_kind(kind) && K % QK_K == 0 && rows * K < ((size_t)1 << 32) &&
-           32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
-           ((((uintptr_t)w0) | ((uintptr_t)w1)) & 15) == 0;
-}
-
-int launch_gemm_x16_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
-                            const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
-                            size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1) {
-    if (max_items > 65535) {
-        return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "grouped tiled GEMM: %zu work items exceed the grid limit",
-                         max_items);
-    }
-    GemmX16Params p = {};
-    p.w[0] = (const uint8_t *)d_w0;
-    p.w[1] = (const uint8_t *)d_w1;
-    p.out[0] = d_out0;
-    p.out[1] = d_out1;
-    p.qs = act.qs;
-    p.ad = act.d;
-    p.sums = act.sums;
-    p.kp = act.kp;
-    p.M = M;
-    p.nb = K / QK_K;
-    p.items = d_items;
-    p.n_items = d_n_items;
-    p.act_index = d_act_index;
-    p.expert_stride = expert_stride;
-    const unsigned weights = d_w1 != nullptr ? 2 : 1;
-    switch (kind) {
-    case MARMOT_HIP_KIND_Q4_K:
-        return x16_launch<MARMOT_HIP_KIND_Q4_K, 2, 4>(dev, p, (unsigned)max_items, weights);
-    case MARMOT_HIP_KIND_Q5_K:
-        return x16_launch<MARMOT_HIP_KIND_Q5_K, 2, 4>(dev, p, (unsigned)max_items, weights);
-    default:
-        return x16_launch<MARMOT_HIP_KIND_Q6_K, 2, 4>(dev, p, (unsigned)max_items, weights);
-    }
+    return kind == MARMOT_HIP_KIND_Q4_K ? x16_launch<MARMOT_HIP_KIND_Q4_K>(dev, p, weights)
+                                        : x16_launch<MARMOT_HIP_KIND_Q5_K>(dev, p, weights);
 }
 
 } // namespace mh

@@ -1,0 +1,895 @@
+// Prompts with packed (Q8_K) activations: K-quant weights x activation codes as a tiled GEMM on the int8 matrix cores, the
+// product of a weight and its sub-block scale cut into two int8 planes.
+//
+// Per 256-value block the reference forms (cpu_vec_dot_q{4,5,6}_k_q8_k, src/backends/cpu/ops/matmul/quantized/
+// vec_dot_impl.h:689-860) y += a.d * (w.d * isum - w.dmin * msum) with isum = sum_j sc_j * (q_j . a_j) and msum = sum_j mn_j *
+// (sum of a over sub-block j). sc * q does not fit int8, but two numbers that do make it up: Q4_K q * (sc & 7) and q * (sc >> 3)
+// (at most 105); Q5_K (0 .. 1953) and Q6_K (-4096 .. 4064) the product itself as 256 * h + l, its high byte and its low byte
+// as signed numbers. One chain of v_mfma_i32_32x32x32_i8 per plane over the whole block gives isum = X + 2^SHIFT * Y exactly
+// (below 2^27), in the matrix time of one fp16 operand, since the int8 instructions run at twice the rate. Beside fp16
+// operands (mh_gemm_int16.hip, which need two for Q6_K) the activations stay the bytes they are packed as: half the reads
+// from LDS, no conversion, direct-to-LDS loads; the price is a shift-add and a conversion per output and block. The sums of
+// 16 codes (at most 2032) and the mins are exact in fp16: one fp16 instruction per block and tile gives msum.
+//
+// What bounds it: vector instructions. Per wavefront and block, 32 rows x 128 tokens, a kernel issues 64 (68) matrix instructions
+// beside 700 (Q6_K), 736 (Q5_K) or 534 (Q4_K) vector ones: 256 or 320 of the fp32 step (one output: shift-add, conversion, two or
+// three multiply-adds), 50 / 16 per 32 values of unpacking (Q6_K, Q5_K / Q4_K), the rest addresses. Hence the tile: what a lane
+// unpacks meets up to four token tiles, and everything else waits in LDS so that two wavefronts fit a SIMD.
+//
+// A wavefront owns 32 weight rows x 32 CT tokens: lane (row j, half kh) unpacks the bytes only it reads, a run of 32 values
+// (a step: 2 CT matrix instructions) ahead of its use, a quarter between every two matrix instructions. A stage is half a block
+// of activation codes (two buffers, one barrier per stage); raw weight blocks go through a private LDS area of the wavefront,
+// whose next block is requested as soon as the last bytes of this one are in registers. The fp32 step of a block is done
+// half at the end of its second stage and half at the beginning of the next block's first, which makes stages equally long.
+// KG = 2: eight wavefronts, two K groups with buffers of their own that take every second block, one stage apart (one does its
+// fp32 step while the other multiplies), sums joined in LDS at the end: for calls that have one tile per compute unit, which
+// would leave a SIMD one wavefront. KG = 1: four wavefronts, two or three workgroups per compute unit; the last tiles of a
+// ragged token count run on as many of the C token tiles as hold a token.
+// Measured (us of whole calls in a row, the quantization of 6 - 17 included; before: the best of the kernels of
+// mh_gemm_int16.hip and mh_gemm_i8.hip; tokens x K x M):
+//          1024 x 14336 x 4096   1000 x 4096 x 14336   1024 x 4096 x 4096   300 x 4096 x 4096
+//   Q6_K   308 / 162             302 / 185             99 / 59              61 / 39
+//   Q5_K   203 / 154             -                     67 / 55              38 / 35
+//   Q4_K   189 / 143             -                     62 / 52              31 / 30
+// and routed experts (E = 128, top 8, H = 2048, F = 768, 2048 tokens) Q6_K 650 / 460, Q4_K 395 / 393.
+#include "mh_rows.h"
+
+#include <type_traits>
+
+namespace mh {
+
+typedef int pl_i32x4 __attribute__((ext_vector_type(4)));
+typedef int pl_i32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 pl_half2 __attribute__((ext_vector_type(2)));
+typedef _Float16 pl_half8 __attribute__((ext_vector_type(8)));
+typedef float pl_float16 __attribute__((ext_vector_type(16)));
+typedef unsigned short pl_u16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t pl_u32x4 __attribute__((ext_vector_type(4)));
+
+struct GemmPlanesParams {
+    const uint8_t *w[3];   // weights: M rows of nb blocks each
+    const int8_t *qs;      // activation codes, rows of kp bytes
+    const float *ad;       // activation block scales [rows][nb]
+    const int16_t *sums;   // sums of 16 codes [rows][16 nb]
+    size_t kp, N, M, nb;
+    void *out[3];
+    const void *bias[3];
+    int bias_is_f16, bias_first, out_is_f16;
+    // grouped (MoE): blockIdx.y selects a work item (expert, first route, routes); activation row of a route through
+    // act_index (null: the route itself), output row = route
+    const int4 *items;
+    const int *n_items;
+    const uint32_t *act_index;
+    size_t expert_stride;
+};
+
+// Per format: 16-byte pieces that cover a row's block from the boundary below its start, whether a minimum exists, and the
+// weight of the second plane
+template <int KIND>
+struct PlanesFormat;
+template <>
+struct PlanesFormat<MARMOT_HIP_KIND_Q4_K> {
+    static constexpr int BYTES = Q4_K_BYTES, PIECES = 9, SHIFT = 3;
+    static constexpr bool MIN = true;
+};
+template <>
+struct PlanesFormat<MARMOT_HIP_KIND_Q5_K> {
+    static constexpr int BYTES = Q5_K_BYTES, PIECES = 11, SHIFT = 8;
+    static constexpr bool MIN = true;
+};
+template <>
+struct PlanesFormat<MARMOT_HIP_KIND_Q6_K> {
+    static constexpr int BYTES = Q6_K_BYTES, PIECES = 14, SHIFT = 8;  // 14 + 210 bytes at most
+    static constexpr bool MIN = false;
+};
+
+constexpr int PLANES_ROWS = 4;  // wavefronts along the rows of a workgroup's tile
+
+template <int KIND, int C, int KG>
+struct PlanesLds {
+    static constexpr int ROWS = 64 / PlanesFormat<KIND>::PIECES;  // whole rows per direct-to-LDS load
+    static constexpr int DMA = (32 + ROWS - 1) / ROWS;            // such loads of a wavefront per block
+    static constexpr int ACT = 32 * C * 128;                      // one stage: 32 C tokens x 128 codes
+    static constexpr int W0 = KG * 2 * ACT;
+    static constexpr int WAVE_W = 32 * 16 * PlanesFormat<KIND>::PIECES;
+    static constexpr int S0 = W0 + PLANES_ROWS * KG * WAVE_W;
+    static constexpr int SUMS = PlanesFormat<KIND>::MIN ? 32 * C * 32 : 0;  // sums of a block as fp16: [token][16]
+    static constexpr int SD = SUMS + 32 * C * 4;                            // then the activation scales [token]
+    static constexpr int OFFS = S0 + 2 * KG * SD;  // lane offsets of the activation loads: [wavefront][load][lane]
+    static constexpr int OFF_N = C + 1 + (PlanesFormat<KIND>::MIN ? 1 : 0);
+    static constexpr int BYTES = OFFS + PLANES_ROWS * KG * OFF_N * 256;
+};
+
+__device__ __forceinline__ pl_u16x2 pl_v(uint32_t v) {
+    return __builtin_bit_cast(pl_u16x2, v);
+}
+__device__ __forceinline__ uint32_t pl_u(pl_u16x2 v) {
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// (a & 0x0f0f0f0f) | (b & 0xf0f0f0f0) in one instruction, whatever is done with the result
+__device__ __forceinline__ uint32_t pl_nibbles(uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(0x0f0f0f0fu), "v"(a), "v"(b));
+    return r;
+}
+// e: products of bytes 0 and 2, o: of bytes 1 and 3, each + 128, as 16-bit numbers: their high bytes and their low bytes - 128
+__device__ __forceinline__ void pl_split(uint32_t e, uint32_t o, int &lo, int &hi) {
+    lo = (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u);
+    hi = (int)__builtin_amdgcn_perm(o, e, 0x07030501u);
+}
+
+// The lane's part of a block: row j, values 16 kh .. 16 kh + 15 of each of the eight runs of 32 values. A half block is four
+// steps; step i unpacks run sub(i) of it, both nibbles of the same 16 bytes one after the other.
+template <int KIND>
+struct PlanesRaw;
+
+template <>
+struct PlanesRaw<MARMOT_HIP_KIND_Q6_K> {
+    uint4 ql, qh;
+    uint32_t scw[2];
+    float d, ndmin;
+    static constexpr int sub(int i) {
+        return (i & 1) * 2 + (i >> 1);
+    }
+    __device__ __forceinline__ void load_low(const uint8_t *at, int hb, int pair, int kh) {
+        __builtin_memcpy(&ql, at + 64 * hb + 32 * pair + 16 * kh, 16);
+    }
+    __device__ __forceinline__ void load_half(const uint8_t *at, int hb, int kh) {
+        __builtin_memcpy(&qh, at + 128 + 32 * hb + 16 * kh, 16);
+        __builtin_memcpy(scw, at + 192 + 8 * hb, 8);
+        scw[0] <<= 8 * (1 - kh);  // bytes 1 and 3: this lane's groups
+        scw[1] <<= 8 * (1 - kh);
+    }
+    __device__ __forceinline__ void load_header(const uint8_t *at, int) {
+        uint16_t v;
+        __builtin_memcpy(&v, at + 208, 2);
+        d = h2f(v);
+        asm volatile("" : "+v"(d));
+        ndmin = 0.0f;
+    }
+    __device__ __forceinline__ pl_half8 mins() const {
+        return pl_half8{};
+    }
+    struct Scale {
+        pl_u16x2 m, c;
+    };
+    __device__ __forceinline__ Scale scale(int, int i) const {
+        const uint32_t word = scw[sub(i) >> 1];
+        const uint32_t m = __builtin_amdgcn_perm(0u, word, (sub(i) & 1) ? 0x09030903u : 0x08010801u);
+        return {pl_v(m), pl_v(m) * pl_u16x2{(unsigned short)-32, (unsigned short)-32} + pl_u16x2{128, 128}};
+    }
+    __device__ __forceinline__ void planes(const Scale &sc, int, int i, int piece, int &lo, int &hi) const {
+        const uint32_t lw[4] = {ql.x, ql.y, ql.z, ql.w};
+        const uint32_t hw[4] = {qh.x, qh.y, qh.z, qh.w};
+        const int s = sub(i);
+        const uint32_t l = (i & 1) ? lw[piece] >> 4 : lw[piece];
+        const uint32_t h = s == 0 ? hw[piece] << 4 : s == 1 ? hw[piece] << 2 : s == 2 ? hw[piece] : hw[piece] >> 2;
+        const uint32_t x = pl_nibbles(l, h);
+        const pl_u16x2 e = pl_v(x & 0x003f003fu), o = pl_v((x >> 8) & 0x003f003fu);
+        pl_split(pl_u(e * sc.m + sc.c), pl_u(o * sc.m + sc.c), lo, hi);
+    }
+};
+
+template <>
+struct PlanesRaw<MARMOT_HIP_KIND_Q4_K> {
+    uint4 q;
+    uint32_t sc, mn;
+    float d, ndmin;
+    static constexpr int sub(int i) {
+        return i;
+    }
+    __device__ __forceinline__ void load_low(const uint8_t *at, int hb, int pair, int kh) {
+        q = *(const uint4 *)(at + 16 + 64 * hb + 32 * pair + 16 * kh);
+    }
+    // 6-bit scales and mins as bytes (get_scale_min_k4, kquant_common.h:29-37)
+    __device__ __forceinline__ void load_half(const uint8_t *at, int hb, int) {
+        const uint4 hdr = *(const uint4 *)at;
+        sc = hb == 0 ? hdr.y & 0x3f3f3f3fu : (hdr.w & 0x0f0f0f0fu) | (((hdr.y >> 6) & 0x03030303u) << 4);
+    }
+    __device__ __forceinline__ void load_header(const uint8_t *at, int kh) {
+        const uint4 hdr = *(const uint4 *)at;
+        d = h2f((uint16_t)(hdr.x & 0xffffu));
+        ndmin = -h2f((uint16_t)(hdr.x >> 16));
+        asm volatile("" : "+v"(d), "+v"(ndmin));  // plain fp32 values: no mixed-precision multiply-adds later
+        mn = kh == 0 ? hdr.z & 0x3f3f3f3fu : ((hdr.w >> 4) & 0x0f0f0f0fu) | (((hdr.z >> 6) & 0x03030303u) << 4);
+        asm volatile("" : "+v"(mn));
+    }
+    // mins as the fp16 operand of the sums: sum 8 kh + e belongs to sub-block 4 kh + e / 2
+    __device__ __forceinline__ pl_half8 mins() const {
+        pl_half8 r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            r[2 * i] = r[2 * i + 1] = (_Float16)(unsigned short)((mn >> (8 * i)) & 0xffu);
+        }
+        return r;
+    }
+    struct Scale {
+        pl_u16x2 lo, hi;
+    };
+    __device__ __forceinline__ uint32_t splat(int i) const {
+        return __builtin_amdgcn_perm(0u, sc, i == 0 ? 0x0c000c00u : i == 1 ? 0x0c010c01u : i == 2 ? 0x0c020c02u : 0x0c030c03u);
+    }
+    __device__ __forceinline__ Scale scale(int, int i) const {
+        const uint32_t v = splat(i);
+        return {pl_v(v & 0x00070007u), pl_v(v >> 3 & 0x00070007u)};
+    }
+    __device__ __forceinline__ void planes(const Scale &s, int, int i, int piece, int &lo, int &hi) const {
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        const pl_u16x2 x = pl_v((i & 1) ? (w[piece] >> 4) & 0x0f0f0f0fu : w[piece] & 0x0f0f0f0fu);
+        lo = (int)pl_u(x * s.lo);
+        hi = (int)pl_u(x * s.hi);
+    }
+};
+
+template <>
+struct PlanesRaw<MARMOT_HIP_KIND_Q5_K> {
+    PlanesRaw<MARMOT_HIP_KIND_Q4_K> k4;
+    uint4 h;  // fifth bits of this lane's 16 positions of every run: bit 4 hb + i
+    float d, ndmin;
+    static constexpr int sub(int i) {
+        return i;
+    }
+    __device__ __forceinline__ void load_low(const uint8_t *at, int hb, int pair, int kh) {
+        k4.load_low(at + 32, hb, pair, kh);
+    }
+    __device__ __forceinline__ void load_half(const uint8_t *at, int hb, int kh) {
+        k4.load_half(at, hb, kh);
+        if (hb == 0) {
+            h = *(const uint4 *)(at + 16 + 16 * kh);
+        }
+    }
+    __device__ __forceinline__ void load_header(const uint8_t *at, int kh) {
+        k4.load_header(at, kh);
+        d = k4.d;
+        ndmin = k4.ndmin;
+    }
+    __device__ __forceinline__ pl_half8 mins() const {
+        return k4.mins();
+    }
+    struct Scale {
+        pl_u16x2 m;
+    };
+    __device__ __forceinline__ Scale scale(int, int i) const {
+        return {pl_v(k4.splat(i))};
+    }
+    __device__ __forceinline__ void planes(const Scale &s, int hb, int i, int piece, int &lo, int &hi) const {
+        const uint32_t w[4] = {k4.q.x, k4.q.y, k4.q.z, k4.q.w};
+        const uint32_t hw[4] = {h.x, h.y, h.z, h.w};
+        const int bit = 4 * hb + i;
+        const uint32_t l = (i & 1) ? w[piece] >> 4 : w[piece];
+        const uint32_t f = bit < 4 ? hw[piece] << (4 - bit) : hw[piece] >> (bit - 4);
+        const uint32_t x = pl_nibbles(l, f);
+        const pl_u16x2 e = pl_v(x & 0x001f001fu), o = pl_v((x >> 8) & 0x001f001fu);
+        const pl_u16x2 c = {128, 128};
+        pl_split(pl_u(e * s.m + c), pl_u(o * s.m + c), lo, hi);
+    }
+};
+
+// 64 x 16 bytes from base + voff (per lane) to LDS address lds_addr + 16 * lane (see dma16_to_lds). The s_nop separates the
+// load from a vector instruction that may have written the scalar base right before it (v_readlane of a spilled scalar
+// register): a memory instruction must not read such a register within five wait states, and the compiler does not look
+// into the assembly to keep them apart.
+__device__ __forceinline__ void planes_dma16(uint32_t lds_addr, const uint8_t *base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(base)
+                 : "memory");
+}
+// The same for the lanes of `mask` only (every lane is active around it): a branch here would be a block of its own, and the
+// compiler moves the arithmetic that belongs before it behind it.
+__device__ __forceinline__ void planes_dma16_of(uint64_t mask, uint32_t lds_addr, const uint8_t *base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(base), "s"(mask)
+                 : "memory");
+}
+// 64 x 4 bytes, to lds_addr + 4 * lane
+__device__ __forceinline__ void planes_dma4(uint32_t lds_addr, const uint8_t *base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(base)
+                 : "memory");
+}
+__device__ __forceinline__ void planes_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int KIND, int C, int KG>
+__global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const GemmPlanesParams p) {
+    using F = PlanesFormat<KIND>;
+    using L = PlanesLds<KIND, C, KG>;
+    constexpr int RG = PLANES_ROWS;
+    constexpr int TOK = 32 * C;
+    constexpr int APW = C;  // direct-to-LDS loads of codes per wavefront and stage, 8 tokens each: the i-th of all wavefronts is tile i
+    static_assert(RG == 4, "a token tile is four loads");
+    warm_kernel_arguments<sizeof(GemmPlanesParams)>();
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gw = wave % RG, kg = wave / RG;  // row group, K group
+    const int which = blockIdx.z;
+    const size_t row0 = (size_t)blockIdx.x * (32 * RG) + 32 * gw;  // this wavefront's first weight row
+    const uint8_t *w = p.w[which];
+    size_t tok0 = (size_t)blockIdx.y * TOK;  // first output row
+    uint32_t toks = (uint32_t)(p.N - tok0 < (size_t)TOK ? p.N - tok0 : (size_t)TOK);
+    if (p.items != nullptr) {
+        if ((int)blockIdx.y >= *p.n_items) {
+            return;
+        }
+        const int4 it = p.items[blockIdx.y];
+        w += (size_t)it.x * p.expert_stride;
+        tok0 = (size_t)it.y;
+        toks = (uint32_t)it.z;
+    }
+    auto act_row = [&](uint32_t t) {  // rows beyond the last token re-read it and are never stored
+        uint32_t row = (uint32_t)tok0 + (t < toks ? t : toks - 1u);
+        return p.act_index != nullptr ? p.act_index[row] : row;
+    };
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_u8_t *)lds;
+
+    // ---- activation codes: load q of a stage brings tokens 8 q .. 8 q + 7, 128 bytes each. Lane l's 16 bytes land in slot l % 8 of
+    // token 8 q + l / 8, which holds chunk (slot ^ swizzle(token)), swizzle(t) = t % 8 ^ (t / 8) % 2: eight, and sixteen, lanes with
+    // consecutive tokens that read one chunk touch different banks.
+    const uint32_t a_group = lds_base + (uint32_t)(kg * 2 * L::ACT);
+    uint32_t *offs = (uint32_t *)(lds + L::OFFS) + wave * (L::OFF_N * 64) + lane;
+#pragma unroll
+    for (int i = 0; i < APW; ++i) {
+        const uint32_t q = (uint32_t)(RG * i + gw);
+        const uint32_t chunk = ((uint32_t)lane & 7u) ^ ((uint32_t)lane >> 3) ^ (q & 1u);
+        offs[64 * i] = act_row(8u * q + ((uint32_t)lane >> 3)) * (uint32_t)p.kp + 16u * chunk;
+    }
+    auto request_acts = [&](uint32_t half, int buffer, int i, uint32_t off) {
+        planes_dma16(a_group + (uint32_t)(buffer * L::ACT + 1024 * (RG * i + gw)), (const uint8_t *)p.qs + (size_t)half * 128u, off);
+    };
+    // ---- scales and sums of a block (tokens wrap around: several lanes then write the same bytes)
+    const uint32_t sd_at = lds_base + (uint32_t)(L::S0 + 2 * kg * L::SD);  // (two blocks)
+    offs[64 * APW] = act_row(((uint32_t)gw * 64u + (uint32_t)lane) % TOK) * (uint32_t)p.nb * 4u;
+    const uint32_t s_tok = (uint32_t)((gw * 64 + lane) >> 1) % TOK;
+    if constexpr (F::MIN) {
+        offs[64 * APW + 64] = act_row(s_tok) * (uint32_t)p.nb * 32u + 16u * (lane & 1);
+    }
+    pl_u32x4 s_next = {};
+    auto request_scales = [&](uint32_t b, uint32_t off) {
+        if (64u * (uint32_t)gw < toks) {
+            planes_dma4(sd_at + (uint32_t)((b / KG & 1u) * L::SD + L::SUMS + 256 * gw), (const uint8_t *)p.ad + (size_t)b * 4u, off);
+        }
+    };
+    auto request_sums = [&](uint32_t b, uint32_t off) {
+        if constexpr (F::MIN) {
+            glb_u8_t *sums = (glb_u8_t *)p.sums + (size_t)b * 32u;
+            asm("" : "+s"(sums));
+            s_next = *(const __attribute__((address_space(1))) pl_u32x4 *)(sums + (size_t)off);
+        }
+    };
+    auto store_block = [&](uint32_t b) {
+        if constexpr (F::MIN) {
+            const uint32_t v[4] = {s_next.x, s_next.y, s_next.z, s_next.w};
+            uint32_t e[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                e[c] = __builtin_bit_cast(uint32_t, pl_half2{(_Float16)(int16_t)(v[c] & 0xffffu), (_Float16)(int16_t)(v[c] >> 16)});
+            }
+            *(uint4 *)(lds + L::S0 + (2 * kg + (b / KG & 1u)) * L::SD + s_tok * 32u + 16u * (lane & 1)) = make_uint4(e[0], e[1], e[2], e[3]);
+        }
+    };
+
+    // ---- weights: load i of a block brings rows ROWS i .. + ROWS - 1 of the wavefront: lane l the 16-byte piece l % PIECES
+    // of row l / PIECES, counted from the 16-byte boundary at or below the row's block; a piece that holds no byte of the
+    // block re-reads the last one that does, lanes behind the last row and rows behind the matrix re-read a row before.
+    const uint32_t row_bytes = (uint32_t)p.nb * F::BYTES;
+    const uint32_t rows = (uint32_t)(row0 < p.M ? (p.M - row0 < 32 ? p.M - row0 : 32) : 0);
+    const uint8_t *wbase = w + (row0 < p.M ? row0 : p.M - 1) * row_bytes;
+    const uint32_t low4 = (uint32_t)((uintptr_t)wbase & 15u);
+    wbase = uniform_pointer(wbase - low4);
+    const uint32_t last_row = rows == 0 ? 0 : rows - 1u;
+    const uint32_t w_r = (uint32_t)lane / F::PIECES < L::ROWS ? (uint32_t)lane / F::PIECES : L::ROWS - 1u;
+    const uint32_t w_piece = 16u * ((uint32_t)lane - F::PIECES * w_r < F::PIECES ? (uint32_t)lane - F::PIECES * w_r : F::PIECES - 1u);
+    const uint32_t w_lds = lds_base + (uint32_t)(L::W0 + wave * L::WAVE_W);
+    const uint32_t w_first = low4 + w_r * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
+    const uint32_t w_last = low4 + last_row * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
+    // Q6_K: the piece that holds the end of the matrix may reach up to 14 bytes behind it (its size need not be a multiple
+    // of 16), and those bytes need not exist. The wavefront of the last row brings the piece before in its place (one
+    // operand more of a minimum that is there anyway) and copies the bytes that exist when the block is read (bring_end).
+    const uint32_t w_end = low4 + (last_row + 1u) * row_bytes;
+    const bool ragged = F::BYTES % 16 != 0 && row0 + 32 >= p.M && (w_end & 15u) != 0;
+    const uint32_t w_most = ragged ? (w_end & ~15u) - 16u : ~0u;
+    const uint32_t end_block = ragged ? (uint32_t)p.nb - 1u : ~0u;
+    auto request_weights = [&](uint32_t b, int i) {
+        uint32_t at = w_first;
+        asm volatile("" : "+v"(at));  // formed at each load: kept in registers, the L::DMA offsets would be spilled
+        at += (uint32_t)i * (L::ROWS * row_bytes);
+        at = at < w_last ? at : w_last;
+        const uint32_t to = w_lds + (uint32_t)(i * L::ROWS * 16 * F::PIECES);
+        if constexpr (F::BYTES % 16 != 0) {
+            at += b * (uint32_t)F::BYTES;
+            const uint32_t last = (at + (uint32_t)F::BYTES - 1u) & ~15u;
+            at = (at & ~15u) + w_piece;
+            at = at < last ? at : last;
+            at = at < w_most ? at : w_most;
+        }
+        const uint8_t *base = F::BYTES % 16 != 0 ? wbase : wbase + (size_t)b * F::BYTES;
+        // (the launcher checks that rows of whole 16-byte pieces start on 16-byte boundaries)
+        // lanes without a row write nothing: the place behind the rows of this load belongs to the next one
+        constexpr int ALL = L::ROWS * F::PIECES, LAST = (32 - L::ROWS * (L::DMA - 1)) * F::PIECES;
+        planes_dma16_of(~0ull >> (64 - (i + 1 < L::DMA ? ALL : LAST)), to, base, at);
+    };
+    // After the loads of block b have arrived: the end of the matrix, two bytes per lane
+    auto bring_end = [&](uint32_t b) {
+        if constexpr (F::BYTES % 16 != 0) {
+            if (b == end_block) {
+                const uint32_t block = low4 + last_row * row_bytes + b * (uint32_t)F::BYTES;
+                const uint32_t from = (w_end & ~15u) + 2u * (uint32_t)lane;
+                if (from < w_end) {
+                    uint8_t *to = lds + L::W0 + wave * L::WAVE_W + last_row * (16 * F::PIECES) + (from - (block & ~15u));
+                    *(uint16_t *)to = *(const __attribute__((address_space(1))) uint16_t *)(wbase + from);
+                }
+            }
+        }
+    };
+    const uint32_t my_row = low4 + ((uint32_t)j < last_row ? (uint32_t)j : last_row) * row_bytes;
+    const uint8_t *my_w = lds + L::W0 + wave * L::WAVE_W + j * (16 * F::PIECES);
+    auto my_block = [&](uint32_t b) {  // (blocks of whole pieces start at the beginning of their place)
+        return F::BYTES % 16 != 0 ? my_w + ((my_row + b * (uint32_t)F::BYTES) & 15u) : my_w;
+    };
+
+    // CT: the token tiles that hold a token
+    auto walk = [&](auto tiles_c) {
+    constexpr int CT = decltype(tiles_c)::value;
+    pl_float16 total[CT];
+#pragma unroll
+    for (int t = 0; t < CT; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            total[t][r] = 0.0f;
+        }
+    }
+    pl_i32x16 X[CT], Y[CT];
+    PlanesRaw<KIND> raw;
+    const uint32_t nb = (uint32_t)p.nb;
+    const uint32_t a_at = a_group + (uint32_t)(j * 128 + 16 * (kh ^ (j & 7) ^ ((j >> 3) & 1)));
+
+    // fp32 step of a block: y += a.d * (w.d * isum - w.dmin * msum)
+    auto finish = [&](uint32_t b, int first, int last) {
+        const uint8_t *sd = lds + L::S0 + (2 * kg + (b / KG & 1u)) * L::SD;
+        pl_half8 sums = {}, mins = {};
+        if constexpr (F::MIN) {
+            sums = *(const pl_half8 *)(sd + (32 * first + j) * 32 + 16 * kh);
+            mins = raw.mins();
+        }
+#pragma unroll
+        for (int t = first; t < last; ++t) {
+            pl_float16 T = {};
+            if constexpr (F::MIN) {
+                T = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, mins, T, 0, 0, 0);
+                if (t + 1 < last) {
+                    sums = *(const pl_half8 *)(sd + (32 * (t + 1) + j) * 32 + 16 * kh);
+                }
+            }
+            float4 da4 = *(const float4 *)(sd + L::SUMS + 4 * (32 * t + 4 * kh));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float da[4] = {da4.x, da4.y, da4.z, da4.w};
+                if (q < 3) {
+                    da4 = *(const float4 *)(sd + L::SUMS + 4 * (32 * t + 8 * (q + 1) + 4 * kh));
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * q + e;
+                    float v = raw.d * (float)((Y[t][r] << F::SHIFT) + X[t][r]);
+                    if constexpr (F::MIN) {
+                        v = __builtin_fmaf(raw.ndmin, T[r], v);
+                    }
+                    total[t][r] = __builtin_fmaf(da[e], v, total[t][r]);
+                }
+            }
+            asm volatile("" : "+v"(total[t]));  // done here: the sums of a block's products are not carried further
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // Blocks kg, kg + KG, ... are this K group's.
+    const uint32_t mine = nb > (uint32_t)kg ? (nb - (uint32_t)kg + KG - 1u) / KG : 0u;
+    const uint32_t stages = 2u * ((nb + KG - 1u) / KG) + (KG > 1 ? 1u : 0u);  // barriers of every wavefront
+    uint32_t passed = 0;
+    pl_i32x4 lo[2], hi[2];
+    // The weights of block b have been requested: unpacks its first step
+    auto first_load = [&](uint32_t b) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        bring_end(b);
+        raw.load_half(my_block(b), 0, kh);
+        raw.load_low(my_block(b), 0, 0, kh);
+    };
+    auto first_step = [&](uint32_t b) {
+        const auto sc = raw.scale(0, 0);
+#pragma unroll
+        for (int piece = 0; piece < 4; ++piece) {
+            int l, h;
+            raw.planes(sc, 0, 0, piece, l, h);
+            lo[0][piece] = l;
+            hi[0][piece] = h;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (mine != 0) {
+#pragma unroll
+        for (int i = 0; i < L::DMA; ++i) {
+            request_weights((uint32_t)kg, i);
+        }
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+            request_acts(2u * (uint32_t)kg, 0, i, offs[64 * i]);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    planes_barrier();
+    if (KG > 1 && kg == 1) {
+        planes_barrier();
+        ++passed;
+    }
+    for (uint32_t ib = 0; ib < mine; ++ib) {
+        const uint32_t b = (uint32_t)kg + KG * ib;
+        const uint32_t bn = ib + 1 < mine ? b + KG : b;  // (the last block is requested again rather than branched around)
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+            constexpr int STEPS = 4 * CT, AHEAD = 2;
+            pl_i32x4 ring[AHEAD];
+            uint32_t a_addr = 0;
+            auto read_a = [&](int st) {
+                const int s = st / CT, t = st % CT;
+                if (t == 0) {
+                    asm volatile("v_xor_b32 %0, %1, %2" : "=v"(a_addr) : "s"(32 * PlanesRaw<KIND>::sub(s)), "v"(a_at));
+                }
+                ring[st % AHEAD] = *(const __attribute__((address_space(3))) pl_i32x4 *)(
+                    (const lds_u8_t *)(uintptr_t)a_addr + hb * L::ACT + t * 4096);
+            };
+            if (hb == 0) {
+                // (Q6_K's blocks are the largest and arrive last: read behind the fp32 step, 3 % of 1024 x 14336 x 4096)
+                if (F::BYTES % 16 == 0) {
+                    first_load(b);
+                }
+                if (ib != 0) {
+                    finish(b - KG, CT / 2, CT);
+                }
+                if (F::BYTES % 16 != 0) {
+                    first_load(b);
+                }
+                first_step(b);
+                raw.load_header(my_block(b), kh);
+            }
+#pragma unroll
+            for (int st = 0; st < AHEAD; ++st) {
+                read_a(st);
+            }
+            uint32_t off = offs[0];  // of the next load of the activations
+            // Steps before fp32 steps of the other K group's wavefront on this SIMD, which fill what matrix instructions leave (2 - 3 %;
+            // independent workgroups are 4 % slower with it)
+            if (KG > 1) {
+                __builtin_amdgcn_s_setprio(1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            typename PlanesRaw<KIND>::Scale sc = {};
+#pragma unroll
+            for (int st = 0; st < STEPS; ++st) {
+                const int s = st / CT, t = st % CT;
+                const pl_i32x4 a = ring[st % AHEAD];
+                const pl_i32x16 zero = {};
+                X[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, lo[s & 1], hb == 0 && s == 0 ? zero : X[t], 0, 0, 0);
+                Y[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, hi[s & 1], hb == 0 && s == 0 ? zero : Y[t], 0, 0, 0);
+                if (st + AHEAD < STEPS) {
+                    read_a(st + AHEAD);
+                }
+                // the next stage's codes, then scales and sums of this block: one load per place
+                if (st < CT) {
+                    request_acts(hb == 0 ? 2u * b + 1u : 2u * bn, hb ^ 1, st, off);
+                    if (st + 1 < CT) {
+                        off = offs[64 * (st + 1)];
+                    } else if (hb == 0) {
+                        off = offs[64 * APW];
+                    }
+                } else if (st == CT && hb == 0) {
+                    request_scales(b, off);
+                    if (F::MIN) {
+                        off = offs[64 * (APW + 1)];
+                    }
+                } else if (st == CT + 1 && hb == 0) {
+                    request_sums(b, off);
+                }
+                // the operands of the next step, a quarter at a time
+                const int hn = s < 3 ? hb : 1, sn = (s + 1) & 3;
+                if (t == 0) {
+                    if (s == 3 && hb == 0) {
+                        store_block(b);
+                        raw.load_half(my_block(b), hn, kh);
+                    }
+                    if (s == 1 || (s == 3 && hb == 0)) {
+                        raw.load_low(my_block(b), hn, sn / 2, kh);
+                    }
+                }
+                // The last bytes of this block have been read: its place is the next one's. (Waited for: the request alone does not keep the
+                // new bytes behind a read that still queues for LDS.)
+                constexpr int FREE = CT == 1 ? 2 : 3 * CT / 2;
+                if (hb == 1 && st == FREE) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                }
+                if (hb == 1) {
+#pragma unroll
+                    for (int i = 0; i < L::DMA; ++i) {
+                        if (st == FREE + i * CT / L::DMA) {
+                            request_weights(bn, i);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int piece = 0; piece < 4; ++piece) {
+                    // (not at once: the bytes are on their way from LDS)
+                    if ((s < 3 || hb == 0) && (piece + 1 < 4 ? piece + 1 : 3) * CT / 4 == t) {
+                        if (piece == 0) {
+                            sc = raw.scale(hn, sn);
+                        }
+                        int l, h;
+                        raw.planes(sc, hn, sn, piece, l, h);
+                        lo[sn & 1][piece] = l;
+                        hi[sn & 1][piece] = h;
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (KG > 1) {
+                __builtin_amdgcn_s_setprio(0);
+            }
+            if (hb == 0) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else {
+                finish(b, 0, CT / 2);
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L::DMA) : "memory");  // all but the weights, the last requests
+            }
+            planes_barrier();
+            ++passed;
+        }
+    }
+    // (the last block's weights were requested once more: they must not land in the LDS of the workgroup that comes after)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (mine != 0) {
+        finish(kg + KG * (mine - 1), CT / 2, CT);
+    }
+    if constexpr (KG > 1) {
+        for (; passed < stages; ++passed) {
+            planes_barrier();
+        }
+        // the K groups' sums meet in LDS: each gives the other half of its token tiles and keeps the other half
+        static_assert(KG == 2 && CT == C && C % 2 == 0, "two K groups, halves of whole token tiles");
+        float *mail = (float *)lds + (size_t)wave * (C / 2) * 1024 + lane * 4;
+        const float *from = (const float *)lds + (size_t)(wave ^ RG) * (C / 2) * 1024 + lane * 4;
+#pragma unroll
+        for (int t = 0; t < C / 2; ++t) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float4 v;
+                v.x = kg == 0 ? total[C / 2 + t][4 * q] : total[t][4 * q];
+                v.y = kg == 0 ? total[C / 2 + t][4 * q + 1] : total[t][4 * q + 1];
+                v.z = kg == 0 ? total[C / 2 + t][4 * q + 2] : total[t][4 * q + 2];
+                v.w = kg == 0 ? total[C / 2 + t][4 * q + 3] : total[t][4 * q + 3];
+                *(float4 *)(mail + (4 * t + q) * 256) = v;
+            }
+        }
+        planes_barrier();
+#pragma unroll
+        for (int t = 0; t < C / 2; ++t) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 v = *(const float4 *)(from + (4 * t + q) * 256);
+                const float add[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * q + e;
+                    // (in the order of K: group 0's sum first)
+                    total[t][r] = kg == 0 ? total[t][r] + add[e] : add[e] + total[C / 2 + t][r];
+                }
+            }
+        }
+    }
+
+    // lane (j, kh) holds weight row row0 + j for tokens 32 t + 8 (r / 4) + 4 kh + r % 4: 32 rows of a token per store
+    if ((uint32_t)j >= rows) {
+        return;
+    }
+    const size_t m = row0 + j;
+    constexpr int OUT = KG > 1 ? C / 2 : CT;  // token tiles this wavefront stores
+    const uint32_t t0 = (uint32_t)(KG > 1 ? kg * OUT : 0);
+    const void *bias_p = p.bias[which];
+    const bool has_bias = bias_p != nullptr;
+    const float bias = !has_bias ? 0.0f : p.bias_is_f16 ? h2f(((const uint16_t *)bias_p)[m]) : ((const float *)bias_p)[m];
+    if (!p.out_is_f16) {
+        float *out = (float *)p.out[which] + tok0 * p.M + m;
+#pragma unroll
+        for (int t = 0; t < OUT; ++t) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t n = (uint32_t)(32 * (t0 + t) + 8 * (r >> 2) + 4 * kh + (r & 3));
+                if (n < toks) {
+                    out[(size_t)n * p.M] = has_bias ? total[t][r] + bias : total[t][r];
+                }
+            }
+        }
+    } else {
+        uint16_t *out = (uint16_t *)p.out[which] + tok0 * p.M + m;
+        const bool bias_first = p.bias_first != 0;
+#pragma unroll
+        for (int t = 0; t < OUT; ++t) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t n = (uint32_t)(32 * (t0 + t) + 8 * (r >> 2) + 4 * kh + (r & 3));
+                if (n < toks) {
+                    // without bias_first: round to the output type, then add the bias in it
+                    const uint16_t first = f2h(has_bias && bias_first ? total[t][r] + bias : total[t][r]);
+                    out[(size_t)n * p.M] = has_bias && !bias_first ? f2h(h2f(first) + bias) : first;
+                }
+            }
+        }
+    }
+    };
+    if constexpr (KG == 1) {
+        const uint32_t tiles = (toks + 31u) / 32u;
+        if (C >= 4 && tiles == 4) {
+            walk(std::integral_constant<int, C < 4 ? 1 : 4>{});
+        } else if (C >= 3 && tiles == 3) {
+            walk(std::integral_constant<int, C < 3 ? 1 : 3>{});
+        } else if (tiles == 2) {
+            walk(std::integral_constant<int, 2>{});
+        } else {
+            walk(std::integral_constant<int, 1>{});
+        }
+    } else {
+        walk(std::integral_constant<int, C>{});
+    }
+}
+
+template <int KIND, int C, int KG>
+static int planes_launch(marmot_hip_device *dev, const GemmPlanesParams &p, unsigned col_tiles, unsigned weights) {
+    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_planes<KIND, C, KG>));
+    const dim3 grid((unsigned)((p.M + 32 * PLANES_ROWS - 1) / (32 * PLANES_ROWS)), col_tiles, weights);
+    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG>), grid, dim3(64 * PLANES_ROWS * KG), (PlanesLds<KIND, C, KG>::BYTES), dev->stream, p);
+    MH_HIP(hipGetLastError());
+    return MARMOT_HIP_SUCCESS;
+}
+
+
+static bool planes_kind(int kind) {
+    return kind == MARMOT_HIP_KIND_Q4_K || kind == MARMOT_HIP_KIND_Q5_K || kind == MARMOT_HIP_KIND_Q6_K;
+}
+
+// Which form (10 C + KG), or none (0), by the tiles a call has. The kernels of mh_gemm_i8.hip split K over workgroups where
+// tiles are few, which pays the partial sums and wins while the chip is mostly empty; two K groups per workgroup want one
+// tile per compute unit, and beyond that workgroups share one (us of whole calls, other kernels / forms):
+//   Q6_K, 64 tokens a tile    64 tiles 128 x 4096 x 4096 31 / (22) 37   104, 800 x 4096 x 1024 47 / (22) 42
+//                             88 tiles 128 x 2048 x 5632 29 / (22) 24   128, 200 x 14336 x 4096 122 / (22) 109
+//   Q4_K, the same            128 tiles 200 x 4096 x 4096 28 / (22) 30  160, 300 x 4096 x 4096 31.5 / (22) 30.3
+//                             224, 128 x 4096 x 14336 31.9 / (22) 30.9  256, 512 x 14336 x 4096 100 / (22) 91
+//   with up to eight blocks   64, 64 x 1024 x 8192 15.8 / (22) 13.9     88, 128 x 2048 x 5632 20.0 / (22) 19.0
+//                             44, 128 x 2048 x 2816: other kernels
+//   128 tokens a tile         Q4_K 192 tiles 300 x 1024 x 8192 22.8 / (42) 20.2   256, 1024 x 14336 x 4096 187 / (42) 142
+//   more tiles than units     Q4_K 308, 800 x 2048 x 5632 49 / (42) 50, (41) 46, (21) 40   784, 800 x 4096 x 14336 167 / 153, 145, 130
+//                             Q6_K 308, 77 / (42) 57, (41) 53, (21) 52   896, 1024 x 4096 x 14336 303 / 186, 178, 204
+// Q4_K and Q5_K: where mh_gemm_int16.hip has a form of 256 x 128 for the call, that one is as fast or faster (1024 x 4096 x 14336
+// Q4_K 156 against 155, Q5_K 162 against 169; 1024 x 1024 x 8192 31 against 35).
+static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t nb, size_t weights) {
+    const size_t cus = (size_t)dev->props.multiProcessorCount;
+    const size_t rows = (M + 127) / 128 * weights;
+    const size_t small = (N + 63) / 64 * rows, large = (N + 127) / 128 * rows;
+    if (small <= cus) {
+        const bool few = kind == MARMOT_HIP_KIND_Q6_K || nb <= 8 ? 3 * small <= cus : 5 * small <= 3 * cus;
+        return few ? 0 : 22;
+    }
+    return large <= cus ? 42 : kind == MARMOT_HIP_KIND_Q6_K ? 41 : 21;
+}
+
+bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights,
+                         const ActScratch &act) {
+    if (dev->knobs.no_gemm_i8 || !planes_kind(kind) || K % QK_K != 0) {
+        return false;
+    }
+    if ((((uintptr_t)act.qs) & 15) != 0 || act.kp % 16 != 0 || N * act.kp >= ((size_t)1 << 32) ||
+        32 * (K / QK_K) * block_bytes(kind) >= ((size_t)1 << 31) || N > (size_t)65535 * 64) {
+        return false;  // 32-bit lane offsets
+    }
+    return planes_form(dev, kind, N, M, K / QK_K, (size_t)weights) != 0;
+}
+
+// The tile of 64 tokens keeps the route name of the kernel that had it before (callers compare names).
+template <int KIND>
+static int planes_launch_kind(marmot_hip_device *dev, const GemmPlanesParams &p, unsigned weights, const char *small_route,
+                              const char *large_route) {
+    const int form = planes_form(dev, KIND, p.N, p.M, p.nb, weights);
+    set_route(form >= 40 ? large_route : small_route);
+    const unsigned t64 = (unsigned)((p.N + 63) / 64), t128 = (unsigned)((p.N + 127) / 128);
+    if (form == 22) {
+        return planes_launch<KIND, 2, 2>(dev, p, t64, weights);
+    }
+    if (form == 42) {
+        return planes_launch<KIND, 4, 2>(dev, p, t128, weights);
+    }
+    if constexpr (KIND == MARMOT_HIP_KIND_Q6_K) {
+        return planes_launch<KIND, 4, 1>(dev, p, t128, weights);
+    } else {
+        return planes_launch<KIND, 2, 1>(dev, p, t64, weights);
+    }
+}
+
+int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
+                       size_t M, int out_dtype) {
+    GemmPlanesParams p = {};
+    for (int i = 0; i < ws.count; ++i) {
+        p.w[i] = (const uint8_t *)ws.w[i];
+        p.out[i] = ws.out[i];
+        p.bias[i] = ws.bias[i];
+    }
+    p.qs = act.qs;
+    p.ad = act.d;
+    p.sums = act.sums;
+    p.kp = act.kp;
+    p.N = N;
+    p.M = M;
+    p.nb = K / QK_K;
+    p.bias_is_f16 = ws.bias_dtype == MARMOT_HIP_DTYPE_F16;
+    p.bias_first = ws.bias_first ? 1 : 0;
+    p.out_is_f16 = out_dtype == MARMOT_HIP_DTYPE_F16;
+    const unsigned weights = (unsigned)ws.count;
+    switch (kind) {
+    case MARMOT_HIP_KIND_Q4_K:
+        return planes_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights, "mmq_q4_k_q8_k_int8_planes_128x64",
+                                                        "mmq_q4_k_q8_k_int8_planes_128x128");
+    case MARMOT_HIP_KIND_Q5_K:
+        return planes_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights, "mmq_q5_k_q8_k_fp16_tile_128x64",
+                                                        "mmq_q5_k_q8_k_int8_planes_128x128");
+    default:
+        return planes_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights, "mmq_q6_k_q8_k_fp16_tile_128x64",
+                                                        "mmq_q6_k_q8_k_int8_planes_128x128");
+    }
+}
+
+// ------------------------------------------------------------------ grouped (MoE)
+bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
+                                   const void *w1) {
+    // (Q6_K rows are loaded from the 16-byte boundary below: the first one must not begin behind it)
+    return !dev->knobs.no_gemm_i8 && planes_kind(kind) && K % QK_K == 0 && rows * K < ((size_t)1 << 32) &&
+           32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
+           ((((uintptr_t)w0) | ((uintptr_t)w1)) & 15) == 0;
+}
+
+int launch_gemm_planes_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
+                               const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
+                               size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1) {
+    if (max_items > 65535) {
+        return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "grouped tiled GEMM: %zu work items exceed the grid limit",
+                         max_items);
+    }
+    GemmPlanesParams p = {};
+    p.w[0] = (const uint8_t *)d_w0;
+    p.w[1] = (const uint8_t *)d_w1;
+    p.out[0] = d_out0;
+    p.out[1] = d_out1;
+    p.qs = act.qs;
+    p.ad = act.d;
+    p.sums = act.sums;
+    p.kp = act.kp;
+    p.M = M;
+    p.nb = K / QK_K;
+    p.items = d_items;
+    p.n_items = d_n_items;
+    p.act_index = d_act_index;
+    p.expert_stride = expert_stride;
+    const unsigned weights = d_w1 != nullptr ? 2 : 1;
+    // Items of 64 routes and three workgroups per compute unit: with items of 128 and two of them, 2048 tokens of 128 experts
+    // take 401 us for 393 (Q4_K), 452 for 460 (Q6_K).
+    switch (kind) {
+    case MARMOT_HIP_KIND_Q4_K:
+        return planes_launch<MARMOT_HIP_KIND_Q4_K, 2, 1>(dev, p, (unsigned)max_items, weights);
+    case MARMOT_HIP_KIND_Q5_K:
+        return planes_launch<MARMOT_HIP_KIND_Q5_K, 2, 1>(dev, p, (unsigned)max_items, weights);
+    default:
+        return planes_launch<MARMOT_HIP_KIND_Q6_K, 2, 1>(dev, p, (unsigned)max_items, weights);
+    }
+}
+
+} // namespace mh

@@ -1078,6 +1078,9 @@ int launch_mmq_set(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
         if (gemm_x16_applies(dev, kind, N, K, M, ws.count, act)) {
             return launch_gemm_x16(dev, kind, ws, act, N, K, M, out_dtype);
         }
+        if (gemm_planes_applies(dev, kind, N, K, M, ws.count, act)) {
+            return launch_gemm_planes(dev, kind, ws, act, N, K, M, out_dtype);
+        }
         return launch_gemm_i8(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }
     if (kind == MARMOT_HIP_KIND_Q6_K && mmq_rows_q6k_applies(dev, ws, N, K, M)) {

@@ -10,7 +10,7 @@
 namespace mh {
 
 constexpr int MOE_ITEM_COLS = 8;   // routes per grouped work item (16 or 32 when experts see many routes, see moe_item_cols)
-// Routes per expert from which prompts take the tiled GEMM (mh_gemm_int16.hip, 64 routes per item) instead of passes of
+// Routes per expert from which prompts take the tiled GEMM (mh_gemm_planes.hip, 64 routes per item) instead of passes of
 // 16 or 32 routes, given two of its tiles per compute unit in both projections (us before / tiled, E = 128, top 8, H = 2048,
 // F = 768: Q4_K 512 tokens = 32 routes per expert 248 / 182, 1024 401 / 260, 2048 729 / 429; Q6_K 512 472 / 285)
 constexpr size_t MOE_TILED_ROUTES = 32;
@@ -579,12 +579,12 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     if (mmq_gu && mmq_dn && routes >= 12 * E) {
         item_cols = (routes >= 24 * E && q45(kind_gate_up) && q45(kind_down)) ? 32 : 16;
     }
-    // Prompts with many routes per expert: the tiled GEMM on integer fp16 operands, 64 routes per item
+    // Prompts with many routes per expert: the tiled GEMM on int8 planes, 64 routes per item
     const size_t tiled_items = routes / 64 + E / 2, two_per_cu = 2 * (size_t)dev->props.multiProcessorCount;
     const bool tiled = routes >= MOE_TILED_ROUTES * E && tiled_items * 2 * ((F + 127) / 128) >= two_per_cu &&
                        tiled_items * ((H + 127) / 128) >= two_per_cu &&
-                       gemm_x16_grouped_supported(dev, kind_gate_up, T, H, F, d_gate, d_up) &&
-                       gemm_x16_grouped_supported(dev, kind_down, routes, F, H, d_down, d_down);
+                       gemm_planes_grouped_supported(dev, kind_gate_up, T, H, F, d_gate, d_up) &&
+                       gemm_planes_grouped_supported(dev, kind_down, routes, F, H, d_down, d_down);
     if (tiled) {
         item_cols = 64;
     }
@@ -677,9 +677,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     }
     const size_t gu_stride = F * ((H + bv_gu - 1) / bv_gu) * block_bytes(kind_gate_up);
     const size_t dn_stride = H * ((F + bv_dn - 1) / bv_dn) * block_bytes(kind_down);
-    // K-quant experts run on the matrix cores (long prompts on the tiled GEMM with integer fp16 operands, else passes on
-    // int8), the 32-value formats on the dot-product matvec
-    st = tiled  ? launch_gemm_x16_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
+    // K-quant experts run on the matrix cores (long prompts on the tiled GEMM on int8 planes, else passes), the 32-value formats on the dot-product matvec
+    st = tiled  ? launch_gemm_planes_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
                                           max_items, H, F, gate_out, up_out)
         : mmq_gu ? launch_mmq_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
                                      max_items, H, F, gate_out, up_out, (int)item_cols)
@@ -715,7 +714,7 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
                                   dev->stream));
         }
     }
-    st = tiled  ? launch_gemm_x16_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags,
+    st = tiled  ? launch_gemm_planes_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags,
                                           max_items, F, H, route_down, nullptr)
         : mmq_dn ? launch_mmq_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags, max_items,
                                      F, H, route_down, nullptr, (int)item_cols)

@@ -1,0 +1,102 @@
+"""Tiled GEMM of K-quant weights and Q8_K activations on int8 planes (mh_gemm_planes.hip) against the CPU oracle, at the edges
+of its forms and of the rule that chooses one (planes_form, 256 compute units): two K groups per workgroup or one, 64 or 128
+tokens per tile, last tiles with one to four token tiles, one block per row (the second K group has none) and odd counts."""
+import numpy as np
+import pytest
+
+from oracle.pyoracle import KIND_Q4_K, KIND_Q5_K, KIND_Q6_K
+from tests.util import assert_matmul_parity, gaussian, random_valid_blocks
+
+pytestmark = pytest.mark.gpu
+
+KINDS = {"q4_k": KIND_Q4_K, "q5_k": KIND_Q5_K, "q6_k": KIND_Q6_K}
+SMALL = {"q4_k": "int8_planes_128x64", "q5_k": "fp16_tile_128x64", "q6_k": "fp16_tile_128x64"}
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from marmot_amd import HipBackend
+
+    b = HipBackend(0)
+    yield b
+    b.close()
+
+
+CASES = [
+    # (kinds, tile, tokens, rows, K)
+    ("q4_k q5_k", "small", 128, 10400, 256),   # two K groups, 64 tokens, the second group without a block
+    ("q4_k q5_k", "small", 97, 12801, 768),    # odd block counts, one row and 33 tokens in the last tiles
+    ("q6_k", "small", 33, 11000, 1280),
+    ("q4_k q5_k q6_k", "large", 257, 6785, 768),   # two K groups, 128 tokens, one token in the last tile
+    ("q4_k q5_k q6_k", "large", 380, 8200, 256),
+    ("q4_k q5_k", "small", 130, 16600, 512),   # one K group, 64 tokens
+    ("q4_k q5_k", "small", 161, 18500, 256),   # (two token tiles in the last one)
+    ("q6_k", "large", 257, 11000, 512),        # one K group, 128 tokens: one, two, three and four token tiles in the last one
+    ("q6_k", "large", 300, 11000, 256),
+    ("q6_k", "large", 340, 11000, 768),
+    ("q6_k", "large", 384, 11001, 512),
+]
+
+
+@pytest.mark.parametrize("name,tile,N,M,K", [(n, t, *rest) for names, t, *rest in CASES for n in names.split()])
+def test_forms_match_oracle(hip, oracle, name, tile, N, M, K):
+    """The bound is the suite's for matmul outputs (1e-3, floored): exact integer block sums on both sides, so only the fp32
+    sum over at most five blocks is ordered differently. Arbitrary block bytes: every nibble, scale (Q6_K: -128 among them,
+    products -4096 .. 4064 in two bytes) and minimum."""
+    kind = KINDS[name]
+    blocks = random_valid_blocks(np.random.default_rng(800 + N), kind, M, K)
+    x, bias = gaussian(801 + N, (N, K)), gaussian(802, (M,))
+    got = hip.linear(x, blocks, kind, M, bias=bias)
+    assert hip.last_route() == f"mmq_{name}_q8_k_{SMALL[name] if tile == 'small' else 'int8_planes_128x128'}"
+    assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, bias=bias, threads=16), what=f"{name} {N} x {K} x {M}")
+
+
+@pytest.mark.parametrize("name,N,M", [("q4_k", 130, 16600), ("q5_k", 130, 16600), ("q6_k", 300, 11000),  # one K group
+                                      ("q4_k", 257, 6800), ("q5_k", 257, 6800), ("q6_k", 257, 6800)])  # two
+@pytest.mark.parametrize("scale", ["largest", "mixed"])
+def test_block_sums_are_exact(hip, name, N, M, scale):
+    """One block per row, activation and block scales of 1, minimum scale 0: the output is the integer block sum rounded
+    once, also where it does not fit 24 bits (sums of one sign at the largest values reach 2^24.9, Q5_K 2^25.9, Q6_K 2^26.9)."""
+    kind, K, rng = KINDS[name], 256, np.random.default_rng(810)
+    bb = {"q4_k": 144, "q5_k": 176, "q6_k": 210}[name]
+    few = rng.integers(0, 256, (4, bb), dtype=np.uint8)  # a few distinct blocks, repeated
+    one, zero = np.float16(1.0).tobytes(), np.float16(0.0).tobytes()
+    if name == "q6_k":
+        few[:, 208:210] = np.frombuffer(one, np.uint8)
+        if scale == "largest":
+            few[:, 192:208] = np.array([127, 128, 127, 128], np.uint8)[:, None]
+            few[:, :192] = np.array([0, 0, 255, 255], np.uint8)[:, None]
+        ql, qh = few[:, :128].astype(np.int64).reshape(4, 2, 2, 32), few[:, 128:192].astype(np.int64).reshape(4, 2, 32)
+        u = np.stack([((ql[:, :, g & 1] >> (4 * (g >> 1))) & 15) | (((qh >> (2 * g)) & 3) << 4) for g in range(4)], axis=2)
+        w = (u - 32).reshape(4, 16, 16) * few[:, 192:208].view(np.int8).astype(np.int64)[:, :, None]
+    else:
+        qs = 16 if name == "q4_k" else 48
+        few[:, 0:2], few[:, 2:4] = np.frombuffer(one, np.uint8), np.frombuffer(zero, np.uint8)
+        if scale == "largest":
+            few[:, 4:] = 0xFF
+        s = few[:, 4:16].astype(np.int64)
+        sc = np.concatenate([s[:, :4] & 63, (s[:, 8:] & 15) | ((s[:, :4] >> 6) << 4)], axis=1)
+        q = few[:, qs:qs + 128].astype(np.int64).reshape(4, 4, 1, 32)
+        q = np.concatenate([q & 15, q >> 4], axis=2).reshape(4, 8, 32)
+        if name == "q5_k":
+            h = few[:, 16:48].astype(np.int64)
+            q = q + np.stack([((h >> b) & 1) << 4 for b in range(8)], axis=1)
+        w = q * sc[:, :, None]
+    codes = (rng.integers(120, 128, (N, K)) if scale == "largest" else rng.integers(-127, 128, (N, K))).astype(np.int8)
+    want = codes.astype(np.int64) @ w.reshape(4, K).T
+    lay = hip.packed_activation_layout(kind, N, K)
+    image = np.zeros(lay.total_bytes, np.uint8)
+    vals = np.zeros((N, lay.values_per_row), np.int8)
+    vals[:, :K] = codes
+    image[lay.values_offset:lay.values_offset + vals.size] = vals.view(np.uint8).reshape(-1)
+    image[lay.scales_offset:lay.scales_offset + 4 * N] = np.ones(N, np.float32).view(np.uint8)
+    sums = codes.reshape(N, 16, 16).sum(axis=2, dtype=np.int16)
+    image[lay.sums_offset:lay.sums_offset + sums.nbytes] = sums.view(np.uint8).reshape(-1)
+    d_w, d_p, d_out = hip.to_device(few[np.arange(M) % 4]), hip.to_device(image), hip.alloc(4 * N * M)
+    try:
+        hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out)
+        got = d_out.download(np.float32, (N, M))
+    finally:
+        for b in (d_w, d_p, d_out):
+            b.free()
+    assert np.array_equal(got, want[:, np.arange(M) % 4].astype(np.float32))
