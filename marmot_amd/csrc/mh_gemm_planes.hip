@@ -31,7 +31,11 @@
 //   Q6_K   308 / 162             302 / 185             99 / 59              61 / 39
 //   Q5_K   203 / 154             -                     67 / 55              38 / 35
 //   Q4_K   189 / 143             -                     62 / 52              31 / 30
-// and routed experts (E = 128, top 8, H = 2048, F = 768, 2048 tokens) Q6_K 650 / 460, Q4_K 395 / 393.
+// and routed experts (E = 128, top 8, H = 2048, F = 768, 2048 tokens) Q6_K 650 / 455, Q4_K 395 / 373.
+// Experts have few blocks per row (3 and 8 there), so a tile is over soon after its first operands have arrived. Their form
+// (LOOP) keeps as many workgroups as the chip holds and has each request the first codes and weights of its next tile during
+// the last block of this one: the calls above 384 -> 373 and 464 -> 455, 1500 tokens of 64 Q5_K experts of 512 228 -> 212. Linears of
+// 16 blocks and more lose up to 4 % to the registers it takes.
 #include "mh_rows.h"
 
 #include <type_traits>
@@ -55,7 +59,8 @@ struct GemmPlanesParams {
     void *out[3];
     const void *bias[3];
     int bias_is_f16, bias_first, out_is_f16;
-    // grouped (MoE): blockIdx.y selects a work item (expert, first route, routes); activation row of a route through
+    uint32_t row_tiles, col_tiles, weights;
+    // grouped (MoE): work items (expert, first route, routes) in the place of col_tiles; activation row of a route through
     // act_index (null: the route itself), output row = route
     const int4 *items;
     const int *n_items;
@@ -85,7 +90,7 @@ struct PlanesFormat<MARMOT_HIP_KIND_Q6_K> {
 
 constexpr int PLANES_ROWS = 4;  // wavefronts along the rows of a workgroup's tile
 
-template <int KIND, int C, int KG>
+template <int KIND, int C, int KG, bool LOOP>
 struct PlanesLds {
     static constexpr int ROWS = 64 / PlanesFormat<KIND>::PIECES;  // whole rows per direct-to-LDS load
     static constexpr int DMA = (32 + ROWS - 1) / ROWS;            // such loads of a wavefront per block
@@ -95,9 +100,11 @@ struct PlanesLds {
     static constexpr int S0 = W0 + PLANES_ROWS * KG * WAVE_W;
     static constexpr int SUMS = PlanesFormat<KIND>::MIN ? 32 * C * 32 : 0;  // sums of a block as fp16: [token][16]
     static constexpr int SD = SUMS + 32 * C * 4;                            // then the activation scales [token]
-    static constexpr int OFFS = S0 + 2 * KG * SD;  // lane offsets of the activation loads: [wavefront][load][lane]
+    static constexpr int OFFS = S0 + 2 * KG * SD;  // lane offsets of the activation loads: [this tile, next][wavefront][load][lane]
     static constexpr int OFF_N = C + 1 + (PlanesFormat<KIND>::MIN ? 1 : 0);
-    static constexpr int BYTES = OFFS + PLANES_ROWS * KG * OFF_N * 256;
+    static constexpr int TABLE = PLANES_ROWS * KG * OFF_N * 256;
+    static constexpr int NEXT = OFFS + (LOOP ? 2 : 1) * TABLE;  // activation rows of the next tile's tokens, per wavefront
+    static constexpr int BYTES = NEXT + (LOOP ? PLANES_ROWS * 128 * C : 0);
 };
 
 __device__ __forceinline__ pl_u16x2 pl_v(uint32_t v) {
@@ -295,10 +302,12 @@ __device__ __forceinline__ void planes_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int KIND, int C, int KG>
-__global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const GemmPlanesParams p) {
+// LOOP: a workgroup goes from tile to tile
+template <int KIND, int C, int KG, bool LOOP = false>
+__global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) void k_gemm_planes(const GemmPlanesParams p) {
     using F = PlanesFormat<KIND>;
-    using L = PlanesLds<KIND, C, KG>;
+    using L = PlanesLds<KIND, C, KG, LOOP>;
+    static_assert(!LOOP || KG == 1, "one K group");
     constexpr int RG = PLANES_ROWS;
     constexpr int TOK = 32 * C;
     constexpr int APW = C;  // direct-to-LDS loads of codes per wavefront and stage, 8 tokens each: the i-th of all wavefronts is tile i
@@ -308,51 +317,78 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int gw = wave % RG, kg = wave / RG;  // row group, K group
-    const int which = blockIdx.z;
-    const size_t row0 = (size_t)blockIdx.x * (32 * RG) + 32 * gw;  // this wavefront's first weight row
-    const uint8_t *w = p.w[which];
-    size_t tok0 = (size_t)blockIdx.y * TOK;  // first output row
-    uint32_t toks = (uint32_t)(p.N - tok0 < (size_t)TOK ? p.N - tok0 : (size_t)TOK);
-    if (p.items != nullptr) {
-        if ((int)blockIdx.y >= *p.n_items) {
-            return;
-        }
-        const int4 it = p.items[blockIdx.y];
-        w += (size_t)it.x * p.expert_stride;
-        tok0 = (size_t)it.y;
-        toks = (uint32_t)it.z;
-    }
-    auto act_row = [&](uint32_t t) {  // rows beyond the last token re-read it and are never stored
-        uint32_t row = (uint32_t)tok0 + (t < toks ? t : toks - 1u);
-        return p.act_index != nullptr ? p.act_index[row] : row;
+    const uint32_t nb = (uint32_t)p.nb;
+    // Tile t of the call: rows fastest, then weights, then tokens (or work items). KG == 1: a workgroup takes every gridDim.x-th.
+    struct Tile {
+        const uint8_t *w;
+        uint32_t which, row0, tok0, toks;  // row0: this wavefront's first weight row; tok0: first output row
     };
+    typedef const __attribute__((address_space(4))) int uniform_int;
+    uint32_t cols = p.col_tiles;
+    if (p.items != nullptr) {
+        cols = (uint32_t)*(uniform_int *)(uintptr_t)p.n_items;
+    }
+    const uint32_t tiles_all = p.row_tiles * p.weights * cols;
+    auto tile_at = [&](uint32_t t) {
+        Tile r;
+        const uint32_t rest = t / p.row_tiles, y = rest / p.weights;
+        r.which = rest - y * p.weights;
+        r.row0 = (t - rest * p.row_tiles) * (32u * RG) + 32u * (uint32_t)gw;
+        r.w = p.w[r.which];
+        if (p.items != nullptr) {
+            uniform_int *it = (uniform_int *)(uintptr_t)(p.items + y);
+            r.w += (size_t)it[0] * p.expert_stride;
+            r.tok0 = (uint32_t)it[1];
+            r.toks = (uint32_t)it[2];
+        } else {
+            r.tok0 = y * TOK;
+            r.toks = (uint32_t)p.N - r.tok0 < (uint32_t)TOK ? (uint32_t)p.N - r.tok0 : (uint32_t)TOK;
+        }
+        return r;
+    };
+    if (blockIdx.x >= tiles_all) {
+        return;
+    }
+    uint32_t tile = blockIdx.x;
+    const Tile first = tile_at(tile);
+    uint32_t toks = first.toks;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_u8_t *)lds;
 
     // ---- activation codes: load q of a stage brings tokens 8 q .. 8 q + 7, 128 bytes each. Lane l's 16 bytes land in slot l % 8 of
     // token 8 q + l / 8, which holds chunk (slot ^ swizzle(token)), swizzle(t) = t % 8 ^ (t / 8) % 2: eight, and sixteen, lanes with
     // consecutive tokens that read one chunk touch different banks.
     const uint32_t a_group = lds_base + (uint32_t)(kg * 2 * L::ACT);
-    uint32_t *offs = (uint32_t *)(lds + L::OFFS) + wave * (L::OFF_N * 64) + lane;
+    uint32_t table = 0;  // this tile's
+    auto offs = [&](uint32_t table, int i) -> uint32_t & {
+        return ((uint32_t *)(lds + L::OFFS + table * (uint32_t)L::TABLE))[wave * (L::OFF_N * 64) + 64 * i + lane];
+    };
+    const uint32_t s_tok = (uint32_t)((gw * 64 + lane) >> 1) % TOK;
+    auto fill_offs = [&](uint32_t table, auto act_row) {  // act_row: the activation row of a tile's token
 #pragma unroll
-    for (int i = 0; i < APW; ++i) {
-        const uint32_t q = (uint32_t)(RG * i + gw);
-        const uint32_t chunk = ((uint32_t)lane & 7u) ^ ((uint32_t)lane >> 3) ^ (q & 1u);
-        offs[64 * i] = act_row(8u * q + ((uint32_t)lane >> 3)) * (uint32_t)p.kp + 16u * chunk;
-    }
+        for (int i = 0; i < APW; ++i) {
+            const uint32_t q = (uint32_t)(RG * i + gw);
+            const uint32_t chunk = ((uint32_t)lane & 7u) ^ ((uint32_t)lane >> 3) ^ (q & 1u);
+            offs(table, i) = act_row(8u * q + ((uint32_t)lane >> 3)) * (uint32_t)p.kp + 16u * chunk;
+        }
+        // scales, sums (tokens wrap around: several lanes then bring the same bytes)
+        offs(table, APW) = act_row(((uint32_t)gw * 64u + (uint32_t)lane) % TOK) * nb * 4u;
+        if constexpr (F::MIN) {
+            offs(table, APW + 1) = act_row(s_tok) * nb * 32u + 16u * (lane & 1);
+        }
+    };
+    fill_offs(0u, [&](uint32_t t) {  // tokens beyond the last one re-read it and are never stored
+        const uint32_t row = first.tok0 + (t < toks ? t : toks - 1u);
+        return p.act_index != nullptr ? p.act_index[row] : row;
+    });
     auto request_acts = [&](uint32_t half, int buffer, int i, uint32_t off) {
         planes_dma16(a_group + (uint32_t)(buffer * L::ACT + 1024 * (RG * i + gw)), (const uint8_t *)p.qs + (size_t)half * 128u, off);
     };
-    // ---- scales and sums of a block (tokens wrap around: several lanes then write the same bytes)
-    const uint32_t sd_at = lds_base + (uint32_t)(L::S0 + 2 * kg * L::SD);  // (two blocks)
-    offs[64 * APW] = act_row(((uint32_t)gw * 64u + (uint32_t)lane) % TOK) * (uint32_t)p.nb * 4u;
-    const uint32_t s_tok = (uint32_t)((gw * 64 + lane) >> 1) % TOK;
-    if constexpr (F::MIN) {
-        offs[64 * APW + 64] = act_row(s_tok) * (uint32_t)p.nb * 32u + 16u * (lane & 1);
-    }
+    // ---- scales and sums of a block, in places that alternate with its number since the workgroup began
+    const uint32_t sd_at = lds_base + (uint32_t)(L::S0 + 2 * kg * L::SD);
     pl_u32x4 s_next = {};
-    auto request_scales = [&](uint32_t b, uint32_t off) {
+    auto request_scales = [&](uint32_t b, uint32_t number, uint32_t off) {
         if (64u * (uint32_t)gw < toks) {
-            planes_dma4(sd_at + (uint32_t)((b / KG & 1u) * L::SD + L::SUMS + 256 * gw), (const uint8_t *)p.ad + (size_t)b * 4u, off);
+            planes_dma4(sd_at + (uint32_t)((number & 1u) * L::SD + L::SUMS + 256 * gw), (const uint8_t *)p.ad + (size_t)b * 4u, off);
         }
     };
     auto request_sums = [&](uint32_t b, uint32_t off) {
@@ -362,7 +398,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
             s_next = *(const __attribute__((address_space(1))) pl_u32x4 *)(sums + (size_t)off);
         }
     };
-    auto store_block = [&](uint32_t b) {
+    auto store_block = [&](uint32_t number) {
         if constexpr (F::MIN) {
             const uint32_t v[4] = {s_next.x, s_next.y, s_next.z, s_next.w};
             uint32_t e[4];
@@ -370,7 +406,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
             for (int c = 0; c < 4; ++c) {
                 e[c] = __builtin_bit_cast(uint32_t, pl_half2{(_Float16)(int16_t)(v[c] & 0xffffu), (_Float16)(int16_t)(v[c] >> 16)});
             }
-            *(uint4 *)(lds + L::S0 + (2 * kg + (b / KG & 1u)) * L::SD + s_tok * 32u + 16u * (lane & 1)) = make_uint4(e[0], e[1], e[2], e[3]);
+            *(uint4 *)(lds + L::S0 + (2 * kg + (number & 1u)) * L::SD + s_tok * 32u + 16u * (lane & 1)) = make_uint4(e[0], e[1], e[2], e[3]);
         }
     };
 
@@ -378,23 +414,29 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
     // of row l / PIECES, counted from the 16-byte boundary at or below the row's block; a piece that holds no byte of the
     // block re-reads the last one that does, lanes behind the last row and rows behind the matrix re-read a row before.
     const uint32_t row_bytes = (uint32_t)p.nb * F::BYTES;
-    const uint32_t rows = (uint32_t)(row0 < p.M ? (p.M - row0 < 32 ? p.M - row0 : 32) : 0);
-    const uint8_t *wbase = w + (row0 < p.M ? row0 : p.M - 1) * row_bytes;
-    const uint32_t low4 = (uint32_t)((uintptr_t)wbase & 15u);
-    wbase = uniform_pointer(wbase - low4);
-    const uint32_t last_row = rows == 0 ? 0 : rows - 1u;
     const uint32_t w_r = (uint32_t)lane / F::PIECES < L::ROWS ? (uint32_t)lane / F::PIECES : L::ROWS - 1u;
     const uint32_t w_piece = 16u * ((uint32_t)lane - F::PIECES * w_r < F::PIECES ? (uint32_t)lane - F::PIECES * w_r : F::PIECES - 1u);
     const uint32_t w_lds = lds_base + (uint32_t)(L::W0 + wave * L::WAVE_W);
-    const uint32_t w_first = low4 + w_r * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
-    const uint32_t w_last = low4 + last_row * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
     // Q6_K: the piece that holds the end of the matrix may reach up to 14 bytes behind it (its size need not be a multiple
     // of 16), and those bytes need not exist. The wavefront of the last row brings the piece before in its place (one
     // operand more of a minimum that is there anyway) and copies the bytes that exist when the block is read (bring_end).
-    const uint32_t w_end = low4 + (last_row + 1u) * row_bytes;
-    const bool ragged = F::BYTES % 16 != 0 && row0 + 32 >= p.M && (w_end & 15u) != 0;
-    const uint32_t w_most = ragged ? (w_end & ~15u) - 16u : ~0u;
-    const uint32_t end_block = ragged ? (uint32_t)p.nb - 1u : ~0u;
+    const uint8_t *wbase;
+    uint32_t low4, last_row, w_first, w_last, w_end, w_most, end_block, my_row;
+    auto aim = [&](const Tile &t) {  // where the weights of tile t are
+        const uint32_t M = (uint32_t)p.M;
+        const uint8_t *at = t.w + (size_t)(t.row0 < M ? t.row0 : M - 1u) * row_bytes;
+        low4 = (uint32_t)((uintptr_t)at & 15u);
+        wbase = uniform_pointer(at - low4);
+        last_row = t.row0 >= M ? 0u : M - t.row0 < 32u ? M - t.row0 - 1u : 31u;
+        w_first = low4 + w_r * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
+        w_last = low4 + last_row * row_bytes + (F::BYTES % 16 != 0 ? 0u : w_piece);
+        w_end = low4 + (last_row + 1u) * row_bytes;
+        const bool ragged = F::BYTES % 16 != 0 && t.row0 + 32u >= M && (w_end & 15u) != 0;
+        w_most = ragged ? (w_end & ~15u) - 16u : ~0u;
+        end_block = ragged ? nb - 1u : ~0u;
+        my_row = low4 + ((uint32_t)j < last_row ? (uint32_t)j : last_row) * row_bytes;
+    };
+    aim(first);
     auto request_weights = [&](uint32_t b, int i) {
         uint32_t at = w_first;
         asm volatile("" : "+v"(at));  // formed at each load: kept in registers, the L::DMA offsets would be spilled
@@ -427,15 +469,21 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
             }
         }
     };
-    const uint32_t my_row = low4 + ((uint32_t)j < last_row ? (uint32_t)j : last_row) * row_bytes;
     const uint8_t *my_w = lds + L::W0 + wave * L::WAVE_W + j * (16 * F::PIECES);
     auto my_block = [&](uint32_t b) {  // (blocks of whole pieces start at the beginning of their place)
         return F::BYTES % 16 != 0 ? my_w + ((my_row + b * (uint32_t)F::BYTES) & 15u) : my_w;
     };
 
+    uint32_t number = 0;  // blocks of this K group so far
+    // (looked up where it is needed: two of them in registers throughout would be spilled)
+    auto look_up = [&](uint32_t t) {
+        asm volatile("" : "+s"(t));
+        return tile_at(t);
+    };
     // CT: the token tiles that hold a token
-    auto walk = [&](auto tiles_c) {
+    auto walk = [&](auto tiles_c, bool first_tile) {
     constexpr int CT = decltype(tiles_c)::value;
+    const bool more = LOOP && tile + gridDim.x < tiles_all;  // another tile of this workgroup
     pl_float16 total[CT];
 #pragma unroll
     for (int t = 0; t < CT; ++t) {
@@ -446,12 +494,11 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
     }
     pl_i32x16 X[CT], Y[CT];
     PlanesRaw<KIND> raw;
-    const uint32_t nb = (uint32_t)p.nb;
     const uint32_t a_at = a_group + (uint32_t)(j * 128 + 16 * (kh ^ (j & 7) ^ ((j >> 3) & 1)));
 
     // fp32 step of a block: y += a.d * (w.d * isum - w.dmin * msum)
-    auto finish = [&](uint32_t b, int first, int last) {
-        const uint8_t *sd = lds + L::S0 + (2 * kg + (b / KG & 1u)) * L::SD;
+    auto finish = [&](uint32_t number, int first, int last) {
+        const uint8_t *sd = lds + L::S0 + (2 * kg + (number & 1u)) * L::SD;
         pl_half8 sums = {}, mins = {};
         if constexpr (F::MIN) {
             sums = *(const pl_half8 *)(sd + (32 * first + j) * 32 + 16 * kh);
@@ -495,7 +542,6 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
     pl_i32x4 lo[2], hi[2];
     // The weights of block b have been requested: unpacks its first step
     auto first_load = [&](uint32_t b) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         bring_end(b);
         raw.load_half(my_block(b), 0, kh);
         raw.load_low(my_block(b), 0, 0, kh);
@@ -511,25 +557,29 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if (mine != 0) {
+    if (first_tile && mine != 0) {
 #pragma unroll
         for (int i = 0; i < L::DMA; ++i) {
             request_weights((uint32_t)kg, i);
         }
 #pragma unroll
         for (int i = 0; i < CT; ++i) {
-            request_acts(2u * (uint32_t)kg, 0, i, offs[64 * i]);
+            request_acts(2u * (uint32_t)kg, 0, i, offs(table, i));
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    planes_barrier();
+    if (first_tile) {
+        planes_barrier();
+    }
     if (KG > 1 && kg == 1) {
         planes_barrier();
         ++passed;
     }
-    for (uint32_t ib = 0; ib < mine; ++ib) {
+    for (uint32_t ib = 0; ib < mine; ++ib, ++number) {
         const uint32_t b = (uint32_t)kg + KG * ib;
-        const uint32_t bn = ib + 1 < mine ? b + KG : b;  // (the last block is requested again rather than branched around)
+        const bool last = ib + 1 == mine;
+        // (behind the workgroup's last block some block is requested again rather than branched around)
+        const uint32_t bn = !last ? b + KG : LOOP ? 0u : b;
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
             constexpr int STEPS = 4 * CT, AHEAD = 2;
@@ -545,23 +595,51 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
             };
             if (hb == 0) {
                 // (Q6_K's blocks are the largest and arrive last: read behind the fp32 step, 3 % of 1024 x 14336 x 4096)
+                if (ib != 0 && F::BYTES % 16 == 0) {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
                 if (F::BYTES % 16 == 0) {
                     first_load(b);
                 }
                 if (ib != 0) {
-                    finish(b - KG, CT / 2, CT);
+                    finish(number - 1u, CT / 2, CT);
+                    if (F::BYTES % 16 != 0) {
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    }
                 }
                 if (F::BYTES % 16 != 0) {
                     first_load(b);
                 }
                 first_step(b);
                 raw.load_header(my_block(b), kh);
+                if (LOOP && ib == 0 && more) {
+                    if (p.act_index != nullptr) {  // read behind the end of this stage
+                        const Tile next = look_up(tile + gridDim.x);
+#pragma unroll
+                        for (int i = 0; i < C / 2; ++i) {
+                            const uint32_t t = 64u * i + (uint32_t)lane;
+                            planes_dma4(lds_base + (uint32_t)(L::NEXT + wave * 128 * C + 256 * i), (const uint8_t *)(p.act_index + next.tok0),
+                                        4u * (t < next.toks ? t : next.toks - 1u));
+                        }
+                    }
+                }
+            }
+            const uint8_t *block = my_block(b);
+            if (LOOP && hb == 1 && last && more) {
+                // from here on the requests are the next tile's
+                const Tile next = look_up(tile + gridDim.x);
+                fill_offs(table ^ 1u, [&](uint32_t t) {
+                    const uint32_t in = t < next.toks ? t : next.toks - 1u;
+                    return p.act_index != nullptr ? ((const uint32_t *)(lds + L::NEXT))[wave * (32 * C) + in] : next.tok0 + in;
+                });
+                table ^= 1u;
+                aim(next);
             }
 #pragma unroll
             for (int st = 0; st < AHEAD; ++st) {
                 read_a(st);
             }
-            uint32_t off = offs[0];  // of the next load of the activations
+            uint32_t off = offs(table, 0);  // of the next load of the activations
             // Steps before fp32 steps of the other K group's wavefront on this SIMD, which fill what matrix instructions leave (2 - 3 %;
             // independent workgroups are 4 % slower with it)
             if (KG > 1) {
@@ -583,14 +661,19 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
                 if (st < CT) {
                     request_acts(hb == 0 ? 2u * b + 1u : 2u * bn, hb ^ 1, st, off);
                     if (st + 1 < CT) {
-                        off = offs[64 * (st + 1)];
+                        off = offs(table, st + 1);
                     } else if (hb == 0) {
-                        off = offs[64 * APW];
+                        off = offs(table, APW);
+                    } else if (LOOP && CT < C && last) {  // the next tile may have more of them
+#pragma unroll
+                        for (int i = CT; i < C; ++i) {
+                            request_acts(2u * bn, hb ^ 1, i, offs(table, i));
+                        }
                     }
                 } else if (st == CT && hb == 0) {
-                    request_scales(b, off);
+                    request_scales(b, number, off);
                     if (F::MIN) {
-                        off = offs[64 * (APW + 1)];
+                        off = offs(table, APW + 1);
                     }
                 } else if (st == CT + 1 && hb == 0) {
                     request_sums(b, off);
@@ -599,11 +682,11 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
                 const int hn = s < 3 ? hb : 1, sn = (s + 1) & 3;
                 if (t == 0) {
                     if (s == 3 && hb == 0) {
-                        store_block(b);
-                        raw.load_half(my_block(b), hn, kh);
+                        store_block(number);
+                        raw.load_half(block, hn, kh);
                     }
                     if (s == 1 || (s == 3 && hb == 0)) {
-                        raw.load_low(my_block(b), hn, sn / 2, kh);
+                        raw.load_low(block, hn, sn / 2, kh);
                     }
                 }
                 // The last bytes of this block have been read: its place is the next one's. (Waited for: the request alone does not keep the
@@ -641,17 +724,18 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
             if (hb == 0) {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
-                finish(b, 0, CT / 2);
+                finish(number, 0, CT / 2);
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L::DMA) : "memory");  // all but the weights, the last requests
             }
             planes_barrier();
             ++passed;
         }
     }
-    // (the last block's weights were requested once more: they must not land in the LDS of the workgroup that comes after)
+    // The first weights of the next tile (in front of the stores, which would be waited for too). Behind the last tile some were
+    // requested all the same, and must not land in the LDS of the workgroup that comes after.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (mine != 0) {
-        finish(kg + KG * (mine - 1), CT / 2, CT);
+        finish(number - 1u, CT / 2, CT);
     }
     if constexpr (KG > 1) {
         for (; passed < stages; ++passed) {
@@ -691,10 +775,14 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
     }
 
     // lane (j, kh) holds weight row row0 + j for tokens 32 t + 8 (r / 4) + 4 kh + r % 4: 32 rows of a token per store
-    if ((uint32_t)j >= rows) {
+    const Tile cur = LOOP ? look_up(tile) : first;
+    if (cur.row0 + (uint32_t)j >= p.M) {
         return;
     }
-    const size_t m = row0 + j;
+    const size_t m = cur.row0 + j, tok0 = cur.tok0;
+    const uint32_t which = cur.which;
+    uint32_t kh4 = 4u * (uint32_t)kh;
+    asm volatile("" : "+v"(kh4));  // (the places of the outputs are not kept from tile to tile)
     constexpr int OUT = KG > 1 ? C / 2 : CT;  // token tiles this wavefront stores
     const uint32_t t0 = (uint32_t)(KG > 1 ? kg * OUT : 0);
     const void *bias_p = p.bias[which];
@@ -706,7 +794,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
         for (int t = 0; t < OUT; ++t) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t n = (uint32_t)(32 * (t0 + t) + 8 * (r >> 2) + 4 * kh + (r & 3));
+                const uint32_t n = 32u * (t0 + t) + 8u * (r >> 2) + kh4 + (r & 3u);
                 if (n < toks) {
                     out[(size_t)n * p.M] = has_bias ? total[t][r] + bias : total[t][r];
                 }
@@ -719,7 +807,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
         for (int t = 0; t < OUT; ++t) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t n = (uint32_t)(32 * (t0 + t) + 8 * (r >> 2) + 4 * kh + (r & 3));
+                const uint32_t n = 32u * (t0 + t) + 8u * (r >> 2) + kh4 + (r & 3u);
                 if (n < toks) {
                     // without bias_first: round to the output type, then add the bias in it
                     const uint16_t first = f2h(has_bias && bias_first ? total[t][r] + bias : total[t][r]);
@@ -730,30 +818,42 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, 2) void k_gemm_planes(const 
     }
     };
     if constexpr (KG == 1) {
-        const uint32_t tiles = (toks + 31u) / 32u;
-        if (C >= 4 && tiles == 4) {
-            walk(std::integral_constant<int, C < 4 ? 1 : 4>{});
-        } else if (C >= 3 && tiles == 3) {
-            walk(std::integral_constant<int, C < 3 ? 1 : 3>{});
-        } else if (tiles == 2) {
-            walk(std::integral_constant<int, 2>{});
-        } else {
-            walk(std::integral_constant<int, 1>{});
+        for (bool first_tile = true;; first_tile = false) {
+            const uint32_t tiles = (toks + 31u) / 32u;
+            if (C >= 4 && tiles == 4) {
+                walk(std::integral_constant<int, C < 4 ? 1 : 4>{}, first_tile);
+            } else if (C >= 3 && tiles == 3) {
+                walk(std::integral_constant<int, C < 3 ? 1 : 3>{}, first_tile);
+            } else if (tiles == 2) {
+                walk(std::integral_constant<int, 2>{}, first_tile);
+            } else {
+                walk(std::integral_constant<int, 1>{}, first_tile);
+            }
+            tile += gridDim.x;
+            if (!LOOP || tile >= tiles_all) {
+                return;
+            }
+            toks = look_up(tile).toks;
         }
     } else {
-        walk(std::integral_constant<int, C>{});
+        walk(std::integral_constant<int, C>{}, true);
     }
 }
 
-template <int KIND, int C, int KG>
-static int planes_launch(marmot_hip_device *dev, const GemmPlanesParams &p, unsigned col_tiles, unsigned weights) {
-    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_planes<KIND, C, KG>));
-    const dim3 grid((unsigned)((p.M + 32 * PLANES_ROWS - 1) / (32 * PLANES_ROWS)), col_tiles, weights);
-    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG>), grid, dim3(64 * PLANES_ROWS * KG), (PlanesLds<KIND, C, KG>::BYTES), dev->stream, p);
+// cols: tiles along the tokens, or work items at most. LOOP: as many workgroups as the chip holds at once (three per compute unit).
+template <int KIND, int C, int KG, bool LOOP = false>
+static int planes_launch(marmot_hip_device *dev, GemmPlanesParams &p, size_t cols, unsigned weights) {
+    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_planes<KIND, C, KG, LOOP>));
+    p.row_tiles = (uint32_t)((p.M + 32 * PLANES_ROWS - 1) / (32 * PLANES_ROWS));
+    p.col_tiles = (uint32_t)cols;
+    p.weights = weights;
+    const size_t tiles = (size_t)p.row_tiles * cols * weights;
+    const size_t places = (size_t)dev->props.multiProcessorCount * 3;
+    const dim3 grid((unsigned)(LOOP && tiles > places ? places : tiles));
+    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG, LOOP>), grid, dim3(64 * PLANES_ROWS * KG), (PlanesLds<KIND, C, KG, LOOP>::BYTES), dev->stream, p);
     MH_HIP(hipGetLastError());
     return MARMOT_HIP_SUCCESS;
 }
-
 
 static bool planes_kind(int kind) {
     return kind == MARMOT_HIP_KIND_Q4_K || kind == MARMOT_HIP_KIND_Q5_K || kind == MARMOT_HIP_KIND_Q6_K;
@@ -798,7 +898,7 @@ bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_
 
 // The tile of 64 tokens keeps the route name of the kernel that had it before (callers compare names).
 template <int KIND>
-static int planes_launch_kind(marmot_hip_device *dev, const GemmPlanesParams &p, unsigned weights, const char *small_route,
+static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsigned weights, const char *small_route,
                               const char *large_route) {
     const int form = planes_form(dev, KIND, p.N, p.M, p.nb, weights);
     set_route(form >= 40 ? large_route : small_route);
@@ -884,11 +984,11 @@ int launch_gemm_planes_grouped(marmot_hip_device *dev, int kind, const void *d_w
     // take 401 us for 393 (Q4_K), 452 for 460 (Q6_K).
     switch (kind) {
     case MARMOT_HIP_KIND_Q4_K:
-        return planes_launch<MARMOT_HIP_KIND_Q4_K, 2, 1>(dev, p, (unsigned)max_items, weights);
+        return planes_launch<MARMOT_HIP_KIND_Q4_K, 2, 1, true>(dev, p, max_items, weights);
     case MARMOT_HIP_KIND_Q5_K:
-        return planes_launch<MARMOT_HIP_KIND_Q5_K, 2, 1>(dev, p, (unsigned)max_items, weights);
+        return planes_launch<MARMOT_HIP_KIND_Q5_K, 2, 1, true>(dev, p, max_items, weights);
     default:
-        return planes_launch<MARMOT_HIP_KIND_Q6_K, 2, 1>(dev, p, (unsigned)max_items, weights);
+        return planes_launch<MARMOT_HIP_KIND_Q6_K, 2, 1, true>(dev, p, max_items, weights);
     }
 }
 

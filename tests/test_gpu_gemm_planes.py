@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from oracle.pyoracle import KIND_Q4_K, KIND_Q5_K, KIND_Q6_K
+from tests.test_gpu_moe import check_moe_stages
 from tests.util import assert_matmul_parity, gaussian, random_valid_blocks
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +101,39 @@ def test_block_sums_are_exact(hip, name, N, M, scale):
         for b in (d_w, d_p, d_out):
             b.free()
     assert np.array_equal(got, want[:, np.arange(M) % 4].astype(np.float32))
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+def test_experts_in_more_tiles_than_the_chip_holds(hip, oracle, name):
+    """About 30 items of 32 tiles in both projections: workgroups go on to a second tile, of the other weight or another expert,
+    ragged last items among them. Stage by stage with the bounds of the expert tests."""
+    E, F, H, k, T = 3, 2048, 4096, 2, 900
+    kind = KINDS[name]
+    gate, up = (hip.quantize_weights(kind, gaussian(820 + i, (E * F, H), 0.02)) for i in range(2))
+    down = hip.quantize_weights(kind, gaussian(822, (E * H, F), 0.02))
+    hidden = gaussian(823, (T, H))
+    vals, ids = oracle.topk(gaussian(824, (T, E)), k)
+    w = oracle.softmax_rows(vals)
+    ref = oracle.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind, threads=16)
+    check_moe_stages(hip, oracle, hidden, gate, up, down, ids, w, F, E, kind, ref, f"experts from tile to tile {name}")
+    hip.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind)
+    assert hip.last_route() == "moe_experts_tiled"
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("H,F,T", [(2048, 256, 8200), (256, 2304, 16500)])  # one block per row: down, gate and up
+def test_experts_of_a_call_and_of_its_halves(hip, name, H, F, T):
+    """A token's result does not depend on the others, bit for bit: the halves of a call fit the chip in one of the two
+    projections, the whole call does not."""
+    E, k, kind = 4, 2, KINDS[name]
+    gate, up = (random_valid_blocks(np.random.default_rng(830 + i), kind, E * F, H) for i in range(2))
+    down = random_valid_blocks(np.random.default_rng(832), kind, E * H, F)
+    hidden, rng = gaussian(833, (T, H)), np.random.default_rng(834)
+    ids = np.argsort(rng.random((T, E)), axis=1)[:, :k].astype(np.int32)
+    w = np.full((T, k), 0.5, np.float32)
+    whole = hip.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind)
+    assert hip.last_route() == "moe_experts_tiled"
+    for part in (slice(0, T // 2), slice(T // 2, T)):
+        got = hip.moe_experts(hidden[part], gate, up, down, ids[part], w[part], F, E, kind, kind)
+        assert hip.last_route() == "moe_experts_tiled"
+        assert np.array_equal(got.view(np.uint32), whole[part].view(np.uint32))
