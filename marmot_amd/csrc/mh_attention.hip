@@ -311,6 +311,49 @@ __global__ __launch_bounds__(128) void k_pa_write(const PaParams p) {
     }
 }
 
+// The same for 16-bit caches where eight values are 16 aligned bytes (pa_write_rows): one workgroup per token, eight values of a
+// row per thread and step, and a wavefront of its own for the look at the call's lengths, which is a chain of loads as long
+// as the copy's. 1024 tokens of 8 heads of 128 beside a prompt: 9.7 -> 7.2 us (a workgroup per row is 8192 small ones).
+constexpr uint32_t PA_WRITE_THREADS = 256;
+__global__ __launch_bounds__(PA_WRITE_THREADS + 64) void k_pa_write_rows(const PaParams p) {
+    const uint32_t t = blockIdx.x;
+    if (threadIdx.x >= PA_WRITE_THREADS) {  // (launched beside k_pa_prompt only)
+        const uint32_t tiled = pa_in_run(p, t, p.meta[t * p.meta_stride[0]]);
+        if (threadIdx.x == PA_WRITE_THREADS) {
+            p.tiled[t] = tiled;
+        }
+        return;
+    }
+    const uint32_t slot = p.meta[t * p.meta_stride[0] + 2 * p.meta_stride[1]];
+    const uint32_t block = slot >> p.shift;
+    if (block >= p.kv_blocks) {
+        return;
+    }
+    const size_t dst0 = (size_t)block * p.kv_stride[0] + (size_t)p.layer_idx * p.kv_stride[1] + (size_t)(slot & p.mask) * p.kv_stride[3];
+    const bool bits16 = p.act_dtype == p.kv_dtype;
+    const uint32_t per_head = p.head_dim / 8u, pieces = p.num_kv_heads * per_head;
+    for (uint32_t i = threadIdx.x; i < 2u * pieces; i += PA_WRITE_THREADS) {
+        const bool is_value = i >= pieces;
+        const uint32_t u = is_value ? i - pieces : i, h = u / per_head, d = 8u * (u - h * per_head);
+        const void *src = is_value ? p.v_new : p.k_new;
+        const size_t from = (size_t)t * (is_value ? p.v_stride[0] : p.k_stride[0]) + (size_t)h * (is_value ? p.v_stride[1] : p.k_stride[1]) + d;
+        uint16_t *dst = (uint16_t *)(is_value ? p.kv_v : p.kv_k) + dst0 + (size_t)h * p.kv_stride[2] + d;
+        if (bits16) {
+            *(uint4 *)dst = *(const uint4 *)((const uint16_t *)src + from);
+        } else {
+            float v[8];
+            pa_load_run<8>(src, p.act_dtype, from, v);
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool f16 = p.kv_dtype == MARMOT_HIP_DTYPE_F16;
+                w[e] = f16 ? (uint32_t)f2h(v[2 * e]) | (uint32_t)f2h(v[2 * e + 1]) << 16 : (uint32_t)pa_f2bf(v[2 * e]) | (uint32_t)pa_f2bf(v[2 * e + 1]) << 16;
+            }
+            *(uint4 *)dst = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+}
+
 // ---- the FLOAT8_E4M3 cache write (paged_attention_ref.c:825-989) in four launches
 // 1. scratch: no new magnitudes, no block touched
 __global__ __launch_bounds__(256) void k_pa_fp8_init(const PaParams p) {
@@ -1309,12 +1352,15 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 }
 
 // ---- prompts: tiles of tokens that share the key / value rows (FLOAT16 or BFLOAT16 cache, rows of 64 or 128 values)
-// One workgroup of four wavefronts per (tile of tokens, key / value head, share of the history). Its 128 rows are the
-// (token, query head) pairs of 128 / group consecutive tokens; wavefront w owns rows 32 w .. + 31, lane l row l % 32.
-// The workgroup walks the histories of the sequences in its tile (one, mostly) in tiles of 64 positions, double-buffered
-// in LDS: keys as rows, values transposed, both requested one tile ahead through registers.
+// One workgroup of eight wavefronts per (tile of tokens, key / value head, share of the history). Its 128 rows are the
+// (token, query head) pairs of 128 / group consecutive tokens; wavefronts w and w + 4 own rows 32 w .. + 31, lane l row l % 32,
+// each for one half (32 positions) of every tile of the history, with a maximum, a sum and outputs of its own; the halves
+// meet in LDS at the end. Two wavefronts per SIMD: one multiplies while the other is at its softmax. The workgroup walks the
+// histories of the sequences in its tile (one, mostly) in tiles of 64 positions: keys as rows in two buffers, values
+// transposed in three, both requested one tile ahead through registers.
 //   * Scores: S[position][row] = K . q as v_mfma_f32_32x32x16 with the key rows as row operand; lane (row, h = l / 32)
-//     receives positions 8 q + 4 h + e in register 4 q + e, so a row's softmax is 16 registers and one exchange.
+//     receives positions 8 q + 4 h + e in register 4 q + e, so a row's softmax is 16 registers and one exchange. Most of the
+//     query's parts wait in LDS (rows of 128): 256 registers hold neither them nor a copy of the outputs beside the rest.
 //   * Output: O[dimension][row] += V^T . P with the weights as column operand: registers 8 i .. 8 i + 7 ARE the operand of
 //     instruction i (the k index of lane half h stands for positions 16 i + 4 h + 0..3 and 16 i + 8 + 4 h + 0..3), and the
 //     transposed values are stored in that order, so no weight moves between lanes.
@@ -1324,10 +1370,13 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 //   * A value that is not finite would reach rows that may not see it (0 x infinity): a tile that holds one takes the
 //     products of its visible positions one by one.
 // The kernel per token reads a history once per token and head group and uses a quarter of its matrix instructions; this
-// one reads it once per 128 / group tokens. Bound by the chain of one wavefront per SIMD (scores, softmax, output): 64
-// positions at a time instead of 32 give it two score chains and half the rescaling. Two sequences x 512 tokens over 2048
-// cached ones, 32 / 8 heads of 128, BFLOAT16 cache, whole call: 756 us per token, 249 with 32 positions at a time and the
-// table entry read in front of each tile, 171 now. Error against 64 bits there: 3.6e-7 per token, 2.2e-7 here.
+// one reads it once per 128 / group tokens. Two sequences x 512 tokens over 2048 cached ones, 32 / 8 heads of 128, BFLOAT16 cache,
+// whole call: 756 us per token; 249 with four wavefronts that own 32 positions at a time and the table entry read in front of
+// each tile; 166 with 64 at a time (one wavefront per SIMD: scores, softmax and output one after the other); 148 with
+// eight wavefronts; 138 - 140 now that one wavefront locates a tile's rows for all and the values' infinities are looked for by two
+// maxima per word. Bound by the issue of vector instructions (about 1300 per SIMD and tile, 5200 clocks, beside 3070 of
+// the matrix cores); 20 us are the start and the end (the query's parts 6, the join of the halves 4, the first tile 8).
+// Error against 64 bits there: 3.6e-7 per token, 2.2e-7 here.
 typedef float pa_float16v __attribute__((ext_vector_type(16)));
 typedef _Float16 pa_half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 pa_bf8 __attribute__((ext_vector_type(8)));
@@ -1339,12 +1388,20 @@ constexpr uint32_t PA_LONG = 512, PA_MANY = 256, PA_ANY_TABLE = 512;
 constexpr size_t PA_PROMPT_WORK = (size_t)3 << 19;
 constexpr uint32_t PA_SHARES = 4;  // of the history of a token that is left over
 
-template <int HD>
+constexpr uint32_t PA_PROMPT_WAVES = 8;
+
+template <int HD, bool BF16>
 struct PaPromptLds {
     static constexpr uint32_t KROW = 2 * HD + 16;   // bytes; 16 of padding: rows 4 banks apart
-    static constexpr uint32_t K = 64 * KROW, V = HD * 128, STAGE = K + V;
-    static constexpr uint32_t TOKENS = 2 * STAGE;  // sequence, length, longest history: 128 words each; four words
-    static constexpr uint32_t BYTES = TOKENS + (3 * PA_PROMPT_ROWS + 4) * 4;
+    static constexpr uint32_t K = 64 * KROW, V = HD * 128;
+    static constexpr uint32_t V0 = 2 * K;          // two buffers of keys, three of values
+    static constexpr uint32_t Q = V0 + 3 * V;      // small parts of the query: [part][16 dimensions][wavefront][lane] x 16 bytes
+    static constexpr uint32_t QPARTS = HD == 128 ? (BF16 ? 2 : 1) : 0;
+    static constexpr uint32_t TOKENS = Q + QPARTS * PA_PROMPT_ROWS * HD * 2;  // sequence, length, longest history: 128 words each; five words
+    static constexpr uint32_t ROWS = TOKENS + (3 * PA_PROMPT_ROWS + 8) * 4;  // two tiles: places of 64 rows; then which of them exist
+    static constexpr uint32_t BYTES = ROWS + (2 * 64 + 2) * 8;
+    static constexpr uint32_t MAIL = PA_PROMPT_WAVES * HD / 64 * 4096;  // at the end: outputs, then maximum and sum of every lane
+    static_assert(MAIL + PA_PROMPT_WAVES * 512 <= Q, "the mail fits the stages");
 };
 
 // byte offset of chunk c (16 bytes: eight positions) of dimension d in the transposed values; the exclusive or spreads
@@ -1363,18 +1420,21 @@ __device__ __forceinline__ pa_float16v pa_mma32(const uint4 a, const uint4 b, co
     }
 }
 
-// (the parts of the query, 64 scores and 64 output registers: one wavefront per SIMD)
 template <int HD, bool BF16>
-__global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
-    using L = PaPromptLds<HD>;
-    constexpr int PARTS = BF16 ? 3 : 2, QC = HD / 16, DB = HD / 32;
-    constexpr int KN = HD / 32, VN = HD / 64;  // per thread and tile: 16-byte key chunks, 4 x 4 blocks of values
+__global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaParams p) {
+    using L = PaPromptLds<HD, BF16>;
+    constexpr int PARTS = BF16 ? 3 : 2, QC = HD / 16, DB = HD / 32, QREGS = PARTS - L::QPARTS;
+    constexpr uint32_t THREADS = 64 * PA_PROMPT_WAVES;
+    constexpr int KN = 64 * HD / 8 / THREADS;   // per thread and tile: 16-byte key chunks
+    constexpr uint32_t VUNITS = 16 * HD / 4;    // of a tile: 4 x 4 blocks of values, one per thread at most
+    static_assert(KN >= 1 && VUNITS <= THREADS && VUNITS % 64 == 0, "a tile's rows over the threads");
     constexpr float UNIT = BF16 ? 1.0f : 16384.0f;
     constexpr uint32_t NONE = 0xFFFFFFFFu;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint32_t *s_seq = (uint32_t *)(lds + L::TOKENS), *s_len = s_seq + PA_PROMPT_ROWS, *s_longest = s_len + PA_PROMPT_ROWS;
     uint32_t *s_odd = s_longest + PA_PROMPT_ROWS;  // per buffer: 1 + number of its tile if that holds a value that is not finite
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u, n = lane & 31u, h = lane >> 5;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 31u, h = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), rows = wave & 3u, half = wave >> 2;
     const uint32_t tt = p.tile_tokens, t0 = (gridDim.x - 1u - blockIdx.x) * tt, kvh = blockIdx.y;  // long histories first
 
     // the tile's tokens: sequence (NONE: not this kernel's), visible positions, and at the first token of a sequence the
@@ -1383,10 +1443,10 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
     static_assert(PA_PROMPT_ROWS == 2 * 64, "tokens of a tile: in the first two wavefronts");
     const unsigned long long any_mine = __builtin_amdgcn_ballot_w64(mine);
     if (lane == 0 && wave < 2u) {
-        s_odd[2 + wave] = any_mine != 0 ? 1u : 0u;
+        s_odd[3 + wave] = any_mine != 0 ? 1u : 0u;
     }
     __syncthreads();
-    if ((s_odd[2] | s_odd[3]) == 0u) {
+    if ((s_odd[3] | s_odd[4]) == 0u) {
         return;
     }
     if (tid < PA_PROMPT_ROWS) {
@@ -1394,7 +1454,7 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         s_seq[tid] = mine ? p.meta[at] : NONE;
         s_len[tid] = mine ? pa_visible(p, p.meta[at + p.meta_stride[1]]) : 0u;
     }
-    if (tid < 2) {
+    if (tid < 3) {
         s_odd[tid] = 0;
     }
     __syncthreads();
@@ -1402,17 +1462,21 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         const uint32_t seq = s_seq[tid];
         uint32_t longest = 0;
         bool first = true;
-        for (uint32_t i = 0; i < tt; ++i) {
-            const uint32_t len = s_len[i];
-            const bool eq = s_seq[i] == seq;
-            first = first && !(eq && i < tid);
-            longest = eq && len > longest ? len : longest;
+        for (uint32_t i = 0; i < tt; i += 4u) {  // (behind the tile's tokens: nobody's)
+            const uint4 lens = *(const uint4 *)(s_len + i), seqs = *(const uint4 *)(s_seq + i);
+            const uint32_t len[4] = {lens.x, lens.y, lens.z, lens.w}, other[4] = {seqs.x, seqs.y, seqs.z, seqs.w};
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) {
+                const bool eq = other[e] == seq;
+                first = first && !(eq && i + e < tid);
+                longest = eq && len[e] > longest ? len[e] : longest;
+            }
         }
         s_longest[tid] = mine && first ? longest : 0u;
     }
     __syncthreads();
 
-    const uint32_t row = 32u * wave + n, tl = row / p.group, g = row - tl * p.group;
+    const uint32_t row = 32u * rows + n, tl = row / p.group, g = row - tl * p.group;
     const bool have = tl < tt;
     const uint32_t row_seq = have ? s_seq[tl] : NONE;
     const uint32_t full_len = row_seq != NONE ? s_len[tl] : 0u;
@@ -1421,9 +1485,9 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
     // the query of this lane's row: dimensions 16 c + 8 h .. + 7, scaled and split. Rows that are not contiguous pass
     // through LDS (element loads in a loop of their own instead of 64 copies of them here).
     float *staged = (float *)lds;  // [128][HD]
-    static_assert(L::TOKENS >= PA_PROMPT_ROWS * HD * 4, "the query rows fit the two stages");
+    static_assert(L::TOKENS >= PA_PROMPT_ROWS * HD * 4, "the query rows fit the stages");
     if (!p.q_vec) {
-        for (uint32_t i = tid; i < PA_PROMPT_ROWS * HD; i += 256u) {
+        for (uint32_t i = tid; i < PA_PROMPT_ROWS * HD; i += THREADS) {
             const uint32_t r = i / HD, token = r / p.group;
             if (token < tt && s_seq[token] != NONE) {
                 staged[i] = pa_load(p.q, p.act_dtype, (size_t)(t0 + token) * p.q_stride[0] +
@@ -1459,11 +1523,11 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
                 const uint2 a = *(const uint2 *)((const uint16_t *)p.q + q_base + d);
                 const uint2 b = *(const uint2 *)((const uint16_t *)p.q + q_base + d + 4u);
                 const uint32_t words[4] = {a.x, a.y, b.x, b.y};
-                const bool half = p.act_dtype == MARMOT_HIP_DTYPE_F16;
+                const bool f16 = p.act_dtype == MARMOT_HIP_DTYPE_F16;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const uint16_t bits = (uint16_t)(words[e >> 1] >> (16 * (e & 1)));
-                    qv[c][e] = half ? h2f(bits) : pa_bf2f(bits);
+                    qv[c][e] = f16 ? h2f(bits) : pa_bf2f(bits);
                 }
             }
         }
@@ -1488,7 +1552,8 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         up = pa_split_exponent(fmaxf(most, pa_xor32(most)));
         unit = ldexpf(1.0f, -up);
     }
-    uint4 qpart[PARTS][QC];
+    uint4 qpart[QREGS][QC];
+    uint8_t *q_small = lds + L::Q + rows * 1024u + 16u * lane;
 #pragma unroll
     for (int c = 0; c < QC; ++c) {
         uint32_t w[PARTS][4];
@@ -1510,7 +1575,12 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         }
 #pragma unroll
         for (int part = 0; part < PARTS; ++part) {
-            qpart[part][c] = make_uint4(w[part][0], w[part][1], w[part][2], w[part][3]);
+            const uint4 v = make_uint4(w[part][0], w[part][1], w[part][2], w[part][3]);
+            if (part < QREGS) {
+                qpart[part][c] = v;
+            } else {  // (both halves' wavefronts hold the same rows)
+                *(uint4 *)(q_small + 4096 * (QC * (part - QREGS) + c)) = v;
+            }
         }
     }
 
@@ -1524,12 +1594,18 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
     for (int d = 0; d < DB; ++d) {
         out[d] = zero;
     }
-    float m = -INFINITY, lsum = 0.0f;  // lsum: of this lane's half of the positions
+    float m = -INFINITY, lsum = 0.0f;  // of this wavefront's positions; lsum: of this lane's part of them
     const size_t head_base = (size_t)p.layer_idx * p.kv_stride[1] + (size_t)kvh * p.kv_stride[2];
-    const uint16_t *keys = (const uint16_t *)p.kv_k + head_base, *values = (const uint16_t *)p.kv_v + head_base;
-    uint32_t count = 0;  // tiles staged so far, over all sequences: buffer = count & 1
+    const uint8_t *keys = (const uint8_t *)((const uint16_t *)p.kv_k + head_base), *values = (const uint8_t *)((const uint16_t *)p.kv_v + head_base);
+    // a thread's part of a tile: 16 bytes of every THREADS / (HD / 8)-th key row, four dimensions of four consecutive value rows.
+    // (The chunk of dimension 4 i + e: that of dimension 4 i with 2 e in an exclusive or, 128 e bytes on.)
+    const uint32_t v_at = pa_vt_chunk(4u * (tid % (HD / 4)), 2u * (tid / HD) + (tid / (HD / 4) & 1u)) + 8u * (tid / (HD / 2) & 1u);
+    const uint32_t v_from = pa_vt_chunk(n, 4u * half + h);
+    uint64_t *s_rows = (uint64_t *)(lds + L::ROWS);
+    // tiles staged so far, over all sequences: keys in buffer count & 1, values at `now`, the ones before at `before`
+    uint32_t count = 0, now = L::V0, before = L::V0 + 2u * L::V;
     pa_uint4 kreg[KN];
-    uint2 vreg[VN][4];
+    uint2 vreg[4];
     uint64_t mask_next = 0;  // positions of the requested tile that exist
 
     for (uint32_t first = 0; first < tt; ++first) {
@@ -1549,156 +1625,142 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
         if (begin >= end) {
             continue;
         }
-        // lane i locates position i of the tile; rows without a block read block 0
+        // The first wavefront locates the rows two tiles ahead, lane i position i; rows without a block read block 0.
         auto table_entry = [&](uint32_t tile) -> uint32_t {
             const uint32_t logical = (64u * tile + lane) >> p.shift;
             return table_row[(size_t)(logical < p.max_blocks ? logical : p.max_blocks - 1u) * p.table_stride[1]];
         };
-        auto request = [&](uint32_t tile, uint32_t tb) {
-            const uint32_t pos = 64u * tile + lane, logical = pos >> p.shift;
+        auto locate = [&](uint32_t tile, uint32_t tb) {
+            const uint32_t pos = 64u * tile + lane, logical = pos >> p.shift, buffer = (tile - begin) & 1u;
             const bool ok = pos < longest && logical < p.max_blocks && tb != PA_NO_BLOCK && tb < p.kv_blocks;
-            mask_next = __builtin_amdgcn_ballot_w64(ok);
-            const size_t off = ok ? (size_t)tb * p.kv_stride[0] + (size_t)(pos & p.mask) * p.kv_stride[3] : 0u;
-            const int lo = (int)(uint32_t)off, hi = (int)(uint32_t)(off >> 32);
-            auto row_of = [&](uint32_t r) -> size_t {
-                return (size_t)(uint32_t)__shfl(lo, (int)r) | ((size_t)(uint32_t)__shfl(hi, (int)r) << 32);
-            };
+            const uint64_t exist = __builtin_amdgcn_ballot_w64(ok);
+            s_rows[64u * buffer + lane] = ok ? 2u * ((uint64_t)tb * p.kv_stride[0] + (uint64_t)(pos & p.mask) * p.kv_stride[3]) : 0u;
+            if (lane == 0) {
+                s_rows[128u + buffer] = exist;
+            }
+        };
+        auto request = [&](uint32_t tile) {
+            const uint32_t buffer = (tile - begin) & 1u;
+            const uint64_t exist = s_rows[128u + buffer];
+            mask_next = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)exist) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(exist >> 32)) << 32;
+            uint32_t tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));  // (places formed from it here, not kept throughout: there are no registers for them)
+            const uint64_t *k_rows = s_rows + 64u * buffer + tid / (HD / 8);
+            const uint8_t *k_base = keys + 16u * (tid % (HD / 8));
 #pragma unroll
             for (int i = 0; i < KN; ++i) {
-                const uint32_t c = tid + 256u * i, r = c / (HD / 8);
-                kreg[i] = *(const pa_uint4 *)(keys + row_of(r) + 8u * (c % (HD / 8)));
+                kreg[i] = *(const pa_uint4 *)(k_base + k_rows[THREADS / (HD / 8) * i]);
             }
-#pragma unroll
-            for (int i = 0; i < VN; ++i) {
-                const uint32_t u = tid + 256u * i, pq = u / (HD / 4);
+            if (VUNITS == THREADS || tid < VUNITS) {
+                const uint64_t *v_rows = s_rows + 64u * buffer + 4u * (tid / (HD / 4));
+                const uint8_t *v_base = values + 8u * (tid % (HD / 4));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    vreg[i][e] = *(const uint2 *)(values + row_of(4u * pq + e) + 4u * (u % (HD / 4)));
+                    vreg[e] = *(const uint2 *)(v_base + v_rows[e]);
                 }
             }
         };
-        auto store = [&](uint32_t number) {
-            uint8_t *stage = lds + (number & 1u) * L::STAGE;
+        auto store = [&](uint32_t number, uint32_t values_at) {
+            uint32_t tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));
+            uint8_t *stage = lds + (number & 1u) * L::K + tid / (HD / 8) * L::KROW + 16u * (tid % (HD / 8));
 #pragma unroll
             for (int i = 0; i < KN; ++i) {
-                const uint32_t c = tid + 256u * i;
-                *(pa_uint4 *)(stage + c / (HD / 8) * L::KROW + 16u * (c % (HD / 8))) = kreg[i];
+                *(pa_uint4 *)(stage + THREADS / (HD / 8) * i * L::KROW) = kreg[i];
             }
-            uint32_t odd = 0;
+            if (VUNITS == THREADS || tid < VUNITS) {
+                if (mask_next != ~0ull) {
 #pragma unroll
-            for (int i = 0; i < VN; ++i) {
-                const uint32_t u = tid + 256u * i, pq = u / (HD / 4), d0 = 4u * (u % (HD / 4));
-                uint2 v[4];
+                    for (int e = 0; e < 4; ++e) {
+                        vreg[e] = (mask_next >> (4u * (tid / (HD / 4)) + e)) & 1u ? vreg[e] : make_uint2(0, 0);
+                    }
+                }
+                // largest halves as unsigned numbers (negative values) and as signed ones (positive values): has one of them all
+                // bits of its exponent set?
+                typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+                typedef short i16x2 __attribute__((ext_vector_type(2)));
+                u16x2 below = {0, 0};
+                i16x2 above = {0, 0};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const bool ok = (mask_next >> (4u * pq + e)) & 1u;
-                    v[e] = ok ? vreg[i][e] : make_uint2(0, 0);
-                    // the top bit of each half: exponent field all ones
-                    constexpr uint32_t ONE = BF16 ? 0x00800080u : 0x04000400u;
-                    odd |= ((v[e].x & 0x7fff7fffu) + ONE) | ((v[e].y & 0x7fff7fffu) + ONE);
+                    below = __builtin_elementwise_max(below, __builtin_elementwise_max(__builtin_bit_cast(u16x2, vreg[e].x), __builtin_bit_cast(u16x2, vreg[e].y)));
+                    above = __builtin_elementwise_max(above, __builtin_elementwise_max(__builtin_bit_cast(i16x2, vreg[e].x), __builtin_bit_cast(i16x2, vreg[e].y)));
                 }
-                const uint32_t chunk = 2u * (pq >> 2) + (pq & 1u), half = 8u * ((pq >> 1) & 1u);
-                uint8_t *vt = stage + L::K + half;
+                constexpr uint32_t ONE = BF16 ? 0x00800080u : 0x04000400u;
+                const uint32_t odd = ((__builtin_bit_cast(uint32_t, below) & 0x7fff7fffu) + ONE) | ((__builtin_bit_cast(uint32_t, above) & 0x7fff7fffu) + ONE);
+                uint8_t *vt = lds + values_at;
                 constexpr uint32_t LOW = 0x05040100u, HIGH = 0x07060302u;
                 auto pair = [](uint32_t b, uint32_t a, uint32_t sel) { return __builtin_amdgcn_perm(b, a, sel); };
-                *(uint2 *)(vt + pa_vt_chunk(d0, chunk)) = make_uint2(pair(v[1].x, v[0].x, LOW), pair(v[3].x, v[2].x, LOW));
-                *(uint2 *)(vt + pa_vt_chunk(d0 + 1u, chunk)) =
-                    make_uint2(pair(v[1].x, v[0].x, HIGH), pair(v[3].x, v[2].x, HIGH));
-                *(uint2 *)(vt + pa_vt_chunk(d0 + 2u, chunk)) =
-                    make_uint2(pair(v[1].y, v[0].y, LOW), pair(v[3].y, v[2].y, LOW));
-                *(uint2 *)(vt + pa_vt_chunk(d0 + 3u, chunk)) =
-                    make_uint2(pair(v[1].y, v[0].y, HIGH), pair(v[3].y, v[2].y, HIGH));
-            }
-            if ((odd & 0x80008000u) != 0u) {
-                s_odd[number & 1u] = number + 1u;
+                *(uint2 *)(vt + v_at) = make_uint2(pair(vreg[1].x, vreg[0].x, LOW), pair(vreg[3].x, vreg[2].x, LOW));
+                *(uint2 *)(vt + (v_at ^ 32u) + 128) = make_uint2(pair(vreg[1].x, vreg[0].x, HIGH), pair(vreg[3].x, vreg[2].x, HIGH));
+                *(uint2 *)(vt + (v_at ^ 64u) + 256) = make_uint2(pair(vreg[1].y, vreg[0].y, LOW), pair(vreg[3].y, vreg[2].y, LOW));
+                *(uint2 *)(vt + (v_at ^ 96u) + 384) = make_uint2(pair(vreg[1].y, vreg[0].y, HIGH), pair(vreg[3].y, vreg[2].y, HIGH));
+                if ((odd & 0x80008000u) != 0u) {
+                    s_odd[number % 3u] = number + 1u;
+                }
             }
         };
-        auto consume = [&](uint32_t tile, uint32_t number, uint64_t mask) {
-            const uint8_t *stage = lds + (number & 1u) * L::STAGE;
-            const bool odd = __builtin_amdgcn_readfirstlane(s_odd[number & 1u]) == number + 1u;
-            const uint32_t p0 = 64u * tile;
-            if (__builtin_amdgcn_ballot_w64(row_len > p0) == 0) {
+        pa_float16v s = zero;
+        uint32_t see = 0;   // the positions of this wavefront's half of a tile that the lane's row sees
+        bool some = false;  // some row sees one of them
+        auto scores = [&](uint32_t tile, uint32_t number, uint64_t mask) {
+            const uint32_t p0 = 64u * tile + 32u * half;
+            some = __builtin_amdgcn_ballot_w64(row_len > p0) != 0;
+            if (!some) {
                 return;
             }
-            pa_float16v s[2] = {zero, zero};
-            uint4 k[2][QC];
+            const uint8_t *stage = lds + (number & 1u) * L::K + (32u * half + n) * L::KROW + 16u * h;
+            uint4 k[QC];
 #pragma unroll
             for (int c = 0; c < QC; ++c) {
-                k[0][c] = *(const uint4 *)(stage + n * L::KROW + 32u * c + 16u * h);
-                k[1][c] = *(const uint4 *)(stage + (32u + n) * L::KROW + 32u * c + 16u * h);
+                k[c] = *(const uint4 *)(stage + 32u * c);
             }
+            s = zero;
 #pragma unroll
             for (int part = PARTS - 1; part >= 0; --part) {  // small parts first
 #pragma unroll
                 for (int c = 0; c < QC; ++c) {
-                    s[0] = pa_mma32<BF16>(k[0][c], qpart[part][c], s[0]);
-                    s[1] = pa_mma32<BF16>(k[1][c], qpart[part][c], s[1]);
+                    const uint4 q = part < QREGS ? qpart[part < QREGS ? part : 0][c] : *(const uint4 *)(q_small + 4096 * (QC * (part - QREGS) + c));
+                    s = pa_mma32<BF16>(k[c], q, s);
                 }
             }
             const uint32_t left = row_len > p0 ? row_len - p0 : 0u;
-            const uint64_t see = mask & (left >= 64u ? ~0ull : (1ull << left) - 1ull);
-            if (__builtin_amdgcn_ballot_w64(see != ~0ull) != 0) {
+            see = (uint32_t)(mask >> (32u * half)) & (left >= 32u ? ~0u : (1u << left) - 1u);
+            if (__builtin_amdgcn_ballot_w64(see != ~0u) != 0) {
+                const uint32_t bits = see >> (4u * h);
 #pragma unroll
-                for (int st = 0; st < 2; ++st) {
-                    const uint32_t bits = (uint32_t)(see >> (32 * st)) >> (4u * h);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        s[st][r] = (bits >> (8 * (r >> 2) + (r & 3))) & 1u ? s[st][r] : -INFINITY;
-                    }
+                for (int r = 0; r < 16; ++r) {
+                    s[r] = (bits >> (8 * (r >> 2) + (r & 3))) & 1u ? s[r] : -INFINITY;
                 }
             }
-            float big = fmaxf(s[0][0], s[1][0]);
+        };
+        auto output = [&](uint32_t number, uint32_t values_at) {
+            if (!some) {
+                return;
+            }
+            const bool odd = __builtin_amdgcn_readfirstlane(s_odd[number % 3u]) == number + 1u;
+            float big = s[0];
 #pragma unroll
             for (int r = 1; r < 16; ++r) {
-                big = fmaxf(big, fmaxf(s[0][r], s[1][r]));
+                big = fmaxf(big, s[r]);
             }
             big = fmaxf(big, pa_xor32(big)) * unit;
             const float m_new = fmaxf(m, big);
             const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
             const float m_use = m_new == -INFINITY && see == 0u ? 0.0f : m_new;  // (a row that sees nothing yet)
             m = m_new;
-            float w[32], sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            float w[16], sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int r = 0; r < 32; ++r) {
-                w[r] = pa_exp(__builtin_fmaf(s[r >> 4][r & 15], unit, -m_use)) * UNIT;
+            for (int r = 0; r < 16; ++r) {
+                w[r] = pa_exp(__builtin_fmaf(s[r], unit, -m_use)) * UNIT;
                 sum[r & 3] += w[r];
             }
             lsum = lsum * corr + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
-            const uint8_t *vt = stage + L::K;
-            if (odd) {
+            const uint8_t *vt = lds + values_at;
+            uint32_t wp[2][PARTS][4];
 #pragma unroll
-                for (int d = 0; d < DB; ++d) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        out[d][r] *= corr;
-                    }
-                }
-                for (uint32_t i = 0; i < 64u; ++i) {
-                    // position i: register 16 (i / 32) + 4 (i / 8 % 4) + i % 4 of lane half (i / 4) % 2
-                    float mine_w = 0.0f;
-#pragma unroll
-                    for (int r = 0; r < 32; ++r) {
-                        mine_w = (uint32_t)r == 4u * (i >> 3) + (i & 3u) ? w[r] : mine_w;
-                    }
-                    const float wi = __shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u)));
-                    if ((see >> i) & 1u) {
-                        const uint32_t chunk = 2u * (i >> 4) + ((i >> 2) & 1u), in = 8u * ((i >> 3) & 1u) + 2u * (i & 3u);
-#pragma unroll
-                        for (int d = 0; d < DB; ++d) {
-#pragma unroll
-                            for (int r = 0; r < 16; ++r) {
-                                const uint32_t dim = 32u * d + 8u * (r >> 2) + 4u * h + (r & 3);
-                                const uint16_t v = *(const uint16_t *)(vt + pa_vt_chunk(dim, chunk) + in);
-                                out[d][r] = __builtin_fmaf(wi, BF16 ? pa_bf2f(v) : h2f(v), out[d][r]);
-                            }
-                        }
-                    }
-                }
-                return;
-            }
-            uint32_t wp[4][PARTS][4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < 2; ++i) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float a = w[8 * i + 2 * e], b = w[8 * i + 2 * e + 1];
@@ -1720,58 +1782,165 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
             }
             // The tile's products are summed by themselves, small parts first, and join the running output in one rounding
             // (a third of the error of a chain through the running output, and the rescaling costs nothing)
+            uint4 v[2][2];
+            auto read_v = [&](int d) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    v[d & 1][i] = *(const uint4 *)(vt + (v_from ^ (32u * i)) + 4096 * d);
+                }
+            };
+            read_v(0);
+            __builtin_amdgcn_s_setprio(1);  // in front of the other half's softmax (0.6 us of 147)
 #pragma unroll
             for (int d = 0; d < DB; ++d) {
                 pa_float16v tile_out = zero;
-                uint4 v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    v[i] = *(const uint4 *)(vt + pa_vt_chunk(32u * d + n, 2u * i + h));
+                if (d + 1 < DB) {
+                    read_v(d + 1);
                 }
+                if (!odd) {
 #pragma unroll
-                for (int part = PARTS - 1; part >= 0; --part) {
+                    for (int part = PARTS - 1; part >= 0; --part) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        tile_out = pa_mma32<BF16>(
-                            v[i], make_uint4(wp[i][part][0], wp[i][part][1], wp[i][part][2], wp[i][part][3]), tile_out);
+                        for (int i = 0; i < 2; ++i) {
+                            tile_out = pa_mma32<BF16>(
+                                v[d & 1][i], make_uint4(wp[i][part][0], wp[i][part][1], wp[i][part][2], wp[i][part][3]), tile_out);
+                        }
+                    }
+                } else {
+                    uint32_t h = lane >> 5;
+                    asm volatile("" : "+v"(h));
+                    for (uint32_t i = 0; i < 32u; ++i) {
+                        // position i: weight 4 (i / 8) + i % 4 of lane half (i / 4) % 2
+                        const uint32_t at = 4u * (i >> 3) + (i & 3u);
+                        float mine_w = 0.0f;
+#pragma unroll
+                        for (int part = PARTS - 1; part >= 0; --part) {
+                            uint32_t word = 0;
+#pragma unroll
+                            for (int r = 0; r < 8; ++r) {
+                                word = (uint32_t)r == at >> 1 ? wp[r >> 2][part][r & 3] : word;
+                            }
+                            const uint16_t bits = (uint16_t)(word >> (16u * (at & 1u)));
+                            mine_w += BF16 ? pa_bf2f(bits) : h2f(bits);
+                        }
+                        const float wi = __shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u)));
+                        if ((see >> i) & 1u) {
+                            const uint32_t chunk = 4u * half + 2u * (i >> 4) + ((i >> 2) & 1u), in = 8u * ((i >> 3) & 1u) + 2u * (i & 3u);
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) {
+                                const uint32_t dim = 32u * d + 8u * (r >> 2) + 4u * h + (r & 3);
+                                const uint16_t one = *(const uint16_t *)(vt + pa_vt_chunk(dim, chunk) + in);
+                                tile_out[r] = __builtin_fmaf(wi, BF16 ? pa_bf2f(one) : h2f(one), tile_out[r]);
+                                __builtin_amdgcn_sched_barrier(0);  // (rare, and short of registers otherwise)
+                            }
+                        }
                     }
                 }
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     out[d][r] = __builtin_fmaf(out[d][r], corr, tile_out[r]);
                 }
+                asm volatile("" : "+v"(out[d]));  // in place, one after the other
+                __builtin_amdgcn_sched_barrier(0);
             }
+            __builtin_amdgcn_s_setprio(0);
         };
-        // A buffer is written after the barrier that follows its last reading: tile k + 1 is stored beside the reading of
-        // tile k, into the buffer that tile k - 1 left before the barrier.
-        request(begin, table_entry(begin));
-        uint32_t entry = table_entry(begin + 1u);
-        store(count);
+        // Between two barriers tile k + 1 is stored, half 0 takes tile k whole, half 1 the output of tile k - 1 and then
+        // the scores of tile k: one uses the matrix cores while the other is at its softmax. Tile k + 1 goes to buffers
+        // last read before the barrier: the keys of tile k - 1, the values of tile k - 2.
+        auto after = [&](uint32_t at) { return at == L::V0 + 2u * L::V ? L::V0 : at + L::V; };
+        uint32_t entry = 0;
+        if (wave == 0u) {
+            const uint32_t entry0 = table_entry(begin), entry1 = table_entry(begin + 1u);
+            entry = table_entry(begin + 2u);
+            locate(begin, entry0);
+            locate(begin + 1u, entry1);
+        }
+        __syncthreads();
+        request(begin);
+        store(count, now);
         uint64_t mask = mask_next;
         __syncthreads();
-        for (uint32_t tile = begin; tile < end; ++tile, ++count) {
+        for (uint32_t tile = begin; tile <= end; ++tile) {
             const bool more = tile + 1u < end;
             if (more) {
-                request(tile + 1u, entry);
-                entry = table_entry(tile + 2u);
+                request(tile + 1u);
+                if (wave == 0u) {
+                    locate(tile + 2u, entry);
+                    entry = table_entry(tile + 3u);
+                }
             }
-            consume(tile, count, mask);
+            if (half == 0u && tile < end) {
+                scores(tile, count, mask);
+            }
+            if (half == 0u ? tile < end : tile != begin) {
+                output(count - half, half == 0u ? now : before);
+            }
+            if (half != 0u && tile < end) {
+                scores(tile, count, mask);
+            }
+            if (tile == end) {
+                break;  // (the stores of the next sequence's first tile go to other buffers than the last output's)
+            }
             if (more) {
-                store(count + 1u);
+                store(count + 1u, after(now));
                 mask = mask_next;
             }
+            ++count;
+            before = now;
+            now = after(now);
             __syncthreads();
         }
     }
 
+    // The halves' sums meet in LDS: each gives half of its dimensions to the other and keeps the other half
     lsum += pa_xor32(lsum);
+    __syncthreads();
+    {
+        float2 *ml = (float2 *)(lds + L::MAIL);
+        ml[tid] = make_float2(m, lsum);
+        float4 *mail = (float4 *)lds + wave * (HD / 64 * 256u) + lane;
+#pragma unroll
+        for (int d = 0; d < DB / 2; ++d) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = half == 0u ? out[DB / 2 + d][4 * q + e] : out[d][4 * q + e];
+                    out[d][4 * q + e] = half == 0u ? out[d][4 * q + e] : out[DB / 2 + d][4 * q + e];
+                }
+                mail[64 * (4 * d + q)] = make_float4(v[0], v[1], v[2], v[3]);
+            }
+        }
+        __syncthreads();
+        const float2 other = ml[tid ^ 256u];
+        const float m_all = fmaxf(m, other.x);
+        const float f_own = m == -INFINITY ? 0.0f : pa_exp(m - m_all), f_other = other.x == -INFINITY ? 0.0f : pa_exp(other.x - m_all);
+        lsum = __builtin_fmaf(other.y, f_other, lsum * f_own);
+        m = m_all;
+        const float4 *from = (const float4 *)lds + (wave ^ 4u) * (HD / 64 * 256u) + lane;
+#pragma unroll
+        for (int d = 0; d < DB / 2; ++d) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 v = from[64 * (4 * d + q)];
+                const float add[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    out[d][4 * q + e] = __builtin_fmaf(add[e], f_other, out[d][4 * q + e] * f_own);
+                }
+            }
+        }
+    }
+    const uint32_t dim0 = half * (HD / 2);
     if (row_seq == NONE) {
         return;
     }
     const bool bad = lsum != lsum;
     if (p.tile_splits > 1u) {
         float *part = p.partial + (((size_t)t * p.num_q_heads + qh) * p.partial_splits + blockIdx.z) * (HD + 2u);
-        if (h == 0) {
+        if (h == 0 && half == 0u) {
             part[0] = m;
             part[1] = lsum;
         }
@@ -1779,10 +1948,10 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
             return;
         }
 #pragma unroll
-        for (int d = 0; d < DB; ++d) {
+        for (int d = 0; d < DB / 2; ++d) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                float2 *dst = (float2 *)(part + 2 + 32 * d + 8 * q + 4 * h);
+                float2 *dst = (float2 *)(part + 2 + dim0 + 32 * d + 8 * q + 4 * h);
                 dst[0] = make_float2(out[d][4 * q], out[d][4 * q + 1]);
                 dst[1] = make_float2(out[d][4 * q + 2], out[d][4 * q + 3]);
             }
@@ -1792,10 +1961,10 @@ __global__ __launch_bounds__(256, 1) void k_pa_prompt(const PaParams p) {
     const float inv = bad ? __uint_as_float(0x7fc00000u) : (lsum > 0.0f ? 1.0f / lsum : 0.0f);
     const size_t base = (size_t)t * p.out_stride[0] + (size_t)qh * p.out_stride[1];
 #pragma unroll
-    for (int d = 0; d < DB; ++d) {
+    for (int d = 0; d < DB / 2; ++d) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const uint32_t dim = 32u * d + 8u * q + 4u * h;
+            const uint32_t dim = dim0 + 32u * d + 8u * q + 4u * h;
             float o[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -1869,10 +2038,28 @@ template <int HD, bool BF16>
 static int pa_launch_prompt(marmot_hip_device *dev, const PaParams &p) {
     MH_TRY(allow_large_lds(dev, (const void *)k_pa_prompt<HD, BF16>));
     const unsigned tiles = (p.token_count + p.tile_tokens - 1) / p.tile_tokens;
-    hipLaunchKernelGGL((k_pa_prompt<HD, BF16>), dim3(tiles, p.num_kv_heads, p.tile_splits), dim3(256), PaPromptLds<HD>::BYTES,
-                       dev->stream, p);
+    hipLaunchKernelGGL((k_pa_prompt<HD, BF16>), dim3(tiles, p.num_kv_heads, p.tile_splits), dim3(64 * PA_PROMPT_WAVES),
+                       (PaPromptLds<HD, BF16>::BYTES),                       dev->stream, p);
     MH_HIP(hipGetLastError());
     return MARMOT_HIP_SUCCESS;
+}
+
+// k_pa_write_rows takes the call: rows of whole 16-byte pieces, in the cache and in the new rows, and more of them than run at once
+// as workgroups of their own (a decode step of 16 tokens of 8 heads is 0.7 % of a layer faster with those: all start together)
+static bool pa_write_rows(const marmot_hip_device *dev, const marmot_hip_paged_attention_t *a, size_t act_size) {
+    if ((size_t)a->token_count * a->num_kv_heads < 4 * (size_t)dev->props.multiProcessorCount) {
+        return false;
+    }
+    bool ok = (a->kv_dtype == MARMOT_HIP_DTYPE_F16 || a->kv_dtype == MARMOT_HIP_DTYPE_BF16) && a->head_dim % 8 == 0 &&
+              a->kv_stride[4] == 1 && a->k_stride[2] == 1 && a->v_stride[2] == 1;
+    ok = ok && (((uintptr_t)a->d_kv_k | (uintptr_t)a->d_kv_v | (uintptr_t)a->d_k_new | (uintptr_t)a->d_v_new) & 15) == 0;
+    for (int i = 0; i < 4; ++i) {
+        ok = ok && (a->kv_stride[i] * 2) % 16 == 0;
+    }
+    for (int i = 0; i < 2; ++i) {
+        ok = ok && (a->k_stride[i] * act_size) % 16 == 0 && (a->v_stride[i] * act_size) % 16 == 0;
+    }
+    return ok;
 }
 
 static bool pa_float_dtype(int d) {
@@ -2089,6 +2276,8 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
             hipLaunchKernelGGL(k_pa_fp8_rescale, per_token, dim3(128), 0, dev->stream, p);
             hipLaunchKernelGGL(k_pa_fp8_store, per_token, dim3(128), 0, dev->stream, p);
         }
+    } else if (pa_write_rows(dev, a, asz)) {
+        hipLaunchKernelGGL(k_pa_write_rows, dim3(a->token_count), dim3(PA_WRITE_THREADS + (prompt ? 64 : 0)), 0, dev->stream, p);
     } else {
         hipLaunchKernelGGL(k_pa_write, per_token, dim3(a->head_dim <= 64 ? 64 : 128), 0, dev->stream, p);
     }

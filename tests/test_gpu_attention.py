@@ -149,6 +149,17 @@ def test_long_context_decode_batch(hip, oracle):
     check(hip, oracle, case, "decode batch")
 
 
+@pytest.mark.parametrize("act,kv", [("f32", "f16"), ("f32", "bf16"), ("f16", "f16"), ("bf16", "bf16"), ("f16", "bf16")])
+@pytest.mark.parametrize("hkv,head_dim,tokens", [(1, 8, 1030), (3, 72, 350), (10, 104, 102), (2, 60, 520), (9, 104, 112)])
+def test_cache_rows_in_pieces(hip, oracle, hkv, head_dim, tokens, act, kv):
+    """The cache write in pieces of eight values (from four rows per compute unit on): one piece per row, heads whose pieces end
+    inside a wavefront, more than one step of the workgroup; rows that are no whole pieces, and fewer rows (one workgroup per
+    row). `check` compares the bits."""
+    case = make_case(900 + hkv, [(0, tokens - 3), (37, 2), (5, 1)], num_q_heads=hkv, num_kv_heads=hkv, head_dim=head_dim,
+                     block_size=16, act=act, kv=kv)
+    check(hip, oracle, case, "pieces")
+
+
 def test_prompt_of_many_tokens_takes_unsplit_histories(hip, oracle):
     """A prompt chunk of 640 tokens on top of 100 positions of history, next to a short second sequence: enough
     (token, heads) pairs that no history is split across workgroups (decode-sized calls above split it)."""
