@@ -23,7 +23,8 @@
 // half at the end of its second stage and half at the beginning of the next block's first, which makes stages equally long.
 // KG = 2: eight wavefronts, two K groups with buffers of their own that take every second block, one stage apart (one does its
 // fp32 step while the other multiplies), sums joined in LDS at the end: for calls that have one tile per compute unit, which
-// would leave a SIMD one wavefront. KG = 1: four wavefronts, two or three workgroups per compute unit; the last tiles of a
+// would leave a SIMD one wavefront. KG = 4 halves the tile's rows besides (RG = 2 wavefronts of them, four K groups): a call of
+// half a chip of 128 x 64 tiles, the k and v projections of a prompt, takes a whole chip of these. KG = 1: four wavefronts, two or three workgroups per compute unit; the last tiles of a
 // ragged token count run on as many of the C token tiles as hold a token.
 // Measured (us of whole calls in a row, the quantization of 6 - 17 included; before: the best of the kernels of
 // mh_gemm_int16.hip and mh_gemm_i8.hip; tokens x K x M):
@@ -88,23 +89,22 @@ struct PlanesFormat<MARMOT_HIP_KIND_Q6_K> {
     static constexpr bool MIN = false;
 };
 
-constexpr int PLANES_ROWS = 4;  // wavefronts along the rows of a workgroup's tile
-
-template <int KIND, int C, int KG, bool LOOP>
+// RG: wavefronts along the rows of a workgroup's tile
+template <int KIND, int C, int KG, bool LOOP, int RG>
 struct PlanesLds {
     static constexpr int ROWS = 64 / PlanesFormat<KIND>::PIECES;  // whole rows per direct-to-LDS load
     static constexpr int DMA = (32 + ROWS - 1) / ROWS;            // such loads of a wavefront per block
     static constexpr int ACT = 32 * C * 128;                      // one stage: 32 C tokens x 128 codes
     static constexpr int W0 = KG * 2 * ACT;
     static constexpr int WAVE_W = 32 * 16 * PlanesFormat<KIND>::PIECES;
-    static constexpr int S0 = W0 + PLANES_ROWS * KG * WAVE_W;
+    static constexpr int S0 = W0 + RG * KG * WAVE_W;
     static constexpr int SUMS = PlanesFormat<KIND>::MIN ? 32 * C * 32 : 0;  // sums of a block as fp16: [token][16]
     static constexpr int SD = SUMS + 32 * C * 4;                            // then the activation scales [token]
     static constexpr int OFFS = S0 + 2 * KG * SD;  // lane offsets of the activation loads: [this tile, next][wavefront][load][lane]
-    static constexpr int OFF_N = C + 1 + (PlanesFormat<KIND>::MIN ? 1 : 0);
-    static constexpr int TABLE = PLANES_ROWS * KG * OFF_N * 256;
+    static constexpr int OFF_N = 4 * C / RG + 1 + (PlanesFormat<KIND>::MIN ? 1 : 0);
+    static constexpr int TABLE = RG * KG * OFF_N * 256;
     static constexpr int NEXT = OFFS + (LOOP ? 2 : 1) * TABLE;  // activation rows of the next tile's tokens, per wavefront
-    static constexpr int BYTES = NEXT + (LOOP ? PLANES_ROWS * 128 * C : 0);
+    static constexpr int BYTES = NEXT + (LOOP ? RG * 128 * C : 0);
 };
 
 __device__ __forceinline__ pl_u16x2 pl_v(uint32_t v) {
@@ -303,15 +303,15 @@ __device__ __forceinline__ void planes_barrier() {
 }
 
 // LOOP: a workgroup goes from tile to tile
-template <int KIND, int C, int KG, bool LOOP = false>
-__global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) void k_gemm_planes(const GemmPlanesParams p) {
+template <int KIND, int C, int KG, bool LOOP = false, int RG = 4>
+__global__ __launch_bounds__(64 * RG * KG, C == 2 && KG == 1 ? 3 : 2) void k_gemm_planes(const GemmPlanesParams p) {
     using F = PlanesFormat<KIND>;
-    using L = PlanesLds<KIND, C, KG, LOOP>;
+    using L = PlanesLds<KIND, C, KG, LOOP, RG>;
     static_assert(!LOOP || KG == 1, "one K group");
-    constexpr int RG = PLANES_ROWS;
     constexpr int TOK = 32 * C;
-    constexpr int APW = C;  // direct-to-LDS loads of codes per wavefront and stage, 8 tokens each: the i-th of all wavefronts is tile i
-    static_assert(RG == 4, "a token tile is four loads");
+    // direct-to-LDS loads of codes per wavefront and stage, 8 tokens each: the i-th of all wavefronts is tile i (RG == 4)
+    constexpr int APW = 4 * C / RG;
+    static_assert(RG == 4 || (RG == 2 && C == 2 && KG == 4), "a token tile is four loads; two wavefronts load the sums of 64 tokens");
     warm_kernel_arguments<sizeof(GemmPlanesParams)>();
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
             request_weights((uint32_t)kg, i);
         }
 #pragma unroll
-        for (int i = 0; i < CT; ++i) {
+        for (int i = 0; i < CT * 4 / RG; ++i) {
             request_acts(2u * (uint32_t)kg, 0, i, offs(table, i));
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
     if (first_tile) {
         planes_barrier();
     }
-    if (KG > 1 && kg == 1) {
+    if (KG > 1 && kg >= KG / 2) {  // (wavefronts w and w + 4 share a SIMD)
         planes_barrier();
         ++passed;
     }
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
         const uint32_t bn = !last ? b + KG : LOOP ? 0u : b;
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
-            constexpr int STEPS = 4 * CT, AHEAD = 2;
+            constexpr int STEPS = 4 * CT, AHEAD = 2, LOADS = CT * 4 / RG;
             pl_i32x4 ring[AHEAD];
             uint32_t a_addr = 0;
             auto read_a = [&](int st) {
@@ -658,9 +658,9 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
                     read_a(st + AHEAD);
                 }
                 // the next stage's codes, then scales and sums of this block: one load per place
-                if (st < CT) {
+                if (st < LOADS) {
                     request_acts(hb == 0 ? 2u * b + 1u : 2u * bn, hb ^ 1, st, off);
-                    if (st + 1 < CT) {
+                    if (st + 1 < LOADS) {
                         off = offs(table, st + 1);
                     } else if (hb == 0) {
                         off = offs(table, APW);
@@ -670,19 +670,21 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
                             request_acts(2u * bn, hb ^ 1, i, offs(table, i));
                         }
                     }
-                } else if (st == CT && hb == 0) {
+                } else if (st == LOADS && hb == 0) {
                     request_scales(b, number, off);
                     if (F::MIN) {
                         off = offs(table, APW + 1);
                     }
-                } else if (st == CT + 1 && hb == 0) {
+                } else if (st == LOADS + 1 && hb == 0) {
                     request_sums(b, off);
                 }
                 // the operands of the next step, a quarter at a time
                 const int hn = s < 3 ? hb : 1, sn = (s + 1) & 3;
                 if (t == 0) {
                     if (s == 3 && hb == 0) {
-                        store_block(number);
+                        if (RG == 4) {
+                            store_block(number);
+                        }
                         raw.load_half(block, hn, kh);
                     }
                     if (s == 1 || (s == 3 && hb == 0)) {
@@ -722,6 +724,9 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
                 __builtin_amdgcn_s_setprio(0);
             }
             if (hb == 0) {
+                if (RG != 4) {  // (requested later than with four)
+                    store_block(number);
+                }
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
                 finish(number, 0, CT / 2);
@@ -741,8 +746,49 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
         for (; passed < stages; ++passed) {
             planes_barrier();
         }
+        static_assert(CT == C, "whole tiles");
+    }
+    if constexpr (KG == 4) {
+        // the K groups' sums meet in LDS: each keeps a quarter of the outputs, half a token tile, and gives away the others
+        static_assert(C == 2 && RG * 4 * 4 * 2048 <= L::W0, "the mail fits the codes' place");
+        float4 *mail = (float4 *)lds + gw * 2048 + lane;  // [to][from][two][lane]
+#pragma unroll
+        for (int to = 0; to < 4; ++to) {
+            if (to != kg) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const pl_float16 &v = total[to >> 1];
+                    const int r = 8 * (to & 1) + 4 * q;
+                    mail[512 * to + 128 * kg + 64 * q] = make_float4(v[r], v[r + 1], v[r + 2], v[r + 3]);
+                }
+            }
+        }
+        planes_barrier();
+        float own[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float low = kg == 0 ? total[0][i] : total[0][8 + i], high = kg == 2 ? total[1][i] : total[1][8 + i];
+            own[i] = kg < 2 ? low : high;
+        }
+#pragma unroll
+        for (int from = 0; from < 4; ++from) {  // in the order of K
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float4 v = make_float4(own[4 * q], own[4 * q + 1], own[4 * q + 2], own[4 * q + 3]);
+                if (from != kg) {
+                    v = mail[512 * kg + 128 * from + 64 * q];
+                }
+                const float add[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    total[0][4 * q + e] = from == 0 ? add[e] : total[0][4 * q + e] + add[e];
+                }
+            }
+        }
+    }
+    if constexpr (KG == 2) {
         // the K groups' sums meet in LDS: each gives the other half of its token tiles and keeps the other half
-        static_assert(KG == 2 && CT == C && C % 2 == 0, "two K groups, halves of whole token tiles");
+        static_assert(C % 2 == 0, "halves of whole token tiles");
         float *mail = (float *)lds + (size_t)wave * (C / 2) * 1024 + lane * 4;
         const float *from = (const float *)lds + (size_t)(wave ^ RG) * (C / 2) * 1024 + lane * 4;
 #pragma unroll
@@ -783,8 +829,8 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
     const uint32_t which = cur.which;
     uint32_t kh4 = 4u * (uint32_t)kh;
     asm volatile("" : "+v"(kh4));  // (the places of the outputs are not kept from tile to tile)
-    constexpr int OUT = KG > 1 ? C / 2 : CT;  // token tiles this wavefront stores
-    const uint32_t t0 = (uint32_t)(KG > 1 ? kg * OUT : 0);
+    constexpr int OUT = KG == 4 ? 1 : KG == 2 ? C / 2 : CT, REGS = KG == 4 ? 8 : 16;  // token tiles this wavefront stores, outputs of one
+    const uint32_t n0 = (uint32_t)(KG == 4 ? 16 * kg : KG == 2 ? 32 * kg * OUT : 0);
     const void *bias_p = p.bias[which];
     const bool has_bias = bias_p != nullptr;
     const float bias = !has_bias ? 0.0f : p.bias_is_f16 ? h2f(((const uint16_t *)bias_p)[m]) : ((const float *)bias_p)[m];
@@ -793,8 +839,8 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
 #pragma unroll
         for (int t = 0; t < OUT; ++t) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t n = 32u * (t0 + t) + 8u * (r >> 2) + kh4 + (r & 3u);
+            for (int r = 0; r < REGS; ++r) {
+                const uint32_t n = n0 + 32u * t + 8u * (r >> 2) + kh4 + (r & 3u);
                 if (n < toks) {
                     out[(size_t)n * p.M] = has_bias ? total[t][r] + bias : total[t][r];
                 }
@@ -806,8 +852,8 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
 #pragma unroll
         for (int t = 0; t < OUT; ++t) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t n = 32u * (t0 + t) + 8u * (r >> 2) + kh4 + (r & 3u);
+            for (int r = 0; r < REGS; ++r) {
+                const uint32_t n = n0 + 32u * t + 8u * (r >> 2) + kh4 + (r & 3u);
                 if (n < toks) {
                     // without bias_first: round to the output type, then add the bias in it
                     const uint16_t first = f2h(has_bias && bias_first ? total[t][r] + bias : total[t][r]);
@@ -841,16 +887,16 @@ __global__ __launch_bounds__(64 * PLANES_ROWS * KG, C == 2 && KG == 1 ? 3 : 2) v
 }
 
 // cols: tiles along the tokens, or work items at most. LOOP: as many workgroups as the chip holds at once (three per compute unit).
-template <int KIND, int C, int KG, bool LOOP = false>
+template <int KIND, int C, int KG, bool LOOP = false, int RG = 4>
 static int planes_launch(marmot_hip_device *dev, GemmPlanesParams &p, size_t cols, unsigned weights) {
-    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_planes<KIND, C, KG, LOOP>));
-    p.row_tiles = (uint32_t)((p.M + 32 * PLANES_ROWS - 1) / (32 * PLANES_ROWS));
+    MH_TRY(allow_large_lds(dev, (const void *)k_gemm_planes<KIND, C, KG, LOOP, RG>));
+    p.row_tiles = (uint32_t)((p.M + 32 * RG - 1) / (32 * RG));
     p.col_tiles = (uint32_t)cols;
     p.weights = weights;
     const size_t tiles = (size_t)p.row_tiles * cols * weights;
     const size_t places = (size_t)dev->props.multiProcessorCount * 3;
     const dim3 grid((unsigned)(LOOP && tiles > places ? places : tiles));
-    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG, LOOP>), grid, dim3(64 * PLANES_ROWS * KG), (PlanesLds<KIND, C, KG, LOOP>::BYTES), dev->stream, p);
+    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG, LOOP, RG>), grid, dim3(64 * RG * KG), (PlanesLds<KIND, C, KG, LOOP, RG>::BYTES), dev->stream, p);
     MH_HIP(hipGetLastError());
     return MARMOT_HIP_SUCCESS;
 }
@@ -860,14 +906,18 @@ static bool planes_kind(int kind) {
 }
 
 // Which form (10 C + KG), or none (0), by the tiles a call has. The kernels of mh_gemm_i8.hip split K over workgroups where
-// tiles are few, which pays the partial sums and wins while the chip is mostly empty; two K groups per workgroup want one
-// tile per compute unit, and beyond that workgroups share one (us of whole calls, other kernels / forms):
-//   Q6_K, 64 tokens a tile    64 tiles 128 x 4096 x 4096 31 / (22) 37   104, 800 x 4096 x 1024 47 / (22) 42
-//                             88 tiles 128 x 2048 x 5632 29 / (22) 24   128, 200 x 14336 x 4096 122 / (22) 109
-//   Q4_K, the same            128 tiles 200 x 4096 x 4096 28 / (22) 30  160, 300 x 4096 x 4096 31.5 / (22) 30.3
+// tiles are few, which pays the partial sums and wins while the chip is mostly empty; K groups in one workgroup want one
+// tile per compute unit, and beyond that workgroups share one (us of whole calls, other kernels / forms; 24: 64 rows, four K
+// groups):
+//   64 x 64, up to a tile     Q6_K 64 tiles 100 x 4096 x 2048 22.1 / (24) 22.8   80, 300 x 4096 x 1024 27.7 / 24.3   128, 128 x
+//   per compute unit          14336 x 4096 65 / 58   256, 1024 x 4096 x 1024 48 / (22) 42, (24) 29   256 x 14336 x 4096 - / 104, 62
+//                             Q4_K 64, 64 x 4096 x 4096 17.7 / (24) 18.4   80, 300 x 4096 x 1024 20.9 / 20.4   88, 64 x 2048 x
+//                             5632 16.3 / 13.9   128, 128 x 4096 x 4096 21.3 / 19.5   128 x 8192 x 4096 27.3 / 30.0   192, 192 x
+//                             8192 x 4096 37 / 32   160, 300 x 14336 x 2048 45 / 49   192, 192 x 14336 x 4096 52 / 48
+//                             (320, 300 x 4096 x 4096: Q6_K (22) 37.5, (24) 42.6; Q4_K 30.1, 35.1)
+//   Q6_K, 64 tokens a tile    104 tiles 800 x 4096 x 1024 47 / (22) 42
+//   Q4_K, the same            160, 300 x 4096 x 4096 31.5 / (22) 30.3
 //                             224, 128 x 4096 x 14336 31.9 / (22) 30.9  256, 512 x 14336 x 4096 100 / (22) 91
-//   with up to eight blocks   64, 64 x 1024 x 8192 15.8 / (22) 13.9     88, 128 x 2048 x 5632 20.0 / (22) 19.0
-//                             44, 128 x 2048 x 2816: other kernels
 //   128 tokens a tile         Q4_K 192 tiles 300 x 1024 x 8192 22.8 / (42) 20.2   256, 1024 x 14336 x 4096 187 / (42) 142
 //   more tiles than units     Q4_K 308, 800 x 2048 x 5632 49 / (42) 50, (41) 46, (21) 40   784, 800 x 4096 x 14336 167 / 153, 145, 130
 //                             Q6_K 308, 77 / (42) 57, (41) 53, (21) 52   896, 1024 x 4096 x 14336 303 / 186, 178, 204
@@ -877,9 +927,12 @@ static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t 
     const size_t cus = (size_t)dev->props.multiProcessorCount;
     const size_t rows = (M + 127) / 128 * weights;
     const size_t small = (N + 63) / 64 * rows, large = (N + 127) / 128 * rows;
+    const size_t least = (N + 63) / 64 * ((M + 63) / 64) * weights;
+    if (least <= cus) {
+        return 4 * least > cus && (kind == MARMOT_HIP_KIND_Q6_K || nb <= 16 || 3 * least > 2 * cus) ? 24 : 0;
+    }
     if (small <= cus) {
-        const bool few = kind == MARMOT_HIP_KIND_Q6_K || nb <= 8 ? 3 * small <= cus : 5 * small <= 3 * cus;
-        return few ? 0 : 22;
+        return kind != MARMOT_HIP_KIND_Q6_K && nb > 8 && 5 * small <= 3 * cus ? 0 : 22;
     }
     return large <= cus ? 42 : kind == MARMOT_HIP_KIND_Q6_K ? 41 : 21;
 }
@@ -905,6 +958,9 @@ static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsig
     const unsigned t64 = (unsigned)((p.N + 63) / 64), t128 = (unsigned)((p.N + 127) / 128);
     if (form == 22) {
         return planes_launch<KIND, 2, 2>(dev, p, t64, weights);
+    }
+    if (form == 24) {
+        return planes_launch<KIND, 2, 4, false, 2>(dev, p, t64, weights);
     }
     if (form == 42) {
         return planes_launch<KIND, 4, 2>(dev, p, t128, weights);

@@ -1,5 +1,5 @@
 """Tiled GEMM of K-quant weights and Q8_K activations on int8 planes (mh_gemm_planes.hip) against the CPU oracle, at the edges
-of its forms and of the rule that chooses one (planes_form, 256 compute units): two K groups per workgroup or one, 64 or 128
+of its forms and of the rule that chooses one (planes_form, 256 compute units): four K groups per workgroup, two or one, 64 or 128
 tokens per tile, last tiles with one to four token tiles, one block per row (the second K group has none) and odd counts."""
 import numpy as np
 import pytest
@@ -28,6 +28,10 @@ CASES = [
     ("q4_k q5_k", "small", 128, 10400, 256),   # two K groups, 64 tokens, the second group without a block
     ("q4_k q5_k", "small", 97, 12801, 768),    # odd block counts, one row and 33 tokens in the last tiles
     ("q6_k", "small", 33, 11000, 1280),
+    ("q4_k q5_k q6_k", "small", 65, 2085, 256),   # four K groups, 64 rows: three without a block, one token and 37 rows in the last tiles
+    ("q4_k q5_k q6_k", "small", 130, 1401, 1280),  # (five blocks, one row in the last tile)
+    ("q4_k q5_k q6_k", "small", 257, 3232, 768),   # (255 tiles of 256)
+    ("q4_k q5_k q6_k", "small", 129, 3700, 4352),  # (more than 16 blocks)
     ("q4_k q5_k q6_k", "large", 257, 6785, 768),   # two K groups, 128 tokens, one token in the last tile
     ("q4_k q5_k q6_k", "large", 380, 8200, 256),
     ("q4_k q5_k", "small", 130, 16600, 512),   # one K group, 64 tokens
@@ -53,7 +57,8 @@ def test_forms_match_oracle(hip, oracle, name, tile, N, M, K):
 
 
 @pytest.mark.parametrize("name,N,M", [("q4_k", 130, 16600), ("q5_k", 130, 16600), ("q6_k", 300, 11000),  # one K group
-                                      ("q4_k", 257, 6800), ("q5_k", 257, 6800), ("q6_k", 257, 6800)])  # two
+                                      ("q4_k", 257, 6800), ("q5_k", 257, 6800), ("q6_k", 257, 6800),  # two
+                                      ("q4_k", 70, 2100), ("q5_k", 70, 2100), ("q6_k", 70, 2100)])  # four
 @pytest.mark.parametrize("scale", ["largest", "mixed"])
 def test_block_sums_are_exact(hip, name, N, M, scale):
     """One block per row, activation and block scales of 1, minimum scale 0: the output is the integer block sum rounded
