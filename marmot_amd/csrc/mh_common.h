@@ -487,7 +487,7 @@ bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_
                                    const void *w1);
 int launch_gemm_planes_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
                                const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
-                               size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1);
+                               size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1, bool swiglu);
 // Tiled int8 GEMM on Q8_0 activations (mh_gemm_i8.hip): Q8_0 and Q4_0 weights, K a multiple of 256, nine rows and more;
 // `scratch` holds the gemm_i8_scratch_bytes of the call for the K-split partial sums
 bool gemm_q23k_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, const void *const *weights, int count,

@@ -678,8 +678,11 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const size_t gu_stride = F * ((H + bv_gu - 1) / bv_gu) * block_bytes(kind_gate_up);
     const size_t dn_stride = H * ((F + bv_dn - 1) / bv_dn) * block_bytes(kind_down);
     // K-quant experts run on the matrix cores (long prompts on the tiled GEMM on int8 planes, else passes), the 32-value formats on the dot-product matvec
+    // Tiled, SwiGLU: the GEMM forms the gated product itself, which is written and read once in the place of two arrays (a call
+    // that looks at the stages gets both)
+    const bool gated = tiled && ffn_type != MARMOT_HIP_FFN_GEGLU && probe == nullptr;
     st = tiled  ? launch_gemm_planes_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
-                                          max_items, H, F, gate_out, up_out)
+                                          max_items, H, F, gate_out, up_out, gated)
         : mmq_gu ? launch_mmq_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
                                      max_items, H, F, gate_out, up_out, (int)item_cols)
                 : launch_matvec_grouped(dev, kind_gate_up, d_gate, d_up, gu_stride, hidden_q, sorted_tokens, items, flags,
@@ -687,7 +690,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     if (st != MARMOT_HIP_SUCCESS) {
         return st;
     }
-    st = launch_quantize_glu_soa(dev, act_dn, gate_out, up_out, ffn_type == MARMOT_HIP_FFN_GEGLU, routes, F, fused_q);
+    st = gated ? launch_quantize_act_soa(dev, act_dn, gate_out, MARMOT_HIP_DTYPE_F32, routes, F, fused_q)
+               : launch_quantize_glu_soa(dev, act_dn, gate_out, up_out, ffn_type == MARMOT_HIP_FFN_GEGLU, routes, F, fused_q);
     if (st != MARMOT_HIP_SUCCESS) {
         return st;
     }
@@ -715,7 +719,7 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
         }
     }
     st = tiled  ? launch_gemm_planes_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags,
-                                          max_items, F, H, route_down, nullptr)
+                                          max_items, F, H, route_down, nullptr, false)
         : mmq_dn ? launch_mmq_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags, max_items,
                                      F, H, route_down, nullptr, (int)item_cols)
                 : launch_matvec_grouped(dev, kind_down, d_down, nullptr, dn_stride, fused_q, nullptr, items, flags,

@@ -142,3 +142,20 @@ def test_experts_of_a_call_and_of_its_halves(hip, name, H, F, T):
         got = hip.moe_experts(hidden[part], gate, up, down, ids[part], w[part], F, E, kind, kind)
         assert hip.last_route() == "moe_experts_tiled"
         assert np.array_equal(got.view(np.uint32), whole[part].view(np.uint32))
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("H,F,T", [(1024, 768, 2100), (2048, 512, 2077)])
+def test_gated_product_in_the_gemm(hip, name, H, F, T):
+    """The call whose GEMM forms the gated product against the one that stores gate and up outputs and forms it when they are
+    packed (a call that looks at the stages): the same sums through the same function, bit for bit. Items of one to 64 routes."""
+    E, k, kind = 6, 2, KINDS[name]
+    gate, up = (hip.quantize_weights(kind, gaussian(840 + i, (E * F, H), 0.02)) for i in range(2))
+    down = hip.quantize_weights(kind, gaussian(842, (E * H, F), 0.02))
+    hidden, rng = gaussian(843, (T, H)), np.random.default_rng(844)
+    ids = np.argsort(rng.random((T, E)) * np.array([1, 1, 1, 2, 3, 6]), axis=1)[:, :k].astype(np.int32)
+    w = np.abs(gaussian(845, (T, k)))
+    got = hip.moe_experts(hidden, gate, up, down, ids, w, F, E, kind, kind)
+    assert hip.last_route() == "moe_experts_tiled"
+    stages = hip.moe_experts_probe(hidden, gate, up, down, ids, w, F, E, kind, kind)
+    assert np.array_equal(got.view(np.uint32), stages["out"].view(np.uint32))
