@@ -1373,7 +1373,7 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 // one reads it once per 128 / group tokens. Two sequences x 512 tokens over 2048 cached ones, 32 / 8 heads of 128, BFLOAT16 cache,
 // whole call: 756 us per token; 249 with four wavefronts that own 32 positions at a time and the table entry read in front of
 // each tile; 166 with 64 at a time (one wavefront per SIMD: scores, softmax and output one after the other); 148 with
-// eight wavefronts; 138 - 140 now that one wavefront locates a tile's rows for all and the values' infinities are looked for by two
+// eight wavefronts; 138 - 147 (by card) now that one wavefront locates a tile's rows for all and the values' infinities are looked for by two
 // maxima per word. Bound by the issue of vector instructions (about 1300 per SIMD and tile, 5200 clocks, beside 3070 of
 // the matrix cores); 20 us are the start and the end (the query's parts 6, the join of the halves 4, the first tile 8).
 // Error against 64 bits there: 3.6e-7 per token, 2.2e-7 here.

@@ -37,8 +37,8 @@
 // (LOOP) keeps as many workgroups as the chip holds and has each request the first codes and weights of its next tile during
 // the last block of this one: the calls above 384 -> 373 and 464 -> 455, 1500 tokens of 64 Q5_K experts of 512 228 -> 212. The
 // gate and up projections share a tile (GLU: 64 rows of each), so that their gated product is formed from sums that are still in
-// registers: 50 MB written and read in the place of 100, 376 -> 350 us for the Q4_K call, its gated packing 28 -> 20 us. Linears of
-// 16 blocks and more lose up to 4 % to the registers it takes.
+// registers: 50 MB written and read in the place of 100, 376 -> 350 us for the Q4_K call, its packing 28 -> 19 us. (Linears
+// of 16 blocks and more would lose up to 4 % to the registers that LOOP takes.)
 #include "mh_rows.h"
 
 #include <type_traits>
