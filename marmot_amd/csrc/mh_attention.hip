@@ -1373,7 +1373,7 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 // one reads it once per 128 / group tokens. Two sequences x 512 tokens over 2048 cached ones, 32 / 8 heads of 128, BFLOAT16 cache,
 // whole call: 756 us per token; 249 with four wavefronts that own 32 positions at a time and the table entry read in front of
 // each tile; 166 with 64 at a time (one wavefront per SIMD: scores, softmax and output one after the other); 148 with
-// eight wavefronts; 138 - 147 (by card) now that one wavefront locates a tile's rows for all and the values' infinities are looked for by two
+// eight wavefronts; 136 - 145 (by card) now that one wavefront locates a tile's rows for all and the values' infinities are looked for by two
 // maxima per word. Bound by the issue of vector instructions (about 1300 per SIMD and tile, 5200 clocks, beside 3070 of
 // the matrix cores); 20 us are the start and the end (the query's parts 6, the join of the halves 4, the first tile 8).
 // Error against 64 bits there: 3.6e-7 per token, 2.2e-7 here.
@@ -1863,6 +1863,9 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
         __syncthreads();
         for (uint32_t tile = begin; tile <= end; ++tile) {
             const bool more = tile + 1u < end;
+            if (half == 0u && tile < end) {
+                scores(tile, count, mask);
+            }
             if (more) {
                 request(tile + 1u);
                 if (wave == 0u) {
@@ -1870,21 +1873,20 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
                     entry = table_entry(tile + 3u);
                 }
             }
-            if (half == 0u && tile < end) {
-                scores(tile, count, mask);
-            }
             if (half == 0u ? tile < end : tile != begin) {
                 output(count - half, half == 0u ? now : before);
             }
-            if (half != 0u && tile < end) {
-                scores(tile, count, mask);
-            }
-            if (tile == end) {
-                break;  // (the stores of the next sequence's first tile go to other buffers than the last output's)
-            }
+            // (the requests behind half 0's scores and the stores in front of half 1's: 1 - 2.5 % of long histories)
+            const uint64_t mask_now = mask;
             if (more) {
                 store(count + 1u, after(now));
                 mask = mask_next;
+            }
+            if (half != 0u && tile < end) {
+                scores(tile, count, mask_now);
+            }
+            if (tile == end) {
+                break;  // (the stores of the next sequence's first tile go to other buffers than the last output's)
             }
             ++count;
             before = now;
