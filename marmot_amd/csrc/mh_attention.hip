@@ -1758,24 +1758,33 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
             }
             lsum = lsum * corr + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
             const uint8_t *vt = lds + values_at;
-            uint32_t wp[2][PARTS][4];
+            // The weights as operands, in parts; or as they are, weight r in word 8 (r / 8) + r % 8 of the first two parts, for a tile with
+            // a value that is not finite: two FLOAT16 parts hold nothing below 2^-39, and 0 x infinity is not what a small weight gives
+            uint32_t wp[2][PARTS][4] = {};
+            if (odd) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+                for (int r = 0; r < 16; ++r) {
+                    wp[r >> 3][(r >> 2) & 1][r & 3] = __float_as_uint(w[r]);
+                }
+            } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float a = w[8 * i + 2 * e], b = w[8 * i + 2 * e + 1];
+                for (int i = 0; i < 2; ++i) {
 #pragma unroll
-                    for (int part = 0; part < PARTS; ++part) {
-                        if constexpr (BF16) {  // eight bits at a time, cut off: the third part is exact
-                            const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
-                            wp[i][part][e] = __builtin_amdgcn_perm(bb, ab, 0x07060302u);
-                            a -= __uint_as_float(ab & 0xFFFF0000u);
-                            b -= __uint_as_float(bb & 0xFFFF0000u);
-                        } else {
-                            const uint16_t ah = f2h(a), bh = f2h(b);
-                            wp[i][part][e] = (uint32_t)ah | ((uint32_t)bh << 16);
-                            a -= h2f(ah);
-                            b -= h2f(bh);
+                    for (int e = 0; e < 4; ++e) {
+                        float a = w[8 * i + 2 * e], b = w[8 * i + 2 * e + 1];
+#pragma unroll
+                        for (int part = 0; part < PARTS; ++part) {
+                            if constexpr (BF16) {  // eight bits at a time, cut off: the third part is exact
+                                const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
+                                wp[i][part][e] = __builtin_amdgcn_perm(bb, ab, 0x07060302u);
+                                a -= __uint_as_float(ab & 0xFFFF0000u);
+                                b -= __uint_as_float(bb & 0xFFFF0000u);
+                            } else {
+                                const uint16_t ah = f2h(a), bh = f2h(b);
+                                wp[i][part][e] = (uint32_t)ah | ((uint32_t)bh << 16);
+                                a -= h2f(ah);
+                                b -= h2f(bh);
+                            }
                         }
                     }
                 }
@@ -1812,18 +1821,12 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
                     for (uint32_t i = 0; i < 32u; ++i) {
                         // position i: weight 4 (i / 8) + i % 4 of lane half (i / 4) % 2
                         const uint32_t at = 4u * (i >> 3) + (i & 3u);
-                        float mine_w = 0.0f;
+                        uint32_t mine_w = 0;
 #pragma unroll
-                        for (int part = PARTS - 1; part >= 0; --part) {
-                            uint32_t word = 0;
-#pragma unroll
-                            for (int r = 0; r < 8; ++r) {
-                                word = (uint32_t)r == at >> 1 ? wp[r >> 2][part][r & 3] : word;
-                            }
-                            const uint16_t bits = (uint16_t)(word >> (16u * (at & 1u)));
-                            mine_w += BF16 ? pa_bf2f(bits) : h2f(bits);
+                        for (int r = 0; r < 16; ++r) {
+                            mine_w = (uint32_t)r == at ? wp[r >> 3][(r >> 2) & 1][r & 3] : mine_w;
                         }
-                        const float wi = __shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u)));
+                        const float wi = __uint_as_float(__shfl(mine_w, (int)(n + 32u * ((i >> 2) & 1u))));
                         if ((see >> i) & 1u) {
                             const uint32_t chunk = 4u * half + 2u * (i >> 4) + ((i >> 2) & 1u), in = 8u * ((i >> 3) & 1u) + 2u * (i & 3u);
 #pragma unroll

@@ -222,6 +222,60 @@ def test_prompt_tiles(prompt_hip, oracle, hq, hkv, block_size, seqs, shuffle, he
     assert np.max(np.abs(g[rest].astype(np.float64) - b[rest])) <= TOLERANCE[act] * vmax, "rows beside the infinite value"
 
 
+def _chosen_scores(seed, seqs, scores, head_dim, act, kv):
+    """A case whose position p has the score scores[p] (0 if absent) plus small noise: dimension 0 of the queries is
+    sqrt(head_dim) and that of the keys the score; values of dimension 5 are 0."""
+    case = make_case(seed, seqs, num_q_heads=8, num_kv_heads=2, head_dim=head_dim, block_size=16, act=act, kv=kv, layers=1,
+                     layer_idx=0, shuffle_tokens=False)
+    q, kn, vn, ck, cv = (to_f32(case[n], t).copy() for n, t in (("q", act), ("k_new", act), ("v_new", act), ("kv_k", kv), ("kv_v", kv)))
+    q *= np.float32(0.25)
+    q[..., 0] = np.sqrt(head_dim)
+    kn[..., 0] = ck[..., 0] = vn[..., 5] = cv[..., 5] = 0.0
+    rows = {(int(s), int(p)): t for t, (s, p, _, _) in enumerate(case["token_meta"])}
+    slots = list(dict.fromkeys(int(s) for s, _, _, _ in case["token_meta"]))
+
+    def place(seq, pos):
+        """Views of the key and value row of a position, of the new rows or of the cache."""
+        if (seq, pos) in rows:
+            return kn[rows[seq, pos]], vn[rows[seq, pos]]
+        b = int(case["block_table"][seq, pos // 16])
+        return ck[b, 0, :, pos % 16], cv[b, 0, :, pos % 16]
+
+    for seq in slots:
+        for pos, score in scores.items():
+            place(seq, pos)[0][:, 0] = score
+
+    def finish():
+        return dict(case, q=to_storage(q, act), k_new=to_storage(kn, act), v_new=to_storage(vn, act), kv_k=to_storage(ck, kv),
+                    kv_v=to_storage(cv, kv))
+
+    return case, slots, place, q, finish
+
+
+@pytest.mark.parametrize("act,kv", [("f32", "f16"), ("f32", "bf16")])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("pos", [5, 37, 70, 100])  # either half of a tile of the history, and of one with new rows
+def test_prompt_tiles_infinite_value_with_a_small_weight(prompt_hip, oracle, pos, head_dim, act, kv):
+    """A value of +inf whose score is 40 below the others: its weight, about 4e-18, is far below what two FLOAT16 parts hold, yet
+    the output is +inf and no NaN. A finite value of its tile, 26 below, keeps a weight of FLOAT32's precision: the score
+    is good to 26 * 2^-21 (the query in two FLOAT16 or three BFLOAT16 parts, FLOAT32 sums), hence 1e-4."""
+    near = pos + 2
+    case, slots, place, _, finish = _chosen_scores(760 + pos, [(90, 70)], {pos: -40.0, near: -26.0}, head_dim, act, kv)
+    place(slots[0], pos)[1][:, 3] = np.inf
+    place(slots[0], near)[1][:, 5] = 1.0
+    case = finish()
+    got, _, _ = run_hip(prompt_hip, case)
+    assert prompt_hip.last_route() == "paged_attention_tiles"
+    ref, _, _ = run_oracle(oracle, case)
+    sees, sees_near = case["token_meta"][:, 1] >= pos, case["token_meta"][:, 1] >= near
+    assert np.all(np.isposinf(ref[sees][:, :, 3])) and np.all(np.isposinf(got[sees][:, :, 3]))
+    assert np.all(np.isfinite(got[~sees])) and not got[~sees_near][:, :, 5].any()
+    small, want = got[sees_near][:, :, 5].astype(np.float64), ref[sees_near][:, :, 5].astype(np.float64)
+    assert np.all(want > 1e-15) and np.max(np.abs(small / want - 1)) <= 1e-4
+    rest = np.arange(head_dim) != 3
+    assert np.max(np.abs(got[:, :, rest].astype(np.float64) - ref[:, :, rest])) <= TOLERANCE[act] * np.abs(ref[:, :, rest]).max()
+
+
 @pytest.mark.parametrize("kv,act", [("f16", "f32"), ("f16", "bf16"), ("bf16", "f32")])
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("tiles", [True, False])
