@@ -1747,8 +1747,11 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
             }
             big = fmaxf(big, pa_xor32(big)) * unit;
             const float m_new = fmaxf(m, big);
-            const float corr = m == -INFINITY ? 0.0f : pa_exp(m - m_new);
-            const float m_use = m_new == -INFINITY && see == 0u ? 0.0f : m_new;  // (a row that sees nothing yet)
+            // While every score so far is -inf, weights are 0, and a sum above 0 says that there were scores at all (then the output is
+            // NaN if it stays so over the whole row: exp(-inf + inf)); the first larger score drops it.
+            const float corr = m == m_new ? 1.0f : pa_exp(m - m_new);
+            const bool lost = m_new == -INFINITY;
+            const float m_use = lost ? 0.0f : m_new;
             m = m_new;
             float w[16], sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -1756,7 +1759,7 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
                 w[r] = pa_exp(__builtin_fmaf(s[r], unit, -m_use)) * UNIT;
                 sum[r & 3] += w[r];
             }
-            lsum = lsum * corr + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
+            lsum = lsum * corr + ((sum[0] + sum[1]) + (sum[2] + sum[3])) + (lost && see != 0u ? 1.0f : 0.0f);
             const uint8_t *vt = lds + values_at;
             // The weights as operands, in parts; or as they are, weight r in word 8 (r / 8) + r % 8 of the first two parts, for a tile with
             // a value that is not finite: two FLOAT16 parts hold nothing below 2^-39, and 0 x infinity is not what a small weight gives
@@ -1921,7 +1924,7 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
         __syncthreads();
         const float2 other = ml[tid ^ 256u];
         const float m_all = fmaxf(m, other.x);
-        const float f_own = m == -INFINITY ? 0.0f : pa_exp(m - m_all), f_other = other.x == -INFINITY ? 0.0f : pa_exp(other.x - m_all);
+        const float f_own = m == m_all ? 1.0f : pa_exp(m - m_all), f_other = other.x == m_all ? 1.0f : pa_exp(other.x - m_all);
         lsum = __builtin_fmaf(other.y, f_other, lsum * f_own);
         m = m_all;
         const float4 *from = (const float4 *)lds + (wave ^ 4u) * (HD / 64 * 256u) + lane;
@@ -1949,7 +1952,7 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
             part[0] = m;
             part[1] = lsum;
         }
-        if (m == -INFINITY && !bad) {  // a share that holds nothing: k_pa_merge leaves its sums alone
+        if (m == -INFINITY && !bad) {  // a share that holds nothing but scores of -inf, if any: k_pa_merge leaves its outputs alone
             return;
         }
 #pragma unroll
@@ -1963,7 +1966,7 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
         }
         return;
     }
-    const float inv = bad ? __uint_as_float(0x7fc00000u) : (lsum > 0.0f ? 1.0f / lsum : 0.0f);
+    const float inv = bad || (m == -INFINITY && lsum > 0.0f) ? __uint_as_float(0x7fc00000u) : (lsum > 0.0f ? 1.0f / lsum : 0.0f);
     const size_t base = (size_t)t * p.out_stride[0] + (size_t)qh * p.out_stride[1];
 #pragma unroll
     for (int d = 0; d < DB / 2; ++d) {
@@ -2015,13 +2018,13 @@ __global__ __launch_bounds__(256) void k_pa_merge(const PaParams p) {
     const size_t out_base = (size_t)t * p.out_stride[0] + (size_t)qh * p.out_stride[1];
     for (uint32_t d = threadIdx.x; d < p.head_dim; d += blockDim.x) {
         float o = 0.0f, total = 0.0f;
-        bool bad = false;  // a share saw a NaN score
+        bool bad = false;  // a share saw a NaN score, or all of them none but -inf (k_pa_prompt: a sum beside that maximum)
         for (uint32_t z = 0; z < splits; ++z) {
-            bad = bad || s_tot[z] != s_tot[z];
+            bad = bad || s_tot[z] != s_tot[z] || (TILES && big == -INFINITY && s_tot[z] > 0.0f);
         }
         if (big != -INFINITY) {
             for (uint32_t z = 0; z < splits; ++z) {
-                const bool empty = TILES && s_big[z] == -INFINITY;  // (k_pa_prompt leaves the sums of such a share unwritten)
+                const bool empty = TILES && s_big[z] == -INFINITY;  // (k_pa_prompt leaves the outputs of such a share unwritten)
                 const float f = s_big[z] == -INFINITY ? 0.0f : pa_exp(s_big[z] - big);
                 total = __builtin_fmaf(s_tot[z], f, total);
                 const float v = part[(size_t)z * (p.head_dim + 2u) + 2 + d];

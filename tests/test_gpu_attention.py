@@ -276,6 +276,40 @@ def test_prompt_tiles_infinite_value_with_a_small_weight(prompt_hip, oracle, pos
     assert np.max(np.abs(got[:, :, rest].astype(np.float64) - ref[:, :, rest])) <= TOLERANCE[act] * np.abs(ref[:, :, rest]).max()
 
 
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("lost,hist,new", [
+    ([32], 0, 70),              # the one position that token 32 sees of its tile's second half
+    (range(32), 0, 40),         # tokens 0 .. 31 see nothing else, the later ones the second half
+    (range(64, 96), 80, 40),    # a half of a later tile
+    (range(128), 0, 140),       # whole tiles: tokens up to 127 see nothing else
+    (range(1500), 1400, 140),   # whole shares of a split history
+    (range(1024, 1560), 1480, 80),  # (the last share)
+])
+def test_prompt_tiles_scores_of_minus_infinity(prompt_hip, lost, hist, new, head_dim, kv):
+    """Scores that overflow to -inf (a query channel of 1e36 against keys of -60000) weigh nothing beside finite ones, wherever
+    they lie; a token that sees nothing else has no maximum to subtract and its output is NaN, as in the reference. The other
+    scores are 0, so every output is the mean of the values in between."""
+    case, slots, place, q, finish = _chosen_scores(780 + hist, [(hist, new)], {p: -60000.0 for p in lost if p < hist + new}, head_dim,
+                                                   "f32", kv)
+    q[...] = 0.0
+    q[..., 0] = 1e36
+    case = finish()
+    got, _, kv_v = run_hip(prompt_hip, case)
+    assert prompt_hip.last_route() == "paged_attention_tiles"
+    v = to_f32(kv_v, kv).astype(np.float64)
+    pos = np.arange(hist + new)
+    rows = v[case["block_table"][slots[0], pos // 16], 0, :, pos % 16]  # [position][kv head][dimension]
+    seen = ~np.isin(pos, list(lost))
+    for t, end in enumerate(case["token_meta"][:, 1].astype(int)):
+        use = rows[:end + 1][seen[:end + 1]]
+        if len(use) == 0:
+            assert np.all(np.isnan(got[t])), f"token {t} sees nothing but -inf"
+        else:
+            want = np.repeat(use.mean(axis=0), 4, axis=0)
+            assert np.max(np.abs(got[t] - want)) <= TOLERANCE["f32"] * np.abs(v).max(), f"token {t}"
+
+
 @pytest.mark.parametrize("kv,act", [("f16", "f32"), ("f16", "bf16"), ("bf16", "f32")])
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("tiles", [True, False])
