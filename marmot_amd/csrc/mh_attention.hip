@@ -1397,8 +1397,8 @@ struct PaPromptLds {
     static constexpr uint32_t V0 = 2 * K;          // two buffers of keys, three of values
     static constexpr uint32_t Q = V0 + 3 * V;      // small parts of the query: [part][16 dimensions][wavefront][lane] x 16 bytes
     static constexpr uint32_t QPARTS = HD == 128 ? (BF16 ? 2 : 1) : 0;
-    static constexpr uint32_t TOKENS = Q + QPARTS * PA_PROMPT_ROWS * HD * 2;  // sequence, length, longest history: 128 words each; five words
-    static constexpr uint32_t ROWS = TOKENS + (3 * PA_PROMPT_ROWS + 8) * 4;  // two tiles: places of 64 rows; then which of them exist
+    static constexpr uint32_t TOKENS = Q + QPARTS * PA_PROMPT_ROWS * HD * 2;  // sequence, length, longest history: 128 words each; nine words
+    static constexpr uint32_t ROWS = TOKENS + (3 * PA_PROMPT_ROWS + 12) * 4;  // two tiles: places of 64 rows; then which of them exist
     static constexpr uint32_t BYTES = ROWS + (2 * 64 + 2) * 8;
     static constexpr uint32_t MAIL = PA_PROMPT_WAVES * HD / 64 * 4096;  // at the end: outputs, then maximum and sum of every lane
     static_assert(MAIL + PA_PROMPT_WAVES * 512 <= Q, "the mail fits the stages");
@@ -1432,7 +1432,8 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
     constexpr uint32_t NONE = 0xFFFFFFFFu;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint32_t *s_seq = (uint32_t *)(lds + L::TOKENS), *s_len = s_seq + PA_PROMPT_ROWS, *s_longest = s_len + PA_PROMPT_ROWS;
-    uint32_t *s_odd = s_longest + PA_PROMPT_ROWS;  // per buffer: 1 + number of its tile if that holds a value that is not finite
+    uint64_t *s_firsts = (uint64_t *)(s_longest + PA_PROMPT_ROWS);  // which tokens are the first of their sequence
+    uint32_t *s_odd = (uint32_t *)(s_firsts + 2);  // per buffer: 1 + number of its tile if that holds a value that is not finite
     const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 31u, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), rows = wave & 3u, half = wave >> 2;
     const uint32_t tt = p.tile_tokens, t0 = (gridDim.x - 1u - blockIdx.x) * tt, kvh = blockIdx.y;  // long histories first
@@ -1472,7 +1473,11 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
                 longest = eq && len[e] > longest ? len[e] : longest;
             }
         }
-        s_longest[tid] = mine && first ? longest : 0u;
+        s_longest[tid] = longest;
+        const uint64_t firsts = __builtin_amdgcn_ballot_w64(mine && first);
+        if (lane == 0) {
+            s_firsts[wave] = firsts;
+        }
     }
     __syncthreads();
 
@@ -1608,7 +1613,21 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
     uint2 vreg[4];
     uint64_t mask_next = 0;  // positions of the requested tile that exist
 
-    for (uint32_t first = 0; first < tt; ++first) {
+    auto uniform64 = [](uint64_t v) {
+        return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+               (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32;
+    };
+    // (a look at every token instead is a chain of as many reads from LDS: 3 of the 30 us of 512 fresh tokens, 128 of them in a tile)
+    uint64_t firsts = uniform64(s_firsts[0]), firsts_high = uniform64(s_firsts[1]);
+    while ((firsts | firsts_high) != 0u) {
+        uint32_t first;
+        if (firsts != 0u) {
+            first = (uint32_t)__builtin_ctzll(firsts);
+            firsts &= firsts - 1u;
+        } else {
+            first = 64u + (uint32_t)__builtin_ctzll(firsts_high);
+            firsts_high &= firsts_high - 1u;
+        }
         const uint32_t longest = __builtin_amdgcn_readfirstlane(s_longest[first]);
         if (longest == 0u) {
             continue;
@@ -1641,9 +1660,7 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
         };
         auto request = [&](uint32_t tile) {
             const uint32_t buffer = (tile - begin) & 1u;
-            const uint64_t exist = s_rows[128u + buffer];
-            mask_next = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)exist) |
-                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(exist >> 32)) << 32;
+            mask_next = uniform64(s_rows[128u + buffer]);
             uint32_t tid = threadIdx.x;
             asm volatile("" : "+v"(tid));  // (places formed from it here, not kept throughout: there are no registers for them)
             const uint64_t *k_rows = s_rows + 64u * buffer + tid / (HD / 8);
