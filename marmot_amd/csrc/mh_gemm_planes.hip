@@ -4,7 +4,7 @@
 // Per 256-value block the reference forms (cpu_vec_dot_q{4,5,6}_k_q8_k, src/backends/cpu/ops/matmul/quantized/
 // vec_dot_impl.h:689-860) y += a.d * (w.d * isum - w.dmin * msum) with isum = sum_j sc_j * (q_j . a_j) and msum = sum_j mn_j *
 // (sum of a over sub-block j). sc * q does not fit int8, but two numbers that do make it up: Q4_K q * (sc & 7) and q * (sc >> 3)
-// (at most 105); Q5_K (0 .. 1953) and Q6_K (-4096 .. 4064) the product itself as 256 * h + l, its high byte and its low byte
+// (at most 105); Q5_K (0 .. 1953) and Q6_K (-4064 .. 4096) the product itself as 256 * h + l, its high byte and its low byte
 // as signed numbers. One chain of v_mfma_i32_32x32x32_i8 per plane over the whole block gives isum = X + 2^SHIFT * Y exactly
 // (below 2^27), in the matrix time of one fp16 operand, since the int8 instructions run at twice the rate. Beside fp16
 // operands (mh_gemm_int16.hip, which need two for Q6_K) the activations stay the bytes they are packed as: half the reads
@@ -24,8 +24,9 @@
 // KG = 2: eight wavefronts, two K groups with buffers of their own that take every second block, one stage apart (one does its
 // fp32 step while the other multiplies), sums joined in LDS at the end: for calls that have one tile per compute unit, which
 // would leave a SIMD one wavefront. KG = 4 halves the tile's rows besides (RG = 2 wavefronts of them, four K groups): a call of
-// half a chip of 128 x 64 tiles, the k and v projections of a prompt, takes a whole chip of these. KG = 1: four wavefronts, two or three workgroups per compute unit; the last tiles of a
-// ragged token count run on as many of the C token tiles as hold a token.
+// half a chip of 128 x 64 tiles, the k and v projections of a prompt, takes a whole chip of these. KG = 1: four wavefronts, two
+// or three workgroups per compute unit; the last tiles of a ragged token count run on as many of the C token tiles as hold a
+// token.
 // Measured (us of whole calls in a row, the quantization of 6 - 17 included; before: the best of the kernels of
 // mh_gemm_int16.hip and mh_gemm_i8.hip; tokens x K x M):
 //          1024 x 14336 x 4096   1000 x 4096 x 14336   1024 x 4096 x 4096   300 x 4096 x 4096
@@ -945,34 +946,52 @@ static bool planes_kind(int kind) {
 
 // Which form (10 C + KG), or none (0), by the tiles a call has. The kernels of mh_gemm_i8.hip split K over workgroups where
 // tiles are few, which pays the partial sums and wins while the chip is mostly empty; K groups in one workgroup want one
-// tile per compute unit, and beyond that workgroups share one (us of whole calls, other kernels / forms; 24: 64 rows, four K
-// groups):
-//   64 x 64, up to a tile     Q6_K 64 tiles 100 x 4096 x 2048 22.1 / (24) 22.8   80, 300 x 4096 x 1024 27.7 / 24.3   128, 128 x
-//   per compute unit          14336 x 4096 65 / 58   256, 1024 x 4096 x 1024 48 / (22) 42, (24) 29   256 x 14336 x 4096 - / 104, 62
-//                             Q4_K 64, 64 x 4096 x 4096 17.7 / (24) 18.4   80, 300 x 4096 x 1024 20.9 / 20.4   88, 64 x 2048 x
-//                             5632 16.3 / 13.9   128, 128 x 4096 x 4096 21.3 / 19.5   128 x 8192 x 4096 27.3 / 30.0   192, 192 x
-//                             8192 x 4096 37 / 32   160, 300 x 14336 x 2048 45 / 49   192, 192 x 14336 x 4096 52 / 48
-//                             (320, 300 x 4096 x 4096: Q6_K (22) 37.5, (24) 42.6; Q4_K 30.1, 35.1)
-//   Q6_K, 64 tokens a tile    104 tiles 800 x 4096 x 1024 47 / (22) 42
-//   Q4_K, the same            160, 300 x 4096 x 4096 31.5 / (22) 30.3
-//                             224, 128 x 4096 x 14336 31.9 / (22) 30.9  256, 512 x 14336 x 4096 100 / (22) 91
-//   128 tokens a tile         Q4_K 192 tiles 300 x 1024 x 8192 22.8 / (42) 20.2   256, 1024 x 14336 x 4096 187 / (42) 142
-//   more tiles than units     Q4_K 308, 800 x 2048 x 5632 49 / (42) 50, (41) 46, (21) 40   784, 800 x 4096 x 14336 167 / 153, 145, 130
-//                             Q6_K 308, 77 / (42) 57, (41) 53, (21) 52   896, 1024 x 4096 x 14336 303 / 186, 178, 204
+// tile per compute unit, and beyond that workgroups share one. Measured as time of the form over time of those kernels (Q6_K from
+// form 42 on: of the fp16 tile that was there), whole calls in a row, about 400 sizes per format; tiles on 256 compute units:
+//   24, 64 x 64, four K groups, up to a tile per compute unit. It takes a whole tile's time for any number of tokens in it.
+//     Q6_K   up to 16 blocks from 65 tiles on 0.95 - 0.55, also at 17 tokens (66 tiles of 4 / 8 / 16 blocks 0.70, 0.83, 0.95)
+//            17 - 23 blocks at 66 tiles 0.94 at 64 tokens, 1.03 at 17; 24 and more 1.03 - 1.31 (80 tiles 1.00 - 1.10), 88 tiles 0.88 - 0.98
+//     Q4_K   up to 8 blocks 0.95 - 0.66. 16 blocks, 66 tiles with 33 / 64 tokens 1.08 / 0.99, 96 with 33 / 48 / 80 1.02, 1.00, 1.02,
+//            128 with 33 / 80 0.98, 0.98; 12 blocks 1.01 / 0.92 and 0.93; beyond 16 blocks 160 tiles 1.03 - 1.09, 172 0.90
+//     Q5_K   up to 8 blocks 0.98 - 0.65. 16 blocks, 66 tiles 1.12 / 1.03, 96 1.04, 1.01, 1.04, 128 1.01, 0.99; 12 blocks
+//            1.09 / 0.98 and 0.98; beyond 16 blocks 160 tiles 1.00 - 1.04, 172 0.84
+//            (One size goes the other way: 1024 x 4096 x 512, 128 tiles, 1.02 for both)
+//   22, 128 x 64, two K groups, up to a tile per compute unit
+//     Q6_K   0.77 (4 blocks) - 0.50
+//     Q4_K   144 - 256 tiles of 4 / 8 / 10 / 12 / 14 / 16 blocks 1.14 - 1.06, 1.06 - 1.02, 1.04 - 1.01, 1.03 - 1.00, 1.02 - 0.99,
+//            1.01 - 0.98, 32 and more 0.98 - 0.91
+//     Q5_K   4 / 5 / 6 / 8 blocks 1.07 - 1.02, 1.04 - 1.00, 1.01 - 0.98, 0.99 - 0.96, 16 and more 0.93 - 0.85
+//            (Both: up to three fifths of the compute units the split of more than 8 blocks fills the chip better)
+//   42, 128 x 128, two K groups, up to a tile per compute unit (130 - 256 of them, 260 - 512 of 128 x 64)
+//     Q6_K   0.76 - 0.46; the forms with one K group over it: 41 1.19 - 1.42, 21 1.01 - 1.54
+//     Q4_K   0.96 - 0.67; 41 1.18 - 1.39, 21 1.00 - 1.26 but for 4 blocks (0.96 - 1.04) and 140 tokens (two tiles for little more
+//            than one: 0.88 of 4 blocks, 0.91 of 16)
+//     Q5_K   0.93 - 0.59; 41 1.17 - 1.37, 21 1.03 - 1.41 but for 140 and 200 tokens of 4 blocks (0.91, 0.95)
+//   more tiles: Q6_K 41, 0.91 - 0.52 (21 against it 0.86 at 258 - 344 tiles of 128 x 128 and few blocks, 0.95 - 1.25 else); Q4_K, Q5_K 21,
+//            0.99 - 0.68 (41 against it 0.97 - 1.21 and, Q5_K, 0.87 - 1.16)
 // Q4_K and Q5_K: where mh_gemm_int16.hip has a form of 256 x 128 for the call, that one is as fast or faster (1024 x 4096 x 14336
-// Q4_K 156 against 155, Q5_K 162 against 169; 1024 x 1024 x 8192 31 against 35).
+// Q4_K 156 us against 155, Q5_K 162 against 169; 1024 x 1024 x 8192 31 against 35).
 static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t nb, size_t weights) {
     const size_t cus = (size_t)dev->props.multiProcessorCount;
-    const size_t rows = (M + 127) / 128 * weights;
-    const size_t small = (N + 63) / 64 * rows, large = (N + 127) / 128 * rows;
-    const size_t least = (N + 63) / 64 * ((M + 63) / 64) * weights;
+    const size_t rows = (M + 127) / 128 * weights, rows64 = (M + 63) / 64 * weights;
+    const size_t small = (N + 63) / 64 * rows, large = (N + 127) / 128 * rows, least = (N + 63) / 64 * rows64;
+    const bool q6 = kind == MARMOT_HIP_KIND_Q6_K, q5 = kind == MARMOT_HIP_KIND_Q5_K;
     if (least <= cus) {
-        return 4 * least > cus && (kind == MARMOT_HIP_KIND_Q6_K || nb <= 16 || 3 * least > 2 * cus) ? 24 : 0;
+        const size_t used = N * rows64;  // 64 per tile if tokens fill them
+        bool takes;
+        if (q6) {
+            takes = nb <= 16 || 3 * least > cus || (nb < 24 && used >= 8 * cus);
+        } else if (nb > 16) {
+            takes = 3 * least > 2 * cus;
+        } else {  // (16 blocks: from 16 and 19 tokens of a row tile per compute unit on)
+            takes = nb <= 8 || 2 * used >= cus * (3 * nb - (q5 ? 10 : 16));
+        }
+        return 4 * least > cus && takes ? 24 : 0;
     }
     if (small <= cus) {
-        return kind != MARMOT_HIP_KIND_Q6_K && nb > 8 && 5 * small <= 3 * cus ? 0 : 22;
+        return q6 || (nb >= (q5 ? 6u : 14u) && (nb <= 8 || 5 * small > 3 * cus)) ? 22 : 0;
     }
-    return large <= cus ? 42 : kind == MARMOT_HIP_KIND_Q6_K ? 41 : 21;
+    return large <= cus ? 42 : q6 ? 41 : 21;
 }
 
 bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights,

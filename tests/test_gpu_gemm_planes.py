@@ -24,14 +24,31 @@ def hip():
 
 
 CASES = [
-    # (kinds, tile, tokens, rows, K)
-    ("q4_k q5_k", "small", 128, 10400, 256),   # two K groups, 64 tokens, the second group without a block
-    ("q4_k q5_k", "small", 97, 12801, 768),    # odd block counts, one row and 33 tokens in the last tiles
+    # (kinds, tile, tokens, rows, K); "other": the kernels of mh_gemm_i8.hip
+    ("q4_k q5_k", "other", 128, 10400, 256),   # few blocks
+    ("q4_k q5_k", "other", 97, 12801, 768),
+    ("q6_k", "small", 128, 10400, 256),        # two K groups, 64 tokens, the second group without a block
+    ("q6_k", "small", 97, 12801, 768),         # odd block counts, one row and 33 tokens in the last tiles
+    ("q4_k", "small", 128, 9900, 3584),
+    ("q4_k", "small", 97, 9985, 3840),
+    ("q4_k", "other", 128, 9900, 3328),        # (13 blocks)
+    ("q5_k", "small", 128, 10400, 1536),
+    ("q5_k", "small", 97, 12801, 1792),
+    ("q5_k", "other", 97, 12801, 1280),        # (5 blocks)
     ("q6_k", "small", 33, 11000, 1280),
     ("q4_k q5_k q6_k", "small", 65, 2085, 256),   # four K groups, 64 rows: three without a block, one token and 37 rows in the last tiles
     ("q4_k q5_k q6_k", "small", 130, 1401, 1280),  # (five blocks, one row in the last tile)
     ("q4_k q5_k q6_k", "small", 257, 3232, 768),   # (255 tiles of 256)
     ("q4_k q5_k q6_k", "small", 129, 3700, 4352),  # (more than 16 blocks)
+    ("q6_k", "small", 17, 8200, 512),              # (17 tokens of two token tiles)
+    ("q6_k", "other", 64, 5440, 6144),             # 85 tiles of 24 blocks
+    ("q6_k", "small", 64, 5441, 6144),             # 86 of them
+    ("q6_k", "other", 17, 4224, 4352),             # 66 tiles of 17 blocks, 17 tokens in each
+    ("q6_k", "small", 32, 4224, 4352),             # 32 tokens
+    ("q4_k", "other", 33, 6144, 4096),             # 16 blocks: 96 tiles of 33 tokens
+    ("q4_k", "small", 33, 8192, 4096),             # 128 of them
+    ("q5_k", "other", 64, 4800, 4096),             # 75 tiles of 64 tokens
+    ("q5_k", "small", 64, 4864, 4096),             # 76 of them
     ("q4_k q5_k q6_k", "large", 257, 6785, 768),   # two K groups, 128 tokens, one token in the last tile
     ("q4_k q5_k q6_k", "large", 380, 8200, 256),
     ("q4_k q5_k", "small", 130, 16600, 512),   # one K group, 64 tokens
@@ -47,12 +64,13 @@ CASES = [
 def test_forms_match_oracle(hip, oracle, name, tile, N, M, K):
     """The bound is the suite's for matmul outputs (1e-3, floored): exact integer block sums on both sides, so only the fp32
     sum over at most five blocks is ordered differently. Arbitrary block bytes: every nibble, scale (Q6_K: -128 among them,
-    products -4096 .. 4064 in two bytes) and minimum."""
+    products -4064 .. 4096 in two bytes) and minimum."""
     kind = KINDS[name]
     blocks = random_valid_blocks(np.random.default_rng(800 + N), kind, M, K)
     x, bias = gaussian(801 + N, (N, K)), gaussian(802, (M,))
     got = hip.linear(x, blocks, kind, M, bias=bias)
-    assert hip.last_route() == f"mmq_{name}_q8_k_{SMALL[name] if tile == 'small' else 'int8_planes_128x128'}"
+    route = {"small": SMALL[name], "large": "int8_planes_128x128", "other": "mfma_tile"}[tile]
+    assert hip.last_route() == f"mmq_{name}_q8_k_{route}"
     assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, bias=bias, threads=16), what=f"{name} {N} x {K} x {M}")
 
 
