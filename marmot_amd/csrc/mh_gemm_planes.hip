@@ -1006,28 +1006,36 @@ bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_
     return planes_form(dev, kind, N, M, K / QK_K, (size_t)weights) != 0;
 }
 
-// The tile of 64 tokens keeps the route name of the kernel that had it before (callers compare names).
+// Rows x tokens of a tile, and the K groups of a workgroup (_k2, _k4)
+#define PLANES_ROUTE(form)                                                                    \
+    (KIND == MARMOT_HIP_KIND_Q4_K ? "mmq_q4_k_q8_k_int8_planes_" form                         \
+     : KIND == MARMOT_HIP_KIND_Q5_K ? "mmq_q5_k_q8_k_int8_planes_" form : "mmq_q6_k_q8_k_int8_planes_" form)
+
 template <int KIND>
-static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsigned weights, const char *small_route,
-                              const char *large_route) {
+static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsigned weights) {
     const int form = planes_form(dev, KIND, p.N, p.M, p.nb, weights);
-    set_route(form >= 40 ? large_route : small_route);
     const unsigned t64 = (unsigned)((p.N + 63) / 64), t128 = (unsigned)((p.N + 127) / 128);
     if (form == 22) {
+        set_route(PLANES_ROUTE("128x64_k2"));
         return planes_launch<KIND, 2, 2>(dev, p, t64, weights);
     }
     if (form == 24) {
+        set_route(PLANES_ROUTE("64x64_k4"));
         return planes_launch<KIND, 2, 4, false, 2>(dev, p, t64, weights);
     }
     if (form == 42) {
+        set_route(PLANES_ROUTE("128x128_k2"));
         return planes_launch<KIND, 4, 2>(dev, p, t128, weights);
     }
     if constexpr (KIND == MARMOT_HIP_KIND_Q6_K) {
+        set_route(PLANES_ROUTE("128x128"));
         return planes_launch<KIND, 4, 1>(dev, p, t128, weights);
     } else {
+        set_route(PLANES_ROUTE("128x64"));
         return planes_launch<KIND, 2, 1>(dev, p, t64, weights);
     }
 }
+#undef PLANES_ROUTE
 
 int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                        size_t M, int out_dtype) {
@@ -1050,14 +1058,11 @@ int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, co
     const unsigned weights = (unsigned)ws.count;
     switch (kind) {
     case MARMOT_HIP_KIND_Q4_K:
-        return planes_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights, "mmq_q4_k_q8_k_int8_planes_128x64",
-                                                        "mmq_q4_k_q8_k_int8_planes_128x128");
+        return planes_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights);
     case MARMOT_HIP_KIND_Q5_K:
-        return planes_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights, "mmq_q5_k_q8_k_fp16_tile_128x64",
-                                                        "mmq_q5_k_q8_k_int8_planes_128x128");
+        return planes_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights);
     default:
-        return planes_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights, "mmq_q6_k_q8_k_fp16_tile_128x64",
-                                                        "mmq_q6_k_q8_k_int8_planes_128x128");
+        return planes_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights);
     }
 }
 

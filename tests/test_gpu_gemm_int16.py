@@ -1,5 +1,6 @@
-"""Tiled GEMM of K-quant weights and Q8_K activations with integer fp16 operands (mh_gemm_int16.hip) against the CPU oracle,
-at the edges of its two tile forms and of the rule that chooses one (x16_form, 256 compute units)."""
+"""Tiled GEMM of Q4_K / Q5_K weights and Q8_K activations with integer fp16 operands (mh_gemm_int16.hip) against the CPU oracle,
+at the edges of its 256 x 128 tile and of the rule that takes it (x16_form, 256 compute units), and the int8 planes beside it
+(mh_gemm_planes.hip) where a Q6_K matrix ends, with several weights in a launch and with FLOAT16 outputs."""
 import numpy as np
 import pytest
 
@@ -23,12 +24,12 @@ def hip():
 
 
 @pytest.mark.parametrize("name,form,N,M,K", [
-    ("q4_k", "256x128", 500, 14335, 512),    # 256 x 128 tiles, the last ones ragged in both directions
-    ("q4_k", "256x128", 449, 14081, 256),    # one block per row, one weight row in the last tile
-    ("q5_k", "256x128", 512, 14336, 768),    # whole tiles, three blocks
-    ("q5_k", "128x64", 129, 16641, 256),    # 128 x 64 tiles, one token and one weight row in the last ones
-    ("q6_k", "128x64", 193, 4229, 1280),    # rows of 5 blocks: every row starts at another offset in its 16-byte piece
-    ("q6_k", "128x64", 64, 16513, 256),     # one token tile, one block
+    ("q4_k", "fp16_tile_256x128", 500, 14335, 512),    # 256 x 128 tiles, the last ones ragged in both directions
+    ("q4_k", "fp16_tile_256x128", 449, 14081, 256),    # one block per row, one weight row in the last tile
+    ("q5_k", "fp16_tile_256x128", 512, 14336, 768),    # whole tiles, three blocks
+    ("q5_k", "int8_planes_128x64", 129, 16641, 256),    # 128 x 64 tiles, one token and one weight row in the last ones
+    ("q6_k", "int8_planes_128x64_k2", 193, 4229, 1280),    # rows of 5 blocks: every row starts at another offset in its 16-byte piece
+    ("q6_k", "int8_planes_128x64_k2", 64, 16513, 256),     # one token tile, one block
 ])
 def test_integer_operand_gemm_matches_oracle(hip, oracle, name, form, N, M, K):
     """The bound is the suite's for matmul outputs (1e-3, floored): exact integer block sums on both sides, so only the
@@ -38,7 +39,7 @@ def test_integer_operand_gemm_matches_oracle(hip, oracle, name, form, N, M, K):
     x = gaussian(701 + N, (N, K))
     bias = gaussian(702, (M,))
     got = hip.linear(x, blocks, kind, M, bias=bias)
-    assert hip.last_route() == f"mmq_{name}_q8_k_fp16_tile_{form}"
+    assert hip.last_route() == f"mmq_{name}_q8_k_{form}"
     assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, bias=bias, threads=16), what=f"{name} {N} x {K} x {M}")
 
 
@@ -76,7 +77,7 @@ def test_end_of_a_q6_k_matrix(hip, oracle, N, M, K):
     try:
         d_w.upload(np.concatenate([blocks.reshape(-1), np.full(64, 0xFF, np.uint8)]))
         hip.linear_d(KIND_Q6_K, d_w, d_x, DT_F32, N, K, M, d_out, DT_F32)
-        assert hip.last_route() == "mmq_q6_k_q8_k_fp16_tile_128x64"
+        assert hip.last_route() == "mmq_q6_k_q8_k_int8_planes_128x64_k2"
         got = d_out.download(np.float32, (N, M))
     finally:
         for b in (d_w, d_x, d_out):
@@ -84,26 +85,28 @@ def test_end_of_a_q6_k_matrix(hip, oracle, N, M, K):
     assert_matmul_parity(got, oracle.matmul(KIND_Q6_K, blocks, x, M, threads=16), what=f"q6_k end {N} x {K} x {M}")
 
 
-@pytest.mark.parametrize("name,form,N,M", [("q4_k", "256x128", 290, 21500), ("q5_k", "256x128", 290, 21500),
-                                           ("q5_k", "128x64", 130, 16600), ("q6_k", "128x64", 130, 6000)])
+@pytest.mark.parametrize("name,form,N,M", [("q4_k", "fp16_tile_256x128", 290, 21500), ("q5_k", "fp16_tile_256x128", 290, 21500),
+                                           ("q5_k", "int8_planes_128x64", 130, 16600),
+                                           ("q6_k", "int8_planes_128x64_k2", 130, 6000)])
 def test_random_blocks(hip, oracle, name, form, N, M):
     """Arbitrary block bytes: every nibble, scale (Q6_K: -128 among them) and minimum."""
     kind, K = KINDS[name], 512
     blocks = random_valid_blocks(np.random.default_rng(730), kind, M, K)
     x = gaussian(731, (N, K))
     got = hip.linear(x, blocks, kind, M)
-    assert hip.last_route() == f"mmq_{name}_q8_k_fp16_tile_{form}"
+    assert hip.last_route() == f"mmq_{name}_q8_k_{form}"
     assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, threads=16), what=f"random blocks {name} {form}")
 
 
-@pytest.mark.parametrize("name,form,N,M", [("q4_k", "256x128", 290, 21500), ("q5_k", "256x128", 290, 21500),
-                                           ("q5_k", "128x64", 130, 16600), ("q6_k", "128x64", 130, 6000)])
+@pytest.mark.parametrize("name,form,N,M", [("q4_k", "fp16_tile_256x128", 290, 21500), ("q5_k", "fp16_tile_256x128", 290, 21500),
+                                           ("q5_k", "int8_planes_128x64", 130, 16600),
+                                           ("q6_k", "int8_planes_128x64_k2", 130, 6000)])
 @pytest.mark.parametrize("large", [False, True])
 def test_block_sums(hip, name, form, N, M, large):
     """One block per row, activation and block scales of 1, minimum scale 0: the output is the integer block sum. Below
-    2^24 it must be exact. Sums of one sign at the largest values go to 2^24.9 (Q5_K 2^25.9, Q6_K 2^26.9): 16 instructions, Q6_K 32,
-    whose roundings are at most one unit in the last place each, and a factor of two for the smaller partial sums of a
-    chain whose parts differ in sign."""
+    2^24 it must be exact. Sums of one sign at the largest values go to 2^24.9 (Q5_K 2^25.9, Q6_K 2^26.9). On int8 planes they are
+    rounded once; on fp16 operands 16 instructions round by at most one unit in the last place each, and a factor of two for
+    the smaller partial sums of a chain whose parts differ in sign."""
     kind, K, rng = KINDS[name], 256, np.random.default_rng(740)
     rows = rng.integers(0, 256, (4, 4096), dtype=np.uint8)  # a few distinct blocks, repeated
     bb = {"q4_k": 144, "q5_k": 176, "q6_k": 210}[name]
@@ -145,26 +148,26 @@ def test_block_sums(hip, name, form, N, M, large):
     d_w, d_p, d_out = hip.to_device(few[np.arange(M) % 4]), hip.to_device(image), hip.alloc(4 * N * M)
     try:
         hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out)
-        assert hip.last_route() == f"mmq_{name}_q8_k_fp16_tile_{form}"
+        assert hip.last_route() == f"mmq_{name}_q8_k_{form}"
         got = d_out.download(np.float32, (N, M))
     finally:
         for b in (d_w, d_p, d_out):
             b.free()
     want = want[:, np.arange(M) % 4]
-    if large:
-        # (a unit in the last place is at most 2^-23 of the value; Q6_K accumulates in quarters, the same relative size)
-        assert np.max(np.abs(got - want) / np.abs(want)) <= 2 * (32 if name == "q6_k" else 16) * 2.0 ** -23
+    if large and form.startswith("fp16"):
+        # (a unit in the last place is at most 2^-23 of the value)
+        assert np.max(np.abs(got - want) / np.abs(want)) <= 2 * 16 * 2.0 ** -23
     else:
         assert np.array_equal(got, want.astype(np.float32))
 
 
-@pytest.mark.parametrize("name,form,N,M,K", [("q4_k", "256x128", 300, 10752, 256), ("q6_k", "128x64", 130, 3000, 512)])
+@pytest.mark.parametrize("name,form,N,M,K", [("q4_k", "fp16_tile_256x128", 300, 10752, 256), ("q6_k", "int8_planes_128x64_k2", 130, 3000, 512)])
 def test_two_weights_in_one_launch(hip, oracle, name, form, N, M, K):
     kind = KINDS[name]
     a, b = (hip.quantize_weights(kind, gaussian(750 + i, (M, K), 0.02)) for i in range(2))
     x = gaussian(752, (N, K))
     got = hip.linear_dual(x, a, b, kind, M)
-    assert hip.last_route() == f"mmq_{name}_q8_k_fp16_tile_{form}"
+    assert hip.last_route() == f"mmq_{name}_q8_k_{form}"
     for g, w in zip(got, (a, b)):
         assert_matmul_parity(g, oracle.matmul(kind, w, x, M, threads=16), what=f"two weights {name}")
 
@@ -179,7 +182,7 @@ def test_three_weights_and_float16_outputs(hip, oracle, dtype):
     biases = [gaussian(764, (M,)).astype(dtype), None, gaussian(765, (M,)).astype(dtype)]
     tol = 1e-3 if dtype == np.float32 else 2e-3
     got = hip.linear_qkv(x, *ws, kind, M, bq=biases[0], bv=biases[2])
-    assert hip.last_route() == "mmq_q6_k_q8_k_fp16_tile_128x64"
+    assert hip.last_route() == "mmq_q6_k_q8_k_int8_planes_128x64_k2"
     for g, r in zip(got, oracle.matmul_qkv(kind, *ws, x, M, bq=biases[0], bv=biases[2])):
         assert g.dtype == dtype
         assert_matmul_parity(g, r, tol=tol, what="three weights")
@@ -189,7 +192,7 @@ def test_three_weights_and_float16_outputs(hip, oracle, dtype):
         dot = None
         for b in (None, bias):
             one = hip.linear(x, w, kind, 6000, bias=b, out_dtype=np.float16, force_pack=True)
-            assert hip.last_route() == "mmq_q6_k_q8_k_fp16_tile_128x64"
+            assert hip.last_route() == "mmq_q6_k_q8_k_int8_planes_128x64_k2"
             ref = oracle.matmul(kind, w, x, 6000, bias=b, out_dtype=np.float16, force_pack=True, threads=16)
             # a product on a tie rounds the other way, and so may the sum with the bias: one unit (2^-10) of each
             dot = one.astype(np.float64) if b is None else dot

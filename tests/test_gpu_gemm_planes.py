@@ -1,6 +1,6 @@
 """Tiled GEMM of K-quant weights and Q8_K activations on int8 planes (mh_gemm_planes.hip) against the CPU oracle, at the edges
-of its forms and of the rule that chooses one (planes_form, 256 compute units): four K groups per workgroup, two or one, 64 or 128
-tokens per tile, last tiles with one to four token tiles, one block per row (the second K group has none) and odd counts."""
+of its forms and of the rule that chooses one (planes_form, 256 compute units): 64 x 64 tiles with four K groups per workgroup, 128
+rows with two or one, 64 or 128 tokens per tile, last tiles with one to four token tiles, one block per row (the second K group has none) and odd counts."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,6 @@ from tests.util import assert_matmul_parity, gaussian, random_valid_blocks
 pytestmark = pytest.mark.gpu
 
 KINDS = {"q4_k": KIND_Q4_K, "q5_k": KIND_Q5_K, "q6_k": KIND_Q6_K}
-SMALL = {"q4_k": "int8_planes_128x64", "q5_k": "fp16_tile_128x64", "q6_k": "fp16_tile_128x64"}
 
 
 @pytest.fixture(scope="module")
@@ -24,53 +23,52 @@ def hip():
 
 
 CASES = [
-    # (kinds, tile, tokens, rows, K); "other": the kernels of mh_gemm_i8.hip
-    ("q4_k q5_k", "other", 128, 10400, 256),   # few blocks
-    ("q4_k q5_k", "other", 97, 12801, 768),
-    ("q6_k", "small", 128, 10400, 256),        # two K groups, 64 tokens, the second group without a block
-    ("q6_k", "small", 97, 12801, 768),         # odd block counts, one row and 33 tokens in the last tiles
-    ("q4_k", "small", 128, 9900, 3584),
-    ("q4_k", "small", 97, 9985, 3840),
-    ("q4_k", "other", 128, 9900, 3328),        # (13 blocks)
-    ("q5_k", "small", 128, 10400, 1536),
-    ("q5_k", "small", 97, 12801, 1792),
-    ("q5_k", "other", 97, 12801, 1280),        # (5 blocks)
-    ("q6_k", "small", 33, 11000, 1280),
-    ("q4_k q5_k q6_k", "small", 65, 2085, 256),   # four K groups, 64 rows: three without a block, one token and 37 rows in the last tiles
-    ("q4_k q5_k q6_k", "small", 130, 1401, 1280),  # (five blocks, one row in the last tile)
-    ("q4_k q5_k q6_k", "small", 257, 3232, 768),   # (255 tiles of 256)
-    ("q4_k q5_k q6_k", "small", 129, 3700, 4352),  # (more than 16 blocks)
-    ("q6_k", "small", 17, 8200, 512),              # (17 tokens of two token tiles)
-    ("q6_k", "other", 64, 5440, 6144),             # 85 tiles of 24 blocks
-    ("q6_k", "small", 64, 5441, 6144),             # 86 of them
-    ("q6_k", "other", 17, 4224, 4352),             # 66 tiles of 17 blocks, 17 tokens in each
-    ("q6_k", "small", 32, 4224, 4352),             # 32 tokens
-    ("q4_k", "other", 33, 6144, 4096),             # 16 blocks: 96 tiles of 33 tokens
-    ("q4_k", "small", 33, 8192, 4096),             # 128 of them
-    ("q5_k", "other", 64, 4800, 4096),             # 75 tiles of 64 tokens
-    ("q5_k", "small", 64, 4864, 4096),             # 76 of them
-    ("q4_k q5_k q6_k", "large", 257, 6785, 768),   # two K groups, 128 tokens, one token in the last tile
-    ("q4_k q5_k q6_k", "large", 380, 8200, 256),
-    ("q4_k q5_k", "small", 130, 16600, 512),   # one K group, 64 tokens
-    ("q4_k q5_k", "small", 161, 18500, 256),   # (two token tiles in the last one)
-    ("q6_k", "large", 257, 11000, 512),        # one K group, 128 tokens: one, two, three and four token tiles in the last one
-    ("q6_k", "large", 300, 11000, 256),
-    ("q6_k", "large", 340, 11000, 768),
-    ("q6_k", "large", 384, 11001, 512),
+    # (kinds, form, tokens, rows, K); mfma_tile: the kernels of mh_gemm_i8.hip
+    ("q4_k q5_k", "mfma_tile", 128, 10400, 256),               # few blocks
+    ("q4_k q5_k", "mfma_tile", 97, 12801, 768),
+    ("q6_k", "128x64_k2", 128, 10400, 256),                    # two K groups, 64 tokens, the second group without a block
+    ("q6_k", "128x64_k2", 97, 12801, 768),                     # odd block counts, one row and 33 tokens in the last tiles
+    ("q4_k", "128x64_k2", 128, 9900, 3584),
+    ("q4_k", "128x64_k2", 97, 9985, 3840),
+    ("q4_k", "mfma_tile", 128, 9900, 3328),                    # (13 blocks)
+    ("q5_k", "128x64_k2", 128, 10400, 1536),
+    ("q5_k", "128x64_k2", 97, 12801, 1792),
+    ("q5_k", "mfma_tile", 97, 12801, 1280),                    # (5 blocks)
+    ("q6_k", "64x64_k4", 33, 11000, 1280),
+    ("q4_k q5_k q6_k", "64x64_k4", 65, 2085, 256),             # four K groups, 64 rows: three without a block, one token and 37 rows in the last tiles
+    ("q4_k q5_k q6_k", "64x64_k4", 130, 1401, 1280),           # (five blocks, one row in the last tile)
+    ("q4_k q5_k q6_k", "64x64_k4", 257, 3232, 768),            # (255 tiles of 256)
+    ("q4_k q5_k q6_k", "64x64_k4", 129, 3700, 4352),           # (more than 16 blocks)
+    ("q6_k", "64x64_k4", 17, 8200, 512),                       # (17 tokens of two token tiles)
+    ("q6_k", "mfma_tile", 64, 5440, 6144),                     # 85 tiles of 24 blocks
+    ("q6_k", "64x64_k4", 64, 5441, 6144),                      # 86 of them
+    ("q6_k", "mfma_tile", 17, 4224, 4352),                     # 66 tiles of 17 blocks, 17 tokens in each
+    ("q6_k", "64x64_k4", 32, 4224, 4352),                      # 32 tokens
+    ("q4_k", "mfma_tile", 33, 6144, 4096),                     # 16 blocks: 96 tiles of 33 tokens
+    ("q4_k", "64x64_k4", 33, 8192, 4096),                      # 128 of them
+    ("q5_k", "mfma_tile", 64, 4800, 4096),                     # 75 tiles of 64 tokens
+    ("q5_k", "64x64_k4", 64, 4864, 4096),                      # 76 of them
+    ("q4_k q5_k q6_k", "128x128_k2", 257, 6785, 768),          # two K groups, 128 tokens, one token in the last tile
+    ("q4_k q5_k q6_k", "128x128_k2", 380, 8200, 256),
+    ("q4_k q5_k", "128x64", 130, 16600, 512),                  # one K group, 64 tokens
+    ("q4_k q5_k", "128x64", 161, 18500, 256),                  # (two token tiles in the last one)
+    ("q6_k", "128x128", 257, 11000, 512),                      # one K group, 128 tokens: one, two, three and four token tiles in the last one
+    ("q6_k", "128x128", 300, 11000, 256),
+    ("q6_k", "128x128", 340, 11000, 768),
+    ("q6_k", "128x128", 384, 11001, 512),
 ]
 
 
-@pytest.mark.parametrize("name,tile,N,M,K", [(n, t, *rest) for names, t, *rest in CASES for n in names.split()])
-def test_forms_match_oracle(hip, oracle, name, tile, N, M, K):
+@pytest.mark.parametrize("name,form,N,M,K", [(n, t, *rest) for names, t, *rest in CASES for n in names.split()])
+def test_forms_match_oracle(hip, oracle, name, form, N, M, K):
     """The bound is the suite's for matmul outputs (1e-3, floored): exact integer block sums on both sides, so only the fp32
-    sum over at most five blocks is ordered differently. Arbitrary block bytes: every nibble, scale (Q6_K: -128 among them,
+    sum over at most 24 blocks is ordered differently. Arbitrary block bytes: every nibble, scale (Q6_K: -128 among them,
     products -4064 .. 4096 in two bytes) and minimum."""
     kind = KINDS[name]
     blocks = random_valid_blocks(np.random.default_rng(800 + N), kind, M, K)
     x, bias = gaussian(801 + N, (N, K)), gaussian(802, (M,))
     got = hip.linear(x, blocks, kind, M, bias=bias)
-    route = {"small": SMALL[name], "large": "int8_planes_128x128", "other": "mfma_tile"}[tile]
-    assert hip.last_route() == f"mmq_{name}_q8_k_{route}"
+    assert hip.last_route() == f"mmq_{name}_q8_k_{'' if form == 'mfma_tile' else 'int8_planes_'}{form}"
     assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, bias=bias, threads=16), what=f"{name} {N} x {K} x {M}")
 
 
