@@ -483,8 +483,8 @@ bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_
 int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                        size_t M, int out_dtype);
 // grouped (MoE): work items of up to 64 routes
-bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
-                                   const void *w1);
+bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, size_t max_items,
+                                   const void *w0, const void *w1);
 int launch_gemm_planes_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
                                const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
                                size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1, bool swiglu);

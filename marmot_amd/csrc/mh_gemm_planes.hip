@@ -1067,21 +1067,17 @@ int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, co
 }
 
 // ------------------------------------------------------------------ grouped (MoE)
-bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, const void *w0,
-                                   const void *w1) {
-    // (Q6_K rows are loaded from the 16-byte boundary below: the first one must not begin behind it)
+bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, size_t max_items,
+                                   const void *w0, const void *w1) {
+    // (Q6_K rows are loaded from the 16-byte boundary below: the first one must not begin behind it. Tiles are counted in 32 bits.)
     return !dev->knobs.no_gemm_i8 && planes_kind(kind) && K % QK_K == 0 && rows * K < ((size_t)1 << 32) &&
-           32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
+           2 * ((M + 63) / 64) * max_items < ((size_t)1 << 31) && 32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
            ((((uintptr_t)w0) | ((uintptr_t)w1)) & 15) == 0;
 }
 
 int launch_gemm_planes_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,
                                const ActScratch &act, const uint32_t *d_act_index, const int4 *d_items, const int *d_n_items,
                                size_t max_items, size_t K, size_t M, void *d_out0, void *d_out1, bool swiglu) {
-    if (max_items > 65535) {
-        return set_error(MARMOT_HIP_ERROR_NOT_IMPLEMENTED, "grouped tiled GEMM: %zu work items exceed the grid limit",
-                         max_items);
-    }
     GemmPlanesParams p = {};
     p.w[0] = (const uint8_t *)d_w0;
     p.w[1] = (const uint8_t *)d_w1;

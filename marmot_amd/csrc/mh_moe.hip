@@ -583,8 +583,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const size_t tiled_items = routes / 64 + E / 2, two_per_cu = 2 * (size_t)dev->props.multiProcessorCount;
     const bool tiled = routes >= MOE_TILED_ROUTES * E && tiled_items * 2 * ((F + 127) / 128) >= two_per_cu &&
                        tiled_items * ((H + 127) / 128) >= two_per_cu &&
-                       gemm_planes_grouped_supported(dev, kind_gate_up, T, H, F, d_gate, d_up) &&
-                       gemm_planes_grouped_supported(dev, kind_down, routes, F, H, d_down, d_down);
+                       gemm_planes_grouped_supported(dev, kind_gate_up, T, H, F, E + routes / 64, d_gate, d_up) &&
+                       gemm_planes_grouped_supported(dev, kind_down, routes, F, H, E + routes / 64, d_down, d_down);
     if (tiled) {
         item_cols = 64;
     }

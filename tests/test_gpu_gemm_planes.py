@@ -175,3 +175,19 @@ def test_gated_product_in_the_gemm(hip, name, H, F, T):
     assert hip.last_route() == "moe_experts_tiled"
     stages = hip.moe_experts_probe(hidden, gate, up, down, ids, w, F, E, kind, kind)
     assert np.array_equal(got.view(np.uint32), stages["out"].view(np.uint32))
+
+
+def test_experts_in_more_items_than_a_grid_dimension_holds(hip):
+    """66048 work items (tiles are counted in one dimension): 4096 tokens 129 times over, each with the bits of the call of 4096."""
+    E, F, H, k, T, times = 8, 256, 256, 8, 4096, 129
+    gate, up = (random_valid_blocks(np.random.default_rng(850 + i), KIND_Q4_K, E * F, H) for i in range(2))
+    down = random_valid_blocks(np.random.default_rng(852), KIND_Q4_K, E * H, F)
+    hidden = gaussian(853, (T, H))
+    ids, w = np.tile(np.arange(E, dtype=np.int32), (T, 1)), np.abs(gaussian(854, (T, k)))
+    want = hip.moe_experts(hidden, gate, up, down, ids, w, F, E, KIND_Q4_K, KIND_Q4_K)
+    assert hip.last_route() == "moe_experts_tiled"
+    got = hip.moe_experts(*(np.tile(a, (times, 1)) if a is hidden else a for a in (hidden, gate, up, down)),
+                          np.tile(ids, (times, 1)), np.tile(w, (times, 1)), F, E, KIND_Q4_K, KIND_Q4_K)
+    assert hip.last_route() == "moe_experts_tiled"
+    for part in got.reshape(times, T, H):
+        assert np.array_equal(part.view(np.uint32), want.view(np.uint32))
