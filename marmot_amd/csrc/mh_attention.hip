@@ -336,7 +336,8 @@ __global__ __launch_bounds__(PA_WRITE_THREADS + 64) void k_pa_write_rows(const P
         const bool is_value = i >= pieces;
         const uint32_t u = is_value ? i - pieces : i, h = u / per_head, d = 8u * (u - h * per_head);
         const void *src = is_value ? p.v_new : p.k_new;
-        const size_t from = (size_t)t * (is_value ? p.v_stride[0] : p.k_stride[0]) + (size_t)h * (is_value ? p.v_stride[1] : p.k_stride[1]) + d;
+        const size_t token_stride = is_value ? p.v_stride[0] : p.k_stride[0], head_stride = is_value ? p.v_stride[1] : p.k_stride[1];
+        const size_t from = (size_t)t * token_stride + (size_t)h * head_stride + d;
         uint16_t *dst = (uint16_t *)(is_value ? p.kv_v : p.kv_k) + dst0 + (size_t)h * p.kv_stride[2] + d;
         if (bits16) {
             *(uint4 *)dst = *(const uint4 *)((const uint16_t *)src + from);
@@ -346,8 +347,9 @@ __global__ __launch_bounds__(PA_WRITE_THREADS + 64) void k_pa_write_rows(const P
             uint32_t w[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const bool f16 = p.kv_dtype == MARMOT_HIP_DTYPE_F16;
-                w[e] = f16 ? (uint32_t)f2h(v[2 * e]) | (uint32_t)f2h(v[2 * e + 1]) << 16 : (uint32_t)pa_f2bf(v[2 * e]) | (uint32_t)pa_f2bf(v[2 * e + 1]) << 16;
+                const float a = v[2 * e], b = v[2 * e + 1];
+                w[e] = p.kv_dtype == MARMOT_HIP_DTYPE_F16 ? (uint32_t)f2h(a) | (uint32_t)f2h(b) << 16
+                                                          : (uint32_t)pa_f2bf(a) | (uint32_t)pa_f2bf(b) << 16;
             }
             *(uint4 *)dst = make_uint4(w[0], w[1], w[2], w[3]);
         }
@@ -1368,14 +1370,18 @@ __global__ __launch_bounds__(256) void k_pa_attend_mfma(const PaParams p) {
 //     are scaled first, see pa_split_exponent, weights by 2^14, so that the parts of small ones are normal numbers) or three
 //     BFLOAT16 parts (24 bits, exact), one instruction per part, fp32 accumulation.
 //   * A value that is not finite would reach rows that may not see it (0 x infinity): a tile that holds one takes the
-//     products of its visible positions one by one.
+//     products of its visible positions one by one, with the weights in fp32.
+//   * Scores of -inf weigh nothing as long as the row has others, in whichever half, tile or share of its history; a row that
+//     has no others is NaN. (The reference looks for the maximum a block of 64 - 256 positions at a time and gives NaN for a row whose
+//     first block holds nothing else.)
 // The kernel per token reads a history once per token and head group and uses a quarter of its matrix instructions; this
 // one reads it once per 128 / group tokens. Two sequences x 512 tokens over 2048 cached ones, 32 / 8 heads of 128, BFLOAT16 cache,
 // whole call: 756 us per token; 249 with four wavefronts that own 32 positions at a time and the table entry read in front of
 // each tile; 166 with 64 at a time (one wavefront per SIMD: scores, softmax and output one after the other); 148 with
-// eight wavefronts; 136 - 145 (by card) now that one wavefront locates a tile's rows for all and the values' infinities are looked for by two
-// maxima per word. Bound by the issue of vector instructions (about 1300 per SIMD and tile, 5200 clocks, beside 3070 of
-// the matrix cores); 20 us are the start and the end (the query's parts 6, the join of the halves 4, the first tile 8).
+// eight wavefronts; 136 - 145 (by card) now that one wavefront locates a tile's rows for all and the values' infinities are
+// looked for by two maxima per word. Bound by the issue port: per SIMD and tile of 6700 clocks 1330 instructions take it for
+// 5300 (counted: 790 vector, 96 matrix, 190 scalar, 90 LDS), the matrix cores are busy for 3070; 20 us are the start and the
+// end (the query's parts 6, the join of the halves 4, the first tile 8).
 // Error against 64 bits there: 3.6e-7 per token, 2.2e-7 here.
 typedef float pa_float16v __attribute__((ext_vector_type(16)));
 typedef _Float16 pa_half8 __attribute__((ext_vector_type(8)));
@@ -1397,8 +1403,10 @@ struct PaPromptLds {
     static constexpr uint32_t V0 = 2 * K;          // two buffers of keys, three of values
     static constexpr uint32_t Q = V0 + 3 * V;      // small parts of the query: [part][16 dimensions][wavefront][lane] x 16 bytes
     static constexpr uint32_t QPARTS = HD == 128 ? (BF16 ? 2 : 1) : 0;
-    static constexpr uint32_t TOKENS = Q + QPARTS * PA_PROMPT_ROWS * HD * 2;  // sequence, length, longest history: 128 words each; nine words
-    static constexpr uint32_t ROWS = TOKENS + (3 * PA_PROMPT_ROWS + 12) * 4;  // two tiles: places of 64 rows; then which of them exist
+    // sequence, length, longest history: 128 words each; nine words
+    static constexpr uint32_t TOKENS = Q + QPARTS * PA_PROMPT_ROWS * HD * 2;
+    // two tiles: places of 64 rows; then which of them exist
+    static constexpr uint32_t ROWS = TOKENS + (3 * PA_PROMPT_ROWS + 12) * 4;
     static constexpr uint32_t BYTES = ROWS + (2 * 64 + 2) * 8;
     static constexpr uint32_t MAIL = PA_PROMPT_WAVES * HD / 64 * 4096;  // at the end: outputs, then maximum and sum of every lane
     static_assert(MAIL + PA_PROMPT_WAVES * 512 <= Q, "the mail fits the stages");
@@ -1601,7 +1609,8 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
     }
     float m = -INFINITY, lsum = 0.0f;  // of this wavefront's positions; lsum: of this lane's part of them
     const size_t head_base = (size_t)p.layer_idx * p.kv_stride[1] + (size_t)kvh * p.kv_stride[2];
-    const uint8_t *keys = (const uint8_t *)((const uint16_t *)p.kv_k + head_base), *values = (const uint8_t *)((const uint16_t *)p.kv_v + head_base);
+    const uint8_t *keys = (const uint8_t *)((const uint16_t *)p.kv_k + head_base);
+    const uint8_t *values = (const uint8_t *)((const uint16_t *)p.kv_v + head_base);
     // a thread's part of a tile: 16 bytes of every THREADS / (HD / 8)-th key row, four dimensions of four consecutive value rows.
     // (The chunk of dimension 4 i + e: that of dimension 4 i with 2 e in an exclusive or, 128 e bytes on.)
     const uint32_t v_at = pa_vt_chunk(4u * (tid % (HD / 4)), 2u * (tid / HD) + (tid / (HD / 4) & 1u)) + 8u * (tid / (HD / 2) & 1u);
@@ -1701,11 +1710,15 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
                 i16x2 above = {0, 0};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    below = __builtin_elementwise_max(below, __builtin_elementwise_max(__builtin_bit_cast(u16x2, vreg[e].x), __builtin_bit_cast(u16x2, vreg[e].y)));
-                    above = __builtin_elementwise_max(above, __builtin_elementwise_max(__builtin_bit_cast(i16x2, vreg[e].x), __builtin_bit_cast(i16x2, vreg[e].y)));
+                    const u16x2 ux = __builtin_bit_cast(u16x2, vreg[e].x), uy = __builtin_bit_cast(u16x2, vreg[e].y);
+                    const i16x2 ix = __builtin_bit_cast(i16x2, vreg[e].x), iy = __builtin_bit_cast(i16x2, vreg[e].y);
+                    below = __builtin_elementwise_max(below, __builtin_elementwise_max(ux, uy));
+                    above = __builtin_elementwise_max(above, __builtin_elementwise_max(ix, iy));
                 }
                 constexpr uint32_t ONE = BF16 ? 0x00800080u : 0x04000400u;
-                const uint32_t odd = ((__builtin_bit_cast(uint32_t, below) & 0x7fff7fffu) + ONE) | ((__builtin_bit_cast(uint32_t, above) & 0x7fff7fffu) + ONE);
+                const uint32_t low = __builtin_bit_cast(uint32_t, below) & 0x7fff7fffu;
+                const uint32_t high = __builtin_bit_cast(uint32_t, above) & 0x7fff7fffu;
+                const uint32_t odd = (low + ONE) | (high + ONE);
                 uint8_t *vt = lds + values_at;
                 constexpr uint32_t LOW = 0x05040100u, HIGH = 0x07060302u;
                 auto pair = [](uint32_t b, uint32_t a, uint32_t sel) { return __builtin_amdgcn_perm(b, a, sel); };
@@ -1738,7 +1751,8 @@ __global__ __launch_bounds__(64 * PA_PROMPT_WAVES, 2) void k_pa_prompt(const PaP
             for (int part = PARTS - 1; part >= 0; --part) {  // small parts first
 #pragma unroll
                 for (int c = 0; c < QC; ++c) {
-                    const uint4 q = part < QREGS ? qpart[part < QREGS ? part : 0][c] : *(const uint4 *)(q_small + 4096 * (QC * (part - QREGS) + c));
+                    const uint4 q = part < QREGS ? qpart[part < QREGS ? part : 0][c]
+                                                 : *(const uint4 *)(q_small + 4096 * (QC * (part - QREGS) + c));
                     s = pa_mma32<BF16>(k[c], q, s);
                 }
             }
@@ -2064,7 +2078,7 @@ static int pa_launch_prompt(marmot_hip_device *dev, const PaParams &p) {
     MH_TRY(allow_large_lds(dev, (const void *)k_pa_prompt<HD, BF16>));
     const unsigned tiles = (p.token_count + p.tile_tokens - 1) / p.tile_tokens;
     hipLaunchKernelGGL((k_pa_prompt<HD, BF16>), dim3(tiles, p.num_kv_heads, p.tile_splits), dim3(64 * PA_PROMPT_WAVES),
-                       (PaPromptLds<HD, BF16>::BYTES),                       dev->stream, p);
+                       (PaPromptLds<HD, BF16>::BYTES), dev->stream, p);
     MH_HIP(hipGetLastError());
     return MARMOT_HIP_SUCCESS;
 }
@@ -2229,13 +2243,15 @@ extern "C" int marmot_hip_paged_attention(marmot_hip_device_t *dev, const marmot
     }
     // Prompts: k_pa_prompt beside the kernel per token. Which tokens it takes is found on the device (pa_in_run): those of
     // calls with PA_PROMPT_WORK (token, head group, position) triples and more, counted with the longest history; a call of
-    // fewer than PA_MANY tokens needs 2 PA_LONG positions too. 32 / 8 heads of 128, whole call, us per token / tiles: fresh
-    // prompts of 100 tokens 15 / 24, 300 41 / 42, 440 63 / 50, 512 77 / 51, 1024 210 / 78; 64 tokens over 4000 112 / 45;
-    // 4 x 8 tokens over 100 15 / 44; 32 / 8 heads of 64, 4 x 100 tokens over 500 151 / 50. It is launched where that can be:
-    // two tokens and more per row of the block table, or PA_ANY_TABLE tokens (a decode step has one token per row at most
-    // and would pay for an empty launch), and room for such a history in the table. A table with more room than the call
-    // needs costs the empty launch: 100 fresh tokens 15.2 / 18.9, 256 in 32 short runs 34.3 / 39.6, 512 decode tokens over
-    // 100 57.5 / 61.0. 16-byte key rows, 8-byte value rows.
+    // fewer than PA_MANY tokens needs 2 PA_LONG positions too. Whole call, us per token / tiles, 32 / 8 heads of 128, FLOAT16:
+    // fresh prompts of 100 tokens 15.5 / 29, 300 41.5 / 41.5, 400 56 / 45, 440 65 / 47, 512 78 / 49, 1024 210 / 65; 16 tokens
+    // of four sequences over 1000 42 / 48, of BFLOAT16 64 tokens over 4000 115 / 45, 4 x 8 over 100 18 / 47; 32 / 8 heads of 64,
+    // 100 tokens 23 / 24, 200 31 / 28, 300 50 / 31, 4 x 100 over 500 138 / 45. (The line, 430 fresh tokens here, is that of slower
+    // tiles: from 300 tokens on, 200 with rows of 64, these would not lose.) It is launched where that can be: two tokens and
+    // more per row of the block table, or PA_ANY_TABLE tokens (a decode step has one token per row at most and would pay for
+    // an empty launch), and room for such a history in the table. A table with more room than the call needs costs the
+    // empty launch: 100 fresh tokens 16.2 / 21.3, 256 in 32 short runs 22.0 / 28.5, 512 decode tokens over 100 54.2 / 56.7.
+    // 16-byte key rows, 8-byte value rows.
     const bool any = dev->knobs.attention_prompt_any, many = a->token_count >= PA_MANY;
     const size_t enough = (PA_PROMPT_WORK + pairs - 1) / pairs, least = many || enough > 2 * PA_LONG ? enough : 2 * PA_LONG;
     const bool runs = a->token_count / 2 >= a->max_seqs;

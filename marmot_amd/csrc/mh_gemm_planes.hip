@@ -11,10 +11,14 @@
 // from LDS, no conversion, direct-to-LDS loads; the price is a shift-add and a conversion per output and block. The sums of
 // 16 codes (at most 2032) and the mins are exact in fp16: one fp16 instruction per block and tile gives msum.
 //
-// What bounds it: vector instructions. Per wavefront and block, 32 rows x 128 tokens, a kernel issues 64 (68) matrix instructions
-// beside 700 (Q6_K), 736 (Q5_K) or 534 (Q4_K) vector ones: 256 or 320 of the fp32 step (one output: shift-add, conversion, two or
-// three multiply-adds), 50 / 16 per 32 values of unpacking (Q6_K, Q5_K / Q4_K), the rest addresses. Hence the tile: what a lane
-// unpacks meets up to four token tiles, and everything else waits in LDS so that two wavefronts fit a SIMD.
+// What bounds it: the issue port, most of all vector instructions. Per wavefront and block, 32 rows x 128 tokens, a kernel issues
+// 64 (68) matrix instructions beside 700 (Q6_K), 736 (Q5_K) or 534 (Q4_K) vector ones: 256 or 320 of the fp32 step (one output:
+// shift-add, conversion, two or three multiply-adds), 50 / 16 per 32 values of unpacking (Q6_K, Q5_K / Q4_K), the rest addresses.
+// Counted for 1024 x 14336 x 4096 (two K groups): 720, 755 and 553 vector instructions with the start and the end shared out; all
+// instructions hold the port for 74, 86 and 78 % of a SIMD's clocks, vector ones for 60, 69 and 61, while the matrix cores are busy
+// for 39, 46 and 53 %. Q6_K waits more: its raw blocks are read from LDS at two-byte offsets (LDS busy for 51 %, Q5_K 26).
+// Hence the tile: what a lane unpacks meets up to four token tiles, and everything else waits in LDS so that two wavefronts
+// fit a SIMD.
 //
 // A wavefront owns 32 weight rows x 32 CT tokens: lane (row j, half kh) unpacks the bytes only it reads, a run of 32 values
 // (a step: 2 CT matrix instructions) ahead of its use, a quarter between every two matrix instructions. A stage is half a block
@@ -411,7 +415,8 @@ __global__ __launch_bounds__(64 * RG * KG, C == 2 && KG == 1 ? 3 : 2) void k_gem
             for (int c = 0; c < 4; ++c) {
                 e[c] = __builtin_bit_cast(uint32_t, pl_half2{(_Float16)(int16_t)(v[c] & 0xffffu), (_Float16)(int16_t)(v[c] >> 16)});
             }
-            *(uint4 *)(lds + L::S0 + (2 * kg + (number & 1u)) * L::SD + s_tok * 32u + 16u * (lane & 1)) = make_uint4(e[0], e[1], e[2], e[3]);
+            uint8_t *sums = lds + L::S0 + (2 * kg + (number & 1u)) * L::SD;
+            *(uint4 *)(sums + s_tok * 32u + 16u * (lane & 1)) = make_uint4(e[0], e[1], e[2], e[3]);
         }
     };
 
@@ -623,8 +628,8 @@ __global__ __launch_bounds__(64 * RG * KG, C == 2 && KG == 1 ? 3 : 2) void k_gem
 #pragma unroll
                         for (int i = 0; i < C / 2; ++i) {
                             const uint32_t t = 64u * i + (uint32_t)lane;
-                            planes_dma4(lds_base + (uint32_t)(L::NEXT + wave * 128 * C + 256 * i), (const uint8_t *)(p.act_index + next.tok0),
-                                        4u * (t < next.toks ? t : next.toks - 1u));
+                            planes_dma4(lds_base + (uint32_t)(L::NEXT + wave * 128 * C + 256 * i),
+                                        (const uint8_t *)(p.act_index + next.tok0), 4u * (t < next.toks ? t : next.toks - 1u));
                         }
                     }
                 }
@@ -696,8 +701,8 @@ __global__ __launch_bounds__(64 * RG * KG, C == 2 && KG == 1 ? 3 : 2) void k_gem
                         raw.load_low(block, hn, sn / 2, kh);
                     }
                 }
-                // The last bytes of this block have been read: its place is the next one's. (Waited for: the request alone does not keep the
-                // new bytes behind a read that still queues for LDS.)
+                // The last bytes of this block have been read: its place is the next one's. (Waited for: the request alone does
+                // not keep the new bytes behind a read that still queues for LDS.)
                 constexpr int FREE = CT == 1 ? 2 : 3 * CT / 2;
                 if (hb == 1 && st == FREE) {
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -867,7 +872,8 @@ __global__ __launch_bounds__(64 * RG * KG, C == 2 && KG == 1 ? 3 : 2) void k_gem
     const uint32_t which = cur.which;
     uint32_t kh4 = 4u * (uint32_t)kh;
     asm volatile("" : "+v"(kh4));  // (the places of the outputs are not kept from tile to tile)
-    constexpr int OUT = KG == 4 ? 1 : KG == 2 ? C / 2 : CT, REGS = KG == 4 || GLU ? 8 : 16;  // token tiles this wavefront stores, outputs of one
+    // token tiles this wavefront stores, outputs of one
+    constexpr int OUT = KG == 4 ? 1 : KG == 2 ? C / 2 : CT, REGS = KG == 4 || GLU ? 8 : 16;
     const uint32_t n0 = (uint32_t)(KG == 4 ? 16 * kg : KG == 2 ? 32 * kg * OUT : GLU ? 16 * (gw >> 1) : 0);
     const void *bias_p = p.bias[which];
     const bool has_bias = bias_p != nullptr;
@@ -935,7 +941,8 @@ static int planes_launch(marmot_hip_device *dev, GemmPlanesParams &p, size_t col
     const size_t tiles = (size_t)p.row_tiles * cols * weights;
     const size_t places = (size_t)dev->props.multiProcessorCount * 3;
     const dim3 grid((unsigned)(LOOP && tiles > places ? places : tiles));
-    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG, LOOP, RG, GLU>), grid, dim3(64 * RG * KG), (PlanesLds<KIND, C, KG, LOOP, RG>::BYTES), dev->stream, p);
+    hipLaunchKernelGGL((k_gemm_planes<KIND, C, KG, LOOP, RG, GLU>), grid, dim3(64 * RG * KG),
+                       (PlanesLds<KIND, C, KG, LOOP, RG>::BYTES), dev->stream, p);
     MH_HIP(hipGetLastError());
     return MARMOT_HIP_SUCCESS;
 }
@@ -1071,8 +1078,8 @@ bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_
                                    const void *w0, const void *w1) {
     // (Q6_K rows are loaded from the 16-byte boundary below: the first one must not begin behind it. Tiles are counted in 32 bits.)
     return !dev->knobs.no_gemm_i8 && planes_kind(kind) && K % QK_K == 0 && rows * K < ((size_t)1 << 32) &&
-           2 * ((M + 63) / 64) * max_items < ((size_t)1 << 31) && 32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
-           ((((uintptr_t)w0) | ((uintptr_t)w1)) & 15) == 0;
+           32 * (K / QK_K) * block_bytes(kind) < ((size_t)1 << 31) && M < ((size_t)1 << 31) &&
+           2 * ((M + 63) / 64) * max_items < ((size_t)1 << 31) && ((((uintptr_t)w0) | ((uintptr_t)w1)) & 15) == 0;
 }
 
 int launch_gemm_planes_grouped(marmot_hip_device *dev, int kind, const void *d_w0, const void *d_w1, size_t expert_stride,

@@ -11,8 +11,13 @@ namespace mh {
 
 constexpr int MOE_ITEM_COLS = 8;   // routes per grouped work item (16 or 32 when experts see many routes, see moe_item_cols)
 // Routes per expert from which prompts take the tiled GEMM (mh_gemm_planes.hip, 64 routes per item) instead of passes of
-// 16 or 32 routes, given two of its tiles per compute unit in both projections (us before / tiled, E = 128, top 8, H = 2048,
-// F = 768: Q4_K 512 tokens = 32 routes per expert 248 / 182, 1024 401 / 260, 2048 729 / 429; Q6_K 512 472 / 285)
+// 16 or 32 routes, given two of its tiles per compute unit in both projections. us of whole calls, passes / tiled, E = 128, top 8,
+// H = 2048, F = 768, at 12, 16, 24, 32, 56 and 128 routes per expert:
+//   Q4_K 137 / 131, 161 / 133, 171 / 143, 210 / 155, 303 / 196, 600 / 361
+//   Q5_K 149 / 152, 174 / 155, 204 / 165, 262 / 174, 364 / 212, 730 / 403
+//   Q6_K 225 / 170, 276 / 173, 376 / 183, 439 / 194, 718 / 240, 1417 / 447
+// (64 experts, top 4, F = 1024: Q4_K 88 / 92, 100 / 89, 107 / 95; Q5_K 99 / 106, 117 / 108, 137 / 114.) The line is that of the kernel
+// this one replaced (248 / 182 at 32 routes); with this one passes lose from 16 routes on, and from 12 on for Q6_K.
 constexpr size_t MOE_TILED_ROUTES = 32;
 constexpr int MOE_MAX_EXPERTS = 1024;
 constexpr int MOE_MAX_TOPK = 64;
@@ -612,6 +617,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     const size_t table_bytes = route_groups > 1 ? route_groups * (E + 1) * sizeof(int) : 0;
     const size_t gate_bytes = routes * F * sizeof(float);
     const size_t o_gate = take(gate_bytes > table_bytes ? gate_bytes : table_bytes);  // the counts lie where gate comes later
+    // (laid out also where the GEMM forms the gated product and leaves it alone: a workspace that held a prompt holds every shorter one,
+    // also in a capture, which may not let it grow)
     const size_t o_up = take(routes * F * sizeof(float));
     const size_t o_down = take(routes * H * sizeof(float));
     void *ws = nullptr;
@@ -677,7 +684,8 @@ static int moe_experts_impl(marmot_hip_device_t *dev, const float *d_hidden, siz
     }
     const size_t gu_stride = F * ((H + bv_gu - 1) / bv_gu) * block_bytes(kind_gate_up);
     const size_t dn_stride = H * ((F + bv_dn - 1) / bv_dn) * block_bytes(kind_down);
-    // K-quant experts run on the matrix cores (long prompts on the tiled GEMM on int8 planes, else passes), the 32-value formats on the dot-product matvec
+    // K-quant experts run on the matrix cores (long prompts on the tiled GEMM on int8 planes, else passes), the 32-value formats on
+    // the dot-product matvec
     // Tiled, SwiGLU: the GEMM forms the gated product itself, which is written and read once in the place of two arrays (a call
     // that looks at the stages gets both)
     const bool gated = tiled && ffn_type != MARMOT_HIP_FFN_GEGLU && probe == nullptr;
