@@ -976,17 +976,22 @@ static bool planes_kind(int kind) {
 //     Q5_K   0.93 - 0.59; 41 1.17 - 1.37, 21 1.03 - 1.41 but for 140 and 200 tokens of 4 blocks (0.91, 0.95)
 //   more tiles: Q6_K 41, 0.91 - 0.52 (21 against it 0.86 at 258 - 344 tiles of 128 x 128 and few blocks, 0.95 - 1.25 else); Q4_K, Q5_K 21,
 //            0.99 - 0.68 (41 against it 0.97 - 1.21 and, Q5_K, 0.87 - 1.16)
+// Several weights in one call: the other kernels take them one after the other, each split by itself, so the lines above that
+// keep few blocks and badly filled tiles away are not theirs (three weights, other kernels / here: Q4_K 128 x 1024 x 4096 37.9 / 13.8
+// us, 33 x 4096 x 2048 36.5 / 17.3, Q5_K 200 x 4096 x 512 40.9 / 21.3).
 // Q4_K and Q5_K: where mh_gemm_int16.hip has a form of 256 x 128 for the call, that one is as fast or faster (1024 x 4096 x 14336
 // Q4_K 156 us against 155, Q5_K 162 against 169; 1024 x 1024 x 8192 31 against 35).
 static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t nb, size_t weights) {
     const size_t cus = (size_t)dev->props.multiProcessorCount;
     const size_t rows = (M + 127) / 128 * weights, rows64 = (M + 63) / 64 * weights;
     const size_t small = (N + 63) / 64 * rows, large = (N + 127) / 128 * rows, least = (N + 63) / 64 * rows64;
-    const bool q6 = kind == MARMOT_HIP_KIND_Q6_K, q5 = kind == MARMOT_HIP_KIND_Q5_K;
+    const bool q6 = kind == MARMOT_HIP_KIND_Q6_K, q5 = kind == MARMOT_HIP_KIND_Q5_K, set = weights > 1;
     if (least <= cus) {
         const size_t used = N * rows64;  // 64 per tile if tokens fill them
         bool takes;
-        if (q6) {
+        if (set) {
+            takes = q6 || nb <= 16 || 3 * least > 2 * cus;
+        } else if (q6) {
             takes = nb <= 16 || 3 * least > cus || (nb < 24 && used >= 8 * cus);
         } else if (nb > 16) {
             takes = 3 * least > 2 * cus;
@@ -996,7 +1001,7 @@ static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t 
         return 4 * least > cus && takes ? 24 : 0;
     }
     if (small <= cus) {
-        return q6 || (nb >= (q5 ? 6u : 14u) && (nb <= 8 || 5 * small > 3 * cus)) ? 22 : 0;
+        return q6 || ((set || nb >= (q5 ? 6u : 14u)) && (nb <= 8 || 5 * small > 3 * cus)) ? 22 : 0;
     }
     return large <= cus ? 42 : q6 ? 41 : 21;
 }

@@ -72,6 +72,25 @@ def test_forms_match_oracle(hip, oracle, name, form, N, M, K):
     assert_matmul_parity(got, oracle.matmul(kind, blocks, x, M, bias=bias, threads=16), what=f"{name} {N} x {K} x {M}")
 
 
+@pytest.mark.parametrize("name,form,N,M,K", [
+    ("q4_k", "128x64_k2", 100, 3700, 1024),
+    ("q4_k", "128x64_k2", 200, 2050, 2048),
+    ("q5_k", "128x64_k2", 130, 3300, 256),
+    ("q4_k", "64x64_k4", 33, 2050, 4096),    # 99 tiles of 33 tokens
+    ("q5_k", "64x64_k4", 200, 500, 4096),
+    ("q6_k", "64x64_k4", 64, 1500, 6144),    # 72 tiles of 24 blocks
+])
+def test_sets_of_weights_have_lines_of_their_own(hip, oracle, name, form, N, M, K):
+    """Three weights in one launch, on forms that one weight with as many tiles leaves to the kernels of mh_gemm_i8.hip."""
+    kind = KINDS[name]
+    ws = [random_valid_blocks(np.random.default_rng(860 + i), kind, M, K) for i in range(3)]
+    x = gaussian(863, (N, K))
+    got = hip.linear_qkv(x, *ws, kind, M)
+    assert hip.last_route() == f"mmq_{name}_q8_k_int8_planes_{form}"
+    for g, r in zip(got, oracle.matmul_qkv(kind, *ws, x, M)):
+        assert_matmul_parity(g, r, what=f"three weights {name} {N} x {K} x {M}")
+
+
 @pytest.mark.parametrize("name,N,M", [("q4_k", 130, 16600), ("q5_k", 130, 16600), ("q6_k", 300, 11000),  # one K group
                                       ("q4_k", 257, 6800), ("q5_k", 257, 6800), ("q6_k", 257, 6800),  # two
                                       ("q4_k", 70, 2100), ("q5_k", 70, 2100), ("q6_k", 70, 2100)])  # four
