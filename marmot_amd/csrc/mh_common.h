@@ -477,11 +477,12 @@ bool gemm_x16_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K
                       const ActScratch &act);
 int launch_gemm_x16(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
                     size_t M, int out_dtype);
-// The same on the int8 matrix cores, scaled weights as two planes (mh_gemm_planes.hip)
+// The same on the int8 matrix cores, scaled weights as two planes (mh_gemm_planes.hip); no_split: the call has no room for the
+// partial sums that launch_gemm_i8 would need
 bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights,
-                         const ActScratch &act);
+                         const ActScratch &act, bool no_split);
 int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
-                       size_t M, int out_dtype);
+                       size_t M, int out_dtype, bool no_split);
 // grouped (MoE): work items of up to 64 routes
 bool gemm_planes_grouped_supported(const marmot_hip_device *dev, int kind, size_t rows, size_t K, size_t M, size_t max_items,
                                    const void *w0, const void *w1);

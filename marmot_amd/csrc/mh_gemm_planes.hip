@@ -978,18 +978,20 @@ static bool planes_kind(int kind) {
 //            0.99 - 0.68 (41 against it 0.97 - 1.21 and, Q5_K, 0.87 - 1.16)
 // Several weights in one call: the other kernels take them one after the other, each split by itself, so the lines above that
 // keep few blocks and badly filled tiles away are not theirs (three weights, other kernels / here: Q4_K 128 x 1024 x 4096 37.9 / 13.8
-// us, 33 x 4096 x 2048 36.5 / 17.3, Q5_K 200 x 4096 x 512 40.9 / 21.3).
+// us, 33 x 4096 x 2048 36.5 / 17.3, Q5_K 200 x 4096 x 512 40.9 / 21.3). Nor are they a call's that has no room for the partial sums of
+// a split (a capture without an eager run before): no_split.
 // Q4_K and Q5_K: where mh_gemm_int16.hip has a form of 256 x 128 for the call, that one is as fast or faster (1024 x 4096 x 14336
 // Q4_K 156 us against 155, Q5_K 162 against 169; 1024 x 1024 x 8192 31 against 35).
-static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t nb, size_t weights) {
+static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t M, size_t nb, size_t weights, bool no_split) {
     const size_t cus = (size_t)dev->props.multiProcessorCount;
     const size_t rows = (M + 127) / 128 * weights, rows64 = (M + 63) / 64 * weights;
     const size_t small = (N + 63) / 64 * rows, large = (N + 127) / 128 * rows, least = (N + 63) / 64 * rows64;
-    const bool q6 = kind == MARMOT_HIP_KIND_Q6_K, q5 = kind == MARMOT_HIP_KIND_Q5_K, set = weights > 1;
+    const bool q6 = kind == MARMOT_HIP_KIND_Q6_K, q5 = kind == MARMOT_HIP_KIND_Q5_K;
+    no_split = no_split || weights > 1;
     if (least <= cus) {
         const size_t used = N * rows64;  // 64 per tile if tokens fill them
         bool takes;
-        if (set) {
+        if (no_split) {
             takes = q6 || nb <= 16 || 3 * least > 2 * cus;
         } else if (q6) {
             takes = nb <= 16 || 3 * least > cus || (nb < 24 && used >= 8 * cus);
@@ -1001,13 +1003,13 @@ static int planes_form(const marmot_hip_device *dev, int kind, size_t N, size_t 
         return 4 * least > cus && takes ? 24 : 0;
     }
     if (small <= cus) {
-        return q6 || ((set || nb >= (q5 ? 6u : 14u)) && (nb <= 8 || 5 * small > 3 * cus)) ? 22 : 0;
+        return q6 || ((no_split || nb >= (q5 ? 6u : 14u)) && (nb <= 8 || 5 * small > 3 * cus)) ? 22 : 0;
     }
     return large <= cus ? 42 : q6 ? 41 : 21;
 }
 
 bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_t K, size_t M, int weights,
-                         const ActScratch &act) {
+                         const ActScratch &act, bool no_split) {
     if (dev->knobs.no_gemm_i8 || !planes_kind(kind) || K % QK_K != 0) {
         return false;
     }
@@ -1015,7 +1017,7 @@ bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_
         32 * (K / QK_K) * block_bytes(kind) >= ((size_t)1 << 31) || N > (size_t)65535 * 64) {
         return false;  // 32-bit lane offsets
     }
-    return planes_form(dev, kind, N, M, K / QK_K, (size_t)weights) != 0;
+    return planes_form(dev, kind, N, M, K / QK_K, (size_t)weights, no_split) != 0;
 }
 
 // Rows x tokens of a tile, and the K groups of a workgroup (_k2, _k4)
@@ -1024,8 +1026,8 @@ bool gemm_planes_applies(const marmot_hip_device *dev, int kind, size_t N, size_
      : KIND == MARMOT_HIP_KIND_Q5_K ? "mmq_q5_k_q8_k_int8_planes_" form : "mmq_q6_k_q8_k_int8_planes_" form)
 
 template <int KIND>
-static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsigned weights) {
-    const int form = planes_form(dev, KIND, p.N, p.M, p.nb, weights);
+static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsigned weights, bool no_split) {
+    const int form = planes_form(dev, KIND, p.N, p.M, p.nb, weights, no_split);
     const unsigned t64 = (unsigned)((p.N + 63) / 64), t128 = (unsigned)((p.N + 127) / 128);
     if (form == 22) {
         set_route(PLANES_ROUTE("128x64_k2"));
@@ -1050,7 +1052,7 @@ static int planes_launch_kind(marmot_hip_device *dev, GemmPlanesParams &p, unsig
 #undef PLANES_ROUTE
 
 int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, const ActScratch &act, size_t N, size_t K,
-                       size_t M, int out_dtype) {
+                       size_t M, int out_dtype, bool no_split) {
     GemmPlanesParams p = {};
     for (int i = 0; i < ws.count; ++i) {
         p.w[i] = (const uint8_t *)ws.w[i];
@@ -1070,11 +1072,11 @@ int launch_gemm_planes(marmot_hip_device *dev, int kind, const WeightSet &ws, co
     const unsigned weights = (unsigned)ws.count;
     switch (kind) {
     case MARMOT_HIP_KIND_Q4_K:
-        return planes_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights);
+        return planes_launch_kind<MARMOT_HIP_KIND_Q4_K>(dev, p, weights, no_split);
     case MARMOT_HIP_KIND_Q5_K:
-        return planes_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights);
+        return planes_launch_kind<MARMOT_HIP_KIND_Q5_K>(dev, p, weights, no_split);
     default:
-        return planes_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights);
+        return planes_launch_kind<MARMOT_HIP_KIND_Q6_K>(dev, p, weights, no_split);
     }
 }
 

@@ -1078,8 +1078,9 @@ int launch_mmq_set(marmot_hip_device *dev, int kind, const WeightSet &ws, const 
         if (gemm_x16_applies(dev, kind, N, K, M, ws.count, act)) {
             return launch_gemm_x16(dev, kind, ws, act, N, K, M, out_dtype);
         }
-        if (gemm_planes_applies(dev, kind, N, K, M, ws.count, act)) {
-            return launch_gemm_planes(dev, kind, ws, act, N, K, M, out_dtype);
+        const bool no_split = scratch == nullptr && gemm_i8_scratch_bytes(dev, kind, N, K, M, ws.count, 0) > workspace_room(dev);
+        if (gemm_planes_applies(dev, kind, N, K, M, ws.count, act, no_split)) {
+            return launch_gemm_planes(dev, kind, ws, act, N, K, M, out_dtype, no_split);
         }
         return launch_gemm_i8(dev, kind, ws, act, N, K, M, out_dtype, scratch);
     }

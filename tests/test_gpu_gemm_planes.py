@@ -4,6 +4,7 @@ rows with two or one, 64 or 128 tokens per tile, last tiles with one to four tok
 import numpy as np
 import pytest
 
+from marmot_amd.capi import DT_F32
 from oracle.pyoracle import KIND_Q4_K, KIND_Q5_K, KIND_Q6_K
 from tests.test_gpu_moe import check_moe_stages
 from tests.util import assert_matmul_parity, gaussian, random_valid_blocks
@@ -210,3 +211,33 @@ def test_experts_in_more_items_than_a_grid_dimension_holds(hip):
     assert hip.last_route() == "moe_experts_tiled"
     for part in got.reshape(times, T, H):
         assert np.array_equal(part.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("name,N,M,K", [("q4_k", 33, 4224, 4096), ("q5_k", 80, 2560, 4096), ("q6_k", 64, 4224, 8192)])
+def test_captured_without_an_eager_run(oracle, name, N, M, K):
+    """Packed activations, on sizes whose K is split over workgroups with partial sums in the workspace: a fresh device object
+    captures the call all the same, on tiles that need none, and splits once it may allocate."""
+    from marmot_amd import HipBackend
+
+    kind, hip = KINDS[name], HipBackend(0)
+    blocks, x = random_valid_blocks(np.random.default_rng(870), kind, M, K), gaussian(871, (N, K))
+    want = oracle.matmul(kind, blocks, x, M, threads=16)
+    bufs = [hip.to_device(blocks), hip.to_device(x), hip.alloc(hip.packed_activation_bytes(kind, N, K)), hip.alloc(4 * N * M)]
+    d_w, d_x, d_p, d_out = bufs
+    try:
+        hip.pack_activations_d(kind, d_x, DT_F32, N, K, d_p)
+        graph = hip.graph_capture(lambda: hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out))
+        assert hip.last_route() == f"mmq_{name}_q8_k_int8_planes_64x64_k4"
+        for _ in range(3):
+            d_out.upload(np.full((N, M), np.nan, np.float32))
+            hip.graph_launch(graph)
+            hip.synchronize()
+            assert_matmul_parity(d_out.download(np.float32, (N, M)), want, what=f"captured {name}")
+            hip.linear_prepacked_d(kind, d_w, d_p, N, K, M, d_out)
+            assert hip.last_route() == f"mmq_{name}_q8_k_mfma_tile"
+            assert_matmul_parity(d_out.download(np.float32, (N, M)), want, what=f"eager {name}")
+        hip.graph_destroy(graph)
+    finally:
+        for b in bufs:
+            b.free()
+        hip.close()
