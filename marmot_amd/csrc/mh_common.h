@@ -216,8 +216,8 @@ struct ActScratch {
 //   MARMOT_HIP_NO_FUSED_QUANT  activation quantization inside the matvec -> separate quantization launch
 //   MARMOT_HIP_NO_GEMM         fp16 prefill GEMM -> fp16 matvec
 //   MARMOT_HIP_NO_GEMM_LOADERS prefill GEMM tile fed by loader wavefronts -> the tile whose wavefronts load for themselves
-//   MARMOT_HIP_NO_GEMM_I8      tiled GEMMs on Q8_K activations (33 rows and more; int8 and integer fp16 operands, experts
-//                              too) -> 32-row passes of the small-batch kernel
+//   MARMOT_HIP_NO_GEMM_I8      tiled GEMMs on Q8_K activations (33 rows and more, Q6_K 17; int8 operands, int8 planes and integer
+//                              fp16 operands, experts too) -> 32-row passes of the small-batch kernel
 //   MARMOT_HIP_MOE_NO_VALIDATE skip the check of the expert ids (the call then does not wait for its route kernel)
 //   MARMOT_HIP_ATTENTION_PROMPT_ANY  prompt tiles for calls of every size (the one switch that turns a route on)
 struct marmot_hip_knobs {
